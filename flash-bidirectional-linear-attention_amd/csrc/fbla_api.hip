@@ -668,4 +668,88 @@ int fbla_elu1_bwd(const void* x, const void* dy, void* dx, int64_t n, int dtype,
   return check_launch(what);
 }
 
+// common checks of the depth-wise convolution entry points; fills `c` (x, y, w, bias and strides are the caller's)
+static int check_dwconv(const char* what, dwconv::Conv& c, int64_t B, int64_t H, int64_t W, int C, int Cw, int K,
+                        int dtype) {
+  if (B < 0 || H < 1 || W < 1 || C < 1 || Cw < 1 || (dtype != kF16 && dtype != kBF16 && dtype != kF32)) {
+    set_error("%s: bad sizes or dtype (B=%lld H=%lld W=%lld C=%d Cw=%d dtype=%d)", what, (long long)B, (long long)H,
+              (long long)W, C, Cw, dtype);
+    return kErrBadArg;
+  }
+  if (!dwconv::supported(C, Cw, K, dtype)) {
+    set_error("%s: needs 3, 5 or 7 taps a side, channels in whole 16-byte pieces and a multiple of the filters "
+              "(K=%d C=%d Cw=%d)", what, K, C, Cw);
+    return kErrUnsupported;
+  }
+  if (H > 0x7fffffffLL / W || B > 0x7fffffffLL / (H * W) || C > 64 * 65535) {
+    set_error("%s: too many tokens or channels", what);
+    return kErrBadArg;
+  }
+  c.B = (int)B;
+  c.H = (int)H;
+  c.W = (int)W;
+  c.C = C;
+  c.Cw = Cw;
+  return kOk;
+}
+static int check_row_strides(const char* what, int C, int dtype, std::initializer_list<int64_t> strides) {
+  const int vec = dtype == kF32 ? 4 : 8;
+  for (int64_t s : strides)
+    if (s < C || s % vec) {
+      set_error("%s: strides must be at least C elements and whole 16-byte pieces (got %lld)", what, (long long)s);
+      return kErrBadArg;
+    }
+  return kOk;
+}
+
+int fbla_dwconv_fwd(const void* x, int64_t x_batch, int64_t x_row, const void* w, const void* bias, void* y,
+                    int64_t y_batch, int64_t y_row, int64_t B, int64_t H, int64_t W, int C, int Cw, int K, int flip,
+                    int dtype, void* stream) {
+  const char* what = "fbla_dwconv_fwd";
+  dwconv::Conv c{x, x_batch, x_row, w, bias, y, y_batch, y_row};
+  int rc = check_dwconv(what, c, B, H, W, C, Cw, K, dtype);
+  if (rc != kOk || B == 0) return rc;
+  if (!x || !w || !y) {
+    set_error("%s: null tensor pointer", what);
+    return kErrBadArg;
+  }
+  if (check_aligned(what, {x, y}) != kOk || check_row_strides(what, C, dtype, {x_batch, x_row, y_batch, y_row}) != kOk)
+    return kErrBadArg;
+  dwconv::forward(c, K, dtype, flip != 0, (hipStream_t)stream);
+  return check_launch(what);
+}
+
+size_t fbla_dwconv_grad_workspace_bytes(int64_t B, int64_t H, int64_t W, int C, int Cw, int K, int dtype) {
+  dwconv::Conv c{};
+  if (check_dwconv("fbla_dwconv_grad_workspace_bytes", c, B, H, W, C, Cw, K, dtype) != kOk || B == 0) return 0;
+  return dwconv::grad_workspace_bytes(c, K, dtype);
+}
+
+int fbla_dwconv_grad(const void* x, int64_t x_batch, int64_t x_row, const void* g, int64_t g_batch, int64_t g_row,
+                     void* dw, void* db, void* workspace, size_t workspace_bytes, int64_t B, int64_t H, int64_t W,
+                     int C, int Cw, int K, int dtype, void* stream) {
+  const char* what = "fbla_dwconv_grad";
+  dwconv::Conv c{x, x_batch, x_row};
+  int rc = check_dwconv(what, c, B, H, W, C, Cw, K, dtype);
+  if (rc != kOk) return rc;
+  if (B == 0) {
+    set_error("%s: empty batch", what);
+    return kErrBadArg;
+  }
+  if (!x || !g || (!dw && !db)) {
+    set_error("%s: null tensor pointer", what);
+    return kErrBadArg;
+  }
+  if (check_aligned(what, {x, g, workspace}) != kOk ||
+      check_row_strides(what, C, dtype, {x_batch, x_row, g_batch, g_row}) != kOk)
+    return kErrBadArg;
+  const size_t need = dwconv::grad_workspace_bytes(c, K, dtype);
+  if (!workspace || workspace_bytes < need) {
+    set_error("%s: workspace too small (%zu < %zu bytes)", what, workspace_bytes, need);
+    return kErrWorkspace;
+  }
+  dwconv::grad(c, g, g_batch, g_row, dw, db, (float*)workspace, K, dtype, (hipStream_t)stream);
+  return check_launch(what);
+}
+
 }  // extern "C"

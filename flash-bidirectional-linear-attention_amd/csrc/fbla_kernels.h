@@ -205,6 +205,27 @@ void elu1_fwd(const void* x0, void* y0, int64_t n0, const void* x1, void* y1, in
 void elu1_bwd(const void* x, const void* g, void* dx, int64_t n, int dtype, hipStream_t st);
 }  // namespace feature
 
+// Depth-wise K x K convolution of token rows on an H x W grid, channels adjacent (fbla_dwconv.hip).
+namespace dwconv {
+// x, y: token t of batch b at x + b * x_batch + t * x_row (elements; multiples of a 16-byte piece), C channels,
+// channel c uses filter c % Cw.  w [Cw, K * K], bias [Cw] or null.
+struct Conv {
+  const void* x;
+  int64_t x_batch, x_row;
+  const void *w, *bias;
+  void* y;
+  int64_t y_batch, y_row;
+  int B, H, W, C, Cw;
+};
+bool supported(int C, int Cw, int K, int dtype);
+// flip: taps in reverse order (the gradient with respect to x of a convolution with these taps)
+void forward(const Conv& a, int K, int dtype, bool flip, hipStream_t st);
+size_t grad_workspace_bytes(const Conv& a, int K, int dtype);
+// dw [Cw, K * K] and db [Cw] (either may be null) from the output's gradient g; fixed summation order
+void grad(const Conv& a, const void* g, int64_t g_batch, int64_t g_row, void* dw, void* db, float* partial, int K,
+          int dtype, hipStream_t st);
+}  // namespace dwconv
+
 // Piecewise (PISA) attention, forward only (fbla_piecewise.hip).
 namespace piecewise {
 size_t chunk_reduce_workspace_bytes(int64_t BH, int64_t T, int K, int V, int chunk, int dtype,

@@ -49,6 +49,9 @@ _SIGNATURES = {
     "fbla_piecewise_fwd": (_i32, [_vp] * 9 + [_sz, _i64, _i64, _i32, _i32, _i32, _i32, _f32, _i32, _vp]),
     "fbla_elu1_fwd": (_i32, [_vp, _vp, _i64, _vp, _vp, _i64, _i32, _vp]),
     "fbla_elu1_bwd": (_i32, [_vp, _vp, _vp, _i64, _i32, _vp]),
+    "fbla_dwconv_fwd": (_i32, [_vp, _i64, _i64, _vp, _vp, _vp] + [_i64] * 5 + [_i32] * 5 + [_vp]),
+    "fbla_dwconv_grad_workspace_bytes": (_sz, [_i64] * 3 + [_i32] * 4),
+    "fbla_dwconv_grad": (_i32, [_vp, _i64, _i64, _vp, _i64, _i64, _vp, _vp, _vp, _sz] + [_i64] * 3 + [_i32] * 4 + [_vp]),
 }
 
 
@@ -413,3 +416,44 @@ def elu1_bwd(x, dy):
         rc = L.fbla_elu1_bwd(_ptr(x), _ptr(dy), _ptr(dx), x.numel(), dtype_code(x), _stream(x.device))
     _check(rc, "fbla_elu1_bwd")
     return dx
+
+
+def _rows(t):
+    """(tensor, batch stride, row stride) of token rows [B, N, C] the depth-wise kernels can read in place: channels
+    adjacent, rows and batches at whole 16-byte pieces; anything else is copied to contiguous memory."""
+    piece = 16 // t.element_size()
+    if t.stride(2) != 1 or t.stride(0) % piece or t.stride(1) % piece or t.stride(1) < t.shape[2] or \
+            t.stride(0) < t.shape[2] or t.data_ptr() % 16:
+        t = t.clone(memory_format=torch.contiguous_format)
+    return t, t.stride(0), t.stride(1)
+
+
+def dwconv_fwd(x, w, bias, H, W, flip=False):
+    """Depth-wise convolution of token rows x [B, H*W, C] with w [Cw, 1, K, K]; returns contiguous [B, H*W, C]."""
+    _require_gpu(x, w, bias)
+    x, x_batch, x_row = _rows(x)
+    B, N, C = x.shape
+    y = torch.empty(B, N, C, dtype=x.dtype, device=x.device)
+    with _on(x.device):
+        rc = lib().fbla_dwconv_fwd(_ptr(x), x_batch, x_row, _ptr(w), _ptr(bias), _ptr(y), N * C, C, B, H, W, C,
+                                   w.shape[0], w.shape[-1], int(flip), dtype_code(x), _stream(x.device))
+    _check(rc, "fbla_dwconv_fwd")
+    return y
+
+
+def dwconv_grad(x, g, w, H, W, with_bias):
+    """(dw, db or None) of dwconv_fwd from its input and its output's gradient, both [B, H*W, C]."""
+    _require_gpu(x, g, w)
+    x, x_batch, x_row = _rows(x)
+    g, g_batch, g_row = _rows(g)
+    B, _, C = x.shape
+    Cw, K, code = w.shape[0], w.shape[-1], dtype_code(x)
+    L = lib()
+    dw = torch.empty_like(w, memory_format=torch.contiguous_format)
+    db = torch.empty(Cw, dtype=w.dtype, device=w.device) if with_bias else None
+    with _on(x.device):
+        ws = _workspace(L.fbla_dwconv_grad_workspace_bytes(B, H, W, C, Cw, K, code), x.device)
+        rc = L.fbla_dwconv_grad(_ptr(x), x_batch, x_row, _ptr(g), g_batch, g_row, _ptr(dw), _ptr(db), _ptr(ws),
+                                ws.numel(), B, H, W, C, Cw, K, code, _stream(x.device))
+    _check(rc, "fbla_dwconv_grad")
+    return dw, db

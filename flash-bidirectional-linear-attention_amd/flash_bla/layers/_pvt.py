@@ -5,6 +5,8 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from flash_bla.ops.depthwise import depthwise_conv_tokens
+
 
 class PvtLinearAttentionBase(nn.Module):
     def _init_common(self, dim, num_patches, num_heads, qkv_bias, attn_drop, proj_drop, sr_ratio, kernel_size):
@@ -38,3 +40,9 @@ class PvtLinearAttentionBase(nn.Module):
             v = v.reshape(B, heads, d, N).transpose(-2, -1)
         v = v.reshape(B * heads, H, W, d).permute(0, 3, 1, 2)
         return self.dwc(v).reshape(B, heads * d, N).transpose(1, 2)
+
+    def _value_conv_tokens(self, v, N, H, W):
+        """The same on token rows (B, n, C), without splitting heads: one filter per channel of a head."""
+        if self.sr_ratio > 1:
+            v = F.interpolate(v.transpose(1, 2), size=N, mode='linear').transpose(1, 2)
+        return depthwise_conv_tokens(v, self.dwc, H, W)

@@ -29,7 +29,10 @@ class FocusedLinearAttention(PvtLinearAttentionBase):
         k, v = self._keys_values(x, H, W)
         scale = F.softplus(self.scale)
         q, k = self._focus(self.q(x), scale), self._focus(k, scale)
+        v_rows = v
         q, k, v = (split_heads(t, self.num_heads) for t in (q, k, v))
-        out = linear_attention(q, k, v) if fast else torch_linear_attention(q, k, v)
-        out = merge_heads(out) + self._value_conv(v, N, H, W)
+        if fast:
+            out = merge_heads(linear_attention(q, k, v)) + self._value_conv_tokens(v_rows, N, H, W)
+        else:
+            out = merge_heads(torch_linear_attention(q, k, v)) + self._value_conv(v, N, H, W)
         return self.proj_drop(self.proj(out))

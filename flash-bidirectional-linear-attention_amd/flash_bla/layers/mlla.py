@@ -4,6 +4,7 @@ import torch
 import torch.nn as nn
 
 from flash_bla.layers._common import check_mode, merge_heads, split_heads, torch_linear_attention
+from flash_bla.ops.depthwise import depthwise_conv_tokens
 from flash_bla.ops.feature_map import elu_plus_one
 from flash_bla.ops.linear_attn.decoupled import decoupled_la
 
@@ -49,8 +50,8 @@ class MambaLikeLinearAttention(nn.Module):
         q, k, v, q_rope, k_rope = (split_heads(t, self.num_heads) for t in (q, k, x, *rot))
         if fast:
             out = decoupled_la(q, k, q_rope, k_rope, v, scale=n ** -1.0)
-        else:
-            out = torch_linear_attention(q, k, v, q_num=q_rope, k_num=k_rope)
+            return merge_heads(out) + depthwise_conv_tokens(x, self.lepe, side, side)
+        out = torch_linear_attention(q, k, v, q_num=q_rope, k_num=k_rope)
         grid = merge_heads(v).reshape(b, side, side, c).permute(0, 3, 1, 2)
         return merge_heads(out) + self.lepe(grid).permute(0, 2, 3, 1).reshape(b, n, c)
 

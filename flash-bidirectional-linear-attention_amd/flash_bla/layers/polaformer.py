@@ -28,6 +28,7 @@ class PolaLinearAttention(PvtLinearAttentionBase):
         k, v = self._keys_values(x, H, W)
         scale = F.softplus(self.scale)
         power = 1 + self.alpha * torch.sigmoid(self.power)
+        v_rows = v
         q, k, v = (split_heads(t, self.num_heads) for t in (q / scale, k / scale, v))
         q_pos, q_neg, k_pos, k_neg = (F.relu(t) ** power for t in (q, -q, k, -k))
         q_same = torch.cat([q_pos, q_neg], dim=-1)
@@ -39,5 +40,6 @@ class PolaLinearAttention(PvtLinearAttentionBase):
             v_same, v_opp = v.chunk(2, dim=-1)
             out = torch.cat([torch_linear_attention(q_same, k_both, v_same),
                              torch_linear_attention(q_opp, k_both, v_opp)], dim=-1)
-        out = (merge_heads(out) + self._value_conv(v, N, H, W)) * gate
+        local = self._value_conv_tokens(v_rows, N, H, W) if fast else self._value_conv(v, N, H, W)
+        out = (merge_heads(out) + local) * gate
         return self.proj_drop(self.proj(out))

@@ -5,6 +5,7 @@ import torch.nn as nn
 
 from flash_bla.layers._common import check_mode, merge_heads, split_heads, torch_linear_attention
 from flash_bla.layers.mlla import RoPE
+from flash_bla.ops.depthwise import depthwise_conv_tokens
 from flash_bla.ops.linear_attn.decoupled import decoupled_la
 
 
@@ -25,7 +26,10 @@ class RALALinearAttention(nn.Module):
         b, n, c = x.shape
         side = int(n ** 0.5)
         q, k, v, gate = self.qkvo(x).chunk(4, dim=-1)
-        lepe = self.lepe(v.reshape(b, side, side, c).permute(0, 3, 1, 2)).permute(0, 2, 3, 1).reshape(b, n, c)
+        if fast:
+            lepe = depthwise_conv_tokens(v, self.lepe, side, side)
+        else:
+            lepe = self.lepe(v.reshape(b, side, side, c).permute(0, 3, 1, 2)).permute(0, 2, 3, 1).reshape(b, n, c)
         q, k, v = (split_heads(t, self.num_heads) for t in (self.elu(q) + 1.0, self.elu(k) + 1.0, v))
         # efficiency reweighting: softmax over tokens of scale * mean(q) . k_j, times n
         eff = torch.softmax(self.scale * q.mean(dim=-2, keepdim=True) @ k.transpose(-1, -2), dim=-1)

@@ -1,0 +1,54 @@
+"""Depth-wise convolution of token rows on their H x W grid: what the vision blocks add to the attention's output
+(LePE: layers/mlla.py:92, layers/rala.py:58; the value convolution: layers/focused_la.py:88-93,
+layers/polaformer.py:97-101).  The reference transposes the tokens to images, runs nn.Conv2d with groups = channels and
+transposes back; the kernels here read and write the tokens in place and share one filter between channels
+`Cw` apart, so heads need no batch of their own.
+"""
+import torch
+import torch.nn.functional as F
+
+from flash_bla import _hip
+
+
+class DepthwiseConvTokensFunction(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x, weight, bias, H, W):
+        weight = weight.contiguous()
+        ctx.save_for_backward(x, weight)
+        ctx.grid, ctx.with_bias = (H, W), bias is not None
+        return _hip.dwconv_fwd(x, weight, None if bias is None else bias.contiguous(), H, W)
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, g):
+        x, weight = ctx.saved_tensors
+        dx = dw = db = None
+        if ctx.needs_input_grad[0]:
+            dx = _hip.dwconv_fwd(g, weight, None, *ctx.grid, flip=True)
+        if ctx.needs_input_grad[1] or (ctx.with_bias and ctx.needs_input_grad[2]):
+            dw, db = _hip.dwconv_grad(x, g, weight, *ctx.grid, ctx.with_bias)
+        return dx, dw, db, None, None
+
+
+def runs_on_tokens(x, conv):
+    """Whether the kernels take the depth-wise nn.Conv2d `conv` on token rows x: GPU tensors of one supported type, odd
+    square filters of 3 to 7 taps a side, stride 1, "same" zero padding, whole 16-byte pieces of channels."""
+    K = conv.kernel_size[0]
+    w = conv.weight
+    return (x.is_cuda and x.numel() > 0 and x.dtype in (torch.float16, torch.bfloat16, torch.float32) and
+            w.dtype == x.dtype and w.device == x.device and conv.kernel_size == (K, K) and K in (3, 5, 7) and
+            conv.padding == (K // 2, K // 2) and conv.padding_mode == 'zeros' and conv.stride == (1, 1) and
+            conv.dilation == (1, 1) and conv.groups == w.shape[0] and w.shape[1] == 1 and
+            x.shape[-1] % w.shape[0] == 0 and x.shape[-1] % (16 // x.element_size()) == 0)
+
+
+def depthwise_conv_tokens(x, conv, H, W):
+    """The depth-wise convolution `conv` (an nn.Conv2d over Cw channels) of token rows x [B, H*W, C], C a multiple of
+    Cw: channel c is convolved with filter c % Cw.  Returns [B, H*W, C].  What the kernels do not take (CPU tensors,
+    other filter shapes) runs as the torch convolution of the transposed tokens."""
+    B, N, C = x.shape
+    if runs_on_tokens(x, conv):
+        return DepthwiseConvTokensFunction.apply(x, conv.weight, conv.bias, H, W)
+    Cw = conv.weight.shape[0]
+    images = x.reshape(B, H, W, C // Cw, Cw).permute(0, 3, 4, 1, 2).reshape(B * (C // Cw), Cw, H, W)
+    return conv(images).reshape(B, C, N).transpose(1, 2)

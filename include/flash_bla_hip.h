@@ -261,6 +261,24 @@ int fbla_elu1_fwd(const void* x0, void* y0, int64_t n0, const void* x1, void* y1
 /* Its derivative: dx = dy * (x > 0 ? 1 : exp(x)), what autograd computes for `F.elu(x) + 1.0`. */
 int fbla_elu1_bwd(const void* x, const void* dy, void* dx, int64_t n, int dtype, void* stream);
 
+/* Depth-wise convolution of token rows on an H x W grid ("same" padding, stride 1): y[b, t, c] = bias[c % Cw] +
+ * sum over the K x K taps of w[c % Cw][tap] * x[b, neighbour of t, c], zero outside the grid.  Replaces the blocks'
+ * nn.Conv2d on a transposed view of the tokens (flash_bla/layers/mlla.py:92, rala.py:58, focused_la.py:88-93,
+ * polaformer.py:97-101), which reads and writes the tokens where they are.  Token t of batch b is the C elements at
+ * x + b * x_batch + t * x_row (strides in elements: whole 16-byte pieces, at least C; likewise y and g); w [Cw, K, K] and
+ * bias [Cw] (or NULL) have the element type of x.  K is 3, 5 or 7, C a multiple of Cw and of 8 (16-bit) or 4 (fp32).
+ * flip != 0 applies the taps in reverse order: with the output's gradient as x and no bias, the gradient of x. */
+int fbla_dwconv_fwd(const void* x, int64_t x_batch, int64_t x_row, const void* w, const void* bias, void* y,
+                    int64_t y_batch, int64_t y_row, int64_t B, int64_t H, int64_t W, int C, int Cw, int K, int flip,
+                    int dtype, void* stream);
+
+/* Gradients of the filters: dw [Cw, K, K] and db [Cw] (either may be NULL) from x and the output's gradient g, summed
+ * in fp32 in a fixed order and rounded once.  workspace: fbla_dwconv_grad_workspace_bytes bytes of device memory. */
+size_t fbla_dwconv_grad_workspace_bytes(int64_t B, int64_t H, int64_t W, int C, int Cw, int K, int dtype);
+int fbla_dwconv_grad(const void* x, int64_t x_batch, int64_t x_row, const void* g, int64_t g_batch, int64_t g_row,
+                     void* dw, void* db, void* workspace, size_t workspace_bytes, int64_t B, int64_t H, int64_t W,
+                     int C, int Cw, int K, int dtype, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

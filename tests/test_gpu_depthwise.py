@@ -1,0 +1,70 @@
+"""Depth-wise convolution of token rows against the same convolution in float64: filter sizes, grids whose width is not a
+multiple of the kernels' strips of 7 or 8 columns (and narrower than the filter), channel counts that end inside a
+64-channel block, filters shared between heads, strided rows (a chunk of a joint projection), both gradients.
+
+Bounds: a value is one fp32 sum of at most 49 products rounded once (u = unit roundoff of the type); a filter gradient is
+an fp32 sum over B*H*W tokens, whose rounding error stays below 2^-24 * sqrt(terms) * 4 of the sum of magnitudes."""
+import pytest
+import torch
+import torch.nn as nn
+import torch.nn.functional as F
+
+from helpers import UNIT_ROUNDOFF
+from flash_bla.ops.depthwise import depthwise_conv_tokens, runs_on_tokens
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [  # B, H, W, heads, Cw, K
+    (2, 9, 7, 1, 64, 3), (1, 5, 8, 2, 32, 5), (3, 4, 15, 3, 24, 5), (2, 1, 1, 1, 8, 3), (1, 2, 2, 2, 8, 7),
+    (2, 17, 23, 1, 136, 7), (1, 56, 56, 2, 32, 3), (4, 3, 29, 5, 16, 5),
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_convolution_and_gradients(shape, dtype):
+    B, H, W, heads, Cw, K = shape
+    C, N = heads * Cw, H * W
+    torch.manual_seed(B * 1000 + W)
+    conv = nn.Conv2d(Cw, Cw, K, padding=K // 2, groups=Cw).cuda().to(dtype)
+    joint = torch.randn(B, N, 3 * C, device="cuda").to(dtype).requires_grad_()
+    x = joint.chunk(3, dim=-1)[1]
+    g = torch.randn(B, N, 2 * C, device="cuda").to(dtype)[..., :C]
+    assert runs_on_tokens(x, conv)
+    y = depthwise_conv_tokens(x, conv, H, W)
+    y.backward(g)
+
+    w64 = conv.weight.detach().double().repeat(heads, 1, 1, 1).requires_grad_()
+    b64 = conv.bias.detach().double().repeat(heads).requires_grad_()
+    image = x.detach().double().transpose(1, 2).reshape(B, C, H, W)
+    rows = image.clone().requires_grad_()
+    ref = F.conv2d(rows, w64, b64, padding=K // 2, groups=C)
+    ref.backward(g.double().transpose(1, 2).reshape(B, C, H, W))
+    u = UNIT_ROUNDOFF[dtype]
+    as_rows = lambda t: t.reshape(B, C, N).transpose(1, 2)  # noqa: E731
+    magnitude = F.conv2d(image.abs(), w64.detach().abs(), b64.detach().abs(), padding=K // 2, groups=C)
+    err = (y.double() - as_rows(ref)).abs()
+    assert (err <= u * as_rows(ref).abs() + 2.0 ** -24 * 50 * as_rows(magnitude)).all(), err.max()
+    dx = joint.grad.chunk(3, dim=-1)[1].double()
+    want = as_rows(rows.grad)
+    assert (dx - want).abs().max() <= (u + 2.0 ** -24 * 50) * want.abs().max()
+    assert joint.grad.chunk(3, dim=-1)[0].abs().max() == 0
+    dw = w64.grad.view(heads, Cw, 1, K, K).sum(0)
+    db = b64.grad.view(heads, Cw).sum(0)
+    terms = B * N * heads
+    slack = 2.0 ** -24 * 4 * terms ** 0.5
+    scale = (x.detach().double().square().mean() * g.double().square().mean()).sqrt() * terms
+    assert ((conv.weight.grad.double() - dw).abs() <= u * dw.abs() + slack * scale).all()
+    assert ((conv.bias.grad.double() - db).abs() <= u * db.abs() + slack * g.double().abs().mean() * terms).all()
+
+
+def test_what_the_kernels_do_not_take_runs_as_the_torch_convolution():
+    for conv, C in ((nn.Conv2d(12, 12, 3, padding=1, groups=12), 12), (nn.Conv2d(16, 16, 9, padding=4, groups=16), 32)):
+        conv = conv.cuda()
+        x = torch.randn(2, 20, C, device="cuda")[..., :C]
+        assert runs_on_tokens(x, conv) == (conv.kernel_size[0] == 3)
+        y = depthwise_conv_tokens(x, conv, 4, 5)
+        rep = C // conv.weight.shape[0]
+        want = F.conv2d(x.double().transpose(1, 2).reshape(2, C, 4, 5), conv.weight.double().repeat(rep, 1, 1, 1),
+                        conv.bias.double().repeat(rep), padding=conv.padding, groups=C).reshape(2, C, 20).transpose(1, 2)
+        assert (y.double() - want).abs().max() <= 1e-5 * want.abs().max()
