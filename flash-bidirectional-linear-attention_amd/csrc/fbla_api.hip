@@ -76,7 +76,7 @@ static int check_aligned(const char* what, std::initializer_list<const void*> pt
 
 static Prob make_prob(const int32_t* cu, int64_t N, int64_t H, int64_t L, int64_t T, int DK, int DV,
                       int flags, float scale, float eps) {
-  Prob p;
+  Prob p{};
   p.cu = cu;
   p.perm = nullptr;
   p.chunk_base = nullptr;
@@ -87,6 +87,7 @@ static Prob make_prob(const int32_t* cu, int64_t N, int64_t H, int64_t L, int64_
   p.T = T;
   p.DK = DK;
   p.DV = DV;
+  p.RK = p.RV = 0;
   p.scale = scale;
   p.eps = eps;
   p.flags = flags;

@@ -49,6 +49,8 @@ struct Prob {
                 // the length of the side they walk.
   int64_t T;    // total tokens (dense: N*L)
   int DK, DV;
+  int RK, RV;   // 16-bit plain operator: row lengths in memory (at least 8) when they are no multiples of 8 and DK, DV
+                // are their next multiples of 8, the shape of the state; else 0 (rows of DK and DV elements)
   float scale;
   float eps;
   int flags;

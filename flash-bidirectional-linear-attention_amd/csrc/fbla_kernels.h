@@ -122,6 +122,7 @@ struct RowsJob {
   bool vec_is_add = false;
   float* mat_out = nullptr;
   float* vec_out = nullptr;
+  int xlen = 0, olen = 0;  // Prob::RK, RV set: elements per row of x and of out
   float add_scale = 1.f;  // factor on addvec (queries / keys when their numbers differ)
   bool map_x = false;          // kElu1 together with kElu1Grad: this job's x rows arrive before the map
   const void* gate = nullptr;  // [rows][DC] mapped rows phi(x): the output is multiplied by min(gate, 1), the

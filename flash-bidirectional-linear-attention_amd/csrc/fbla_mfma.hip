@@ -149,6 +149,42 @@ template <typename T> __device__ __forceinline__ uint32_t phi_pair(uint32_t w) {
   return pack2<T>(Ops<T>::lo(e) + 1.f, Ops<T>::hi(e) + 1.f);
 }
 
+// Rows whose length is no multiple of eight elements (PAD = 2: Prob::RK / RV elements in memory, inside operands of the
+// next multiple of eight).  Their 16-byte pieces start on any element.  The last piece of a row is moved back to end with
+// the row, so that no access leaves the row, and its elements are moved to their places in registers.
+typedef u32x4 u32x4_any __attribute__((aligned(2)));
+typedef uint32_t u32_any __attribute__((aligned(2)));
+// first element of piece `ch` of a row of `len` (>= 8) elements, and how far back it was moved
+__device__ __forceinline__ int ragged_first(int ch, int len) { return min(8 * ch, len - 8); }
+__device__ __forceinline__ int ragged_shift(int ch, int len) { return 8 * ch - ragged_first(ch, len); }
+// a moved-back piece as loaded: its first `back` (0..7) elements belong to the piece before it; zeros behind the row
+__device__ __forceinline__ u32x4 ragged_in(u32x4 w, int back) {
+  const uint32_t b = (back & 1) * 16;
+  const uint32_t t0 = __builtin_amdgcn_alignbit(w[1], w[0], b), t1 = __builtin_amdgcn_alignbit(w[2], w[1], b),
+                 t2 = __builtin_amdgcn_alignbit(w[3], w[2], b), t3 = w[3] >> b;
+  auto pick = [](bool c, uint32_t x, uint32_t y) { return c ? x : y; };
+  const bool two = back & 2, four = back & 4;
+  const uint32_t u0 = pick(two, t1, t0), u1 = pick(two, t2, t1), u2 = pick(two, t3, t2), u3 = pick(two, 0u, t3);
+  return u32x4{pick(four, u2, u0), pick(four, u3, u1), pick(four, 0u, u2), pick(four, 0u, u3)};
+}
+// what a moved-back piece stores: the last `back` elements of the piece before it (which stores the same values there),
+// then its own
+__device__ __forceinline__ u32x4 ragged_out(u32x4 prev, u32x4 w, int back) {
+  const int n = 8 - back;  // elements of (prev, w) to drop; 8: the piece is whole
+  const uint32_t b = (n & 1) * 16;
+  const uint32_t t0 = __builtin_amdgcn_alignbit(prev[1], prev[0], b), t1 = __builtin_amdgcn_alignbit(prev[2], prev[1], b),
+                 t2 = __builtin_amdgcn_alignbit(prev[3], prev[2], b), t3 = __builtin_amdgcn_alignbit(w[0], prev[3], b),
+                 t4 = __builtin_amdgcn_alignbit(w[1], w[0], b), t5 = __builtin_amdgcn_alignbit(w[2], w[1], b),
+                 t6 = __builtin_amdgcn_alignbit(w[3], w[2], b);
+  // values, not places (a conditional between two variables would keep them in memory)
+  auto pick = [](bool c, uint32_t x, uint32_t y) { return c ? x : y; };
+  const bool two = n & 2, four = n & 4, whole = back == 0;
+  const uint32_t u0 = pick(two, t1, t0), u1 = pick(two, t2, t1), u2 = pick(two, t3, t2), u3 = pick(two, t4, t3),
+                 u4 = pick(two, t5, t4), u5 = pick(two, t6, t5);
+  return u32x4{pick(whole, w[0], pick(four, u2, u0)), pick(whole, w[1], pick(four, u3, u1)),
+               pick(whole, w[2], pick(four, u4, u2)), pick(whole, w[3], pick(four, u5, u3))};
+}
+
 typedef short i16x4 __attribute__((ext_vector_type(4)));
 // Eight tokens of one feature (an MFMA operand fragment of one k-step) out of a row-major tile:
 // two transposing reads, `off0` / `off1` are this lane's byte offsets for x = 0 / 1.
@@ -173,7 +209,7 @@ template <int C> struct RowWords { uint32_t w[8][C / 2]; };
 // lane's constant offset (its half-wave's first row, 0 or 8, times step, plus its feature
 // column).  No branch, no per-row address arithmetic in vector registers: the loads of the
 // next step can stay in flight while the current one is multiplied.
-template <typename T, int C>
+template <typename T, int C, bool ANY = false>
 __device__ __forceinline__ void load_rows(RowWords<C>& dst, const T* __restrict__ tile, uint32_t step,
                                           uint32_t voff) {
   // byte arithmetic in 32 bits on top of a uniform 64-bit base: the scalar-base + vector-offset
@@ -184,7 +220,7 @@ __device__ __forceinline__ void load_rows(RowWords<C>& dst, const T* __restrict_
   for (int j = 0; j < 8; ++j) {
     const char* row = base + (size_t)((uint32_t)j * step_b);
     if constexpr (C == 2) {
-      dst.w[j][0] = load_stream<uint32_t, kNtStateLoad>(row + voff_b);
+      dst.w[j][0] = load_stream<std::conditional_t<ANY, u32_any, uint32_t>, kNtStateLoad>(row + voff_b);
     } else {
       u32x2 x = load_stream<u32x2, kNtStateLoad>(row + voff_b);
       dst.w[j][0] = x[0];
@@ -195,7 +231,7 @@ __device__ __forceinline__ void load_rows(RowWords<C>& dst, const T* __restrict_
 
 // The same with a bounds check per row, for chunks shorter than one tile: rows at or past
 // `rows` (relative to the tile) are not read and come back as zero.
-template <typename T, int C>
+template <typename T, int C, bool ANY = false>
 __device__ __forceinline__ void load_rows_checked(RowWords<C>& dst, const T* __restrict__ tile,
                                                   uint32_t step, int rel0, int col, int rows) {
 #pragma unroll
@@ -203,7 +239,8 @@ __device__ __forceinline__ void load_rows_checked(RowWords<C>& dst, const T* __r
 #pragma unroll
     for (int c = 0; c < C / 2; ++c) dst.w[j][c] = 0u;
     if (rel0 + j < rows) {
-      const uint32_t* src = reinterpret_cast<const uint32_t*>(tile + (size_t)(rel0 + j) * step + col);
+      using W = std::conditional_t<ANY, u32_any, uint32_t>;
+      const W* src = reinterpret_cast<const W*>(tile + (size_t)(rel0 + j) * step + col);
 #pragma unroll
       for (int c = 0; c < C / 2; ++c) dst.w[j][c] = src[c];
     }
@@ -227,6 +264,15 @@ __device__ __forceinline__ void keep_rows(RowWords<C>& r, uint32_t keep) {
   for (int j = 0; j < 8; ++j)
 #pragma unroll
     for (int c = 0; c < C / 2; ++c) r.w[j][c] &= keep;
+}
+
+// the last element of an odd row: a lane whose second feature does not exist loaded the pair before it
+template <int C>
+__device__ __forceinline__ void shift_rows(RowWords<C>& r, uint32_t bits) {
+#pragma unroll
+  for (int j = 0; j < 8; ++j)
+#pragma unroll
+    for (int c = 0; c < C / 2; ++c) r.w[j][c] >>= bits;
 }
 
 // token-pair packing: operand c gets feature c of tokens (2i, 2i+1) in dword i
@@ -261,7 +307,7 @@ struct BlockStats {
 };
 
 // FMAP = true: the key rows arrive before the feature map and are mapped (phi_pair) as they are used.
-template <typename T, int DK, int DV, bool SPLIT_KD, int TILES, bool SCALED, bool STATS = false, bool PAD = false,
+template <typename T, int DK, int DV, bool SPLIT_KD, int TILES, bool SCALED, bool STATS = false, int PAD = 0,
           bool FMAP = false>
 __global__ __launch_bounds__(kThreads, (DK == 64 && DV == 64 && !SCALED) ? 3 : 2) void state_kernel(Prob p, const T* __restrict__ kn,
                                                          const T* __restrict__ v,
@@ -273,7 +319,10 @@ __global__ __launch_bounds__(kThreads, (DK == 64 && DV == 64 && !SCALED) ? 3 : 2
                                                          BlockStats stats) {
   static_assert(!STATS || (TILES == 1 && !SCALED && !SPLIT_KD && !PAD), "block statistics: plain variant only");
   static_assert(!FMAP || (!SCALED && !SPLIT_KD && !PAD && !STATS), "feature map on load: plain variant only");
-  const int dk = PAD ? p.DK : DK, dv = PAD ? p.DV : DV;  // row lengths in memory
+  constexpr bool RAG = PAD == 2;  // rows of p.RK / p.RV elements
+  static_assert(!RAG || (!SCALED && !SPLIT_KD), "rows of any length: plain variant only");
+  const int dk = PAD ? p.DK : DK, dv = PAD ? p.DV : DV;  // shape of the state
+  const int rk = RAG ? p.RK : dk, rv = RAG ? p.RV : dv;  // row lengths in memory
   // The state is tiled into 64 x 64 blocks (64 accumulator registers per lane); a block is
   // owned by G waves that take interleaved token tiles.  For a 128 x 128 state the four
   // waves of the workgroup therefore read the same tokens, each the 64 key and 64 value
@@ -314,11 +363,15 @@ __global__ __launch_bounds__(kThreads, (DK == 64 && DV == 64 && !SCALED) ? 3 : 2
   const int pp = lane & 31, kb = lane >> 5;
   const int blk = wave / G, g = wave % G, bk = blk / VB, bv = blk % VB;
   // this lane's feature columns inside its block, and whether they exist
-  const bool k_ok = !PAD || 64 * bk + CK * pp < dk, v_ok = !PAD || 64 * bv + CV * pp < dv;
-  const int kcol0 = k_ok ? CK * pp : 0, vcol0 = v_ok ? CV * pp : 0;
+  const bool k_ok = !PAD || 64 * bk + CK * pp < rk, v_ok = !PAD || 64 * bv + CV * pp < rv;
+  // (RAG: the lane with the last element of an odd row loads the pair that ends with it; columns count from the row's
+  // first element, since that pair may start in the block before)
+  const bool k_odd = RAG && 64 * bk + CK * pp == rk - 1, v_odd = RAG && 64 * bv + CV * pp == rv - 1;
+  const int kcol0 = RAG ? (k_ok ? 64 * bk + CK * pp - (k_odd ? 1 : 0) : 0) : k_ok ? CK * pp : 0;
+  const int vcol0 = RAG ? (v_ok ? 64 * bv + CV * pp - (v_odd ? 1 : 0) : 0) : v_ok ? CV * pp : 0;
   const uint32_t k_keep = k_ok ? ~0u : 0u, v_keep = v_ok ? ~0u : 0u;
-  const T* kcol = kn + 64 * bk;
-  const T* vcol = v + 64 * bv;
+  const T* kcol = kn + (RAG ? 0 : 64 * bk);
+  const T* vcol = v + (RAG ? 0 : 64 * bv);
   const T* kdcol = kd + 64 * bk;
 
   f32x16 acc[CK][CV];
@@ -347,7 +400,7 @@ __global__ __launch_bounds__(kThreads, (DK == 64 && DV == 64 && !SCALED) ? 3 : 2
   // first `lo` rows were already part of the previous tile and are zeroed before use.  Every
   // tile therefore reads 16 valid rows with the same address pattern (chunks shorter than
   // one tile take the checked path below).
-  const uint32_t kstep = (uint32_t)(rstride * dk), vstep = (uint32_t)(rstride * dv);
+  const uint32_t kstep = (uint32_t)(rstride * rk), vstep = (uint32_t)(rstride * rv);
   const uint32_t kvoff = (uint32_t)(8 * kb) * kstep + (uint32_t)kcol0;
   const uint32_t vvoff = (uint32_t)(8 * kb) * vstep + (uint32_t)vcol0;
   const uint32_t tvoff = (uint32_t)(8 * kb) * (uint32_t)rstride;
@@ -356,8 +409,8 @@ __global__ __launch_bounds__(kThreads, (DK == 64 && DV == 64 && !SCALED) ? 3 : 2
     for (int u = 0; u < TILES; ++u) {
       const int tb = min(tok + 16 * u, t_end - 16);
       const int64_t row = row0 + (int64_t)tb * rstride;
-      load_rows<T, CK>(b.k[u], kcol + row * dk, kstep, kvoff);
-      load_rows<T, CV>(b.v[u], vcol + row * dv, vstep, vvoff);
+      load_rows<T, CK, RAG>(b.k[u], kcol + row * rk, kstep, kvoff);
+      load_rows<T, CV, RAG>(b.v[u], vcol + row * rv, vstep, vvoff);
       if constexpr (SPLIT_KD) load_rows<T, CK>(b.d[u], kdcol + row * dk, kstep, kvoff);
       if constexpr (SCALED) {
         const float* ts = tokscal + row;
@@ -374,8 +427,8 @@ __global__ __launch_bounds__(kThreads, (DK == 64 && DV == 64 && !SCALED) ? 3 : 2
     for (int u = 0; u < TILES; ++u) {
       const int rows = t_end - (tok + 16 * u);
       const int64_t row = row0 + (int64_t)(tok + 16 * u) * rstride;
-      load_rows_checked<T, CK>(b.k[u], kcol + row * dk, kstep, 8 * kb, kcol0, rows);
-      load_rows_checked<T, CV>(b.v[u], vcol + row * dv, vstep, 8 * kb, vcol0, rows);
+      load_rows_checked<T, CK, RAG>(b.k[u], kcol + row * rk, kstep, 8 * kb, kcol0, rows);
+      load_rows_checked<T, CV, RAG>(b.v[u], vcol + row * rv, vstep, 8 * kb, vcol0, rows);
       if constexpr (SPLIT_KD) load_rows_checked<T, CK>(b.d[u], kdcol + row * dk, kstep, 8 * kb, kcol0, rows);
       if constexpr (SCALED) {
 #pragma unroll
@@ -404,6 +457,10 @@ __global__ __launch_bounds__(kThreads, (DK == 64 && DV == 64 && !SCALED) ? 3 : 2
       for (int u = 0; u < TILES; ++u) {
         keep_rows<CK>(b.k[u], k_keep);
         keep_rows<CV>(b.v[u], v_keep);
+        if constexpr (RAG) {
+          shift_rows<CK>(b.k[u], k_odd ? 16 : 0);
+          shift_rows<CV>(b.v[u], v_odd ? 16 : 0);
+        }
         if constexpr (SPLIT_KD) keep_rows<CK>(b.d[u], k_keep);
       }
     }
@@ -579,7 +636,7 @@ struct State128Layout {
 
 // STATS = true additionally writes the mean key and the value sum of every 64-token block (a
 // step of this kernel), like state_kernel's STATS.
-template <typename T, bool PAD, bool STATS = false>
+template <typename T, int PAD, bool STATS = false>
 __global__ __launch_bounds__(kThreads, 2) void state128_kernel(Prob p, const T* __restrict__ kn,
                                                                const T* __restrict__ v,
                                                                float* __restrict__ partial,
@@ -589,7 +646,9 @@ __global__ __launch_bounds__(kThreads, 2) void state128_kernel(Prob p, const T* 
   static_assert(!STATS || !PAD, "block statistics: full head dims only");
   using LY = State128Layout;
   constexpr int ROWB = 256;
-  const int dk = PAD ? p.DK : 128, dv = PAD ? p.DV : 128;  // row lengths in memory
+  constexpr bool RAG = PAD == 2;
+  const int dk = PAD ? p.DK : 128, dv = PAD ? p.DV : 128;  // shape of the state
+  const int rk = RAG ? p.RK : dk, rv = RAG ? p.RV : dv;    // row lengths in memory
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int wg_item = packed_item(p, blockIdx.x, p.H * nchunks);
   const int wg_nh = wg_item / nchunks, c = wg_item - wg_nh * nchunks;
@@ -623,22 +682,26 @@ __global__ __launch_bounds__(kThreads, 2) void state128_kernel(Prob p, const T* 
   // tensors with more than 65536 heads away from this kernel).  Rows past the end of the chunk
   // and chunks past the head dim are not read and count as zeros.
   const int prow = tid >> 4, pch = tid & 15;
-  const uint32_t krow_b = (uint32_t)rstride * (uint32_t)dk * 2u, vrow_b = (uint32_t)rstride * (uint32_t)dv * 2u;
-  const uint32_t kvoff = (uint32_t)prow * krow_b + (uint32_t)pch * 16u;
-  const uint32_t vvoff = PAD ? (uint32_t)prow * vrow_b + (uint32_t)pch * 16u : kvoff;
-  const bool k_piece = !PAD || pch * 8 < dk, v_piece = !PAD || pch * 8 < dv;
+  const uint32_t krow_b = (uint32_t)rstride * (uint32_t)rk * 2u, vrow_b = (uint32_t)rstride * (uint32_t)rv * 2u;
+  const bool k_piece = !PAD || pch * 8 < rk, v_piece = !PAD || pch * 8 < rv;
+  const uint32_t kvoff = (uint32_t)prow * krow_b + (RAG ? 2u * (uint32_t)ragged_first(pch, rk) : (uint32_t)pch * 16u);
+  const uint32_t vvoff = PAD ? (uint32_t)prow * vrow_b + (RAG ? 2u * (uint32_t)ragged_first(pch, rv) : (uint32_t)pch * 16u)
+                             : kvoff;
+  const int kback = RAG && k_piece ? ragged_shift(pch, rk) : 0, vback = RAG && v_piece ? ragged_shift(pch, rv) : 0;
   auto load_step = [&](u32x4(&dst)[4], const T* src, int tok0, int rowlen, uint32_t row_b, uint32_t voff, bool has) {
     const char* tp = reinterpret_cast<const char*>(src) + ((row0 + (int64_t)tok0 * rstride) * rowlen) * (int64_t)sizeof(T);
     const int rows = t_end - tok0;  // rows of this step that exist (may be <= 0)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       dst[i] = u32x4{0u, 0u, 0u, 0u};
-      if (has && prow + 16 * i < rows) dst[i] = load_stream<u32x4, kNtStateLoad>(tp + (size_t)(16 * i) * row_b + voff);
+      if (has && prow + 16 * i < rows)
+        dst[i] = load_stream<std::conditional_t<RAG, u32x4_any, u32x4>, kNtStateLoad>(tp + (size_t)(16 * i) * row_b + voff);
     }
   };
-  auto stash_step = [&](const u32x4(&src)[4], unsigned char* tiles) {
+  auto stash_step = [&](const u32x4(&src)[4], unsigned char* tiles, int back) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) *reinterpret_cast<u32x4*>(tiles + swz<ROWB>(prow + 16 * i, pch)) = src[i];
+    for (int i = 0; i < 4; ++i)
+      *reinterpret_cast<u32x4*>(tiles + swz<ROWB>(prow + 16 * i, pch)) = RAG ? ragged_in(src[i], back) : src[i];
   };
 
   f32x16 acc[2][2];
@@ -669,17 +732,17 @@ __global__ __launch_bounds__(kThreads, 2) void state128_kernel(Prob p, const T* 
     }
   }
 
-  u32x4 rk[4], rv[4];
-  load_step(rk, kn, t_begin, dk, krow_b, kvoff, k_piece);
-  load_step(rv, v, t_begin, dv, vrow_b, vvoff, v_piece);
+  u32x4 krows[4], vrows[4];
+  load_step(krows, kn, t_begin, rk, krow_b, kvoff, k_piece);
+  load_step(vrows, v, t_begin, rv, vrow_b, vvoff, v_piece);
   int buf = 0;
   for (int base = t_begin; base < t_end; base += 64) {
     unsigned char* kt = ksteps + buf * LY::kStep;
     unsigned char* vt = vsteps + buf * LY::kStep;
-    stash_step(rk, kt);
-    stash_step(rv, vt);
-    load_step(rk, kn, base + 64, dk, krow_b, kvoff, k_piece);
-    load_step(rv, v, base + 64, dv, vrow_b, vvoff, v_piece);
+    stash_step(krows, kt, kback);
+    stash_step(vrows, vt, vback);
+    load_step(krows, kn, base + 64, rk, krow_b, kvoff, k_piece);
+    load_step(vrows, v, base + 64, rv, vrow_b, vvoff, v_piece);
     __syncthreads();  // the step is in LDS; every wave is done with the other buffer's previous step
     float kstep = 0.f, vstep = 0.f;  // this step's sums (STATS: the step is a block of the statistics)
 #pragma unroll
@@ -755,7 +818,7 @@ __global__ __launch_bounds__(kThreads, 2) void state128_kernel(Prob p, const T* 
 // operand's remaining rows and columns are zero.
 // PAIR = true (DR = DC = 64): the matrix in memory is 32 x 32 and the operand is
 // blockdiag(M, M): a 64-wide row then holds two independent 32-wide rows.
-template <typename T, int DR, int DC, int NT = kThreads, bool PAD = false, bool PAIR = false>
+template <typename T, int DR, int DC, int NT = kThreads, int PAD = 0, bool PAIR = false>
 __device__ __forceinline__ float build_operand(unsigned char* lds_opnd, float* lds_max,
                                                const float* __restrict__ mat, int ld_r, int ld_c,
                                                int nsum = 1, int64_t sum_stride = 0,
@@ -937,12 +1000,14 @@ template <int DR, int DC, bool DEN, int WAVES, bool GATE = false> struct RowsLay
 // streams full 128-byte rows at the cost of multiplying zeros.  `chunk` counts row pairs; an
 // odd length leaves the second half of the last pair out.  No partial sums in the prologue.
 // FMAP = true: the rows of x arrive before the feature map and are mapped (phi_pair) on their way into LDS.
-template <typename T, int DR, int DC, bool NORM, bool DEN, int WAVES, bool PAD = false,
+template <typename T, int DR, int DC, bool NORM, bool DEN, int WAVES, int PAD = 0,
           int PF = (DR == 128 && DC == 128) ? FBLA_ROWS_PF128 : FBLA_ROWS_PF, bool PAIR = false, bool FMAP = false,
           bool GATE = false>
 __global__ __launch_bounds__(WAVES * 64, (FBLA_ROWS_OCC4 && DR == 64 && DC == 64 && !DEN && !GATE) ? 4 : 1) void rows_kernel(Prob p, RowsJob job0, RowsJob job1,
                                                           int wgs_per_job, int chunk, int nchunks,
                                                           int dr_true, int dc_true) {
+  constexpr bool RAG = PAD == 2;
+  static_assert(!RAG || (!DEN && !GATE), "rows of any length: plain rows only");
   static_assert(!PAIR || (DR == 64 && DC == 64 && !PAD), "pair mode: two 32-wide rows per 64-wide row");
   static_assert(!FMAP || (!DEN && !PAD && !PAIR), "feature map on load: plain rows only");
   static_assert(!GATE || (!DEN && !PAD && !PAIR && DR == DC), "gated output: plain square tiles only");
@@ -954,6 +1019,7 @@ __global__ __launch_bounds__(WAVES * 64, (FBLA_ROWS_OCC4 && DR == 64 && DC == 64
   const RowsJob& job = second ? job1 : job0;
   // FMAP and GATE together (pass B of a backward given the rows before the map): a job maps its x rows
   // when job.map_x is set, and its gate rows arrive before the map too
+  const int xlen = RAG ? job.xlen : dr, olen = RAG ? job.olen : dc;  // row lengths in memory
   const bool map_x = FMAP && (!GATE || job.map_x);
   const int wg = second ? blockIdx.x - wgs_per_job : blockIdx.x;
   constexpr int NT = WAVES * 64;
@@ -1001,7 +1067,7 @@ __global__ __launch_bounds__(WAVES * 64, (FBLA_ROWS_OCC4 && DR == 64 && DC == 64
       return (row0 + 2 * (int64_t)tok) * 32 + ch * 8;
     } else {
       if (tok >= t_end || (PAD && ch * 8 >= rowlen)) return -1;
-      return (row0 + (int64_t)tok * rstride) * rowlen + ch * 8;
+      return (row0 + (int64_t)tok * rstride) * rowlen + (RAG ? ragged_first(ch, rowlen) : ch * 8);
     }
   };
 
@@ -1025,9 +1091,9 @@ __global__ __launch_bounds__(WAVES * 64, (FBLA_ROWS_OCC4 && DR == 64 && DC == 64
 #pragma unroll
     for (int i = 0; i < XI; ++i) {
       const int q = lane + 64 * i, row = q / XCH, ch = q % XCH;
-      const int64_t off = piece(tok0 + row, ch, dr);
+      const int64_t off = piece(tok0 + row, ch, xlen);
       if (off >= 0) {
-        dst[i] = load_stream<u32x4, kNtRowsLoad>(src + off);
+        dst[i] = load_stream<std::conditional_t<RAG, u32x4_any, u32x4>, kNtRowsLoad>(src + off);
       } else {
         dst[i] = u32x4{0u, 0u, 0u, 0u};
       }
@@ -1037,7 +1103,8 @@ __global__ __launch_bounds__(WAVES * 64, (FBLA_ROWS_OCC4 && DR == 64 && DC == 64
 #pragma unroll
     for (int i = 0; i < XI; ++i) {
       const int q = lane + 64 * i, row = q / XCH, ch = q % XCH;
-      *reinterpret_cast<u32x4*>(dstb + swz<XROWB>(row, ch)) = src[i];
+      // (a piece past the row's end was not read: it is zero however far it is shifted)
+      *reinterpret_cast<u32x4*>(dstb + swz<XROWB>(row, ch)) = RAG ? ragged_in(src[i], ragged_shift(ch, xlen) & 7) : src[i];
     }
   };
   // Whole tiles of plain rows (every tile but a ragged last one): a wave-uniform tile address
@@ -1271,8 +1338,14 @@ __global__ __launch_bounds__(WAVES * 64, (FBLA_ROWS_OCC4 && DR == 64 && DC == 64
 #pragma unroll
       for (int i = 0; i < OI; ++i) {
         const int q = lane + 64 * i, row = q / OCH, ch = q % OCH;
-        const int64_t off = piece(t0 + row, ch, dc);
-        if (off >= 0) store_row16<kNtRowsStore>(out + off, wout[i]);
+        const int64_t off = piece(t0 + row, ch, olen);
+        if constexpr (RAG) {
+          const int back = ragged_shift(ch, olen);
+          const u32x4 prev = *reinterpret_cast<const u32x4*>(stage + swz<OROWB>(row, ch > 0 ? ch - 1 : 0));
+          if (off >= 0) *reinterpret_cast<u32x4_any*>(out + off) = ragged_out(prev, wout[i], back);
+        } else if (off >= 0) {
+          store_row16<kNtRowsStore>(out + off, wout[i]);
+        }
       }
     }
     t0 += t_stride;
@@ -1311,15 +1384,17 @@ struct Rows128Layout {
   static_assert(2 * kTotal <= 160 * 1024, "two workgroups per CU");
 };
 
-template <typename T, bool NORM, bool PAD>
+template <typename T, bool NORM, int PAD>
 __global__ __launch_bounds__(kThreads, 2) void rows128_kernel(Prob p, RowsJob job0, RowsJob job1, int wgs_per_job,
                                                               int chunk, int nchunks, int dr_true, int dc_true) {
   using LY = Rows128Layout;
   constexpr int KS = 8, ROWB = 256, NT = kThreads;
+  constexpr bool RAG = PAD == 2;
   const int dr = PAD ? dr_true : 128, dc = PAD ? dc_true : 128;
   const int dpk = PAD ? (p.DK <= 64 ? 64 : 128) : p.DK;  // padded length of the km / dkm vector
   const bool second = (int)blockIdx.x >= wgs_per_job;
   const RowsJob& job = second ? job1 : job0;
+  const int xlen = RAG ? job.xlen : dr, olen = RAG ? job.olen : dc;  // row lengths in memory
   const int wg = second ? blockIdx.x - wgs_per_job : blockIdx.x;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   uint32_t* lds_km = reinterpret_cast<uint32_t*>(smem + LY::kKm);
@@ -1359,20 +1434,23 @@ __global__ __launch_bounds__(kThreads, 2) void rows128_kernel(Prob p, RowsJob jo
   // i-th distance plus the lane's one constant byte offset (32 bits: the host keeps packed
   // tensors with more than 65536 heads away from this kernel).
   const int prow = tid >> 4, pch = tid & 15;
-  const uint32_t xrow_b = (uint32_t)rstride * (uint32_t)dr * 2u, orow_b = (uint32_t)rstride * (uint32_t)dc * 2u;
-  const uint32_t xvoff = (uint32_t)prow * xrow_b + (uint32_t)pch * 16u;
-  const uint32_t ovoff = PAD ? (uint32_t)prow * orow_b + (uint32_t)pch * 16u : xvoff;
-  const bool x_piece = !PAD || pch * 8 < dr, o_piece = !PAD || pch * 8 < dc;
+  const uint32_t xrow_b = (uint32_t)rstride * (uint32_t)xlen * 2u, orow_b = (uint32_t)rstride * (uint32_t)olen * 2u;
+  const uint32_t xvoff = (uint32_t)prow * xrow_b + (RAG ? 2u * (uint32_t)ragged_first(pch, xlen) : (uint32_t)pch * 16u);
+  const uint32_t ovoff = PAD ? (uint32_t)prow * orow_b + (RAG ? 2u * (uint32_t)ragged_first(pch, olen) : (uint32_t)pch * 16u)
+                             : xvoff;
+  const bool x_piece = !PAD || pch * 8 < xlen, o_piece = !PAD || pch * 8 < olen;
+  const int xback = RAG && x_piece ? ragged_shift(pch, xlen) : 0, oback = RAG && o_piece ? ragged_shift(pch, olen) : 0;
   auto step_ptr = [&](const void* base, int tok0, int rowlen) -> const char* {
     return reinterpret_cast<const char*>(base) + ((row0 + (int64_t)tok0 * rstride) * rowlen) * (int64_t)sizeof(T);
   };
   auto load_step = [&](u32x4(&dst)[4], int tok0) {
-    const char* tp = step_ptr(x, tok0, dr);
+    const char* tp = step_ptr(x, tok0, xlen);
     const int rows = t_end - tok0;  // rows of this step that exist (may be <= 0)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       dst[i] = u32x4{0u, 0u, 0u, 0u};
-      if (x_piece && prow + 16 * i < rows) dst[i] = load_stream<u32x4, kNtRowsLoad>(tp + (size_t)(16 * i) * xrow_b + xvoff);
+      if (x_piece && prow + 16 * i < rows)
+        dst[i] = load_stream<std::conditional_t<RAG, u32x4_any, u32x4>, kNtRowsLoad>(tp + (size_t)(16 * i) * xrow_b + xvoff);
     }
   };
 
@@ -1430,6 +1508,10 @@ __global__ __launch_bounds__(kThreads, 2) void rows128_kernel(Prob p, RowsJob jo
   for (int base = t_begin; base < t_end; base += 64) {
     unsigned char* xt = smem + LY::kX + buf * LY::kStep;
     float* zrow = lds_z + 64 * buf;
+    if constexpr (RAG) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) rx[i] = ragged_in(rx[i], xback);
+    }
 #pragma unroll
     for (int i = 0; i < 4; ++i) *reinterpret_cast<u32x4*>(xt + swz<ROWB>(prow + 16 * i, pch)) = rx[i];
     if constexpr (NORM) {
@@ -1483,13 +1565,20 @@ __global__ __launch_bounds__(kThreads, 2) void rows128_kernel(Prob p, RowsJob jo
     }
     __syncthreads();  // the output rows are complete
     {
-      char* tp = const_cast<char*>(step_ptr(out, base, dc));
+      char* tp = const_cast<char*>(step_ptr(out, base, olen));
       const int rows = t_end - base;
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        if (o_piece && prow + 16 * i < rows)
-          store_row16<kNtRowsStore>(tp + (size_t)(16 * i) * orow_b + ovoff,
-                                    *reinterpret_cast<const u32x4*>(ostage + swz<ROWB>(prow + 16 * i, pch)));
+        if (o_piece && prow + 16 * i < rows) {
+          const u32x4 w = *reinterpret_cast<const u32x4*>(ostage + swz<ROWB>(prow + 16 * i, pch));
+          char* at = tp + (size_t)(16 * i) * orow_b + ovoff;
+          if constexpr (RAG) {
+            const u32x4 prev = *reinterpret_cast<const u32x4*>(ostage + swz<ROWB>(prow + 16 * i, pch > 0 ? pch - 1 : 0));
+            *reinterpret_cast<u32x4_any*>(at) = ragged_out(prev, w, oback);
+          } else {
+            store_row16<kNtRowsStore>(at, w);
+          }
+        }
     }
     buf ^= 1;
   }
@@ -1546,7 +1635,7 @@ template <int DK, int DV, bool NORM, bool DEN, bool FUSED, bool LO = true> struc
 // before the store.  `chunk` counts row pairs.
 // GATE = true: q are the mapped rows phi(x) and dq is wanted with respect to x: times min(q, 1).
 // FMAP = true (with GATE): q are the rows x themselves and are mapped on their way into LDS.
-template <typename T, int DK, int DV, bool NORM, bool DEN, bool FUSED, bool LO = true, bool PAD = false,
+template <typename T, int DK, int DV, bool NORM, bool DEN, bool FUSED, bool LO = true, int PAD = 0,
           bool PAIR = false, bool GATE = false, bool FMAP = false>
 __global__ __launch_bounds__(kThreads, (FBLA_BWDA_OCC3 && FUSED && !DEN && !LO) ? 3 : 2) void bwd_a_kernel(
     Prob p, const T* __restrict__ qn, const T* __restrict__ qd, const T* __restrict__ dout,
@@ -1558,7 +1647,10 @@ __global__ __launch_bounds__(kThreads, (FBLA_BWDA_OCC3 && FUSED && !DEN && !LO) 
   constexpr int CK = DK / 32, CV = DV / 32;
   static_assert(!FUSED || (DK == 64 && DV == 64), "the fused form exists for 64 x 64 tiles (128 x 128: bwd_a128_kernel)");
   static_assert(!PAIR || (DK == 64 && DV == 64 && FUSED && !PAD), "pair mode: two 32-wide rows per 64-wide row");
+  constexpr bool RAG = PAD == 2;
+  static_assert(!RAG || (!DEN && FUSED), "rows of any length: the fused plain form only");
   const int dk = PAD ? p.DK : (PAIR ? 32 : DK), dv = PAD ? p.DV : (PAIR ? 32 : DV);
+  const int rk = RAG ? p.RK : dk, rv = RAG ? p.RV : dv;  // row lengths in memory
   constexpr int QROWB = DK * 2, GROWB = DV * 2;
   constexpr int QCH = QROWB / 16, GCH = GROWB / 16;
   constexpr int QI = 32 * QCH / 64, GI = 32 * GCH / 64;
@@ -1595,7 +1687,7 @@ __global__ __launch_bounds__(kThreads, (FBLA_BWDA_OCC3 && FUSED && !DEN && !LO) 
       return (row0 + 2 * (int64_t)tok) * 32 + ch * 8;
     } else {
       if (tok >= t_end || (PAD && ch * 8 >= rowlen)) return -1;
-      return (row0 + (int64_t)tok * rstride) * rowlen + ch * 8;
+      return (row0 + (int64_t)tok * rstride) * rowlen + (RAG ? ragged_first(ch, rowlen) : ch * 8);
     }
   };
 
@@ -1630,39 +1722,48 @@ __global__ __launch_bounds__(kThreads, (FBLA_BWDA_OCC3 && FUSED && !DEN && !LO) 
 #pragma unroll
     for (int i = 0; i < QI; ++i) {
       const int q = lane + 64 * i, row = q / QCH, ch = q % QCH;
-      const int64_t off = piece(tok0 + row, ch, dk);
-      dst[i] = off >= 0 ? load_stream<u32x4, kNtPassALoad>(src + off) : u32x4{0u, 0u, 0u, 0u};
+      const int64_t off = piece(tok0 + row, ch, rk);
+      dst[i] = u32x4{0u, 0u, 0u, 0u};
+      if (off >= 0) dst[i] = load_stream<std::conditional_t<RAG, u32x4_any, u32x4>, kNtPassALoad>(src + off);
     }
   };
   auto load_g = [&](u32x4(&dst)[GI], const T* src, int tok0) {
 #pragma unroll
     for (int i = 0; i < GI; ++i) {
       const int q = lane + 64 * i, row = q / GCH, ch = q % GCH;
-      const int64_t off = piece(tok0 + row, ch, dv);
-      dst[i] = off >= 0 ? load_stream<u32x4, kNtPassALoad>(src + off) : u32x4{0u, 0u, 0u, 0u};
+      const int64_t off = piece(tok0 + row, ch, rv);
+      dst[i] = u32x4{0u, 0u, 0u, 0u};
+      if (off >= 0) dst[i] = load_stream<std::conditional_t<RAG, u32x4_any, u32x4>, kNtPassALoad>(src + off);
     }
   };
   auto stash_q = [&](const u32x4(&src)[QI], unsigned char* dstb) {
 #pragma unroll
     for (int i = 0; i < QI; ++i) {
       const int q = lane + 64 * i;
-      *reinterpret_cast<u32x4*>(dstb + swz<QROWB>(q / QCH, q % QCH)) = src[i];
+      *reinterpret_cast<u32x4*>(dstb + swz<QROWB>(q / QCH, q % QCH)) =
+          RAG ? ragged_in(src[i], ragged_shift(q % QCH, rk) & 7) : src[i];
     }
   };
   auto stash_g = [&](const u32x4(&src)[GI], unsigned char* dstb) {
 #pragma unroll
     for (int i = 0; i < GI; ++i) {
       const int q = lane + 64 * i;
-      *reinterpret_cast<u32x4*>(dstb + swz<GROWB>(q / GCH, q % GCH)) = src[i];
+      *reinterpret_cast<u32x4*>(dstb + swz<GROWB>(q / GCH, q % GCH)) =
+          RAG ? ragged_in(src[i], ragged_shift(q % GCH, rv) & 7) : src[i];
     }
   };
   auto store_q = [&](const unsigned char* srcb, T* dst, int tok0) {
 #pragma unroll
     for (int i = 0; i < QI; ++i) {
       const int q = lane + 64 * i, row = q / QCH, ch = q % QCH;
-      const int64_t off = piece(tok0 + row, ch, dk);
-      if (off >= 0)
-        store_row16<kNtPassAStore>(dst + off, *reinterpret_cast<const u32x4*>(srcb + swz<QROWB>(row, ch)));
+      const int64_t off = piece(tok0 + row, ch, rk);
+      const u32x4 w = *reinterpret_cast<const u32x4*>(srcb + swz<QROWB>(row, ch));
+      if constexpr (RAG) {
+        const u32x4 prev = *reinterpret_cast<const u32x4*>(srcb + swz<QROWB>(row, ch > 0 ? ch - 1 : 0));
+        if (off >= 0) *reinterpret_cast<u32x4_any*>(dst + off) = ragged_out(prev, w, ragged_shift(ch, rk));
+      } else if (off >= 0) {
+        store_row16<kNtPassAStore>(dst + off, w);
+      }
     }
   };
   // Whole tiles of plain rows: a wave-uniform tile address plus one constant byte offset per
@@ -1995,7 +2096,7 @@ struct BwdA128Layout {
   static_assert(2 * kTotal <= 160 * 1024, "two workgroups per CU");
 };
 
-template <typename T, bool NORM, bool PAD>
+template <typename T, bool NORM, int PAD>
 __global__ __launch_bounds__(256, 2) void bwd_a128_kernel(
     Prob p, const T* __restrict__ qn, const T* __restrict__ dout, const float* __restrict__ S,
     const float* __restrict__ km, T* __restrict__ dqn, float* __restrict__ partial, float* fin_mat,
@@ -2003,7 +2104,9 @@ __global__ __launch_bounds__(256, 2) void bwd_a128_kernel(
   using LY = BwdA128Layout;
   constexpr bool LO = !std::is_same<T, _Float16>::value;  // see launch_bwd_a
   constexpr int KS = 8, ROWB = 256, NT = 256;
+  constexpr bool RAG = PAD == 2;
   const int dk = PAD ? p.DK : 128, dv = PAD ? p.DV : 128;
+  const int rk = RAG ? p.RK : dk, rv = RAG ? p.RV : dv;  // row lengths in memory
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
 
   const int wg_item = packed_item(p, blockIdx.x, p.H * nchunks);
@@ -2044,10 +2147,12 @@ __global__ __launch_bounds__(256, 2) void bwd_a128_kernel(
   // address plus a uniform i-th distance plus the lane's one constant byte offset (32 bits: the
   // host keeps packed tensors with more than 65536 heads away from this kernel).
   const int prow = tid >> 4, pch = tid & 15;
-  const uint32_t qrow_b = (uint32_t)rstride * (uint32_t)dk * 2u, grow_b = (uint32_t)rstride * (uint32_t)dv * 2u;
-  const uint32_t qvoff = (uint32_t)prow * qrow_b + (uint32_t)pch * 16u;
-  const uint32_t gvoff = PAD ? (uint32_t)prow * grow_b + (uint32_t)pch * 16u : qvoff;
-  const bool q_piece = !PAD || pch * 8 < dk, g_piece = !PAD || pch * 8 < dv;  // the chunk exists in a row
+  const uint32_t qrow_b = (uint32_t)rstride * (uint32_t)rk * 2u, grow_b = (uint32_t)rstride * (uint32_t)rv * 2u;
+  const uint32_t qvoff = (uint32_t)prow * qrow_b + (RAG ? 2u * (uint32_t)ragged_first(pch, rk) : (uint32_t)pch * 16u);
+  const uint32_t gvoff = PAD ? (uint32_t)prow * grow_b + (RAG ? 2u * (uint32_t)ragged_first(pch, rv) : (uint32_t)pch * 16u)
+                             : qvoff;
+  const bool q_piece = !PAD || pch * 8 < rk, g_piece = !PAD || pch * 8 < rv;  // the chunk exists in a row
+  const int qback = RAG && q_piece ? ragged_shift(pch, rk) : 0, gback = RAG && g_piece ? ragged_shift(pch, rv) : 0;
   auto step_ptr = [&](const void* src, int tok0, int rowlen) -> const char* {
     return reinterpret_cast<const char*>(src) + ((row0 + (int64_t)tok0 * rstride) * rowlen) * (int64_t)sizeof(T);
   };
@@ -2057,12 +2162,14 @@ __global__ __launch_bounds__(256, 2) void bwd_a128_kernel(
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       dst[i] = u32x4{0u, 0u, 0u, 0u};
-      if (has && prow + 16 * i < rows) dst[i] = load_stream<u32x4, kNtPassALoad>(tp + (size_t)(16 * i) * row_b + voff);
+      if (has && prow + 16 * i < rows)
+        dst[i] = load_stream<std::conditional_t<RAG, u32x4_any, u32x4>, kNtPassALoad>(tp + (size_t)(16 * i) * row_b + voff);
     }
   };
-  auto stash_step = [&](const u32x4(&src)[4], unsigned char* tiles) {
+  auto stash_step = [&](const u32x4(&src)[4], unsigned char* tiles, int back) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) *reinterpret_cast<u32x4*>(tiles + swz<ROWB>(prow + 16 * i, pch)) = src[i];
+    for (int i = 0; i < 4; ++i)
+      *reinterpret_cast<u32x4*>(tiles + swz<ROWB>(prow + 16 * i, pch)) = RAG ? ragged_in(src[i], back) : src[i];
   };
 
   f32x16 acc[2][2];
@@ -2075,8 +2182,8 @@ __global__ __launch_bounds__(256, 2) void bwd_a128_kernel(
   float dkm = 0.f;  // row 64 bk + 32 bv + ntok, this half-wave's tokens
 
   u32x4 rq[4], rg[4];
-  load_step(rq, qn, t_begin, dk, qrow_b, qvoff, q_piece);
-  load_step(rg, dout, t_begin, dv, grow_b, gvoff, g_piece);
+  load_step(rq, qn, t_begin, rk, qrow_b, qvoff, q_piece);
+  load_step(rg, dout, t_begin, rv, grow_b, gvoff, g_piece);
 
   // g_t = dO_t S^T: contraction over dv, M(r = dv, c = dk) = S[c][r]
   const float denorm = build_operand<T, 128, 128, NT, PAD>(smem, lds_max, S + (int64_t)nh * dk * dv, 1, dv, 1, 0,
@@ -2114,8 +2221,8 @@ __global__ __launch_bounds__(256, 2) void bwd_a128_kernel(
   const int kpos = (ntok & 16) | ((ntok & 2) << 2) | ((ntok & 1) << 2) | ((ntok >> 2) & 3);
 
   for (int base = t_begin; base < t_end; base += 64) {
-    stash_step(rq, qtile);
-    stash_step(rg, gtile);
+    stash_step(rq, qtile, qback);
+    stash_step(rg, gtile, gback);
     __syncthreads();
 
     // ---- token view: this lane gets columns 64 kb + 16 blk + 0..15 of token ntok of both tiles
@@ -2133,8 +2240,8 @@ __global__ __launch_bounds__(256, 2) void bwd_a128_kernel(
     }
     // the next step's rows are requested here, not at the top of the step: their 32 registers are
     // then free during the token view, whose LDS reads need buffers to be in flight ahead of the products
-    load_step(rq, qn, base + 64, dk, qrow_b, qvoff, q_piece);
-    load_step(rg, dout, base + 64, dv, grow_b, gvoff, g_piece);
+    load_step(rq, qn, base + 64, rk, qrow_b, qvoff, q_piece);
+    load_step(rg, dout, base + 64, rv, grow_b, gvoff, g_piece);
     float rz[2] = {1.f, 1.f}, dz[2] = {0.f, 0.f};
     if constexpr (NORM) {
 #pragma unroll
@@ -2225,13 +2332,20 @@ __global__ __launch_bounds__(256, 2) void bwd_a128_kernel(
     __syncthreads();  // dq rows, dO / z and dz are complete
 
     {
-      char* tp = const_cast<char*>(step_ptr(dqn, base, dk));
+      char* tp = const_cast<char*>(step_ptr(dqn, base, rk));
       const int rows = t_end - base;
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        if (q_piece && prow + 16 * i < rows)
-          store_row16<kNtPassAStore>(tp + (size_t)(16 * i) * qrow_b + qvoff,
-                                     *reinterpret_cast<const u32x4*>(dqtile + swz<ROWB>(prow + 16 * i, pch)));
+        if (q_piece && prow + 16 * i < rows) {
+          const u32x4 w = *reinterpret_cast<const u32x4*>(dqtile + swz<ROWB>(prow + 16 * i, pch));
+          char* at = tp + (size_t)(16 * i) * qrow_b + qvoff;
+          if constexpr (RAG) {
+            const u32x4 prev = *reinterpret_cast<const u32x4*>(dqtile + swz<ROWB>(prow + 16 * i, pch > 0 ? pch - 1 : 0));
+            *reinterpret_cast<u32x4_any*>(at) = ragged_out(prev, w, qback);
+          } else {
+            store_row16<kNtPassAStore>(at, w);
+          }
+        }
     }
 
     // ---- feature view: dS block (bk, bv) += q~^T (dO / z) over both tiles
@@ -2295,12 +2409,13 @@ __global__ __launch_bounds__(256, 2) void bwd_a128_kernel(
 // The kernels tile a head into 64-wide blocks: a head dim runs as the next of 64 / 128 above
 // it, the padded variants (PAD) when it is not one of the two.
 static int tiled_dim(int d) { return d <= 64 ? 64 : 128; }
+static bool ragged(const Prob& p) { return p.RK > 0; }  // (the plan sets both row lengths)
 static bool padded(const Prob& p) { return p.DK != tiled_dim(p.DK) || p.DV != tiled_dim(p.DV); }
 
 // Dense tensors with 32 x 32 heads: the row-parallel kernels take two tokens per 64-wide row
 // (PAIR variants) instead of padding every row to 64.
 bool pair_mode(const Prob& p, int dtype) {
-  return (dtype == kF16 || dtype == kBF16) && !p.cu && p.DK == 32 && p.DV == 32;
+  return (dtype == kF16 || dtype == kBF16) && !p.cu && !ragged(p) && p.DK == 32 && p.DV == 32;
 }
 
 // 16-bit inputs with head dims that are multiples of 8 (16-byte row pieces) up to 128.
@@ -2468,7 +2583,7 @@ template <typename K> static int reserve_lds(K kernel, int bytes, bool& done) {
   return kOk;
 }
 
-template <typename T, int DK, int DV, bool PAD>
+template <typename T, int DK, int DV, int PAD>
 static void launch_state(const Prob& p, const T* kn, const T* v, const T* kd, float* partial,
                          const float* tokscal, int64_t total_rows, float* fm, float* fv, int chunk,
                          int nchunks, BlockStats bs, hipStream_t st) {
@@ -2494,6 +2609,10 @@ static void launch_state(const Prob& p, const T* kn, const T* v, const T* kd, fl
       return;
     }
   }
+  if constexpr (PAD == 2) {  // (the plan has checked: plain operator)
+    state_kernel<T, DK, DV, false, TL, false, false, PAD><<<grid, block, 0, st>>>(p, kn, v, kd, partial, nullptr, 0, fm, fv, chunk, nchunks, bs);
+    return;
+  } else {
   if (p.flags & kElu1) {  // (the plan has checked: 64 x 64, plain operator)
     if constexpr (DK == 64 && DV == 64 && !PAD)
       state_kernel<T, 64, 64, false, 1, false, false, false, true><<<grid, block, 0, st>>>(p, kn, v, kd, partial, nullptr, 0, fm, fv, chunk, nchunks, bs);
@@ -2508,9 +2627,10 @@ static void launch_state(const Prob& p, const T* kn, const T* v, const T* kd, fl
     state_kernel<T, DK, DV, true, TL, false, false, PAD><<<grid, block, 0, st>>>(p, kn, v, kd, partial, nullptr, 0, fm, fv, chunk, nchunks, bs);
   else
     state_kernel<T, DK, DV, false, TL, false, false, PAD><<<grid, block, 0, st>>>(p, kn, v, kd, partial, nullptr, 0, fm, fv, chunk, nchunks, bs);
+  }
 }
 
-template <typename T, bool PAD>
+template <typename T, int PAD>
 static void run_state_dims(const Prob& p, const T* a, const T* b, const T* c, float* partial,
                            const float* ts, int64_t rows, float* fm, float* fv, int chunk, int nchunks,
                            BlockStats bs, hipStream_t st) {
@@ -2526,11 +2646,12 @@ static void run_state(const Prob& p, const void* kn, const void* v, const void* 
                       const float* ts, int64_t rows, float* fm, float* fv, int chunk, int nchunks,
                       BlockStats bs, hipStream_t st) {
   const T *a = (const T*)kn, *b = (const T*)v, *c = (const T*)kd;
-  if (padded(p)) run_state_dims<T, true>(p, a, b, c, partial, ts, rows, fm, fv, chunk, nchunks, bs, st);
-  else run_state_dims<T, false>(p, a, b, c, partial, ts, rows, fm, fv, chunk, nchunks, bs, st);
+  if (ragged(p)) run_state_dims<T, 2>(p, a, b, c, partial, ts, rows, fm, fv, chunk, nchunks, bs, st);
+  else if (padded(p)) run_state_dims<T, 1>(p, a, b, c, partial, ts, rows, fm, fv, chunk, nchunks, bs, st);
+  else run_state_dims<T, 0>(p, a, b, c, partial, ts, rows, fm, fv, chunk, nchunks, bs, st);
 }
 
-template <typename T, int DR, int DC, bool NORM, bool DEN, int WAVES, bool PAD, bool PAIR = false, bool FMAP = false,
+template <typename T, int DR, int DC, bool NORM, bool DEN, int WAVES, int PAD, bool PAIR = false, bool FMAP = false,
           bool GATE = false>
 static int launch_rows_k(const Prob& p, const RowsJob& job, const RowsJob* job2, int chunk,
                          int nchunks, int dr, int dc, hipStream_t st) {
@@ -2546,7 +2667,7 @@ static int launch_rows_k(const Prob& p, const RowsJob& job, const RowsJob* job2,
   return kOk;
 }
 
-template <typename T, bool NORM, bool PAD>
+template <typename T, bool NORM, int PAD>
 static int launch_rows128(const Prob& p, const RowsJob& job, const RowsJob* job2, int chunk, int nchunks, int dr,
                           int dc, hipStream_t st) {
   auto kernel = rows128_kernel<T, NORM, PAD>;
@@ -2566,7 +2687,7 @@ static bool use_rows128(const Prob& p) {
   return on == 1 && !(p.flags & kDecoupled) && !(p.cu && p.H > 65536);
 }
 
-template <typename T, int DR, int DC, bool PAD>
+template <typename T, int DR, int DC, int PAD>
 static int launch_rows(const Prob& p, const RowsJob& job, const RowsJob* job2, int dr, int dc,
                        hipStream_t st) {
   // 128 x 128 operands fill 64 KiB of LDS: one 8-wave workgroup per CU instead of
@@ -2594,8 +2715,9 @@ static int launch_rows(const Prob& p, const RowsJob& job, const RowsJob* job2, i
     }
   }
   if (!norm) return launch_rows_k<T, DR, DC, false, false, WAVES, PAD>(p, job, job2, chunk, nchunks, dr, dc, st);
-  if (!den) return launch_rows_k<T, DR, DC, true, false, WAVES, PAD>(p, job, job2, chunk, nchunks, dr, dc, st);
-  return launch_rows_k<T, DR, DC, true, true, WAVES, PAD>(p, job, job2, chunk, nchunks, dr, dc, st);
+  if (!den || PAD == 2) return launch_rows_k<T, DR, DC, true, false, WAVES, PAD>(p, job, job2, chunk, nchunks, dr, dc, st);
+  if constexpr (PAD != 2) return launch_rows_k<T, DR, DC, true, true, WAVES, PAD>(p, job, job2, chunk, nchunks, dr, dc, st);
+  return kErrUnsupported;  // (not reached)
 }
 
 // two tokens per row: chunks are counted in row pairs
@@ -2612,7 +2734,7 @@ static int launch_rows_pair(const Prob& p, const RowsJob& job, const RowsJob* jo
   return launch_rows_k<T, 64, 64, true, true, 4, false, true>(p, job, job2, chunk, nchunks, 32, 32, st);
 }
 
-template <typename T, bool PAD>
+template <typename T, int PAD>
 static int run_rows_dims(const Prob& p, const RowsJob& job, const RowsJob* job2, int dr, int dc,
                          hipStream_t st) {
   const int DR = tiled_dim(dr), DC = tiled_dim(dc);
@@ -2626,8 +2748,9 @@ template <typename T>
 static int run_rows(const Prob& p, const RowsJob& job, const RowsJob* job2, int dr, int dc,
                     hipStream_t st) {
   if (pair_mode(p, kF16) && job.pnchunks == 0) return launch_rows_pair<T>(p, job, job2, st);
-  if (padded(p)) return run_rows_dims<T, true>(p, job, job2, dr, dc, st);
-  return run_rows_dims<T, false>(p, job, job2, dr, dc, st);
+  if (ragged(p)) return run_rows_dims<T, 2>(p, job, job2, dr, dc, st);
+  if (padded(p)) return run_rows_dims<T, 1>(p, job, job2, dr, dc, st);
+  return run_rows_dims<T, 0>(p, job, job2, dr, dc, st);
 }
 
 // Packed batches, which kernels keep the workgroups of a sequence on one XCD (packed_item):
@@ -2722,7 +2845,7 @@ int rows2(const Prob& p_, int dtype, const RowsJob& job0, const RowsJob& job1, i
   return run_rows<__bf16>(p, job0, &job1, DR, DC, st);
 }
 
-template <typename T, int DK, int DV, bool NORM, bool DEN, bool FUSED, bool PAD, bool PAIR = false, bool GATE = false,
+template <typename T, int DK, int DV, bool NORM, bool DEN, bool FUSED, int PAD, bool PAIR = false, bool GATE = false,
           bool FMAP = false>
 static int launch_bwd_a(const Prob& p, const T* qn, const T* qd, const T* dout, const float* S,
                         const float* km, T* dqn, T* dqd, float* partial, float* tokscal,
@@ -2749,7 +2872,7 @@ static int launch_bwd_a(const Prob& p, const T* qn, const T* qd, const T* dout, 
   return kOk;
 }
 
-template <typename T, bool NORM, bool PAD>
+template <typename T, bool NORM, int PAD>
 static int launch_bwd_a128(const Prob& p, const T* q, const T* dout, const float* S, const float* km, T* dq,
                            float* partial, float* fm, float* fv, int chunk, int nchunks, hipStream_t st) {
   using LY = BwdA128Layout;
@@ -2762,7 +2885,7 @@ static int launch_bwd_a128(const Prob& p, const T* q, const T* dout, const float
   return kOk;
 }
 
-template <typename T, bool PAD, bool PAIR = false>
+template <typename T, int PAD, bool PAIR = false>
 static int run_bwd_a_pad(const Prob& p, const void* qn, const void* qd, const void* dout, const float* S,
                          const float* km, void* dqn, void* dqd, float* partial, float* fm, float* fv,
                          int chunk, int nchunks, hipStream_t st) {
@@ -2789,8 +2912,9 @@ static int run_bwd_a_pad(const Prob& p, const void* qn, const void* qd, const vo
   }
   if (!(p.flags & kNormalize))
     return launch_bwd_a<T, 64, 64, false, false, true, PAD, PAIR>(p, a, b, c, S, km, x, y, partial, nullptr, 0, fm, fv, chunk, nchunks, st);
-  if (p.flags & kDecoupled)
-    return launch_bwd_a<T, 64, 64, true, true, true, PAD, PAIR>(p, a, b, c, S, km, x, y, partial, nullptr, 0, fm, fv, chunk, nchunks, st);
+  if constexpr (PAD != 2)
+    if (p.flags & kDecoupled)
+      return launch_bwd_a<T, 64, 64, true, true, true, PAD, PAIR>(p, a, b, c, S, km, x, y, partial, nullptr, 0, fm, fv, chunk, nchunks, st);
   return launch_bwd_a<T, 64, 64, true, false, true, PAD, PAIR>(p, a, b, c, S, km, x, y, partial, nullptr, 0, fm, fv, chunk, nchunks, st);
 }
 
@@ -2800,9 +2924,10 @@ static int run_bwd_a(const Prob& p, const void* qn, const void* qd, const void* 
                      int chunk, int nchunks, hipStream_t st) {
   // pair mode: the chunk (a multiple of 128 tokens) becomes a count of row pairs
   if (pair_mode(p, kF16))
-    return run_bwd_a_pad<T, false, true>(p, qn, qd, dout, S, km, dqn, dqd, partial, fm, fv, chunk / 2, nchunks, st);
-  if (padded(p) || tiled_dim(p.DK) != tiled_dim(p.DV)) return run_bwd_a_pad<T, true>(p, qn, qd, dout, S, km, dqn, dqd, partial, fm, fv, chunk, nchunks, st);
-  return run_bwd_a_pad<T, false>(p, qn, qd, dout, S, km, dqn, dqd, partial, fm, fv, chunk, nchunks, st);
+    return run_bwd_a_pad<T, 0, true>(p, qn, qd, dout, S, km, dqn, dqd, partial, fm, fv, chunk / 2, nchunks, st);
+  if (ragged(p)) return run_bwd_a_pad<T, 2>(p, qn, qd, dout, S, km, dqn, dqd, partial, fm, fv, chunk, nchunks, st);
+  if (padded(p) || tiled_dim(p.DK) != tiled_dim(p.DV)) return run_bwd_a_pad<T, 1>(p, qn, qd, dout, S, km, dqn, dqd, partial, fm, fv, chunk, nchunks, st);
+  return run_bwd_a_pad<T, 0>(p, qn, qd, dout, S, km, dqn, dqd, partial, fm, fv, chunk, nchunks, st);
 }
 
 int bwd_a(const Prob& p_, int dtype, const void* qn, const void* qd, const void* dout, const float* S,
@@ -2814,7 +2939,7 @@ int bwd_a(const Prob& p_, int dtype, const void* qn, const void* qd, const void*
   return run_bwd_a<__bf16>(p, qn, qd, dout, S, km, dqn, dqd, partial, fin_mat, fin_vec, chunk, nchunks, st);
 }
 
-template <typename T, int DK, int DV, bool PAD>
+template <typename T, int DK, int DV, int PAD>
 static int launch_bwd_tokens(const Prob& p, const void* qn, const void* qd, const void* dout, const float* S,
                              const float* km, void* dqn, void* dqd, float* tokscal, int64_t total_rows,
                              int chunk, int nchunks, hipStream_t st) {
@@ -2831,7 +2956,7 @@ static int launch_bwd_tokens(const Prob& p, const void* qn, const void* qd, cons
                                                            nchunks, st);
 }
 
-template <typename T, bool PAD>
+template <typename T, int PAD>
 static int run_bwd_tokens_dims(const Prob& p, const void* qn, const void* qd, const void* dout, const float* S,
                                const float* km, void* dqn, void* dqd, float* tokscal, int64_t total_rows,
                                int chunk, int nchunks, hipStream_t st) {
@@ -2854,8 +2979,8 @@ static int run_bwd_tokens(const Prob& p, const void* qn, const void* qd, const v
   const int chunk = chunk_for(p, big == 2 ? 1 : 2, 1, 512, 128, false);
   const int nchunks = (int)cdiv64(p.L, chunk);
   if (padded(p))
-    return run_bwd_tokens_dims<T, true>(p, qn, qd, dout, S, km, dqn, dqd, tokscal, total_rows, chunk, nchunks, st);
-  return run_bwd_tokens_dims<T, false>(p, qn, qd, dout, S, km, dqn, dqd, tokscal, total_rows, chunk, nchunks, st);
+    return run_bwd_tokens_dims<T, 1>(p, qn, qd, dout, S, km, dqn, dqd, tokscal, total_rows, chunk, nchunks, st);
+  return run_bwd_tokens_dims<T, 0>(p, qn, qd, dout, S, km, dqn, dqd, tokscal, total_rows, chunk, nchunks, st);
 }
 
 // token view of the backward alone: dq and the per-row scalars 1/z_t, dz_t

@@ -1088,7 +1088,7 @@ int select_blocks(const float* qc, const float* kc, const float* bias, int32_t* 
 }
 
 static Prob dense_prob(int64_t BH, int64_t T, int K, int V) {
-  Prob p;
+  Prob p{};
   p.cu = nullptr;
   p.perm = nullptr;
   p.chunk_base = nullptr;

@@ -217,3 +217,34 @@ def test_head_dims_between_row_lengths_are_widened(variant, DK, DV, dtype):
     need = _hip.lib().fbla_la_workspace_bytes(0, B, H, L, DK, DV, code, flags)
     if widened:
         assert need >= 3 * B * H * L * min(DK, DV) * (4 if dtype == torch.float32 else 2)
+
+
+# rows that are no whole number of 16-byte pieces: every remainder of 8 on both sides of the 64-wide tile, odd and even,
+# the last element alone in its block (65), mixed tiles, one side whole
+RAGGED_DIMS = [(9, 15), (63, 57), (58, 60), (65, 67), (100, 121), (127, 126), (66, 35), (12, 113), (64, 101), (89, 128)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("dims", RAGGED_DIMS)
+def test_rows_of_any_length_dense(dims, dtype):
+    for i, L in enumerate((1, 15, 63, 257, 1301)):
+        _check_dense("linear" if i % 2 == 0 else "simple", 2, 3, L, dims[0], dims[1], dtype, 50 * i + dims[0])
+
+
+@pytest.mark.parametrize("dims", RAGGED_DIMS)
+def test_rows_of_any_length_packed_and_cross(dims):
+    from flash_bla.ops.linear_attn.fused import linear_attention
+    test_packed(dims, torch.bfloat16 if dims[0] % 2 else torch.float16)
+    dtype, (lq, lk), (DK, DV) = torch.bfloat16, (70, 333), dims
+    q, _, _, do = make_qkv((2, 2, lq, DK), (2, 2, lq, DV), dtype, DK)
+    k, _, v, _ = make_qkv((2, 2, lk, DK), (2, 2, lk, DV), dtype, DV)
+    leaves = [t.cuda().requires_grad_() for t in (q, k, v)]
+    o = linear_attention(*leaves)
+    o.backward(do.cuda())
+    ref = [t.double().requires_grad_() for t in (q, k, v)]
+    z = ref[0] @ ref[1].mean(-2, keepdim=True).transpose(-1, -2) + 1e-6
+    want = (ref[0] @ (ref[1].transpose(-1, -2) @ ref[2] / lk)) / z
+    want.backward(do.double())
+    assert_parity(o, want.detach().numpy(), dtype, f"o {dims}")
+    for name, a, b in zip(("dq", "dk", "dv"), leaves, ref):
+        assert_parity(a.grad, b.grad.numpy(), dtype, f"{name} {dims}")
