@@ -753,4 +753,44 @@ int fbla_dwconv_grad(const void* x, int64_t x_batch, int64_t x_row, const void* 
   return check_launch(what);
 }
 
+static int check_linear(const char* what, int64_t tokens, int M, int N, int dtype) {
+  if (tokens < 1 || M < 1 || N < 1 || (dtype != kF16 && dtype != kBF16 && dtype != kF32)) {
+    set_error("%s: bad sizes or dtype (tokens=%lld M=%d N=%d dtype=%d)", what, (long long)tokens, M, N, dtype);
+    return kErrBadArg;
+  }
+  // the bound on the product keeps the result's indexes in 31 bits, the one on the tokens the chunks' lengths
+  if (dtype == kF32 || M % 8 || N % 8 || (int64_t)M * N > (1 << 28) || tokens > (1LL << 30)) {
+    set_error("%s: needs 16-bit elements, rows of whole 16-byte pieces and at most 2^28 weights and 2^30 tokens "
+              "(tokens=%lld M=%d N=%d dtype=%d)", what, (long long)tokens, M, N, dtype);
+    return kErrUnsupported;
+  }
+  return kOk;
+}
+
+size_t fbla_linear_wgrad_workspace_bytes(int64_t tokens, int M, int N, int dtype) {
+  if (check_linear("fbla_linear_wgrad_workspace_bytes", tokens, M, N, dtype) != kOk) return 0;
+  return linear::wgrad_workspace_bytes(tokens, M, N);
+}
+
+int fbla_linear_wgrad(const void* g, int64_t g_row, const void* x, int64_t x_row, void* dw, void* db, void* workspace,
+                      size_t workspace_bytes, int64_t tokens, int M, int N, int dtype, void* stream) {
+  const char* what = "fbla_linear_wgrad";
+  const int rc = check_linear(what, tokens, M, N, dtype);
+  if (rc != kOk) return rc;
+  if (!g || !x || !dw) {
+    set_error("%s: null tensor pointer", what);
+    return kErrBadArg;
+  }
+  if (check_aligned(what, {g, x, workspace}) != kOk || check_row_strides(what, M, dtype, {g_row}) != kOk ||
+      check_row_strides(what, N, dtype, {x_row}) != kOk)
+    return kErrBadArg;
+  const size_t need = linear::wgrad_workspace_bytes(tokens, M, N);
+  if (!workspace || workspace_bytes < need) {
+    set_error("%s: workspace too small (%zu < %zu bytes)", what, workspace_bytes, need);
+    return kErrWorkspace;
+  }
+  linear::wgrad(g, g_row, x, x_row, tokens, M, N, dw, db, (float*)workspace, dtype, (hipStream_t)stream);
+  return check_launch(what);
+}
+
 }  // extern "C"

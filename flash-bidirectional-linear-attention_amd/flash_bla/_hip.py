@@ -52,6 +52,8 @@ _SIGNATURES = {
     "fbla_dwconv_fwd": (_i32, [_vp, _i64, _i64, _vp, _vp, _vp] + [_i64] * 5 + [_i32] * 5 + [_vp]),
     "fbla_dwconv_grad_workspace_bytes": (_sz, [_i64] * 3 + [_i32] * 4),
     "fbla_dwconv_grad": (_i32, [_vp, _i64, _i64, _vp, _i64, _i64, _vp, _vp, _vp, _sz] + [_i64] * 3 + [_i32] * 4 + [_vp]),
+    "fbla_linear_wgrad_workspace_bytes": (_sz, [_i64] + [_i32] * 3),
+    "fbla_linear_wgrad": (_i32, [_vp, _i64, _vp, _i64, _vp, _vp, _vp, _sz, _i64] + [_i32] * 3 + [_vp]),
 }
 
 
@@ -456,4 +458,32 @@ def dwconv_grad(x, g, w, H, W, with_bias):
         rc = L.fbla_dwconv_grad(_ptr(x), x_batch, x_row, _ptr(g), g_batch, g_row, _ptr(dw), _ptr(db), _ptr(ws),
                                 ws.numel(), B, H, W, C, Cw, K, code, _stream(x.device))
     _check(rc, "fbla_dwconv_grad")
+    return dw, db
+
+
+def _token_rows(t):
+    """(tensor, row stride) of t [..., C] as rows the projection kernels can read in place: channels adjacent, whole
+    16-byte pieces between the rows; anything else is copied to contiguous memory."""
+    rows = t.reshape(-1, t.shape[-1])
+    if rows.stride(1) != 1 or rows.stride(0) % 8 or rows.stride(0) < rows.shape[1] or rows.data_ptr() % 16:
+        rows = rows.clone(memory_format=torch.contiguous_format)
+    return rows, rows.stride(0)
+
+
+def linear_wgrad(g, x, with_bias):
+    """(dw [M, N], db [M] or None) of y = x W^T + b from the output's gradient g [..., M] and x [..., N] (16-bit)."""
+    _require_gpu(g, x)
+    g, g_row = _token_rows(g)
+    x, x_row = _token_rows(x)
+    (T, M), N, code = g.shape, x.shape[1], dtype_code(x)
+    if x.shape[0] != T or g.dtype != x.dtype or g.device != x.device:
+        raise ValueError("linear_wgrad: g and x must agree in tokens, dtype and device")
+    L, dev = lib(), x.device
+    dw = torch.empty(M, N, dtype=x.dtype, device=dev)
+    db = torch.empty(M, dtype=x.dtype, device=dev) if with_bias else None
+    with _on(dev):
+        ws = _workspace(L.fbla_linear_wgrad_workspace_bytes(T, M, N, code), dev)
+        rc = L.fbla_linear_wgrad(_ptr(g), g_row, _ptr(x), x_row, _ptr(dw), _ptr(db), _ptr(ws), ws.numel(), T, M, N,
+                                 code, _stream(dev))
+    _check(rc, "fbla_linear_wgrad")
     return dw, db

@@ -6,6 +6,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from flash_bla.ops.depthwise import depthwise_conv_tokens
+from flash_bla.ops.projection import TokenLinear
 
 
 class PvtLinearAttentionBase(nn.Module):
@@ -13,9 +14,9 @@ class PvtLinearAttentionBase(nn.Module):
         assert dim % num_heads == 0, f"dim {dim} should be divided by num_heads {num_heads}."
         self.dim, self.num_heads, self.sr_ratio = dim, num_heads, sr_ratio
         head_dim = dim // num_heads
-        self.kv = nn.Linear(dim, dim * 2, bias=qkv_bias)
+        self.kv = TokenLinear(dim, dim * 2, bias=qkv_bias)
         self.attn_drop = nn.Dropout(attn_drop)
-        self.proj = nn.Linear(dim, dim)
+        self.proj = TokenLinear(dim, dim)
         self.proj_drop = nn.Dropout(proj_drop)
         if sr_ratio > 1:
             self.sr = nn.Conv2d(dim, dim, kernel_size=sr_ratio, stride=sr_ratio)

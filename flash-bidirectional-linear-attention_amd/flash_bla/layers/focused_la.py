@@ -6,6 +6,7 @@ import torch.nn.functional as F
 from flash_bla.layers._common import check_mode, merge_heads, split_heads, torch_linear_attention
 from flash_bla.layers._pvt import PvtLinearAttentionBase
 from flash_bla.ops.linear_attn.fused import linear_attention
+from flash_bla.ops.projection import TokenLinear
 
 
 class FocusedLinearAttention(PvtLinearAttentionBase):
@@ -13,7 +14,7 @@ class FocusedLinearAttention(PvtLinearAttentionBase):
                  sr_ratio=1, focusing_factor=3, kernel_size=5):
         super().__init__()
         self._init_common(dim, num_patches, num_heads, qkv_bias, attn_drop, proj_drop, sr_ratio, kernel_size)
-        self.q = nn.Linear(dim, dim, bias=qkv_bias)
+        self.q = TokenLinear(dim, dim, bias=qkv_bias)
         self.focusing_factor = focusing_factor
 
     def _focus(self, t, scale):

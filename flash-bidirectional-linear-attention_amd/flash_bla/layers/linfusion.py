@@ -13,6 +13,7 @@ import torch.nn.functional as F
 from flash_bla.layers._common import check_mode, torch_linear_attention
 from flash_bla.ops.linear_attn.fused import linear_attention
 from flash_bla.ops.linear_attn.varlen import varlen_linear_attention
+from flash_bla.ops.projection import TokenLinear
 
 
 _CU_CACHE = {}
@@ -34,8 +35,8 @@ def get_none_linear_projection(query_dim, mid_dim=None):
     if mid_dim == -1:
         return nn.Identity()
     width = mid_dim or query_dim
-    return nn.Sequential(nn.Linear(query_dim, width), nn.LayerNorm(width), nn.LeakyReLU(inplace=True),
-                         nn.Linear(width, query_dim))
+    return nn.Sequential(TokenLinear(query_dim, width), nn.LayerNorm(width), nn.LeakyReLU(inplace=True),
+                         TokenLinear(width, query_dim))
 
 
 class GeneralizedLinearAttention(nn.Module):
@@ -44,10 +45,10 @@ class GeneralizedLinearAttention(nn.Module):
         super().__init__()
         inner = out_dim if out_dim is not None else dim_head * heads
         self.heads = out_dim // dim_head if out_dim is not None else heads
-        self.to_q = nn.Linear(query_dim, inner, bias=bias)
-        self.to_k = nn.Linear(query_dim, inner, bias=bias)
-        self.to_v = nn.Linear(query_dim, inner, bias=bias)
-        self.to_out = nn.ModuleList([nn.Linear(inner, out_dim or query_dim, bias=out_bias), nn.Dropout(dropout)])
+        self.to_q = TokenLinear(query_dim, inner, bias=bias)
+        self.to_k = TokenLinear(query_dim, inner, bias=bias)
+        self.to_v = TokenLinear(query_dim, inner, bias=bias)
+        self.to_out = nn.ModuleList([TokenLinear(inner, out_dim or query_dim, bias=out_bias), nn.Dropout(dropout)])
         self.add_non_linear_model(projection_mid_dim)
 
     def add_non_linear_model(self, mid_dim=None):

@@ -7,6 +7,7 @@ from flash_bla.layers._common import check_mode, merge_heads, split_heads, torch
 from flash_bla.ops.depthwise import depthwise_conv_tokens
 from flash_bla.ops.feature_map import elu_plus_one
 from flash_bla.ops.linear_attn.decoupled import decoupled_la
+from flash_bla.ops.projection import TokenLinear
 
 
 class RoPE(nn.Module):
@@ -32,7 +33,7 @@ class MambaLikeLinearAttention(nn.Module):
     def __init__(self, dim, input_resolution, num_heads, qkv_bias=True, **kwargs):
         super().__init__()
         self.dim, self.input_resolution, self.num_heads = dim, input_resolution, num_heads
-        self.qk = nn.Linear(dim, dim * 2, bias=qkv_bias)
+        self.qk = TokenLinear(dim, dim * 2, bias=qkv_bias)
         self.elu = nn.ELU()
         self.lepe = nn.Conv2d(dim, dim, 3, padding=1, groups=dim)
         self.rope = RoPE(shape=(input_resolution[0], input_resolution[1], dim))

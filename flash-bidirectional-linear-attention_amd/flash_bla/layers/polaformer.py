@@ -9,6 +9,7 @@ import torch.nn.functional as F
 from flash_bla.layers._common import check_mode, merge_heads, split_heads, torch_linear_attention
 from flash_bla.layers._pvt import PvtLinearAttentionBase
 from flash_bla.ops.linear_attn.paired import paired_linear_attention
+from flash_bla.ops.projection import TokenLinear
 
 
 class PolaLinearAttention(PvtLinearAttentionBase):
@@ -17,7 +18,7 @@ class PolaLinearAttention(PvtLinearAttentionBase):
         super().__init__()
         self.head_dim = self._init_common(dim, num_patches, num_heads, qkv_bias, attn_drop, proj_drop, sr_ratio,
                                           kernel_size)
-        self.qg = nn.Linear(dim, 2 * dim, bias=qkv_bias)
+        self.qg = TokenLinear(dim, 2 * dim, bias=qkv_bias)
         self.power = nn.Parameter(torch.zeros(1, num_heads, 1, self.head_dim))
         self.alpha = alpha
 

@@ -7,6 +7,7 @@ from flash_bla.layers._common import check_mode, merge_heads, split_heads, torch
 from flash_bla.layers.mlla import RoPE
 from flash_bla.ops.depthwise import depthwise_conv_tokens
 from flash_bla.ops.linear_attn.decoupled import decoupled_la
+from flash_bla.ops.projection import TokenLinear
 
 
 class RALALinearAttention(nn.Module):
@@ -15,11 +16,11 @@ class RALALinearAttention(nn.Module):
         self.dim, self.input_resolution, self.num_heads = dim, input_resolution, num_heads
         self.head_dim = dim // num_heads
         self.scale = self.head_dim ** -0.5
-        self.qkvo = nn.Linear(dim, dim * 4, bias=qkv_bias)
+        self.qkvo = TokenLinear(dim, dim * 4, bias=qkv_bias)
         self.elu = nn.ELU()
         self.lepe = nn.Conv2d(dim, dim, 5, padding=2, groups=dim)
         self.rope = RoPE(shape=(input_resolution[0], input_resolution[1], self.head_dim))
-        self.proj = nn.Linear(dim, dim)
+        self.proj = TokenLinear(dim, dim)
 
     def forward(self, x, mode='triton'):
         fast = check_mode(mode)

@@ -1,0 +1,72 @@
+"""Weight and bias gradients of the blocks' projections against float64: results that end inside a 128 x 128 tile, token
+counts around a step of 64 and a chunk of 256, strided rows, an expanded gradient.  Bound: products of 16-bit values are
+exact in fp32, so a gradient is an fp32 sum of `tokens` terms, whose error stays below 2^-24 * sqrt(tokens) * 4 of the root
+mean square of its terms times tokens, and one rounding to the type."""
+import pytest
+import torch
+import torch.nn as nn
+
+from helpers import UNIT_ROUNDOFF
+from flash_bla.ops import projection
+from flash_bla.ops.projection import TokenLinear, runs_on_rows
+
+
+def _gradients(layer, x, g, x64=None):
+    y = layer(x)
+    y.backward(g)
+    return y, layer.weight.grad, None if layer.bias is None else layer.bias.grad
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("tokens,N,M,bias,layout", [
+    (1, 8, 8, True, "plain"), (63, 64, 136, True, "plain"), (64, 72, 128, False, "plain"), (257, 128, 120, True, "strided"),
+    (511, 256, 264, True, "expanded"), (4096 + 65, 64, 128, True, "strided"), (3000, 640, 640, False, "plain")])
+def test_weight_gradient(tokens, N, M, bias, layout, dtype, monkeypatch):
+    monkeypatch.setattr(projection, "splits_tokens", lambda *a: True)
+    torch.manual_seed(tokens)
+    layer = TokenLinear(N, M, bias=bias).cuda().to(dtype)
+    wide = torch.randn(1, tokens, 2 * N if layout == "strided" else N, device="cuda").to(dtype).requires_grad_()
+    x = wide[..., :N]
+    g = torch.randn(1, tokens, 3 * M if layout == "strided" else M, device="cuda").to(dtype)[..., -M:]
+    if layout == "expanded":
+        g = g[:, :1].expand(1, tokens, M)
+    assert runs_on_rows(x, layer.weight, layer.bias)
+    y, dw, db = _gradients(layer, x, g)
+    x64, g64 = x.detach().double().reshape(tokens, N), g.double().reshape(tokens, M)
+    slack = 2.0 ** -24 * 4 * tokens ** 0.5
+    u = UNIT_ROUNDOFF[dtype]
+    want = g64.t() @ x64
+    rms = (g64.square().t() @ x64.square() / tokens).sqrt()
+    assert ((dw.double() - want).abs() <= u * want.abs() + slack * rms * tokens ** 0.5 + 2.0 ** -24).all()
+    if bias:
+        want, rms = g64.sum(0), (g64.square().mean(0)).sqrt()
+        assert ((db.double() - want).abs() <= u * want.abs() + slack * rms * tokens ** 0.5 + 2.0 ** -24).all()
+    assert torch.equal(y, nn.functional.linear(x, layer.weight, layer.bias))
+    dx = wide.grad[..., :N]
+    assert torch.equal(dx, g @ layer.weight) and (layout != "strided" or wide.grad[..., N:].abs().max() == 0)
+
+
+@pytest.mark.gpu
+def test_gradient_of_the_gradient(monkeypatch):
+    monkeypatch.setattr(projection, "splits_tokens", lambda *a: True)
+    torch.manual_seed(0)
+    layer = TokenLinear(16, 8).cuda().half()
+    plain = nn.Linear(16, 8).cuda().half()
+    plain.load_state_dict(layer.state_dict())
+    results = []
+    for f in (layer, plain):
+        x = torch.linspace(-1, 1, 96, device="cuda").half().reshape(6, 16).requires_grad_()
+        dw, = torch.autograd.grad(f(x).square().sum(), f.weight, create_graph=True)
+        dw.square().sum().backward()
+        results.append((x.grad, f.weight.grad))
+    for a, b in zip(*results):
+        torch.testing.assert_close(a, b, rtol=2e-2, atol=2e-2 * b.abs().max().item())
+
+
+def test_other_calls_are_plain_linear():
+    layer = TokenLinear(16, 8)
+    x = torch.randn(3, 16)
+    assert not runs_on_rows(x, layer.weight, layer.bias)
+    assert torch.equal(layer(x), nn.functional.linear(x, layer.weight, layer.bias))
+    assert isinstance(layer, nn.Linear) and list(layer.state_dict()) == ["weight", "bias"]
