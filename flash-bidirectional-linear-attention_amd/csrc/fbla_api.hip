@@ -793,4 +793,139 @@ int fbla_linear_wgrad(const void* g, int64_t g_row, const void* x, int64_t x_row
   return check_launch(what);
 }
 
+static int check_blocks(const char* what, blocks::Shape& s, int64_t B, int64_t N, int64_t Nk, int heads, int d, int unit,
+                        int dtype) {
+  if (B < 1 || N < 1 || Nk < 1 || heads < 1 || d < 1 || (dtype != kF16 && dtype != kBF16 && dtype != kF32)) {
+    set_error("%s: bad sizes or dtype (B=%lld N=%lld Nk=%lld heads=%d d=%d dtype=%d)", what, (long long)B, (long long)N,
+              (long long)Nk, heads, d, dtype);
+    return kErrBadArg;
+  }
+  const int64_t n = N > Nk ? N : Nk;
+  if (d % (unit * blocks::vec_of(dtype)) || heads > (1 << 20) / d || n > 0x7fffffffLL / B ||
+      B * n > 0x7fffffffLL / ((int64_t)heads * d / blocks::vec_of(dtype))) {
+    set_error("%s: needs head dims of whole 16-byte pieces, at most 2^20 channels and 2^31 pieces "
+              "(B=%lld N=%lld Nk=%lld heads=%d d=%d dtype=%d)", what, (long long)B, (long long)N, (long long)Nk, heads, d, dtype);
+    return kErrUnsupported;
+  }
+  s = {(int)B, (int)N, (int)Nk, heads, d};
+  return kOk;
+}
+static int check_tensors(const char* what, std::initializer_list<const void*> ptrs) {
+  for (const void* p : ptrs)
+    if (!p) {
+      set_error("%s: null tensor pointer", what);
+      return kErrBadArg;
+    }
+  return check_aligned(what, ptrs);
+}
+
+int fbla_polarity_fwd(const void* qg, const void* kv, const void* pe, const void* scale, const void* power, void* q_same,
+                      void* q_opp, void* k_both, void* v_heads, int64_t B, int64_t N, int64_t Nk, int heads, int d, int dtype,
+                      void* stream) {
+  const char* what = "fbla_polarity_fwd";
+  blocks::Shape s;
+  int rc = check_blocks(what, s, B, N, Nk, heads, d, 1, dtype);
+  if (rc == kOk) rc = check_tensors(what, {qg, kv, pe, scale, power, q_same, q_opp, k_both, v_heads});
+  if (rc != kOk) return rc;
+  blocks::polarity_fwd(s, {qg, kv, pe, scale, power}, q_same, q_opp, k_both, v_heads, dtype, (hipStream_t)stream);
+  return check_launch(what);
+}
+
+size_t fbla_polarity_bwd_workspace_bytes(int64_t B, int64_t N, int64_t Nk, int heads, int d, int dtype) {
+  blocks::Shape s;
+  if (check_blocks("fbla_polarity_bwd_workspace_bytes", s, B, N, Nk, heads, d, 1, dtype) != kOk) return 0;
+  return blocks::polarity_bwd_workspace_bytes(s, dtype);
+}
+
+int fbla_polarity_bwd(const void* qg, const void* kv, const void* pe, const void* scale, const void* power,
+                      const void* dq_same, const void* dq_opp, const void* dk_both, const void* dv_heads, const void* dv_rows,
+                      const void* dgate, void* dqg, void* dkv, void* dpe, void* dscale, void* dpower, void* workspace,
+                      size_t workspace_bytes, int64_t B, int64_t N, int64_t Nk, int heads, int d, int dtype, void* stream) {
+  const char* what = "fbla_polarity_bwd";
+  blocks::Shape s;
+  int rc = check_blocks(what, s, B, N, Nk, heads, d, 1, dtype);
+  if (rc == kOk)
+    rc = check_tensors(what, {qg, kv, pe, scale, power, dq_same, dq_opp, dk_both, dv_heads, dv_rows, dgate, dqg, dkv, dpe,
+                              dscale, dpower, workspace});
+  if (rc != kOk) return rc;
+  const size_t need = blocks::polarity_bwd_workspace_bytes(s, dtype);
+  if (workspace_bytes < need) {
+    set_error("%s: workspace too small (%zu < %zu bytes)", what, workspace_bytes, need);
+    return kErrWorkspace;
+  }
+  blocks::polarity_bwd(s, {qg, kv, pe, scale, power}, {dq_same, dq_opp, dk_both, dv_heads, dv_rows, dgate}, dqg, dkv, dpe,
+                       dscale, dpower, (float*)workspace, dtype, (hipStream_t)stream);
+  return check_launch(what);
+}
+
+static int check_rotation(const char* what, int rot_channels, int heads, int d, int dtype) {
+  if (rot_channels < 1 || (heads * d) % rot_channels || rot_channels % blocks::vec_of(dtype)) {
+    set_error("%s: the rotation's channels must be whole 16-byte pieces and divide the tokens' (%d, %d)", what, rot_channels,
+              heads * d);
+    return kErrBadArg;
+  }
+  return kOk;
+}
+
+int fbla_rotary_fwd(const void* qk, const void* x, const float* rot, int rot_channels, void* q, void* k, void* q_rot,
+                    void* k_rot, void* v, int64_t B, int64_t N, int heads, int d, int dtype, void* stream) {
+  const char* what = "fbla_rotary_fwd";
+  blocks::Shape s;
+  int rc = check_blocks(what, s, B, N, N, heads, d, 1, dtype);
+  if (rc == kOk) rc = check_rotation(what, rot_channels, heads, d, dtype);
+  if (rc == kOk) rc = check_tensors(what, {qk, x, rot, q, k, q_rot, k_rot, v});
+  if (rc != kOk) return rc;
+  blocks::rotary_fwd(s, qk, x, rot, rot_channels, q, k, q_rot, k_rot, v, dtype, (hipStream_t)stream);
+  return check_launch(what);
+}
+
+int fbla_rotary_bwd(const void* qk, const float* rot, int rot_channels, const void* dq, const void* dk, const void* dq_rot,
+                    const void* dk_rot, const void* dv, const void* dv_rows, void* dqk, void* dx, int64_t B, int64_t N,
+                    int heads, int d, int dtype, void* stream) {
+  const char* what = "fbla_rotary_bwd";
+  blocks::Shape s;
+  int rc = check_blocks(what, s, B, N, N, heads, d, 1, dtype);
+  if (rc == kOk) rc = check_rotation(what, rot_channels, heads, d, dtype);
+  if (rc == kOk) rc = check_tensors(what, {qk, rot, dq, dk, dq_rot, dk_rot, dv, dv_rows, dqk, dx});
+  if (rc != kOk) return rc;
+  blocks::rotary_bwd(s, qk, rot, rot_channels, {dq, dk, dq_rot, dk_rot, dv, dv_rows}, dqk, dx, dtype, (hipStream_t)stream);
+  return check_launch(what);
+}
+
+static int check_merge(const char* what, blocks::Shape& s, const void* o2, const void* gate, int64_t gate_row, int64_t B,
+                       int64_t N, int heads, int d, int dtype) {
+  int rc = check_blocks(what, s, B, N, N, heads, d, o2 ? 2 : 1, dtype);
+  if (rc == kOk && gate) rc = check_row_strides(what, heads * d, dtype, {gate_row});
+  if (rc == kOk) rc = check_aligned(what, {o2, gate});
+  return rc;
+}
+
+int fbla_merge_fwd(const void* o, const void* o2, const void* local, const void* gate, int64_t gate_row, void* out, int64_t B,
+                   int64_t N, int heads, int d, int dtype, void* stream) {
+  const char* what = "fbla_merge_fwd";
+  blocks::Shape s;
+  int rc = check_merge(what, s, o2, gate, gate_row, B, N, heads, d, dtype);
+  if (rc == kOk) rc = check_tensors(what, {o, local, out});
+  if (rc != kOk) return rc;
+  blocks::merge_fwd(s, {o, o2, local, gate, gate_row}, out, dtype, (hipStream_t)stream);
+  return check_launch(what);
+}
+
+int fbla_merge_bwd(const void* dout, const void* o, const void* o2, const void* local, const void* gate, int64_t gate_row,
+                   void* d_o, void* d_o2, void* dlocal, void* dgate, int64_t B, int64_t N, int heads, int d, int dtype,
+                   void* stream) {
+  const char* what = "fbla_merge_bwd";
+  blocks::Shape s;
+  int rc = check_merge(what, s, d_o2, gate, gate_row, B, N, heads, d, dtype);
+  if (rc == kOk) rc = check_tensors(what, {dout, d_o});
+  if (rc == kOk && gate) rc = check_tensors(what, {o, local, dlocal, dgate});
+  if (rc != kOk) return rc;
+  if (gate && !o2 != !d_o2) {
+    set_error("%s: one or two tensors of heads, on both sides alike", what);
+    return kErrBadArg;
+  }
+  blocks::merge_bwd(s, {o, o2, local, gate, gate_row}, dout, d_o, d_o2, dlocal, dgate, dtype, (hipStream_t)stream);
+  return check_launch(what);
+}
+
 }  // extern "C"

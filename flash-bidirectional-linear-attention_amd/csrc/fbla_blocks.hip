@@ -1,0 +1,529 @@
+// What the vision blocks do between their projections and the attention operators, one launch a direction:
+//
+//   polarity features (layers/polaformer.py:63-84): q / scale and (k + positional) / scale, positive and negative parts to a
+//     learned power, the same-sign and opposite-sign pairings and the values as contiguous heads;
+//   rotary features (layers/mlla.py:74-81): elu + 1 of q and k, their 2-D rotation, the values, all as contiguous heads;
+//   merged heads (polaformer.py:92-104, mlla.py:88-92): heads back to token rows, plus the convolution's rows, times a gate.
+//
+// All of it is elementwise on token rows and bound by HBM: a lane owns 16 bytes of channels of one token (the next lanes the
+// next channels), everything is computed from them in fp32 and rounded once, and nothing between the projection's rows and the
+// operator's heads is written.  Training steps with torch operators in their place and with these: polarity (64 x 28x28 x
+// 256, bf16) 2.77 -> 0.83 ms, of it here 51 us features (231 MB, 4.6 TB/s), 77 + 9 us their gradients (385 MB), 19 + 32 us the
+// merge; rotary (64 x 56x56 x 64) 0.83 -> 0.48 ms, of it 33 us features (205 MB, 6.2 TB/s), 44 us gradients (308 MB, 7 TB/s).
+#include <hip/hip_runtime.h>
+
+#include "fbla_kernels.h"
+
+namespace fbla {
+namespace blocks {
+
+namespace {
+
+constexpr int kThreads = 256;
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+template <typename T> struct Piece {
+  static constexpr int kVec = 16 / sizeof(T);
+  union {
+    u32x4 w;
+    T e[kVec];
+  };
+};
+template <typename T> __device__ __forceinline__ Piece<T> load(const T* p) {
+  Piece<T> v;
+  v.w = *reinterpret_cast<const u32x4*>(p);
+  return v;
+}
+template <typename T> __device__ __forceinline__ void store(T* p, const Piece<T>& v) {
+  *reinterpret_cast<u32x4*>(p) = v.w;
+}
+
+// a^p for a >= 0 (0 for a = 0, p > 0).  16-bit results: the hardware's exp2 and log2, whose error (2^-22 of p log2 a) is far
+// below the result's rounding.
+template <typename T> __device__ __forceinline__ float power_of(float a, float p) {
+  if constexpr (sizeof(T) == 4) return powf(a, p);
+  else return __builtin_amdgcn_exp2f(p * __builtin_amdgcn_logf(a));
+}
+template <typename T> __device__ __forceinline__ float log_of(float a) {
+  if constexpr (sizeof(T) == 4) return logf(a);
+  else return __builtin_amdgcn_logf(a) * 0.693147180559945309f;
+}
+template <typename T> __device__ __forceinline__ float exp_of(float x) {
+  if constexpr (sizeof(T) == 4) return expf(x);
+  else return __builtin_amdgcn_exp2f(x * 1.44269504088896341f);
+}
+
+// first element of head row (b, h, t) of a [B, heads, n, width] tensor
+__device__ __forceinline__ int64_t head_row(const Shape& s, uint32_t b, uint32_t h, uint32_t t, uint32_t n, int width) {
+  return (((int64_t)b * s.heads + h) * n + t) * width;
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+// polarity features
+// ---------------------------------------------------------------------------------------------------------------
+template <typename T>
+__device__ __forceinline__ void split_signs(const float (&y)[Piece<T>::kVec], const Piece<T>& power, Piece<T>& pos,
+                                            Piece<T>& neg) {
+#pragma unroll
+  for (int j = 0; j < Piece<T>::kVec; ++j) {
+    const float r = power_of<T>(fabsf(y[j]), (float)power.e[j]);
+    pos.e[j] = (T)(y[j] < 0.f ? 0.f : r);  // NaN goes to both
+    neg.e[j] = (T)(y[j] > 0.f ? 0.f : r);
+  }
+}
+
+// pieces [0, q_pieces) are the queries' (gate half untouched), the others the keys' and values'
+template <typename T>
+__global__ __launch_bounds__(kThreads) void polarity_fwd_kernel(Shape s, Polarity<const T> a, T* __restrict__ q_same,
+                                                                T* __restrict__ q_opp, T* __restrict__ k_both,
+                                                                T* __restrict__ v_heads, uint32_t q_wgs) {
+  constexpr int V = Piece<T>::kVec;
+  const bool keys = blockIdx.x >= q_wgs;
+  const uint32_t i = (keys ? blockIdx.x - q_wgs : blockIdx.x) * kThreads + threadIdx.x;
+  const uint32_t pieces = s.heads * s.d / V, n = keys ? s.Nk : s.N;
+  const uint32_t row = i / pieces, c = i % pieces * V;
+  if (row >= (uint32_t)s.B * n) return;
+  const uint32_t b = row / n, t = row % n, h = c / s.d, j0 = c % s.d, C = s.heads * s.d;
+  const Piece<T> scale = load(a.scale + c), power = load(a.power + c);
+  const T* src = (keys ? a.kv : a.qg) + (int64_t)row * 2 * C + c;
+  const Piece<T> x = load(src);
+  float y[V];
+#pragma unroll
+  for (int j = 0; j < V; ++j) y[j] = (float)x.e[j];
+  if (keys) {
+    const Piece<T> pe = load(a.pe + (int64_t)t * C + c), v = load(src + C);
+#pragma unroll
+    for (int j = 0; j < V; ++j) y[j] += (float)pe.e[j];
+    store(v_heads + head_row(s, b, h, t, n, s.d) + j0, v);
+  }
+#pragma unroll
+  for (int j = 0; j < V; ++j) y[j] /= (float)scale.e[j];
+  Piece<T> pos, neg;
+  split_signs<T>(y, power, pos, neg);
+  const int64_t at = head_row(s, b, h, t, n, 2 * s.d) + j0;
+  if (keys) {
+    store(k_both + at, pos);
+    store(k_both + at + s.d, neg);
+  } else {
+    store(q_same + at, pos);
+    store(q_same + at + s.d, neg);
+    store(q_opp + at, neg);
+    store(q_opp + at + s.d, pos);
+  }
+}
+
+// One piece's gradients: dx = the gradient of x (q, or k and its positional term alike), added to `dscale` the gradient of
+// -scale * scale, to `dpower` that of the power.
+template <typename T>
+__device__ __forceinline__ void polarity_piece_bwd(const float (&x)[Piece<T>::kVec], const float (&inv)[Piece<T>::kVec],
+                                                   const float (&power)[Piece<T>::kVec], const float (&gpos)[Piece<T>::kVec],
+                                                   const float (&gneg)[Piece<T>::kVec], float (&dx)[Piece<T>::kVec],
+                                                   float (&dscale)[Piece<T>::kVec], float (&dpower)[Piece<T>::kVec]) {
+#pragma unroll
+  for (int j = 0; j < Piece<T>::kVec; ++j) {
+    const float y = x[j] * inv[j], a = fabsf(y);
+    const float g = y < 0.f ? gneg[j] : gpos[j];
+    const float w = power_of<T>(a, power[j] - 1.f);
+    const bool zero = a == 0.f;  // both parts are cut off there: no gradient
+    const float dy = zero ? 0.f : (y < 0.f ? -g : g) * power[j] * w;
+    dx[j] = dy * inv[j];
+    dscale[j] += dy * x[j];
+    dpower[j] += zero ? 0.f : g * (w * a) * log_of<T>(a);
+  }
+}
+
+// Workgroup = `lanes` pieces of channels (at most 64, blockIdx.y picks them) times kThreads / lanes rows; it walks rows
+// gridDim.x apart and keeps the sums over tokens (gradients of scale and power) in registers.  Workgroups [0, q_wgs) take the
+// queries, the others the keys: rows there are (token, batch group), a lane adds its token's gradients over the batches of the
+// group (gradient of the positional term).  partial: [workgroup][2][C], pe_partial: [group][Nk][C].
+template <typename T>
+__global__ __launch_bounds__(kThreads) void polarity_bwd_kernel(Shape s, Polarity<const T> a, PolarityGrads<const T> g,
+                                                                T* __restrict__ dqg, T* __restrict__ dkv,
+                                                                float* __restrict__ partial, float* __restrict__ pe_partial,
+                                                                int q_wgs, int groups) {
+  constexpr int V = Piece<T>::kVec;
+  const int C = s.heads * s.d, pieces = C / V;
+  const int lanes = min(pieces - (int)blockIdx.y * 64, 64), rows = kThreads / lanes;
+  const int lane = threadIdx.x % lanes, r = threadIdx.x / lanes;
+  const bool keys = (int)blockIdx.x >= q_wgs;
+  const uint32_t wg = keys ? blockIdx.x - q_wgs : blockIdx.x, wgs = keys ? gridDim.x - q_wgs : q_wgs;
+  const int c = (blockIdx.y * 64 + lane) * V, h = c / s.d, j0 = c % s.d;
+  float dscale[V], dpower[V], inv[V], power[V];
+  {
+    const Piece<T> sc = load(a.scale + c), pw = load(a.power + c);
+#pragma unroll
+    for (int j = 0; j < V; ++j) {
+      dscale[j] = dpower[j] = 0.f;
+      inv[j] = 1.f / (float)sc.e[j];
+      power[j] = (float)pw.e[j];
+    }
+  }
+  if (r < rows && !keys) {
+    const uint32_t total = (uint32_t)s.B * s.N;
+    for (uint32_t row = wg * rows + r; row < total; row += wgs * rows) {
+      const uint32_t b = row / s.N, t = row % s.N;
+      const int64_t at = head_row(s, b, h, t, s.N, 2 * s.d) + j0;
+      const Piece<T> x = load(a.qg + (int64_t)row * 2 * C + c);
+      const Piece<T> s0 = load(g.q_same + at), s1 = load(g.q_same + at + s.d), o0 = load(g.q_opp + at),
+                     o1 = load(g.q_opp + at + s.d), gate = load(g.gate + (int64_t)row * C + c);
+      float xf[V], gpos[V], gneg[V], dx[V];
+#pragma unroll
+      for (int j = 0; j < V; ++j) {
+        xf[j] = (float)x.e[j];
+        gpos[j] = (float)s0.e[j] + (float)o1.e[j];
+        gneg[j] = (float)s1.e[j] + (float)o0.e[j];
+      }
+      polarity_piece_bwd<T>(xf, inv, power, gpos, gneg, dx, dscale, dpower);
+      Piece<T> out;
+#pragma unroll
+      for (int j = 0; j < V; ++j) out.e[j] = (T)dx[j];
+      T* to = dqg + (int64_t)row * 2 * C + c;
+      store(to, out);
+      store(to + C, gate);
+    }
+  }
+  if (r < rows && keys) {
+    const uint32_t total = (uint32_t)s.Nk * groups;
+    for (uint32_t item = wg * rows + r; item < total; item += wgs * rows) {
+      const uint32_t t = item / groups, group = item % groups;
+      const Piece<T> pe = load(a.pe + (int64_t)t * C + c);
+      float dpe[V];
+#pragma unroll
+      for (int j = 0; j < V; ++j) dpe[j] = 0.f;
+      for (uint32_t b = group; b < (uint32_t)s.B; b += groups) {
+        const int64_t row = (int64_t)b * s.Nk + t, at = head_row(s, b, h, t, s.Nk, 2 * s.d) + j0;
+        const Piece<T> x = load(a.kv + row * 2 * C + c);
+        const Piece<T> g0 = load(g.k_both + at), g1 = load(g.k_both + at + s.d),
+                       vh = load(g.v_heads + head_row(s, b, h, t, s.Nk, s.d) + j0), vr = load(g.v_rows + row * C + c);
+        float xf[V], gpos[V], gneg[V], dx[V];
+#pragma unroll
+        for (int j = 0; j < V; ++j) {
+          xf[j] = (float)x.e[j] + (float)pe.e[j];
+          gpos[j] = (float)g0.e[j];
+          gneg[j] = (float)g1.e[j];
+        }
+        polarity_piece_bwd<T>(xf, inv, power, gpos, gneg, dx, dscale, dpower);
+        Piece<T> out, v;
+#pragma unroll
+        for (int j = 0; j < V; ++j) {
+          out.e[j] = (T)dx[j];
+          dpe[j] += dx[j];
+          v.e[j] = (T)((float)vh.e[j] + (float)vr.e[j]);
+        }
+        T* to = dkv + row * 2 * C + c;
+        store(to, out);
+        store(to + C, v);
+      }
+      float* to = pe_partial + ((int64_t)group * s.Nk + t) * C + c;
+#pragma unroll
+      for (int j = 0; j < V; j += 4) *reinterpret_cast<f32x4*>(to + j) = f32x4{dpe[j], dpe[j + 1], dpe[j + 2], dpe[j + 3]};
+    }
+  }
+  // the rows of the workgroup, in order
+  __shared__ float sums[kThreads * V];
+  float* out = partial + (int64_t)blockIdx.x * 2 * C;
+#pragma unroll
+  for (int which = 0; which < 2; ++which) {
+    __syncthreads();
+    if (r < rows)
+#pragma unroll
+      for (int j = 0; j < V; ++j) sums[(r * lanes + lane) * V + j] = which ? dpower[j] : dscale[j];
+    __syncthreads();
+    for (int i = threadIdx.x; i < lanes * V; i += kThreads) {
+      float v = 0.f;
+      for (int q = 0; q < rows; ++q) v += sums[q * lanes * V + i];
+      out[which * C + blockIdx.y * 64 * V + i] = v;
+    }
+  }
+}
+
+// Sums over the partials in order, four neighbouring results per lane, 16 lanes of a column; workgroups [0, stat_wgs): the
+// 2 C sums of scale and power, the others the Nk C sums of the positional term.
+template <typename T>
+__global__ __launch_bounds__(kThreads) void polarity_finish_kernel(int C, int wgs, const float* __restrict__ partial,
+                                                                   const T* __restrict__ scale, T* __restrict__ dscale,
+                                                                   T* __restrict__ dpower, int stat_wgs, int groups,
+                                                                   int64_t pe_count, const float* __restrict__ pe_partial,
+                                                                   T* __restrict__ dpe) {
+  constexpr int kParts = 16, kLanes = kThreads / kParts;
+  __shared__ f32x4 sums[kParts][kLanes];
+  const bool stats = (int)blockIdx.x < stat_wgs;
+  const int lane = threadIdx.x % kLanes, part = threadIdx.x / kLanes;
+  const int64_t at = ((int64_t)(stats ? blockIdx.x : blockIdx.x - stat_wgs) * kLanes + lane) * 4;
+  const int64_t count = stats ? 2 * C : pe_count;
+  const int terms = stats ? wgs : groups;
+  const float* src = stats ? partial : pe_partial;
+  f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+  if (at < count)
+#pragma unroll 4
+    for (int i = part; i < terms; i += kParts) {
+      const f32x4 v = *reinterpret_cast<const f32x4*>(src + (int64_t)i * count + at);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) sum[j] += v[j];
+    }
+  sums[part][lane] = sum;
+  __syncthreads();
+  if (part != 0 || at >= count) return;
+  for (int i = 1; i < kParts; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) sum[j] += sums[i][lane][j];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int64_t c = at + j;
+    if (!stats) dpe[c] = (T)sum[j];
+    else if (c >= C) dpower[c - C] = (T)sum[j];
+    else {
+      const float inv = 1.f / (float)scale[c];
+      dscale[c] = (T)(-sum[j] * inv * inv);
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+// rotary features
+// ---------------------------------------------------------------------------------------------------------------
+template <typename T> __device__ __forceinline__ float phi(float x) { return x > 0.f ? x + 1.f : exp_of<T>(x); }
+
+// cos and sin of the piece's channel pairs: rot [N][rot_channels / 2][2]
+template <typename T>
+__device__ __forceinline__ void load_rotation(const float* __restrict__ rot, int rot_channels, uint32_t t, uint32_t c,
+                                              float (&cs)[Piece<T>::kVec]) {
+  const float* p = rot + (int64_t)t * rot_channels + c % rot_channels;
+#pragma unroll
+  for (int j = 0; j < Piece<T>::kVec; j += 4) {
+    const f32x4 v = *reinterpret_cast<const f32x4*>(p + j);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) cs[j + e] = v[e];
+  }
+}
+
+template <typename T>
+__global__ __launch_bounds__(kThreads) void rotary_fwd_kernel(Shape s, const T* __restrict__ qk, const T* __restrict__ x,
+                                                              const float* __restrict__ rot, int rot_channels,
+                                                              T* __restrict__ q, T* __restrict__ k, T* __restrict__ q_rot,
+                                                              T* __restrict__ k_rot, T* __restrict__ v) {
+  constexpr int V = Piece<T>::kVec;
+  const uint32_t C = s.heads * s.d, pieces = C / V, i = blockIdx.x * kThreads + threadIdx.x;
+  const uint32_t row = i / pieces, c = i % pieces * V;
+  if (row >= (uint32_t)s.B * s.N) return;
+  const uint32_t b = row / s.N, t = row % s.N;
+  const Piece<T> in[2] = {load(qk + (int64_t)row * 2 * C + c), load(qk + (int64_t)row * 2 * C + C + c)};
+  const Piece<T> vin = load(x + (int64_t)row * C + c);
+  float cs[V];
+  load_rotation<T>(rot, rot_channels, t, c, cs);
+  const int64_t at = head_row(s, b, c / s.d, t, s.N, s.d) + c % s.d;
+#pragma unroll
+  for (int w = 0; w < 2; ++w) {
+    Piece<T> plain, turned;
+#pragma unroll
+    for (int j = 0; j < V; j += 2) {
+      const float re = phi<T>((float)in[w].e[j]), im = phi<T>((float)in[w].e[j + 1]);
+      plain.e[j] = (T)re;
+      plain.e[j + 1] = (T)im;
+      turned.e[j] = (T)(re * cs[j] - im * cs[j + 1]);
+      turned.e[j + 1] = (T)(re * cs[j + 1] + im * cs[j]);
+    }
+    store((w ? k : q) + at, plain);
+    store((w ? k_rot : q_rot) + at, turned);
+  }
+  store(v + at, vin);
+}
+
+template <typename T>
+__global__ __launch_bounds__(kThreads) void rotary_bwd_kernel(Shape s, const T* __restrict__ qk,
+                                                              const float* __restrict__ rot, int rot_channels,
+                                                              RotaryGrads<const T> g, T* __restrict__ dqk,
+                                                              T* __restrict__ dx) {
+  constexpr int V = Piece<T>::kVec;
+  const uint32_t C = s.heads * s.d, pieces = C / V, i = blockIdx.x * kThreads + threadIdx.x;
+  const uint32_t row = i / pieces, c = i % pieces * V;
+  if (row >= (uint32_t)s.B * s.N) return;
+  const uint32_t b = row / s.N, t = row % s.N;
+  const int64_t at = head_row(s, b, c / s.d, t, s.N, s.d) + c % s.d, from = (int64_t)row * 2 * C + c;
+  const Piece<T> in[2] = {load(qk + from), load(qk + from + C)};
+  const Piece<T> plain[2] = {load(g.q + at), load(g.k + at)}, turned[2] = {load(g.q_rot + at), load(g.k_rot + at)};
+  const Piece<T> vh = load(g.v + at), vr = load(g.v_rows + (int64_t)row * C + c);
+  float cs[V];
+  load_rotation<T>(rot, rot_channels, t, c, cs);
+#pragma unroll
+  for (int w = 0; w < 2; ++w) {
+    Piece<T> out;
+#pragma unroll
+    for (int j = 0; j < V; j += 2) {
+      const float gre = (float)turned[w].e[j], gim = (float)turned[w].e[j + 1];
+      const float re = (float)plain[w].e[j] + gre * cs[j] + gim * cs[j + 1];
+      const float im = (float)plain[w].e[j + 1] + gim * cs[j] - gre * cs[j + 1];
+      const float x0 = (float)in[w].e[j], x1 = (float)in[w].e[j + 1];
+      out.e[j] = (T)(x0 > 0.f ? re : re * exp_of<T>(x0));
+      out.e[j + 1] = (T)(x1 > 0.f ? im : im * exp_of<T>(x1));
+    }
+    store(dqk + from + (w ? C : 0), out);
+  }
+  Piece<T> v;
+#pragma unroll
+  for (int j = 0; j < V; ++j) v.e[j] = (T)((float)vh.e[j] + (float)vr.e[j]);
+  store(dx + (int64_t)row * C + c, v);
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+// merged heads
+// ---------------------------------------------------------------------------------------------------------------
+// Where the piece of channels c of token (b, t) lies in the heads: o [B, heads, N, d], or with o2 the channels of a head in
+// two halves o, o2 [B, heads, N, d / 2].
+template <typename T>
+__device__ __forceinline__ T* head_piece(const Shape& s, T* o, T* o2, uint32_t b, uint32_t t, uint32_t c) {
+  const uint32_t h = c / s.d, j = c % s.d;
+  if (!o2) return o + head_row(s, b, h, t, s.N, s.d) + j;
+  const uint32_t half = s.d / 2;
+  return j < half ? o + head_row(s, b, h, t, s.N, half) + j : o2 + head_row(s, b, h, t, s.N, half) + j - half;
+}
+
+template <typename T>
+__global__ __launch_bounds__(kThreads) void merge_fwd_kernel(Shape s, Merge<const T> a, T* __restrict__ out) {
+  constexpr int V = Piece<T>::kVec;
+  const uint32_t C = s.heads * s.d, pieces = C / V, i = blockIdx.x * kThreads + threadIdx.x;
+  const uint32_t row = i / pieces, c = i % pieces * V;
+  if (row >= (uint32_t)s.B * s.N) return;
+  const Piece<T> o = load(head_piece<const T>(s, a.o, a.o2, row / s.N, row % s.N, c));
+  const Piece<T> l = load(a.local + (int64_t)row * C + c);
+  Piece<T> r;
+#pragma unroll
+  for (int j = 0; j < V; ++j) r.e[j] = (T)((float)o.e[j] + (float)l.e[j]);
+  if (a.gate) {
+    const Piece<T> gate = load(a.gate + (int64_t)row * a.gate_row + c);
+#pragma unroll
+    for (int j = 0; j < V; ++j) r.e[j] = (T)(((float)o.e[j] + (float)l.e[j]) * (float)gate.e[j]);
+  }
+  store(out + (int64_t)row * C + c, r);
+}
+
+// dlocal = dout * gate (also as heads), dgate = dout * (heads + local); without a gate dlocal is dout and is not written
+template <typename T>
+__global__ __launch_bounds__(kThreads) void merge_bwd_kernel(Shape s, Merge<const T> a, const T* __restrict__ dout,
+                                                             T* __restrict__ d_o, T* __restrict__ d_o2,
+                                                             T* __restrict__ dlocal, T* __restrict__ dgate) {
+  constexpr int V = Piece<T>::kVec;
+  const uint32_t C = s.heads * s.d, pieces = C / V, i = blockIdx.x * kThreads + threadIdx.x;
+  const uint32_t row = i / pieces, c = i % pieces * V;
+  if (row >= (uint32_t)s.B * s.N) return;
+  const uint32_t b = row / s.N, t = row % s.N;
+  const int64_t at = (int64_t)row * C + c;
+  Piece<T> g = load(dout + at);
+  if (a.gate) {
+    const Piece<T> gate = load(a.gate + (int64_t)row * a.gate_row + c), l = load(a.local + at),
+                   o = load(head_piece<const T>(s, a.o, a.o2, b, t, c));
+    Piece<T> dg;
+#pragma unroll
+    for (int j = 0; j < V; ++j) {
+      dg.e[j] = (T)((float)g.e[j] * ((float)o.e[j] + (float)l.e[j]));
+      g.e[j] = (T)((float)g.e[j] * (float)gate.e[j]);
+    }
+    store(dgate + at, dg);
+    store(dlocal + at, g);
+  }
+  store(head_piece<T>(s, d_o, d_o2, b, t, c), g);
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+unsigned wgs_for(int64_t rows, int C, int vec) { return (unsigned)cdiv64(rows * (C / vec), kThreads); }
+template <typename F> void by_type(int dtype, F&& f) {
+  if (dtype == kF16) f(_Float16{});
+  else if (dtype == kBF16) f(__bf16{});
+  else f(float{});
+}
+template <typename T, template <typename> class S> S<const T> typed(const S<const void>& a) {
+  return __builtin_bit_cast(S<const T>, a);  // the same pointers, to elements of the tensors' type
+}
+
+// Split of the polarity gradient: about two workgroups per CU for each side (each costs 2 C partial sums); the batches of a
+// token in as many groups as give the keys that many workgroups.
+struct Split {
+  int q_wgs, k_wgs, groups, channel_wgs;
+};
+Split polarity_split(const Shape& s, int vec) {
+  const int pieces = s.heads * s.d / vec, channel_wgs = (pieces + 63) / 64;
+  const int rows = kThreads / (pieces < 64 ? pieces : 64);
+  const int64_t most = 512 / channel_wgs < 1 ? 1 : 512 / channel_wgs;
+  const int64_t q = cdiv64((int64_t)s.B * s.N, rows);
+  int64_t groups = cdiv64(most * rows, s.Nk);
+  groups = groups < s.B ? groups : s.B;
+  const int64_t k = cdiv64(s.Nk * groups, rows);
+  return {(int)(q < most ? q : most), (int)(k < most ? k : most), (int)groups, channel_wgs};
+}
+
+}  // namespace
+
+int vec_of(int dtype) { return dtype == kF32 ? 4 : 8; }
+
+void polarity_fwd(const Shape& s, const Polarity<const void>& a, void* q_same, void* q_opp, void* k_both, void* v_heads,
+                  int dtype, hipStream_t st) {
+  by_type(dtype, [&](auto tag) {
+    using T = decltype(tag);
+    const int C = s.heads * s.d;
+    const unsigned q_wgs = wgs_for((int64_t)s.B * s.N, C, Piece<T>::kVec),
+                   k_wgs = wgs_for((int64_t)s.B * s.Nk, C, Piece<T>::kVec);
+    polarity_fwd_kernel<T><<<dim3(q_wgs + k_wgs), dim3(kThreads), 0, st>>>(s, typed<T, Polarity>(a), (T*)q_same, (T*)q_opp,
+                                                                          (T*)k_both, (T*)v_heads, q_wgs);
+  });
+}
+
+size_t polarity_bwd_workspace_bytes(const Shape& s, int dtype) {
+  const Split w = polarity_split(s, vec_of(dtype));
+  const size_t C = (size_t)s.heads * s.d;
+  return sizeof(float) * (2 * C * (w.q_wgs + w.k_wgs) + C * w.groups * s.Nk);
+}
+
+void polarity_bwd(const Shape& s, const Polarity<const void>& a, const PolarityGrads<const void>& g, void* dqg, void* dkv,
+                  void* dpe, void* dscale, void* dpower, float* workspace, int dtype, hipStream_t st) {
+  by_type(dtype, [&](auto tag) {
+    using T = decltype(tag);
+    const Split w = polarity_split(s, Piece<T>::kVec);
+    const int C = s.heads * s.d, wgs = w.q_wgs + w.k_wgs;
+    float* pe_partial = workspace + (int64_t)2 * C * wgs;
+    polarity_bwd_kernel<T><<<dim3((unsigned)wgs, (unsigned)w.channel_wgs), dim3(kThreads), 0, st>>>(
+        s, typed<T, Polarity>(a), typed<T, PolarityGrads>(g), (T*)dqg, (T*)dkv, workspace, pe_partial, w.q_wgs, w.groups);
+    const int64_t pe_count = (int64_t)s.Nk * C;
+    const int stat_wgs = (2 * C + 63) / 64;
+    polarity_finish_kernel<T><<<dim3((unsigned)(stat_wgs + cdiv64(pe_count, 64))), dim3(kThreads), 0, st>>>(
+        C, wgs, workspace, (const T*)a.scale, (T*)dscale, (T*)dpower, stat_wgs, w.groups, pe_count, pe_partial, (T*)dpe);
+  });
+}
+
+void rotary_fwd(const Shape& s, const void* qk, const void* x, const float* rot, int rot_channels, void* q, void* k,
+                void* q_rot, void* k_rot, void* v, int dtype, hipStream_t st) {
+  by_type(dtype, [&](auto tag) {
+    using T = decltype(tag);
+    rotary_fwd_kernel<T><<<dim3(wgs_for((int64_t)s.B * s.N, s.heads * s.d, Piece<T>::kVec)), dim3(kThreads), 0, st>>>(
+        s, (const T*)qk, (const T*)x, rot, rot_channels, (T*)q, (T*)k, (T*)q_rot, (T*)k_rot, (T*)v);
+  });
+}
+
+void rotary_bwd(const Shape& s, const void* qk, const float* rot, int rot_channels, const RotaryGrads<const void>& g,
+                void* dqk, void* dx, int dtype, hipStream_t st) {
+  by_type(dtype, [&](auto tag) {
+    using T = decltype(tag);
+    rotary_bwd_kernel<T><<<dim3(wgs_for((int64_t)s.B * s.N, s.heads * s.d, Piece<T>::kVec)), dim3(kThreads), 0, st>>>(
+        s, (const T*)qk, rot, rot_channels, typed<T, RotaryGrads>(g), (T*)dqk, (T*)dx);
+  });
+}
+
+void merge_fwd(const Shape& s, const Merge<const void>& a, void* out, int dtype, hipStream_t st) {
+  by_type(dtype, [&](auto tag) {
+    using T = decltype(tag);
+    merge_fwd_kernel<T><<<dim3(wgs_for((int64_t)s.B * s.N, s.heads * s.d, Piece<T>::kVec)), dim3(kThreads), 0, st>>>(
+        s, typed<T, Merge>(a), (T*)out);
+  });
+}
+
+void merge_bwd(const Shape& s, const Merge<const void>& a, const void* dout, void* d_o, void* d_o2, void* dlocal, void* dgate,
+               int dtype, hipStream_t st) {
+  by_type(dtype, [&](auto tag) {
+    using T = decltype(tag);
+    merge_bwd_kernel<T><<<dim3(wgs_for((int64_t)s.B * s.N, s.heads * s.d, Piece<T>::kVec)), dim3(kThreads), 0, st>>>(
+        s, typed<T, Merge>(a), (const T*)dout, (T*)d_o, (T*)d_o2, (T*)dlocal, (T*)dgate);
+  });
+}
+
+}  // namespace blocks
+}  // namespace fbla

@@ -235,6 +235,43 @@ void wgrad(const void* g, int64_t g_row, const void* x, int64_t x_row, int64_t t
            float* workspace, int dtype, hipStream_t st);
 }  // namespace linear
 
+// Elementwise work of the vision blocks around the attention operators (fbla_blocks.hip).  Rows are [B, N, C] with
+// C = heads * d, joint projections [B, N, 2 C], heads [B, heads, N, width]; all contiguous, d in whole 16-byte pieces.
+namespace blocks {
+struct Shape {
+  int B, N, Nk, heads, d;  // Nk: tokens of the keys (polarity features only)
+};
+template <typename P> struct Polarity {
+  P *qg, *kv, *pe, *scale, *power;  // [B,N,2C], [B,Nk,2C], [Nk,C], [C], [C]
+};
+template <typename P> struct PolarityGrads {
+  P *q_same, *q_opp, *k_both, *v_heads, *v_rows, *gate;  // heads of 2d, 2d, 2d, d; rows of C
+};
+template <typename P> struct RotaryGrads {
+  P *q, *k, *q_rot, *k_rot, *v, *v_rows;
+};
+template <typename P> struct Merge {
+  P *o, *o2;    // heads of d, or (o2 not null) two tensors of heads of d / 2
+  P *local;     // rows
+  P *gate;      // rows gate_row elements apart, or null
+  int64_t gate_row;
+};
+int vec_of(int dtype);  // elements of a piece
+void polarity_fwd(const Shape& s, const Polarity<const void>& a, void* q_same, void* q_opp, void* k_both, void* v_heads,
+                  int dtype, hipStream_t st);
+size_t polarity_bwd_workspace_bytes(const Shape& s, int dtype);
+void polarity_bwd(const Shape& s, const Polarity<const void>& a, const PolarityGrads<const void>& g, void* dqg, void* dkv,
+                  void* dpe, void* dscale, void* dpower, float* workspace, int dtype, hipStream_t st);
+// rot: fp32 [N, rot_channels / 2, 2] (cos, sin), channel c turned by entry c % rot_channels
+void rotary_fwd(const Shape& s, const void* qk, const void* x, const float* rot, int rot_channels, void* q, void* k,
+                void* q_rot, void* k_rot, void* v, int dtype, hipStream_t st);
+void rotary_bwd(const Shape& s, const void* qk, const float* rot, int rot_channels, const RotaryGrads<const void>& g,
+                void* dqk, void* dx, int dtype, hipStream_t st);
+void merge_fwd(const Shape& s, const Merge<const void>& a, void* out, int dtype, hipStream_t st);
+void merge_bwd(const Shape& s, const Merge<const void>& a, const void* dout, void* d_o, void* d_o2, void* dlocal, void* dgate,
+               int dtype, hipStream_t st);
+}  // namespace blocks
+
 // Piecewise (PISA) attention, forward only (fbla_piecewise.hip).
 namespace piecewise {
 size_t chunk_reduce_workspace_bytes(int64_t BH, int64_t T, int K, int V, int chunk, int dtype,

@@ -54,6 +54,13 @@ _SIGNATURES = {
     "fbla_dwconv_grad": (_i32, [_vp, _i64, _i64, _vp, _i64, _i64, _vp, _vp, _vp, _sz] + [_i64] * 3 + [_i32] * 4 + [_vp]),
     "fbla_linear_wgrad_workspace_bytes": (_sz, [_i64] + [_i32] * 3),
     "fbla_linear_wgrad": (_i32, [_vp, _i64, _vp, _i64, _vp, _vp, _vp, _sz, _i64] + [_i32] * 3 + [_vp]),
+    "fbla_polarity_fwd": (_i32, [_vp] * 9 + [_i64] * 3 + [_i32] * 3 + [_vp]),
+    "fbla_polarity_bwd_workspace_bytes": (_sz, [_i64] * 3 + [_i32] * 3),
+    "fbla_polarity_bwd": (_i32, [_vp] * 17 + [_sz] + [_i64] * 3 + [_i32] * 3 + [_vp]),
+    "fbla_rotary_fwd": (_i32, [_vp] * 3 + [_i32] + [_vp] * 5 + [_i64] * 2 + [_i32] * 3 + [_vp]),
+    "fbla_rotary_bwd": (_i32, [_vp] * 2 + [_i32] + [_vp] * 8 + [_i64] * 2 + [_i32] * 3 + [_vp]),
+    "fbla_merge_fwd": (_i32, [_vp] * 4 + [_i64, _vp] + [_i64] * 2 + [_i32] * 3 + [_vp]),
+    "fbla_merge_bwd": (_i32, [_vp] * 5 + [_i64] + [_vp] * 4 + [_i64] * 2 + [_i32] * 3 + [_vp]),
 }
 
 
@@ -487,3 +494,115 @@ def linear_wgrad(g, x, with_bias):
                                  code, _stream(dev))
     _check(rc, "fbla_linear_wgrad")
     return dw, db
+
+
+def _whole(*tensors):
+    """The tensors in contiguous, 16-byte aligned memory (copies where they are not)."""
+    return _aligned(*(t if t is None else t.contiguous() for t in tensors))
+
+
+def polarity_fwd(qg, kv, pe, scale, power, heads):
+    """Polarity features of qg [B, N, 2C] and kv [B, n, 2C]: (q_same, q_opp [B, heads, N, 2d], k_both [B, heads, n, 2d],
+    v [B, heads, n, d]).  pe [1, n, C], scale [1, 1, C], power [1, heads, 1, d]."""
+    _require_gpu(qg, kv, pe, scale, power)
+    qg, kv, pe, scale, power = _whole(qg, kv, pe, scale, power)
+    B, N, C2 = qg.shape
+    n, d = kv.shape[1], C2 // 2 // heads
+    q_same = torch.empty(B, heads, N, 2 * d, dtype=qg.dtype, device=qg.device)
+    q_opp = torch.empty_like(q_same)
+    k_both = torch.empty(B, heads, n, 2 * d, dtype=qg.dtype, device=qg.device)
+    v = torch.empty(B, heads, n, d, dtype=qg.dtype, device=qg.device)
+    with _on(qg.device):
+        rc = lib().fbla_polarity_fwd(_ptr(qg), _ptr(kv), _ptr(pe), _ptr(scale), _ptr(power), _ptr(q_same), _ptr(q_opp),
+                                     _ptr(k_both), _ptr(v), B, N, n, heads, d, dtype_code(qg), _stream(qg.device))
+    _check(rc, "fbla_polarity_fwd")
+    return q_same, q_opp, k_both, v
+
+
+def polarity_bwd(qg, kv, pe, scale, power, heads, dq_same, dq_opp, dk_both, dv, dv_rows, dgate):
+    """Gradients (dqg, dkv, dpe, dscale, dpower) of polarity_fwd; dv_rows [B, n, C] and dgate [B, N, C] are the gradients of
+    kv's and qg's second halves as rows."""
+    tensors = qg, kv, pe, scale, power, dq_same, dq_opp, dk_both, dv, dv_rows, dgate
+    _require_gpu(*tensors)
+    tensors = _whole(*tensors)
+    qg, kv, pe, scale, power = tensors[:5]
+    B, N, C2 = qg.shape
+    n, d, code, L = kv.shape[1], C2 // 2 // heads, dtype_code(qg), lib()
+    grads = tuple(torch.empty_like(t) for t in tensors[:5])
+    with _on(qg.device):
+        ws = _workspace(L.fbla_polarity_bwd_workspace_bytes(B, N, n, heads, d, code), qg.device)
+        rc = L.fbla_polarity_bwd(*(_ptr(t) for t in tensors + grads), _ptr(ws), ws.numel(), B, N, n, heads, d, code,
+                                 _stream(qg.device))
+    _check(rc, "fbla_polarity_bwd")
+    return grads
+
+
+def rotary_fwd(qk, x, rotations, heads):
+    """Rotary features of qk [B, N, 2C] and the values x [B, N, C]: (q, k, q_rot, k_rot, v) [B, heads, N, d]; rotations
+    fp32 [..., pairs, 2] over the N tokens."""
+    _require_gpu(qk, x, rotations)
+    qk, x, rotations = _whole(qk, x, rotations)
+    B, N, C = x.shape
+    out = tuple(torch.empty(B, heads, N, C // heads, dtype=x.dtype, device=x.device) for _ in range(5))
+    with _on(x.device):
+        rc = lib().fbla_rotary_fwd(_ptr(qk), _ptr(x), _ptr(rotations), 2 * rotations.shape[-2], *(_ptr(t) for t in out), B, N,
+                                   heads, C // heads, dtype_code(x), _stream(x.device))
+    _check(rc, "fbla_rotary_fwd")
+    return out
+
+
+def rotary_bwd(qk, rotations, heads, dq, dk, dq_rot, dk_rot, dv, dv_rows):
+    """Gradients (dqk, dx) of rotary_fwd; dv_rows [B, N, C] is added to the values' gradient."""
+    tensors = qk, rotations, dq, dk, dq_rot, dk_rot, dv, dv_rows
+    _require_gpu(*tensors)
+    qk, rotations, *rest = _whole(*tensors)
+    B, N, C = dv_rows.shape
+    dqk, dx = torch.empty_like(qk), torch.empty_like(rest[-1])
+    with _on(qk.device):
+        rc = lib().fbla_rotary_bwd(_ptr(qk), _ptr(rotations), 2 * rotations.shape[-2], *(_ptr(t) for t in rest), _ptr(dqk),
+                                   _ptr(dx), B, N, heads, C // heads, dtype_code(qk), _stream(qk.device))
+    _check(rc, "fbla_rotary_bwd")
+    return dqk, dx
+
+
+def merge_fwd(o, o2, local, gate):
+    """(heads + local) * gate as rows [B, N, C]: o [B, heads, N, d], or o and o2 [B, heads, N, d / 2] each; gate or None."""
+    _require_gpu(o, o2, local, gate)
+    o, o2, local = _whole(o, o2, local)
+    gate, _, gate_row = _rows_of_batches(gate)
+    B, heads, N, d = o.shape
+    d = d if o2 is None else 2 * d
+    out = torch.empty_like(local)
+    with _on(o.device):
+        rc = lib().fbla_merge_fwd(_ptr(o), _ptr(o2), _ptr(local), _ptr(gate), gate_row, _ptr(out), B, N, heads, d,
+                                  dtype_code(o), _stream(o.device))
+    _check(rc, "fbla_merge_fwd")
+    return out
+
+
+def merge_bwd(dout, heads, halves, o, o2, local, gate):
+    """Gradients (do, do2 or None, dlocal, dgate or None) of merge_fwd; without a gate o, o2 and local are not looked at."""
+    _require_gpu(dout, o, o2, local, gate)
+    dout, o, o2, local = _whole(dout, o, o2, local)
+    gate, _, gate_row = _rows_of_batches(gate)
+    B, N, C = dout.shape
+    d = C // heads
+    d_o = torch.empty(B, heads, N, d // 2 if halves else d, dtype=dout.dtype, device=dout.device)
+    d_o2 = torch.empty_like(d_o) if halves else None
+    dlocal, dgate = (torch.empty_like(dout), torch.empty_like(dout)) if gate is not None else (dout, None)
+    with _on(dout.device):
+        rc = lib().fbla_merge_bwd(_ptr(dout), _ptr(o), _ptr(o2), _ptr(local), _ptr(gate), gate_row, _ptr(d_o), _ptr(d_o2),
+                                  _ptr(dlocal) if gate is not None else None, _ptr(dgate), B, N, heads, d, dtype_code(dout),
+                                  _stream(dout.device))
+    _check(rc, "fbla_merge_bwd")
+    return d_o, d_o2, dlocal, dgate
+
+
+def _rows_of_batches(t):
+    """As _rows, for rows that lie at one distance over all batches; None stays None."""
+    if t is None:
+        return None, 0, 0
+    t, batch, row = _rows(t)
+    if batch != row * t.shape[1]:
+        t = t.clone(memory_format=torch.contiguous_format)
+    return t, t.stride(0), t.stride(1)

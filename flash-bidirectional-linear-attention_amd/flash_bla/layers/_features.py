@@ -1,0 +1,136 @@
+"""What the vision blocks do between their projections and the attention operators, one HIP launch a direction: polarity
+features (layers/polaformer.py:63-84), rotary features (layers/mlla.py:74-81) and heads merged back to rows
+(polaformer.py:92-104, mlla.py:88-92).  The reference composes them of torch operators; the compositions here are what runs
+when the kernels do not take a call, and what a gradient of the gradient is made of.
+"""
+import torch
+import torch.nn.functional as F
+
+from flash_bla import _hip
+from flash_bla.layers._common import merge_heads, split_heads
+from flash_bla.ops.feature_map import elu_plus_one
+from flash_bla.ops.projection import plain_tensors
+
+
+def _takes(heads, channels, unit, *tensors):
+    """Ordinary GPU tensors of one supported type whose heads (or their `unit` parts) are whole 16-byte pieces."""
+    x = tensors[0]
+    piece = unit * 16 // x.element_size()
+    return (x.is_cuda and x.dtype in (torch.float16, torch.bfloat16, torch.float32) and channels // heads % piece == 0 and
+            all(t is None or (t.dtype == x.dtype and t.device == x.device and 0 < t.numel() < 1 << 31) for t in tensors) and
+            plain_tensors(*tensors))
+
+
+def differentiable_gradients(formula, inputs, grads):
+    """Gradients of formula(*inputs) that can be differentiated again."""
+    wanted = [t for t in inputs if torch.is_tensor(t) and t.requires_grad]
+    with torch.enable_grad():
+        out = formula(*inputs)
+        pairs = [(o, g) for o, g in zip(out, grads) if o is not None and o.requires_grad]
+        got = iter(torch.autograd.grad([o for o, _ in pairs], wanted, [g for _, g in pairs], create_graph=True,
+                                       allow_unused=True))
+    return tuple(next(got) if torch.is_tensor(t) and t.requires_grad else None for t in inputs)
+
+
+def polarity_formula(qg, kv, pe, scale, power, heads):
+    q, gate = qg.chunk(2, dim=-1)
+    k, v_rows = kv.chunk(2, dim=-1)
+    q, k, v = (split_heads(t, heads) for t in (q / scale, (k + pe) / scale, v_rows))
+    q_pos, q_neg, k_pos, k_neg = (F.relu(t) ** power for t in (q, -q, k, -k))
+    return (torch.cat([q_pos, q_neg], dim=-1), torch.cat([q_neg, q_pos], dim=-1), torch.cat([k_pos, k_neg], dim=-1), v,
+            v_rows, gate)
+
+
+class PolarityFeaturesFunction(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, qg, kv, pe, scale, power, heads):
+        ctx.save_for_backward(qg, kv, pe, scale, power)
+        ctx.heads = heads
+        return (*_hip.polarity_fwd(qg, kv, pe, scale, power, heads), kv.chunk(2, dim=-1)[1], qg.chunk(2, dim=-1)[1])
+
+    @staticmethod
+    def backward(ctx, *grads):
+        inputs = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            return differentiable_gradients(polarity_formula, (*inputs, ctx.heads), grads)
+        return (*_hip.polarity_bwd(*inputs, ctx.heads, *grads), None)
+
+
+def polarity_features(qg, kv, pe, scale, power, heads):
+    """qg [B, N, 2C] (queries | gate), kv [B, n, 2C] (keys | values), pe [1, n, C], scale [1, 1, C], power [1, heads, 1, d]
+    (at least 1).  Returns (q_same, q_opp [B, heads, N, 2d], k_both [B, heads, n, 2d], v [B, heads, n, d], the values as rows
+    [B, n, C], the gate [B, N, C])."""
+    C = qg.shape[-1] // 2
+    if _takes(heads, C, 1, qg, kv, pe, scale, power) and pe.shape == (1, kv.shape[1], C) and scale.shape == (1, 1, C):
+        return PolarityFeaturesFunction.apply(qg, kv, pe, scale, power, heads)
+    return polarity_formula(qg, kv, pe, scale, power, heads)
+
+
+def rotate(x, rotations):
+    """Neighbouring channels of x as complex numbers times rotations [..., pairs, 2]; fp32."""
+    pairs = torch.view_as_complex(x.float().reshape(*x.shape[:-1], -1, 2))
+    return torch.view_as_real(torch.view_as_complex(rotations) * pairs).flatten(-2)
+
+
+def rotary_formula(qk, x, rotations, side, heads, features=lambda t: F.elu(t) + 1.0):
+    b, n, c = x.shape
+    q, k = features(qk).chunk(2, dim=-1)
+    rot = [rotate(t.reshape(b, side, side, c), rotations).reshape(b, n, c).to(x.dtype) for t in (q, k)]
+    return (*(split_heads(t, heads) for t in (q, k, *rot, x)), x)
+
+
+class RotaryFeaturesFunction(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, qk, x, rotations, side, heads):
+        ctx.save_for_backward(qk, x, rotations)
+        ctx.side, ctx.heads = side, heads
+        return (*_hip.rotary_fwd(qk, x, rotations, heads), x.view_as(x))
+
+    @staticmethod
+    def backward(ctx, *grads):
+        qk, x, rotations = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            return differentiable_gradients(rotary_formula, (qk, x, rotations, ctx.side, ctx.heads), grads)
+        return (*_hip.rotary_bwd(qk, rotations, ctx.heads, *grads), None, None, None)
+
+
+def rotary_features(qk, x, rotations, side, heads):
+    """qk [B, N, 2C] (queries | keys before elu + 1), x [B, N, C] (the values), N = side * side, rotations
+    [side, side, C / 2, 2].  Returns (q, k, q_rot, k_rot, v [B, heads, N, d], the values as rows)."""
+    if (_takes(heads, x.shape[-1], 1, x, qk) and plain_tensors(rotations) and rotations.dtype == torch.float32 and
+            rotations.device == x.device and not rotations.requires_grad and
+            rotations.shape == (side, side, x.shape[2] // 2, 2) and x.shape[1] == side * side):
+        return RotaryFeaturesFunction.apply(qk, x, rotations, side, heads)
+    return rotary_formula(qk, x, rotations, side, heads, elu_plus_one)
+
+
+def merge_formula(o, o2, local, gate):
+    out = merge_heads(o if o2 is None else torch.cat((o, o2), dim=-1)) + local
+    return (out if gate is None else out * gate,)
+
+
+class MergeHeadsFunction(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, o, o2, local, gate):
+        ctx.heads, ctx.halves = o.shape[1], o2 is not None
+        ctx.save_for_backward(*((o, o2, local, gate) if gate is not None else (None,) * 4))
+        return _hip.merge_fwd(o, o2, local, gate)
+
+    @staticmethod
+    def backward(ctx, g):
+        o, o2, local, gate = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            if gate is not None:
+                return differentiable_gradients(merge_formula, (o, o2, local, gate), (g,))
+            do = split_heads(g, ctx.heads)
+            return (*(do.chunk(2, dim=-1) if ctx.halves else (do, None)), g, None)
+        return _hip.merge_bwd(g, ctx.heads, ctx.halves, o, o2, local, gate)
+
+
+def merge_heads_with(o, o2, local, gate=None):
+    """(heads + local) * gate as rows [B, N, C]: o [B, heads, N, d], or the halves o, o2 [B, heads, N, d / 2] of each head;
+    local [B, N, C]; gate [B, N, C] or None."""
+    heads, C = o.shape[1], local.shape[-1]
+    if _takes(heads, C, 1 if o2 is None else 2, o, o2, local, gate):
+        return MergeHeadsFunction.apply(o, o2, local, gate)
+    return merge_formula(o, o2, local, gate)[0]

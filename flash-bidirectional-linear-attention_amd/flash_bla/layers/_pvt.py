@@ -26,11 +26,14 @@ class PvtLinearAttentionBase(nn.Module):
         self.positional_encoding = nn.Parameter(torch.zeros(1, num_patches // (sr_ratio * sr_ratio), dim))
         return head_dim
 
-    def _keys_values(self, x, H, W):
+    def _joint_keys_values(self, x, H, W):
         B, N, C = x.shape
         if self.sr_ratio > 1:
             x = self.norm(self.sr(x.transpose(1, 2).reshape(B, C, H, W)).flatten(2).transpose(1, 2))
-        k, v = self.kv(x).chunk(2, dim=-1)
+        return self.kv(x)
+
+    def _keys_values(self, x, H, W):
+        k, v = self._joint_keys_values(x, H, W).chunk(2, dim=-1)
         return k + self.positional_encoding, v
 
     def _value_conv(self, v, N, H, W):

@@ -4,6 +4,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from flash_bla.layers._common import check_mode, merge_heads, split_heads, torch_linear_attention
+from flash_bla.layers._features import merge_heads_with
 from flash_bla.layers._pvt import PvtLinearAttentionBase
 from flash_bla.ops.linear_attn.fused import linear_attention
 from flash_bla.ops.projection import TokenLinear
@@ -33,7 +34,7 @@ class FocusedLinearAttention(PvtLinearAttentionBase):
         v_rows = v
         q, k, v = (split_heads(t, self.num_heads) for t in (q, k, v))
         if fast:
-            out = merge_heads(linear_attention(q, k, v)) + self._value_conv_tokens(v_rows, N, H, W)
+            out = merge_heads_with(linear_attention(q, k, v), None, self._value_conv_tokens(v_rows, N, H, W))
         else:
             out = merge_heads(torch_linear_attention(q, k, v)) + self._value_conv(v, N, H, W)
         return self.proj_drop(self.proj(out))

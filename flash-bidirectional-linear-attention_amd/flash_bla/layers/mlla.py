@@ -3,7 +3,8 @@ elu+1 features, 2-D rotary numerator features, depth-wise conv positional term."
 import torch
 import torch.nn as nn
 
-from flash_bla.layers._common import check_mode, merge_heads, split_heads, torch_linear_attention
+from flash_bla.layers._common import check_mode, merge_heads, split_heads, torch_linear_attention, untouched
+from flash_bla.layers._features import merge_heads_with, rotary_features, rotate
 from flash_bla.ops.depthwise import depthwise_conv_tokens
 from flash_bla.ops.feature_map import elu_plus_one
 from flash_bla.ops.linear_attn.decoupled import decoupled_la
@@ -25,8 +26,7 @@ class RoPE(nn.Module):
         self.register_buffer('rotations', torch.stack([angles.cos(), angles.sin()], dim=-1))
 
     def forward(self, x):
-        pairs = torch.view_as_complex(x.float().reshape(*x.shape[:-1], -1, 2))
-        return torch.view_as_real(torch.view_as_complex(self.rotations) * pairs).flatten(-2)
+        return rotate(x, self.rotations)
 
 
 class MambaLikeLinearAttention(nn.Module):
@@ -43,15 +43,16 @@ class MambaLikeLinearAttention(nn.Module):
         b, n, c = x.shape
         side = int(n ** 0.5)
         qk = self.qk(x)
-        if fast:  # one launch over the joint projection
-            q, k = elu_plus_one(qk).chunk(2, dim=-1)
+        if fast and untouched(self.rope, RoPE):
+            q, k, q_rope, k_rope, v, x_rows = rotary_features(qk, x, self.rope.rotations, side, self.num_heads)
         else:
-            q, k = (self.elu(t) + 1.0 for t in qk.chunk(2, dim=-1))
-        rot = [self.rope(t.reshape(b, side, side, c)).reshape(b, n, c).to(x.dtype) for t in (q, k)]
-        q, k, v, q_rope, k_rope = (split_heads(t, self.num_heads) for t in (q, k, x, *rot))
+            q, k = elu_plus_one(qk).chunk(2, dim=-1) if fast else (self.elu(t) + 1.0 for t in qk.chunk(2, dim=-1))
+            rot = [self.rope(t.reshape(b, side, side, c)).reshape(b, n, c).to(x.dtype) for t in (q, k)]
+            q, k, v, q_rope, k_rope = (split_heads(t, self.num_heads) for t in (q, k, x, *rot))
+            x_rows = x
         if fast:
             out = decoupled_la(q, k, q_rope, k_rope, v, scale=n ** -1.0)
-            return merge_heads(out) + depthwise_conv_tokens(x, self.lepe, side, side)
+            return merge_heads_with(out, None, depthwise_conv_tokens(x_rows, self.lepe, side, side))
         out = torch_linear_attention(q, k, v, q_num=q_rope, k_num=k_rope)
         grid = merge_heads(v).reshape(b, side, side, c).permute(0, 3, 1, 2)
         return merge_heads(out) + self.lepe(grid).permute(0, 2, 3, 1).reshape(b, n, c)

@@ -6,7 +6,8 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from flash_bla.layers._common import check_mode, merge_heads, split_heads, torch_linear_attention
+from flash_bla.layers._common import check_mode, merge_heads, torch_linear_attention
+from flash_bla.layers._features import merge_heads_with, polarity_features, polarity_formula
 from flash_bla.layers._pvt import PvtLinearAttentionBase
 from flash_bla.ops.linear_attn.paired import paired_linear_attention
 from flash_bla.ops.projection import TokenLinear
@@ -25,22 +26,17 @@ class PolaLinearAttention(PvtLinearAttentionBase):
     def forward(self, x, H, W, mode='triton'):
         fast = check_mode(mode)
         N = x.shape[1]
-        q, gate = self.qg(x).chunk(2, dim=-1)
-        k, v = self._keys_values(x, H, W)
         scale = F.softplus(self.scale)
         power = 1 + self.alpha * torch.sigmoid(self.power)
-        v_rows = v
-        q, k, v = (split_heads(t, self.num_heads) for t in (q / scale, k / scale, v))
-        q_pos, q_neg, k_pos, k_neg = (F.relu(t) ** power for t in (q, -q, k, -k))
-        q_same = torch.cat([q_pos, q_neg], dim=-1)
-        q_opp = torch.cat([q_neg, q_pos], dim=-1)
-        k_both = torch.cat([k_pos, k_neg], dim=-1)
+        features = polarity_features if fast else polarity_formula
+        q_same, q_opp, k_both, v, v_rows, gate = features(self.qg(x), self._joint_keys_values(x, H, W),
+                                                          self.positional_encoding, scale, power, self.num_heads)
         if fast:  # both pairings on one state pass over the shared keys and values
-            out = torch.cat(paired_linear_attention(q_same, q_opp, k_both, v), dim=-1)
+            o_same, o_opp = paired_linear_attention(q_same, q_opp, k_both, v)
+            out = merge_heads_with(o_same, o_opp, self._value_conv_tokens(v_rows, N, H, W), gate)
         else:
             v_same, v_opp = v.chunk(2, dim=-1)
             out = torch.cat([torch_linear_attention(q_same, k_both, v_same),
                              torch_linear_attention(q_opp, k_both, v_opp)], dim=-1)
-        local = self._value_conv_tokens(v_rows, N, H, W) if fast else self._value_conv(v, N, H, W)
-        out = (merge_heads(out) + local) * gate
+            out = (merge_heads(out) + self._value_conv(v, N, H, W)) * gate
         return self.proj_drop(self.proj(out))

@@ -4,6 +4,7 @@ import torch
 import torch.nn as nn
 
 from flash_bla.layers._common import check_mode, merge_heads, split_heads, torch_linear_attention
+from flash_bla.layers._features import merge_heads_with
 from flash_bla.layers.mlla import RoPE
 from flash_bla.ops.depthwise import depthwise_conv_tokens
 from flash_bla.ops.linear_attn.decoupled import decoupled_la
@@ -40,8 +41,8 @@ class RALALinearAttention(nn.Module):
         k_rope = self.rope(k.reshape(grid)).reshape(k.shape).to(x.dtype).contiguous()
         if fast:
             out = decoupled_la(q, k.contiguous(), q_rope, k_rope, v, scale=n ** -1.0)
-        else:
-            out = torch_linear_attention(q, k, v, q_num=q_rope, k_num=k_rope)
+            return self.proj(merge_heads_with(out, None, lepe, gate))
+        out = torch_linear_attention(q, k, v, q_num=q_rope, k_num=k_rope)
         return self.proj((merge_heads(out) + lepe) * gate)
 
     def extra_repr(self):

@@ -288,6 +288,41 @@ size_t fbla_linear_wgrad_workspace_bytes(int64_t tokens, int M, int N, int dtype
 int fbla_linear_wgrad(const void* g, int64_t g_row, const void* x, int64_t x_row, void* dw, void* db, void* workspace,
                       size_t workspace_bytes, int64_t tokens, int M, int N, int dtype, void* stream);
 
+/* What the vision blocks do between their projections and the attention operators.  Rows are [B, N, C], C = heads * d,
+ * joint projections [B, N, 2 C], heads [B, heads, N, width]; contiguous, one element type, d in whole 16-byte pieces.
+ *
+ * Polarity features (flash_bla/layers/polaformer.py:63-84): with y = q / scale of qg's first half (the second half is the
+ * gate and is not read) or (k + pe) / scale of kv's first half, pos = relu(y)^power and neg = relu(-y)^power;
+ * q_same = pos | neg, q_opp = neg | pos, k_both = pos | neg as heads of 2 d, v_heads = kv's second half as heads of d.
+ * pe [Nk, C], scale [C], power [heads, d] (at least 1).  The backward takes the gradients of the four outputs, of the
+ * values as rows (dv_rows [B, Nk, C], added to dv) and of the gate as rows (dgate, copied into dqg). */
+int fbla_polarity_fwd(const void* qg, const void* kv, const void* pe, const void* scale, const void* power, void* q_same,
+                      void* q_opp, void* k_both, void* v_heads, int64_t B, int64_t N, int64_t Nk, int heads, int d, int dtype,
+                      void* stream);
+size_t fbla_polarity_bwd_workspace_bytes(int64_t B, int64_t N, int64_t Nk, int heads, int d, int dtype);
+int fbla_polarity_bwd(const void* qg, const void* kv, const void* pe, const void* scale, const void* power,
+                      const void* dq_same, const void* dq_opp, const void* dk_both, const void* dv_heads, const void* dv_rows,
+                      const void* dgate, void* dqg, void* dkv, void* dpe, void* dscale, void* dpower, void* workspace,
+                      size_t workspace_bytes, int64_t B, int64_t N, int64_t Nk, int heads, int d, int dtype, void* stream);
+
+/* Rotary features (flash_bla/layers/mlla.py:74-81): q, k = elu(x) + 1 of the halves of qk, q_rot, k_rot = their channel
+ * pairs turned by rot (fp32 [N, rot_channels / 2, 2]: cos, sin; channel c uses entry c % rot_channels), v = x, all as heads.
+ * The backward adds dv_rows [B, N, C] to the values' gradient. */
+int fbla_rotary_fwd(const void* qk, const void* x, const float* rot, int rot_channels, void* q, void* k, void* q_rot,
+                    void* k_rot, void* v, int64_t B, int64_t N, int heads, int d, int dtype, void* stream);
+int fbla_rotary_bwd(const void* qk, const float* rot, int rot_channels, const void* dq, const void* dk, const void* dq_rot,
+                    const void* dk_rot, const void* dv, const void* dv_rows, void* dqk, void* dx, int64_t B, int64_t N,
+                    int heads, int d, int dtype, void* stream);
+
+/* Heads back to rows: out = (heads + local) * gate (flash_bla/layers/polaformer.py:92-104; without a gate mlla.py:88-92).
+ * o2 not NULL: the channels of a head are the halves o | o2 of d / 2 each (whole 16-byte pieces).  gate: rows gate_row
+ * elements apart, or NULL; then the backward writes d_o alone (dlocal is dout). */
+int fbla_merge_fwd(const void* o, const void* o2, const void* local, const void* gate, int64_t gate_row, void* out, int64_t B,
+                   int64_t N, int heads, int d, int dtype, void* stream);
+int fbla_merge_bwd(const void* dout, const void* o, const void* o2, const void* local, const void* gate, int64_t gate_row,
+                   void* d_o, void* d_o2, void* dlocal, void* dgate, int64_t B, int64_t N, int heads, int d, int dtype,
+                   void* stream);
+
 #ifdef __cplusplus
 }
 #endif

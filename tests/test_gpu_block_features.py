@@ -1,0 +1,132 @@
+"""The vision blocks' fused elementwise steps against their torch compositions in float64: channel counts that fill one
+64-piece block of the gradient kernel, end inside one and need several, heads of one piece and more, fewer keys than queries,
+one token, batches that split into groups, zeros and negative zeros, gates that are part of a wider row.
+
+Bounds: a value is computed in fp32 from inputs that are exact in float64 and rounded once (u); the powers' exponent
+p log2 a, at most 2^6 here, carries the fp32 functions' 2^-22 to 2^-16 of the value; a turned
+channel is a difference of two products, each off by a few 2^-24 of the pair's length: 2^-22 of the largest result; sums over
+tokens (a few hundred terms) stay within 2^-16 of the largest result."""
+import pytest
+import torch
+
+from helpers import UNIT_ROUNDOFF
+from flash_bla.layers import MambaLikeLinearAttention, PolaLinearAttention
+from flash_bla.layers import _features as features
+
+DTYPES = [torch.float16, torch.bfloat16, torch.float32]
+
+
+def _check(function, formula, inputs, dtype):
+    """Outputs and gradients of function(*inputs) against formula in float64 on the same values."""
+    rest = [t for t in inputs if not torch.is_tensor(t)]
+    ours = [t.detach().requires_grad_(t.requires_grad) for t in inputs if torch.is_tensor(t)]
+    exact = [t.detach().double().requires_grad_(t.requires_grad) for t in ours]
+    out, want = function(*ours, *rest), formula(*exact, *rest)
+    assert len(out) == len(want)
+    grads = [torch.randn(o.shape, device="cuda").to(dtype) for o in out]
+    leaves = [t for t in ours if t.requires_grad]
+    got = torch.autograd.grad(out, leaves, grads)
+    ref = torch.autograd.grad(want, [t for t in exact if t.requires_grad], [g.double() for g in grads])
+    u = UNIT_ROUNDOFF[dtype]
+    for name, a, b in [("out", a, b) for a, b in zip(out, want)] + [("grad", a, b) for a, b in zip(got, ref)]:
+        assert a.shape == b.shape and a.dtype == dtype
+        slack = 2.0 ** -16 * (b.abs() if name == "out" else b.abs().max()) + 2.0 ** -22 * b.abs().max()
+        assert ((a.double() - b).abs() <= u * b.abs() + slack).all(), (name, (a.double() - b).abs().max())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("B,N,Nk,heads,d", [(1, 1, 1, 1, 8), (2, 33, 33, 8, 64), (3, 20, 5, 5, 24), (9, 49, 49, 2, 32),
+                                            (2, 7, 7, 10, 64), (37, 4, 1, 3, 40)])
+def test_polarity_features(B, N, Nk, heads, d, dtype):
+    torch.manual_seed(N * heads)
+    C = heads * d
+    # half-width inputs: fifth powers of the largest stay inside fp16's range
+    values = lambda *shape: (0.5 * torch.randn(shape, device="cuda")).to(dtype).requires_grad_()  # noqa: E731
+    qg, kv, pe = values(B, N, 2 * C), values(B, Nk, 2 * C), values(1, Nk, C)
+    with torch.no_grad():
+        qg.view(-1)[::7] = 0.0
+        qg.view(-1)[1::11] = -0.0
+    scale = (0.5 + torch.rand(1, 1, C, device="cuda")).to(dtype).requires_grad_()
+    power = (1 + 4 * torch.rand(1, heads, 1, d, device="cuda")).to(dtype).requires_grad_()
+    assert features._takes(heads, C, 1, qg, kv, pe, scale, power)
+
+    _check(features.polarity_features, features.polarity_formula, (qg, kv, pe, scale, power, heads), dtype)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("B,side,heads,d", [(1, 1, 1, 8), (3, 5, 3, 24), (2, 14, 2, 32), (2, 3, 10, 64)])
+def test_rotary_features(B, side, heads, d, dtype):
+    torch.manual_seed(side)
+    C = heads * d
+    qk = torch.randn(B, side * side, 2 * C, device="cuda").to(dtype).requires_grad_()
+    x = torch.randn(B, side * side, C, device="cuda").to(dtype).requires_grad_()
+    angles = torch.randn(side, side, C // 2, device="cuda")
+    rotations = torch.stack([angles.cos(), angles.sin()], dim=-1)
+
+    def exact(qk, x, side, heads):
+        q, k = (torch.nn.functional.elu(qk) + 1).chunk(2, dim=-1)
+        cos, sin = rotations.double().reshape(side * side, C // 2, 2).unbind(-1)
+        turn = lambda t: torch.stack([t[..., ::2] * cos - t[..., 1::2] * sin,  # noqa: E731
+                                      t[..., ::2] * sin + t[..., 1::2] * cos], dim=-1).flatten(-2)
+        return (*(features.split_heads(t, heads) for t in (q, k, turn(q), turn(k), x)), x)
+    _check(lambda qk, x, side, heads: features.rotary_features(qk, x, rotations, side, heads), exact, (qk, x, side, heads),
+           dtype)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("halves", [False, True])
+@pytest.mark.parametrize("gated", [False, True])
+@pytest.mark.parametrize("B,N,heads,d", [(1, 1, 1, 16), (3, 21, 5, 48), (2, 50, 10, 64)])
+def test_merged_heads(B, N, heads, d, gated, halves, dtype):
+    torch.manual_seed(N)
+    values = lambda *shape: torch.randn(shape, device="cuda").to(dtype).requires_grad_()  # noqa: E731
+    tensors = [values(B, heads, N, d // 2 if halves else d) for _ in range(1 + halves)] + [values(B, N, heads * d)]
+    tensors += [values(B, N, 4 * heads * d)] if gated else []
+
+    def arguments(*t):
+        return t[0], t[1] if halves else None, t[1 + halves], t[-1][..., -heads * d:] if gated else None
+    _check(lambda *t: (features.merge_heads_with(*arguments(*t)),), lambda *t: features.merge_formula(*arguments(*t)),
+           tensors, dtype)
+
+
+@pytest.mark.gpu
+def test_not_a_number_and_infinity_pass_through():
+    """A NaN reaches both parts, an infinity its own, as relu and pow give them."""
+    x = torch.randn(1, 1, 64, device="cuda")
+    x[0, 0, 3], x[0, 0, 4], x[0, 0, 5] = float("nan"), float("inf"), -float("inf")
+    pe, one = torch.zeros(1, 1, 32, device="cuda"), torch.ones(1, 1, 32, device="cuda")
+    args = (x, x.clone(), pe, one, 2 * one.reshape(1, 1, 1, 32), 1)
+    for a, b in zip(features.polarity_features(*args), features.polarity_formula(*args)):
+        torch.testing.assert_close(a, b, equal_nan=True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("make,extra", [(lambda: PolaLinearAttention(24, 4, num_heads=2), (2, 2)),
+                                        (lambda: MambaLikeLinearAttention(24, (2, 2), 2), ())])
+def test_heads_that_are_no_whole_pieces_run_as_torch_operators(make, extra):
+    """12 channels a head in fp16: no 16-byte pieces, the compositions run."""
+    torch.manual_seed(0)
+    block = make().cuda().half()
+    if hasattr(block, "rope"):
+        block.rope.float()
+    x = torch.randn(2, 4, 24, device="cuda", dtype=torch.float16, requires_grad=True)
+    y = block(x, *extra)
+    y.square().sum().backward()
+    exact = block.double()(x.detach().double(), *extra, mode="torch") if extra else None
+    assert torch.isfinite(x.grad).all() and (exact is None or (y.double() - exact).norm() <= 5e-3 * exact.norm())
+
+
+@pytest.mark.gpu
+def test_gradient_of_the_gradient():
+    torch.manual_seed(0)
+    results = []
+    for f in (features.merge_heads_with, lambda *t: features.merge_formula(*t)[0]):
+        t = [torch.linspace(-1, 1, 64, device="cuda").reshape(s).requires_grad_()
+             for s in ((1, 2, 4, 8), (1, 4, 16), (1, 4, 16))]
+        g = torch.autograd.grad(f(t[0], None, t[1], t[2]).square().sum(), t, create_graph=True)
+        results.append(torch.autograd.grad(sum(x.square().sum() for x in g), t))
+    for a, b in zip(*results):
+        torch.testing.assert_close(a, b)
