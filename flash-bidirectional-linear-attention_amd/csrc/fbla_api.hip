@@ -928,4 +928,34 @@ int fbla_merge_bwd(const void* dout, const void* o, const void* o2, const void* 
   return check_launch(what);
 }
 
+static int check_interpolate(const char* what, int64_t B, int64_t from, int64_t to, int C, int dtype) {
+  blocks::Shape s;
+  const int rc = check_blocks(what, s, B, from, to, 1, C, 1, dtype);
+  if (rc == kOk && from * to >= (1 << 28)) {  // the places are whole numbers of 32 bits
+    set_error("%s: too many tokens (%lld to %lld)", what, (long long)from, (long long)to);
+    return kErrUnsupported;
+  }
+  return rc;
+}
+
+int fbla_interpolate_fwd(const void* x, int64_t x_batch, int64_t x_row, void* y, int64_t B, int64_t from, int64_t to, int C,
+                         int dtype, void* stream) {
+  const char* what = "fbla_interpolate_fwd";
+  int rc = check_interpolate(what, B, from, to, C, dtype);
+  if (rc == kOk) rc = check_tensors(what, {x, y});
+  if (rc == kOk) rc = check_row_strides(what, C, dtype, {x_batch, x_row});
+  if (rc != kOk) return rc;
+  blocks::interpolate_fwd(x, x_batch, x_row, (int)B, (int)from, (int)to, C, y, dtype, (hipStream_t)stream);
+  return check_launch(what);
+}
+
+int fbla_interpolate_bwd(const void* g, void* dx, int64_t B, int64_t from, int64_t to, int C, int dtype, void* stream) {
+  const char* what = "fbla_interpolate_bwd";
+  int rc = check_interpolate(what, B, from, to, C, dtype);
+  if (rc == kOk) rc = check_tensors(what, {g, dx});
+  if (rc != kOk) return rc;
+  blocks::interpolate_bwd(g, (int)B, (int)from, (int)to, C, dx, dtype, (hipStream_t)stream);
+  return check_launch(what);
+}
+
 }  // extern "C"

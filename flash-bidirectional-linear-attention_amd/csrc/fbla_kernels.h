@@ -270,6 +270,10 @@ void rotary_bwd(const Shape& s, const void* qk, const float* rot, int rot_channe
 void merge_fwd(const Shape& s, const Merge<const void>& a, void* out, int dtype, hipStream_t st);
 void merge_bwd(const Shape& s, const Merge<const void>& a, const void* dout, void* d_o, void* d_o2, void* dlocal, void* dgate,
                int dtype, hipStream_t st);
+// x: token t of batch b at x + b * x_batch + t * x_row; y [B, to, C], g likewise, dx [B, from, C]; from * to below 2^28
+void interpolate_fwd(const void* x, int64_t x_batch, int64_t x_row, int B, int from, int to, int C, void* y, int dtype,
+                     hipStream_t st);
+void interpolate_bwd(const void* g, int B, int from, int to, int C, void* dx, int dtype, hipStream_t st);
 }  // namespace blocks
 
 // Piecewise (PISA) attention, forward only (fbla_piecewise.hip).

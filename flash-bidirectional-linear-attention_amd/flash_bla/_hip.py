@@ -61,6 +61,8 @@ _SIGNATURES = {
     "fbla_rotary_bwd": (_i32, [_vp] * 2 + [_i32] + [_vp] * 8 + [_i64] * 2 + [_i32] * 3 + [_vp]),
     "fbla_merge_fwd": (_i32, [_vp] * 4 + [_i64, _vp] + [_i64] * 2 + [_i32] * 3 + [_vp]),
     "fbla_merge_bwd": (_i32, [_vp] * 5 + [_i64] + [_vp] * 4 + [_i64] * 2 + [_i32] * 3 + [_vp]),
+    "fbla_interpolate_fwd": (_i32, [_vp, _i64, _i64, _vp] + [_i64] * 3 + [_i32] * 2 + [_vp]),
+    "fbla_interpolate_bwd": (_i32, [_vp] * 2 + [_i64] * 3 + [_i32] * 2 + [_vp]),
 }
 
 
@@ -606,3 +608,27 @@ def _rows_of_batches(t):
     if batch != row * t.shape[1]:
         t = t.clone(memory_format=torch.contiguous_format)
     return t, t.stride(0), t.stride(1)
+
+
+def interpolate_fwd(x, tokens):
+    """Token rows x [B, n, C] linearly interpolated to [B, tokens, C]."""
+    _require_gpu(x)
+    x, x_batch, x_row = _rows(x)
+    B, n, C = x.shape
+    y = torch.empty(B, tokens, C, dtype=x.dtype, device=x.device)
+    with _on(x.device):
+        rc = lib().fbla_interpolate_fwd(_ptr(x), x_batch, x_row, _ptr(y), B, n, tokens, C, dtype_code(x), _stream(x.device))
+    _check(rc, "fbla_interpolate_fwd")
+    return y
+
+
+def interpolate_bwd(g, n):
+    """Gradient [B, n, C] of interpolate_fwd from the output's gradient g [B, tokens, C]."""
+    _require_gpu(g)
+    g, = _whole(g)
+    B, tokens, C = g.shape
+    dx = torch.empty(B, n, C, dtype=g.dtype, device=g.device)
+    with _on(g.device):
+        rc = lib().fbla_interpolate_bwd(_ptr(g), _ptr(dx), B, n, tokens, C, dtype_code(g), _stream(g.device))
+    _check(rc, "fbla_interpolate_bwd")
+    return dx

@@ -134,3 +134,29 @@ def merge_heads_with(o, o2, local, gate=None):
     if _takes(heads, C, 1 if o2 is None else 2, o, o2, local, gate):
         return MergeHeadsFunction.apply(o, o2, local, gate)
     return merge_formula(o, o2, local, gate)[0]
+
+
+def interpolate_formula(rows, tokens):
+    return (F.interpolate(rows.transpose(1, 2), size=tokens, mode='linear').transpose(1, 2),)
+
+
+class InterpolateTokensFunction(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, rows, tokens):
+        ctx.n = rows.shape[1]
+        return _hip.interpolate_fwd(rows, tokens)
+
+    @staticmethod
+    def backward(ctx, g):
+        if torch.is_grad_enabled():  # linear in the rows: the gradient is that of any rows
+            rows = torch.zeros(g.shape[0], ctx.n, g.shape[2], dtype=g.dtype, device=g.device, requires_grad=True)
+            return differentiable_gradients(interpolate_formula, (rows, g.shape[1]), (g,))
+        return _hip.interpolate_bwd(g, ctx.n), None
+
+
+def interpolate_tokens(rows, tokens):
+    """Token rows [B, n, C] linearly interpolated to [B, tokens, C] (corners not aligned)."""
+    if (_takes(1, rows.shape[-1], 1, rows) and tokens > 0 and rows.shape[1] * tokens < 1 << 28 and
+            rows.shape[0] * tokens * rows.shape[2] < 1 << 31):
+        return InterpolateTokensFunction.apply(rows, tokens)
+    return interpolate_formula(rows, tokens)[0]

@@ -5,6 +5,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from flash_bla.layers._features import interpolate_tokens
 from flash_bla.ops.depthwise import depthwise_conv_tokens
 from flash_bla.ops.projection import TokenLinear
 
@@ -48,5 +49,5 @@ class PvtLinearAttentionBase(nn.Module):
     def _value_conv_tokens(self, v, N, H, W):
         """The same on token rows (B, n, C), without splitting heads: one filter per channel of a head."""
         if self.sr_ratio > 1:
-            v = F.interpolate(v.transpose(1, 2), size=N, mode='linear').transpose(1, 2)
+            v = interpolate_tokens(v, N)
         return depthwise_conv_tokens(v, self.dwc, H, W)

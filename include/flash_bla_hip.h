@@ -323,6 +323,14 @@ int fbla_merge_bwd(const void* dout, const void* o, const void* o2, const void* 
                    void* d_o, void* d_o2, void* dlocal, void* dgate, int64_t B, int64_t N, int heads, int d, int dtype,
                    void* stream);
 
+/* Linear interpolation of token rows from `from` to `to` tokens, the corners not aligned: what
+ * F.interpolate(mode='linear', size=to) gives for the transposed rows (flash_bla/layers/focused_la.py:88-91,
+ * polaformer.py:95-98).  x: token t of batch b is the C elements at x + b * x_batch + t * x_row (whole 16-byte pieces, at
+ * least C); y and g [B, to, C], dx [B, from, C] contiguous; from * to below 2^28, C in whole 16-byte pieces. */
+int fbla_interpolate_fwd(const void* x, int64_t x_batch, int64_t x_row, void* y, int64_t B, int64_t from, int64_t to, int C,
+                         int dtype, void* stream);
+int fbla_interpolate_bwd(const void* g, void* dx, int64_t B, int64_t from, int64_t to, int C, int dtype, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

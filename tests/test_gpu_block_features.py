@@ -93,6 +93,17 @@ def test_merged_heads(B, N, heads, d, gated, halves, dtype):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("B,n,tokens,C", [(1, 1, 1, 8), (2, 1, 5, 24), (3, 7, 28, 64), (2, 49, 200, 40), (1, 30, 11, 16),
+                                          (2, 5, 5, 8), (1, 3, 1, 8)])
+def test_interpolated_tokens(B, n, tokens, C, dtype):
+    torch.manual_seed(n)
+    kv = torch.randn(B, n, 2 * C, device="cuda").to(dtype).requires_grad_()
+    _check(lambda t: (features.interpolate_tokens(t[..., C:], tokens),),
+           lambda t: features.interpolate_formula(t[..., C:], tokens), [kv], dtype)
+
+
+@pytest.mark.gpu
 def test_not_a_number_and_infinity_pass_through():
     """A NaN reaches both parts, an infinity its own, as relu and pow give them."""
     x = torch.randn(1, 1, 64, device="cuda")
