@@ -31,9 +31,3 @@ def check_mode(mode):
     if mode != "torch" and mode not in FAST_MODES:
         raise NotImplementedError(f"unknown mode {mode!r}")
     return mode != "torch"
-
-
-def untouched(module, kind):
-    """Whether `module` is a plain `kind` that a fused path may stand in for: no subclass, no hooks of its own."""
-    return type(module) is kind and not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or
-                                         module._backward_pre_hooks)

@@ -3,8 +3,9 @@ elu+1 features, 2-D rotary numerator features, depth-wise conv positional term."
 import torch
 import torch.nn as nn
 
-from flash_bla.layers._common import check_mode, merge_heads, split_heads, torch_linear_attention, untouched
+from flash_bla.layers._common import check_mode, merge_heads, split_heads, torch_linear_attention
 from flash_bla.layers._features import merge_heads_with, rotary_features, rotate
+from flash_bla.ops._check import untouched
 from flash_bla.ops.depthwise import depthwise_conv_tokens
 from flash_bla.ops.feature_map import elu_plus_one
 from flash_bla.ops.linear_attn.decoupled import decoupled_la

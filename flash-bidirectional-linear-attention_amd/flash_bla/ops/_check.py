@@ -33,3 +33,9 @@ def check_dense(name, q, k, v, extra=()):
         raise TypeError(f"{name}: dtype must be float16, bfloat16, or float32")
     if not (0 < q.shape[-1] <= 128 and 0 < v.shape[-1] <= 128):
         raise ValueError(f"{name}: key_dim and value_dim must be between 1 and 128")
+
+
+def untouched(module, kind):
+    """Whether `module` is a plain `kind` that a fused path may stand in for: no subclass, no hooks of its own."""
+    return type(module) is kind and not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or
+                                         module._backward_pre_hooks)

@@ -5,26 +5,36 @@ transposes back; the kernels here read and write the tokens in place and share o
 `Cw` apart, so heads need no batch of their own.
 """
 import torch
+import torch.nn as nn
 import torch.nn.functional as F
 
 from flash_bla import _hip
+from flash_bla.ops._check import untouched
+from flash_bla.ops.projection import plain_tensors
 
 
 class DepthwiseConvTokensFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, weight, bias, H, W):
-        weight = weight.contiguous()
         ctx.save_for_backward(x, weight)
         ctx.grid, ctx.with_bias = (H, W), bias is not None
-        return _hip.dwconv_fwd(x, weight, None if bias is None else bias.contiguous(), H, W)
+        return _hip.dwconv_fwd(x, weight.contiguous(), None if bias is None else bias.contiguous(), H, W)
 
     @staticmethod
-    @torch.autograd.function.once_differentiable
     def backward(ctx, g):
         x, weight = ctx.saved_tensors
         dx = dw = db = None
+        if torch.is_grad_enabled():  # the gradient is to be differentiated again: of torch's convolution
+            bias = torch.zeros(weight.shape[0], dtype=g.dtype, device=g.device, requires_grad=True)
+            with torch.enable_grad():
+                y = _convolution_of_images(x, *ctx.grid, weight.shape[0], lambda images: F.conv2d(
+                    images, weight, bias, padding=weight.shape[-1] // 2, groups=weight.shape[0]))
+                leaves = [t for t in (x, weight, bias) if t.requires_grad]
+                got = iter(torch.autograd.grad(y, leaves, g, create_graph=True))
+            dx, dw, db = (next(got) if t.requires_grad else None for t in (x, weight, bias))
+            return dx, dw, db if ctx.with_bias else None, None, None
         if ctx.needs_input_grad[0]:
-            dx = _hip.dwconv_fwd(g, weight, None, *ctx.grid, flip=True)
+            dx = _hip.dwconv_fwd(g, weight.contiguous(), None, *ctx.grid, flip=True)
         if ctx.needs_input_grad[1] or (ctx.with_bias and ctx.needs_input_grad[2]):
             dw, db = _hip.dwconv_grad(x, g, weight, *ctx.grid, ctx.with_bias)
         return dx, dw, db, None, None
@@ -32,11 +42,12 @@ class DepthwiseConvTokensFunction(torch.autograd.Function):
 
 def runs_on_tokens(x, conv):
     """Whether the kernels take the depth-wise nn.Conv2d `conv` on token rows x: GPU tensors of one supported type, odd
-    square filters of 3 to 7 taps a side, stride 1, "same" zero padding, whole 16-byte pieces of channels."""
+    square filters of 3 to 7 taps a side, stride 1, "same" zero padding, whole 16-byte pieces of channels; a module
+    without hooks."""
     K = conv.kernel_size[0]
     w = conv.weight
-    return (x.is_cuda and x.numel() > 0 and x.dtype in (torch.float16, torch.bfloat16, torch.float32) and
-            w.dtype == x.dtype and w.device == x.device and conv.kernel_size == (K, K) and K in (3, 5, 7) and
+    return (untouched(conv, nn.Conv2d) and plain_tensors(x, w, conv.bias) and x.is_cuda and x.numel() > 0 and
+            x.dtype in (torch.float16, torch.bfloat16, torch.float32) and w.dtype == x.dtype and w.device == x.device and conv.kernel_size == (K, K) and K in (3, 5, 7) and
             conv.padding == (K // 2, K // 2) and conv.padding_mode == 'zeros' and conv.stride == (1, 1) and
             conv.dilation == (1, 1) and conv.groups == w.shape[0] and w.shape[1] == 1 and
             x.shape[-1] % w.shape[0] == 0 and x.shape[-1] % (16 // x.element_size()) == 0)
@@ -49,6 +60,10 @@ def depthwise_conv_tokens(x, conv, H, W):
     B, N, C = x.shape
     if runs_on_tokens(x, conv):
         return DepthwiseConvTokensFunction.apply(x, conv.weight, conv.bias, H, W)
-    Cw = conv.weight.shape[0]
+    return _convolution_of_images(x, H, W, conv.weight.shape[0], conv)
+
+
+def _convolution_of_images(x, H, W, Cw, convolve):
+    B, N, C = x.shape
     images = x.reshape(B, H, W, C // Cw, Cw).permute(0, 3, 4, 1, 2).reshape(B * (C // Cw), Cw, H, W)
-    return conv(images).reshape(B, C, N).transpose(1, 2)
+    return convolve(images).reshape(B, C, N).transpose(1, 2)

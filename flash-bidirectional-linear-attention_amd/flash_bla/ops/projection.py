@@ -34,9 +34,11 @@ class TokenLinearFunction(torch.autograd.Function):
 def plain_tensors(*tensors):
     """Whether these are ordinary tensors in an ordinary eager call: nothing that traces, maps, casts or carries a tangent
     through torch's own operators."""
-    return (all(t is None or type(t) in (torch.Tensor, nn.Parameter) for t in tensors) and
-            not torch.is_autocast_enabled() and not torch.compiler.is_compiling() and
-            forward_ad._current_level < 0 and not torch._C._are_functorch_transforms_active())
+    for t in tensors:
+        if t is not None and type(t) is not torch.Tensor and type(t) is not nn.Parameter:
+            return False
+    return not (torch.is_autocast_enabled() or torch.compiler.is_compiling() or forward_ad._current_level >= 0 or
+                torch._C._are_functorch_transforms_active())
 
 
 # Results beyond these are enough tiles for the library's GEMM.  Measured in bf16, library's gradient + bias sum against the

@@ -68,3 +68,19 @@ def test_what_the_kernels_do_not_take_runs_as_the_torch_convolution():
         want = F.conv2d(x.double().transpose(1, 2).reshape(2, C, 4, 5), conv.weight.double().repeat(rep, 1, 1, 1),
                         conv.bias.double().repeat(rep), padding=conv.padding, groups=C).reshape(2, C, 20).transpose(1, 2)
         assert (y.double() - want).abs().max() <= 1e-5 * want.abs().max()
+
+
+def test_hooks_run_and_the_gradient_has_a_gradient():
+    torch.manual_seed(0)
+    conv = nn.Conv2d(8, 8, 3, padding=1, groups=8).cuda()
+    x = torch.randn(2, 12, 16, device="cuda", requires_grad=True)
+    g, = torch.autograd.grad(depthwise_conv_tokens(x, conv, 3, 4).square().sum(), x, create_graph=True)
+    ours = torch.autograd.grad(g.square().sum(), (x, conv.weight, conv.bias))
+    seen = []
+    conv.register_forward_hook(lambda *a: seen.append(1))
+    assert not runs_on_tokens(x, conv)
+    g, = torch.autograd.grad(depthwise_conv_tokens(x, conv, 3, 4).square().sum(), x, create_graph=True)
+    want = torch.autograd.grad(g.square().sum(), (x, conv.weight, conv.bias))
+    assert seen
+    for a, b in zip(ours, want):  # fp32 sums of 9 products, twice: a few 2^-24 of the largest
+        assert (a - b).abs().max() <= 2.0 ** -18 * b.abs().max()
