@@ -958,4 +958,52 @@ int fbla_interpolate_bwd(const void* g, void* dx, int64_t B, int64_t from, int64
   return check_launch(what);
 }
 
+static int check_row(const char* what, int C, int dtype) {
+  if (C > blocks::most_row_channels(dtype)) {
+    set_error("%s: at most %d channels (got %d)", what, blocks::most_row_channels(dtype), C);
+    return kErrUnsupported;
+  }
+  return kOk;
+}
+
+int fbla_focus_fwd(const void* q, const void* kv, const void* pe, const void* scale, void* q_out, void* k_out, void* v_out,
+                   int64_t B, int64_t N, int64_t Nk, int heads, int d, int dtype, void* stream) {
+  const char* what = "fbla_focus_fwd";
+  blocks::Shape s;
+  int rc = check_blocks(what, s, B, N, Nk, heads, d, 1, dtype);
+  if (rc == kOk) rc = check_row(what, heads * d, dtype);
+  if (rc == kOk) rc = check_tensors(what, {q, kv, pe, scale, q_out, k_out, v_out});
+  if (rc != kOk) return rc;
+  blocks::focus_fwd(s, {q, kv, pe, scale}, q_out, k_out, v_out, dtype, (hipStream_t)stream);
+  return check_launch(what);
+}
+
+size_t fbla_focus_bwd_workspace_bytes(int64_t B, int64_t N, int64_t Nk, int heads, int d, int dtype) {
+  const char* what = "fbla_focus_bwd_workspace_bytes";
+  blocks::Shape s;
+  if (check_blocks(what, s, B, N, Nk, heads, d, 1, dtype) != kOk || check_row(what, heads * d, dtype) != kOk) return 0;
+  return blocks::focus_bwd_workspace_bytes(s, dtype);
+}
+
+int fbla_focus_bwd(const void* q, const void* kv, const void* pe, const void* scale, const void* dq_heads,
+                   const void* dk_heads, const void* dv_heads, const void* dv_rows, void* dq, void* dkv, void* dpe,
+                   void* dscale, void* workspace, size_t workspace_bytes, int64_t B, int64_t N, int64_t Nk, int heads, int d,
+                   int dtype, void* stream) {
+  const char* what = "fbla_focus_bwd";
+  blocks::Shape s;
+  int rc = check_blocks(what, s, B, N, Nk, heads, d, 1, dtype);
+  if (rc == kOk) rc = check_row(what, heads * d, dtype);
+  if (rc == kOk)
+    rc = check_tensors(what, {q, kv, pe, scale, dq_heads, dk_heads, dv_heads, dv_rows, dq, dkv, dpe, dscale, workspace});
+  if (rc != kOk) return rc;
+  const size_t need = blocks::focus_bwd_workspace_bytes(s, dtype);
+  if (workspace_bytes < need) {
+    set_error("%s: workspace too small (%zu < %zu bytes)", what, workspace_bytes, need);
+    return kErrWorkspace;
+  }
+  blocks::focus_bwd(s, {q, kv, pe, scale}, {dq_heads, dk_heads, dv_heads, dv_rows}, dq, dkv, dpe, dscale, (float*)workspace,
+                    dtype, (hipStream_t)stream);
+  return check_launch(what);
+}
+
 }  // extern "C"

@@ -2,6 +2,7 @@
 //
 //   polarity features (layers/polaformer.py:63-84): q / scale and (k + positional) / scale, positive and negative parts to a
 //     learned power, the same-sign and opposite-sign pairings and the values as contiguous heads;
+//   focused features (layers/focused_la.py:56-74): relu features cubed at constant length, the values, as contiguous heads;
 //   rotary features (layers/mlla.py:74-81): elu + 1 of q and k, their 2-D rotation, the values, all as contiguous heads;
 //   token interpolation (focused_la.py:88-91, polaformer.py:95-98): reduced values back to the queries' length;
 //   merged heads (polaformer.py:92-104, mlla.py:88-92): heads back to token rows, plus the convolution's rows, times a gate.
@@ -12,6 +13,8 @@
 // 256, bf16) 2.77 -> 0.83 ms, of it here 51 us features (231 MB, 4.6 TB/s), 77 + 9 us their gradients (385 MB), 19 + 32 us the
 // merge; rotary (64 x 56x56 x 64) 0.83 -> 0.48 ms, of it 33 us features (205 MB, 6.2 TB/s), 44 us gradients (308 MB, 7 TB/s).
 #include <hip/hip_runtime.h>
+
+#include <type_traits>
 
 #include "fbla_kernels.h"
 
@@ -240,9 +243,10 @@ __global__ __launch_bounds__(kThreads) void polarity_bwd_kernel(Shape s, Polarit
 }
 
 // Sums over the partials in order, four neighbouring results per lane, 16 lanes of a column; workgroups [0, stat_wgs): the
-// 2 C sums of scale and power, the others the Nk C sums of the positional term.
+// `stats` C sums of the scale (times its reciprocal square or, `over` 1, its reciprocal) and the power, the others the Nk C
+// sums of the positional term.
 template <typename T>
-__global__ __launch_bounds__(kThreads) void polarity_finish_kernel(int C, int wgs, const float* __restrict__ partial,
+__global__ __launch_bounds__(kThreads) void features_finish_kernel(int C, int stats_of, int over, int wgs, const float* __restrict__ partial,
                                                                    const T* __restrict__ scale, T* __restrict__ dscale,
                                                                    T* __restrict__ dpower, int stat_wgs, int groups,
                                                                    int64_t pe_count, const float* __restrict__ pe_partial,
@@ -252,7 +256,7 @@ __global__ __launch_bounds__(kThreads) void polarity_finish_kernel(int C, int wg
   const bool stats = (int)blockIdx.x < stat_wgs;
   const int lane = threadIdx.x % kLanes, part = threadIdx.x / kLanes;
   const int64_t at = ((int64_t)(stats ? blockIdx.x : blockIdx.x - stat_wgs) * kLanes + lane) * 4;
-  const int64_t count = stats ? 2 * C : pe_count;
+  const int64_t count = stats ? (int64_t)stats_of * C : pe_count;
   const int terms = stats ? wgs : groups;
   const float* src = stats ? partial : pe_partial;
   f32x4 sum = {0.f, 0.f, 0.f, 0.f};
@@ -276,7 +280,7 @@ __global__ __launch_bounds__(kThreads) void polarity_finish_kernel(int C, int wg
     else if (c >= C) dpower[c - C] = (T)sum[j];
     else {
       const float inv = 1.f / (float)scale[c];
-      dscale[c] = (T)(-sum[j] * inv * inv);
+      dscale[c] = (T)(over == 1 ? -sum[j] * inv : -sum[j] * inv * inv);
     }
   }
 }
@@ -491,6 +495,221 @@ __global__ __launch_bounds__(kThreads) void interpolate_bwd_kernel(const T* __re
 }
 
 // ---------------------------------------------------------------------------------------------------------------
+// rows that are normalised over all their channels
+// ---------------------------------------------------------------------------------------------------------------
+// `lanes` (a power of two, 8 .. 64) neighbouring lanes share a row, PER pieces each: piece p of lane l is piece p lanes + l.
+// The row stays in registers between the sums and the result.
+__device__ __forceinline__ float row_sum(float v, int lanes) {
+  for (int m = 1; m < lanes; m *= 2) v += __shfl_xor(v, m);
+  return v;
+}
+__device__ __forceinline__ float row_max(float v, int lanes) {
+  for (int m = 1; m < lanes; m *= 2) v = fmaxf(v, __shfl_xor(v, m));
+  return v;
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+// focused features (layers/focused_la.py:56-74)
+// ---------------------------------------------------------------------------------------------------------------
+// t = (relu(x) + 1e-6) / scale; the feature is t^3 brought to t's length over all channels of the token.  With s = t / max t
+// (nothing under- or overflows) and n = |s|, m = |s^3|: feature = s^3 |t| / m, and for its gradient g, G = sum g s^3:
+// dt = 3 n s^2 g / m + G (s / (n m) - 3 n s^5 / m^3).
+// 64 x 28x28 x 256, bf16: 39 us (154 MB, 4 TB/s) and 83 + 9 us (231 MB), torch's operators 1.0 ms together.
+// Rows of workgroup [0, q_wgs): the queries, the others the keys with the values beside them.
+template <typename T> __device__ __forceinline__ float focus_input(float x, float scale) {
+  return ((x < 0.f ? 0.f : x) + 1e-6f) / scale;
+}
+
+template <typename T, int PER>
+__global__ __launch_bounds__(kThreads) void focus_fwd_kernel(Shape s, Focus<const T> a, int lanes, unsigned q_wgs,
+                                                             T* __restrict__ q_out, T* __restrict__ k_out,
+                                                             T* __restrict__ v_out) {
+  constexpr int V = Piece<T>::kVec;
+  const bool keys = blockIdx.x >= q_wgs;
+  const int lane = threadIdx.x % lanes, per_wg = kThreads / lanes, C = s.heads * s.d;
+  const uint32_t n = keys ? s.Nk : s.N;
+  const uint32_t row = (keys ? blockIdx.x - q_wgs : blockIdx.x) * per_wg + threadIdx.x / lanes;
+  const bool real = row < (uint32_t)s.B * n;
+  const uint32_t b = row / n, tok = row % n;
+  float t[PER][V], top = 0.f;
+#pragma unroll
+  for (int p = 0; p < PER; ++p) {
+    const int c = (p * lanes + lane) * V;
+#pragma unroll
+    for (int j = 0; j < V; ++j) t[p][j] = 0.f;
+    if (!real || c >= C) continue;
+    const Piece<T> x = load((keys ? a.kv + (int64_t)row * 2 * C : a.q + (int64_t)row * C) + c), sc = load(a.scale + c);
+    Piece<T> pe;
+    pe.w = u32x4{0u, 0u, 0u, 0u};
+    if (keys) {
+      pe = load(a.pe + (int64_t)tok * C + c);
+      store(v_out + head_row(s, b, c / s.d, tok, n, s.d) + c % s.d, load(a.kv + (int64_t)row * 2 * C + C + c));
+    }
+#pragma unroll
+    for (int j = 0; j < V; ++j) {
+      t[p][j] = focus_input<T>((float)x.e[j] + (float)pe.e[j], (float)sc.e[j]);
+      top = fmaxf(top, t[p][j]);
+    }
+  }
+  top = row_max(top, lanes);
+  const float down = 1.f / top;
+  float n2 = 0.f, m2 = 0.f;
+#pragma unroll
+  for (int p = 0; p < PER; ++p)
+#pragma unroll
+    for (int j = 0; j < V; ++j) {
+      const float v = t[p][j] * down, cube = v * v * v;
+      n2 = fmaf(v, v, n2);
+      m2 = fmaf(cube, cube, m2);
+      t[p][j] = cube;
+    }
+  const float r = top * sqrtf(row_sum(n2, lanes) / row_sum(m2, lanes));
+#pragma unroll
+  for (int p = 0; p < PER; ++p) {
+    const int c = (p * lanes + lane) * V;
+    if (!real || c >= C) continue;
+    Piece<T> out;
+#pragma unroll
+    for (int j = 0; j < V; ++j) out.e[j] = (T)(t[p][j] * r);
+    store((keys ? k_out : q_out) + head_row(s, b, c / s.d, tok, n, s.d) + c % s.d, out);
+  }
+}
+
+// Sums over tokens and batches as in polarity_bwd_kernel; partial: [workgroup][C]
+template <typename T, int PER>
+__global__ __launch_bounds__(kThreads) void focus_bwd_kernel(Shape s, Focus<const T> a, FocusGrads<const T> g, int lanes,
+                                                             T* __restrict__ dq, T* __restrict__ dkv,
+                                                             float* __restrict__ partial, float* __restrict__ pe_partial,
+                                                             int q_wgs, int groups) {
+  constexpr int V = Piece<T>::kVec;
+  const bool keys = (int)blockIdx.x >= q_wgs;
+  const int lane = threadIdx.x % lanes, per_wg = kThreads / lanes, C = s.heads * s.d, own = threadIdx.x / lanes;
+  const uint32_t wg = keys ? blockIdx.x - q_wgs : blockIdx.x, wgs = keys ? gridDim.x - q_wgs : q_wgs;
+  const uint32_t n = keys ? s.Nk : s.N;
+  // queries: items are rows, one "batch" each; keys: items are (token, batch group)
+  const uint32_t items = keys ? n * groups : (uint32_t)s.B * n;
+  float inv[PER][V], dscale[PER][V];
+#pragma unroll
+  for (int p = 0; p < PER; ++p) {
+    const int c = (p * lanes + lane) * V;
+    Piece<T> sc;
+    sc.w = u32x4{0u, 0u, 0u, 0u};
+    if (c < C) sc = load(a.scale + c);
+#pragma unroll
+    for (int j = 0; j < V; ++j) {
+      inv[p][j] = c < C ? 1.f / (float)sc.e[j] : 0.f;
+      dscale[p][j] = 0.f;
+    }
+  }
+  // every group of lanes makes the same number of trips, so that all lanes of a wave reach the shuffles
+  for (uint32_t first = wg * per_wg; first < items; first += wgs * per_wg) {
+    const uint32_t item = first + own;
+    const bool real = item < items;
+    const uint32_t tok = keys ? item / groups : item % n;
+    const uint32_t b0 = keys ? item % groups : item / n, b_step = keys ? groups : s.B;
+    float dpe[PER][V];
+#pragma unroll
+    for (int p = 0; p < PER; ++p)
+#pragma unroll
+      for (int j = 0; j < V; ++j) dpe[p][j] = 0.f;
+    const uint32_t trips = keys ? (s.B + groups - 1) / groups : 1;
+    for (uint32_t trip = 0; trip < trips; ++trip) {
+      const uint32_t b = b0 + trip * b_step;
+      const bool here = real && b < (uint32_t)s.B;
+      const int64_t row = (int64_t)b * n + tok;
+      float t[PER][V], gf[PER][V], top = 0.f;
+      uint32_t positive[PER];
+#pragma unroll
+      for (int p = 0; p < PER; ++p) {
+        const int c = (p * lanes + lane) * V;
+        positive[p] = 0;
+#pragma unroll
+        for (int j = 0; j < V; ++j) t[p][j] = gf[p][j] = 0.f;
+        if (!here || c >= C) continue;
+        const int64_t head = head_row(s, b, c / s.d, tok, n, s.d) + c % s.d;
+        const Piece<T> x = load((keys ? a.kv + row * 2 * C : a.q + row * C) + c), gi = load((keys ? g.k : g.q) + head);
+        Piece<T> pe;
+        pe.w = u32x4{0u, 0u, 0u, 0u};
+        if (keys) {
+          pe = load(a.pe + (int64_t)tok * C + c);
+          const Piece<T> vh = load(g.v + head), vr = load(g.v_rows + row * C + c);
+          Piece<T> v;
+#pragma unroll
+          for (int j = 0; j < V; ++j) v.e[j] = (T)((float)vh.e[j] + (float)vr.e[j]);
+          store(dkv + row * 2 * C + C + c, v);
+        }
+#pragma unroll
+        for (int j = 0; j < V; ++j) {
+          const float xf = (float)x.e[j] + (float)pe.e[j];
+          if (!(xf <= 0.f)) positive[p] |= 1u << j;
+          t[p][j] = ((xf < 0.f ? 0.f : xf) + 1e-6f) * inv[p][j];
+          top = fmaxf(top, t[p][j]);
+          gf[p][j] = (float)gi.e[j];
+        }
+      }
+      top = row_max(top, lanes);
+      const float down = 1.f / top;
+      float n2 = 0.f, m2 = 0.f, G = 0.f;
+#pragma unroll
+      for (int p = 0; p < PER; ++p)
+#pragma unroll
+        for (int j = 0; j < V; ++j) {
+          const float v = t[p][j] * down, cube = v * v * v;
+          n2 = fmaf(v, v, n2);
+          m2 = fmaf(cube, cube, m2);
+          G = fmaf(gf[p][j], cube, G);
+        }
+      n2 = row_sum(n2, lanes);
+      m2 = row_sum(m2, lanes);
+      G = row_sum(G, lanes);
+      const float nn = sqrtf(n2), mm = sqrtf(m2);
+      const float c2 = 3.f * nn / mm, c1 = G / (nn * mm), c5 = G * 3.f * nn / (mm * m2);
+#pragma unroll
+      for (int p = 0; p < PER; ++p) {
+        const int c = (p * lanes + lane) * V;
+        if (!here || c >= C) continue;
+        Piece<T> out;
+#pragma unroll
+        for (int j = 0; j < V; ++j) {
+          const float v = t[p][j] * down, v2 = v * v;
+          const float dt = c2 * v2 * gf[p][j] + c1 * v - c5 * v2 * v2 * v;
+          dscale[p][j] = fmaf(dt, t[p][j], dscale[p][j]);
+          const float dx = (positive[p] >> j & 1) ? dt * inv[p][j] : 0.f;
+          dpe[p][j] += dx;
+          out.e[j] = (T)dx;
+        }
+        store((keys ? dkv + row * 2 * C : dq + row * C) + c, out);
+      }
+    }
+    if (keys && real) {
+#pragma unroll
+      for (int p = 0; p < PER; ++p) {
+        const int c = (p * lanes + lane) * V;
+        if (c >= C) continue;
+        float* to = pe_partial + ((int64_t)b0 * n + tok) * C + c;
+#pragma unroll
+        for (int j = 0; j < V; j += 4)
+          *reinterpret_cast<f32x4*>(to + j) = f32x4{dpe[p][j], dpe[p][j + 1], dpe[p][j + 2], dpe[p][j + 3]};
+      }
+    }
+  }
+  __shared__ float sums[kThreads * V];
+#pragma unroll
+  for (int p = 0; p < PER; ++p) {
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < V; ++j) sums[threadIdx.x * V + j] = dscale[p][j];
+    __syncthreads();
+    for (int i = threadIdx.x; i < lanes * V; i += kThreads) {
+      const int c = p * lanes * V + i;
+      float v = 0.f;
+      for (int q = 0; q < per_wg; ++q) v += sums[q * lanes * V + i];
+      if (c < C) partial[(int64_t)blockIdx.x * C + c] = v;
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------------------------------------------
 unsigned wgs_for(int64_t rows, int C, int vec) { return (unsigned)cdiv64(rows * (C / vec), kThreads); }
 template <typename F> void by_type(int dtype, F&& f) {
   if (dtype == kF16) f(_Float16{});
@@ -550,8 +769,8 @@ void polarity_bwd(const Shape& s, const Polarity<const void>& a, const PolarityG
         s, typed<T, Polarity>(a), typed<T, PolarityGrads>(g), (T*)dqg, (T*)dkv, workspace, pe_partial, w.q_wgs, w.groups);
     const int64_t pe_count = (int64_t)s.Nk * C;
     const int stat_wgs = (2 * C + 63) / 64;
-    polarity_finish_kernel<T><<<dim3((unsigned)(stat_wgs + cdiv64(pe_count, 64))), dim3(kThreads), 0, st>>>(
-        C, wgs, workspace, (const T*)a.scale, (T*)dscale, (T*)dpower, stat_wgs, w.groups, pe_count, pe_partial, (T*)dpe);
+    features_finish_kernel<T><<<dim3((unsigned)(stat_wgs + cdiv64(pe_count, 64))), dim3(kThreads), 0, st>>>(
+        C, 2, 2, wgs, workspace, (const T*)a.scale, (T*)dscale, (T*)dpower, stat_wgs, w.groups, pe_count, pe_partial, (T*)dpe);
   });
 }
 
@@ -587,6 +806,71 @@ void merge_bwd(const Shape& s, const Merge<const void>& a, const void* dout, voi
     using T = decltype(tag);
     merge_bwd_kernel<T><<<dim3(wgs_for((int64_t)s.B * s.N, s.heads * s.d, Piece<T>::kVec)), dim3(kThreads), 0, st>>>(
         s, typed<T, Merge>(a), (const T*)dout, (T*)d_o, (T*)d_o2, (T*)dlocal, (T*)dgate);
+  });
+}
+
+// Lanes and pieces of a row that is normalised over its channels
+struct Lanes {
+  int lanes, per;
+};
+static Lanes row_lanes(int C, int vec) {
+  const int pieces = C / vec;
+  int lanes = 8;
+  while (lanes < 64 && lanes < pieces) lanes *= 2;
+  return {lanes, (pieces + lanes - 1) / lanes};
+}
+int most_row_channels(int dtype) { return 64 * 4 * vec_of(dtype); }
+template <typename F> static void by_pieces(int per, F&& f) {
+  if (per == 1) f(std::integral_constant<int, 1>());
+  else if (per == 2) f(std::integral_constant<int, 2>());
+  else f(std::integral_constant<int, 4>());
+}
+
+void focus_fwd(const Shape& s, const Focus<const void>& a, void* q, void* k, void* v, int dtype, hipStream_t st) {
+  by_type(dtype, [&](auto tag) {
+    using T = decltype(tag);
+    const Lanes l = row_lanes(s.heads * s.d, Piece<T>::kVec);
+    const int rows = kThreads / l.lanes;
+    const unsigned q_wgs = (unsigned)cdiv64((int64_t)s.B * s.N, rows), k_wgs = (unsigned)cdiv64((int64_t)s.B * s.Nk, rows);
+    by_pieces(l.per, [&](auto per) {
+      focus_fwd_kernel<T, decltype(per)::value><<<dim3(q_wgs + k_wgs), dim3(kThreads), 0, st>>>(
+          s, typed<T, Focus>(a), l.lanes, q_wgs, (T*)q, (T*)k, (T*)v);
+    });
+  });
+}
+
+// as polarity_split, for rows of whole tokens
+static Split focus_split(const Shape& s, int vec) {
+  const int rows = kThreads / row_lanes(s.heads * s.d, vec).lanes;
+  const int64_t most = 512, q = cdiv64((int64_t)s.B * s.N, rows);
+  int64_t groups = cdiv64(most * rows, s.Nk);
+  groups = groups < s.B ? groups : s.B;
+  const int64_t k = cdiv64(s.Nk * groups, rows);
+  return {(int)(q < most ? q : most), (int)(k < most ? k : most), (int)groups, 1};
+}
+
+size_t focus_bwd_workspace_bytes(const Shape& s, int dtype) {
+  const Split w = focus_split(s, vec_of(dtype));
+  const size_t C = (size_t)s.heads * s.d;
+  return sizeof(float) * C * ((size_t)w.q_wgs + w.k_wgs + (size_t)w.groups * s.Nk);
+}
+
+void focus_bwd(const Shape& s, const Focus<const void>& a, const FocusGrads<const void>& g, void* dq, void* dkv, void* dpe,
+               void* dscale, float* workspace, int dtype, hipStream_t st) {
+  by_type(dtype, [&](auto tag) {
+    using T = decltype(tag);
+    const Split w = focus_split(s, Piece<T>::kVec);
+    const int C = s.heads * s.d, wgs = w.q_wgs + w.k_wgs;
+    const Lanes l = row_lanes(C, Piece<T>::kVec);
+    float* pe_partial = workspace + (int64_t)C * wgs;
+    by_pieces(l.per, [&](auto per) {
+      focus_bwd_kernel<T, decltype(per)::value><<<dim3((unsigned)wgs), dim3(kThreads), 0, st>>>(
+          s, typed<T, Focus>(a), typed<T, FocusGrads>(g), l.lanes, (T*)dq, (T*)dkv, workspace, pe_partial, w.q_wgs, w.groups);
+    });
+    const int64_t pe_count = (int64_t)s.Nk * C;
+    const int stat_wgs = (C + 63) / 64;
+    features_finish_kernel<T><<<dim3((unsigned)(stat_wgs + cdiv64(pe_count, 64))), dim3(kThreads), 0, st>>>(
+        C, 1, 1, wgs, workspace, (const T*)a.scale, (T*)dscale, nullptr, stat_wgs, w.groups, pe_count, pe_partial, (T*)dpe);
   });
 }
 

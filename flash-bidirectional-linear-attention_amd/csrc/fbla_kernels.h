@@ -256,7 +256,18 @@ template <typename P> struct Merge {
   P *gate;      // rows gate_row elements apart, or null
   int64_t gate_row;
 };
+template <typename P> struct Focus {
+  P *q, *kv, *pe, *scale;  // [B,N,C], [B,Nk,2C], [Nk,C], [C]
+};
+template <typename P> struct FocusGrads {
+  P *q, *k, *v, *v_rows;  // heads of d; rows of C
+};
 int vec_of(int dtype);  // elements of a piece
+int most_row_channels(int dtype);  // of rows that are normalised over their channels (focus_*)
+void focus_fwd(const Shape& s, const Focus<const void>& a, void* q, void* k, void* v, int dtype, hipStream_t st);
+size_t focus_bwd_workspace_bytes(const Shape& s, int dtype);
+void focus_bwd(const Shape& s, const Focus<const void>& a, const FocusGrads<const void>& g, void* dq, void* dkv, void* dpe,
+               void* dscale, float* workspace, int dtype, hipStream_t st);
 void polarity_fwd(const Shape& s, const Polarity<const void>& a, void* q_same, void* q_opp, void* k_both, void* v_heads,
                   int dtype, hipStream_t st);
 size_t polarity_bwd_workspace_bytes(const Shape& s, int dtype);

@@ -61,6 +61,9 @@ _SIGNATURES = {
     "fbla_rotary_bwd": (_i32, [_vp] * 2 + [_i32] + [_vp] * 8 + [_i64] * 2 + [_i32] * 3 + [_vp]),
     "fbla_merge_fwd": (_i32, [_vp] * 4 + [_i64, _vp] + [_i64] * 2 + [_i32] * 3 + [_vp]),
     "fbla_merge_bwd": (_i32, [_vp] * 5 + [_i64] + [_vp] * 4 + [_i64] * 2 + [_i32] * 3 + [_vp]),
+    "fbla_focus_fwd": (_i32, [_vp] * 7 + [_i64] * 3 + [_i32] * 3 + [_vp]),
+    "fbla_focus_bwd_workspace_bytes": (_sz, [_i64] * 3 + [_i32] * 3),
+    "fbla_focus_bwd": (_i32, [_vp] * 13 + [_sz] + [_i64] * 3 + [_i32] * 3 + [_vp]),
     "fbla_interpolate_fwd": (_i32, [_vp, _i64, _i64, _vp] + [_i64] * 3 + [_i32] * 2 + [_vp]),
     "fbla_interpolate_bwd": (_i32, [_vp] * 2 + [_i64] * 3 + [_i32] * 2 + [_vp]),
 }
@@ -632,3 +635,38 @@ def interpolate_bwd(g, n):
         rc = lib().fbla_interpolate_bwd(_ptr(g), _ptr(dx), B, n, tokens, C, dtype_code(g), _stream(g.device))
     _check(rc, "fbla_interpolate_bwd")
     return dx
+
+
+def focus_fwd(q, kv, pe, scale, heads):
+    """Focused features of q [B, N, C] and kv [B, n, 2C]: (q, k, v) as [B, heads, tokens, d]."""
+    _require_gpu(q, kv, pe, scale)
+    q, kv, pe, scale = _whole(q, kv, pe, scale)
+    B, N, C = q.shape
+    n = kv.shape[1]
+    out = tuple(torch.empty(B, heads, t, C // heads, dtype=q.dtype, device=q.device) for t in (N, n, n))
+    with _on(q.device):
+        rc = lib().fbla_focus_fwd(_ptr(q), _ptr(kv), _ptr(pe), _ptr(scale), *(_ptr(t) for t in out), B, N, n, heads,
+                                  C // heads, dtype_code(q), _stream(q.device))
+    _check(rc, "fbla_focus_fwd")
+    return out
+
+
+def focus_bwd(q, kv, pe, scale, heads, dq_heads, dk_heads, dv_heads, dv_rows):
+    """Gradients (dq, dkv, dpe, dscale) of focus_fwd; dv_rows [B, n, C] is added to the values' gradient."""
+    tensors = q, kv, pe, scale, dq_heads, dk_heads, dv_heads, dv_rows
+    _require_gpu(*tensors)
+    tensors = _whole(*tensors)
+    q, kv = tensors[:2]
+    (B, N, C), n, code, L = q.shape, kv.shape[1], dtype_code(q), lib()
+    grads = tuple(torch.empty_like(t) for t in tensors[:4])
+    with _on(q.device):
+        ws = _workspace(L.fbla_focus_bwd_workspace_bytes(B, N, n, heads, C // heads, code), q.device)
+        rc = L.fbla_focus_bwd(*(_ptr(t) for t in tensors + grads), _ptr(ws), ws.numel(), B, N, n, heads, C // heads, code,
+                              _stream(q.device))
+    _check(rc, "fbla_focus_bwd")
+    return grads
+
+
+def most_row_channels(t):
+    """The widest row of t's type that focus_fwd takes."""
+    return 4096 // t.element_size()

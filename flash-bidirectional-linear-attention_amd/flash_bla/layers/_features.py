@@ -1,6 +1,6 @@
 """What the vision blocks do between their projections and the attention operators, one HIP launch a direction: polarity
-features (layers/polaformer.py:63-84), rotary features (layers/mlla.py:74-81) and heads merged back to rows
-(polaformer.py:92-104, mlla.py:88-92).  The reference composes them of torch operators; the compositions here are what runs
+features (layers/polaformer.py:63-84), focused features (layers/focused_la.py:56-74), rotary
+features (layers/mlla.py:74-81) and heads merged back to rows (polaformer.py:92-104, mlla.py:88-92).  The reference composes them of torch operators; the compositions here are what runs
 when the kernels do not take a call, and what a gradient of the gradient is made of.
 """
 import torch
@@ -11,14 +11,19 @@ from flash_bla.layers._common import merge_heads, split_heads
 from flash_bla.ops.feature_map import elu_plus_one
 from flash_bla.ops.projection import plain_tensors
 
+_TYPES = (torch.float16, torch.bfloat16, torch.float32)
+
 
 def _takes(heads, channels, unit, *tensors):
     """Ordinary GPU tensors of one supported type whose heads (or their `unit` parts) are whole 16-byte pieces."""
     x = tensors[0]
-    piece = unit * 16 // x.element_size()
-    return (x.is_cuda and x.dtype in (torch.float16, torch.bfloat16, torch.float32) and channels // heads % piece == 0 and
-            all(t is None or (t.dtype == x.dtype and t.device == x.device and 0 < t.numel() < 1 << 31) for t in tensors) and
-            plain_tensors(*tensors))
+    dtype, device = x.dtype, x.device
+    if not x.is_cuda or dtype not in _TYPES or channels // heads % (unit * 16 // x.element_size()):
+        return False
+    for t in tensors:
+        if t is not None and (t.dtype != dtype or t.device != device or not 0 < t.numel() < 1 << 31):
+            return False
+    return plain_tensors(*tensors)
 
 
 def differentiable_gradients(formula, inputs, grads):
@@ -64,6 +69,45 @@ def polarity_features(qg, kv, pe, scale, power, heads):
     if _takes(heads, C, 1, qg, kv, pe, scale, power) and pe.shape == (1, kv.shape[1], C) and scale.shape == (1, 1, C):
         return PolarityFeaturesFunction.apply(qg, kv, pe, scale, power, heads)
     return polarity_formula(qg, kv, pe, scale, power, heads)
+
+
+def focus(t, scale, factor):
+    """relu features sharpened by an element-wise power at constant norm."""
+    t = (F.relu(t) + 1e-6) / scale
+    norm = t.norm(dim=-1, keepdim=True)
+    t = t ** factor
+    return t / t.norm(dim=-1, keepdim=True) * norm
+
+
+def focus_formula(q, kv, pe, scale, heads, factor=3):
+    k, v_rows = kv.chunk(2, dim=-1)
+    q, k = focus(q, scale, factor), focus(k + pe, scale, factor)
+    return (*(split_heads(t, heads) for t in (q, k, v_rows)), v_rows)
+
+
+class FocusedFeaturesFunction(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, q, kv, pe, scale, heads):
+        ctx.save_for_backward(q, kv, pe, scale)
+        ctx.heads = heads
+        return (*_hip.focus_fwd(q, kv, pe, scale, heads), kv.chunk(2, dim=-1)[1])
+
+    @staticmethod
+    def backward(ctx, *grads):
+        inputs = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            return differentiable_gradients(focus_formula, (*inputs, ctx.heads), grads)
+        return (*_hip.focus_bwd(*inputs, ctx.heads, *grads), None)
+
+
+def focused_features(q, kv, pe, scale, heads, factor):
+    """q [B, N, C], kv [B, n, 2C] (keys | values), pe [1, n, C], scale [1, 1, C].  Returns (q, k, v [B, heads, tokens, d],
+    the values as rows [B, n, C]).  The kernels know the cube."""
+    C = q.shape[-1]
+    if (factor == 3 and _takes(heads, C, 1, q, kv, pe, scale) and C <= _hip.most_row_channels(q) and
+            pe.shape == (1, kv.shape[1], C) and scale.shape == (1, 1, C)):
+        return FocusedFeaturesFunction.apply(q, kv, pe, scale, heads)
+    return focus_formula(q, kv, pe, scale, heads, factor)
 
 
 def rotate(x, rotations):

@@ -33,10 +33,6 @@ class PvtLinearAttentionBase(nn.Module):
             x = self.norm(self.sr(x.transpose(1, 2).reshape(B, C, H, W)).flatten(2).transpose(1, 2))
         return self.kv(x)
 
-    def _keys_values(self, x, H, W):
-        k, v = self._joint_keys_values(x, H, W).chunk(2, dim=-1)
-        return k + self.positional_encoding, v
-
     def _value_conv(self, v, N, H, W):
         """v: (B, heads, n, d) -> depth-wise conv on the H x W grid -> (B, N, C)."""
         B, heads, n, d = v.shape

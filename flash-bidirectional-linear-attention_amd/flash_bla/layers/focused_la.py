@@ -1,10 +1,9 @@
 """FLatten focused linear attention (counterpart of flash_bla/layers/focused_la.py:13-96)."""
-import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from flash_bla.layers._common import check_mode, merge_heads, split_heads, torch_linear_attention
-from flash_bla.layers._features import merge_heads_with
+from flash_bla.layers._common import check_mode, merge_heads, torch_linear_attention
+from flash_bla.layers._features import focus_formula, focused_features, merge_heads_with
 from flash_bla.layers._pvt import PvtLinearAttentionBase
 from flash_bla.ops.linear_attn.fused import linear_attention
 from flash_bla.ops.projection import TokenLinear
@@ -18,21 +17,13 @@ class FocusedLinearAttention(PvtLinearAttentionBase):
         self.q = TokenLinear(dim, dim, bias=qkv_bias)
         self.focusing_factor = focusing_factor
 
-    def _focus(self, t, scale):
-        """relu features sharpened by an element-wise power at constant norm."""
-        t = (F.relu(t) + 1e-6) / scale
-        norm = t.norm(dim=-1, keepdim=True)
-        t = t ** self.focusing_factor
-        return t / t.norm(dim=-1, keepdim=True) * norm
-
     def forward(self, x, H, W, mode='triton'):
         fast = check_mode(mode)
         N = x.shape[1]
-        k, v = self._keys_values(x, H, W)
-        scale = F.softplus(self.scale)
-        q, k = self._focus(self.q(x), scale), self._focus(k, scale)
-        v_rows = v
-        q, k, v = (split_heads(t, self.num_heads) for t in (q, k, v))
+        kv = self._joint_keys_values(x, H, W)
+        features = focused_features if fast else focus_formula
+        q, k, v, v_rows = features(self.q(x), kv, self.positional_encoding, F.softplus(self.scale), self.num_heads,
+                                   self.focusing_factor)
         if fast:
             out = merge_heads_with(linear_attention(q, k, v), None, self._value_conv_tokens(v_rows, N, H, W))
         else:

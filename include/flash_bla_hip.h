@@ -331,6 +331,18 @@ int fbla_interpolate_fwd(const void* x, int64_t x_batch, int64_t x_row, void* y,
                          int dtype, void* stream);
 int fbla_interpolate_bwd(const void* g, void* dx, int64_t B, int64_t from, int64_t to, int C, int dtype, void* stream);
 
+/* Focused features (flash_bla/layers/focused_la.py:56-74, focusing factor 3): with t = (relu(x) + 1e-6) / scale of q
+ * [B, N, C] or of kv's first half plus pe, the feature t^3 |t| / |t^3| (lengths over the C channels) as heads of d, and kv's
+ * second half as heads v_out.  C in whole
+ * 16-byte pieces, at most 2048 (16-bit) or 1024 (fp32).  The backward adds dv_rows [B, Nk, C] to the values' gradient. */
+int fbla_focus_fwd(const void* q, const void* kv, const void* pe, const void* scale, void* q_out, void* k_out, void* v_out,
+                   int64_t B, int64_t N, int64_t Nk, int heads, int d, int dtype, void* stream);
+size_t fbla_focus_bwd_workspace_bytes(int64_t B, int64_t N, int64_t Nk, int heads, int d, int dtype);
+int fbla_focus_bwd(const void* q, const void* kv, const void* pe, const void* scale, const void* dq_heads,
+                   const void* dk_heads, const void* dv_heads, const void* dv_rows, void* dq, void* dkv, void* dpe,
+                   void* dscale, void* workspace, size_t workspace_bytes, int64_t B, int64_t N, int64_t Nk, int heads, int d,
+                   int dtype, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -104,6 +104,23 @@ def test_interpolated_tokens(B, n, tokens, C, dtype):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("B,N,Nk,heads,d", [(1, 1, 1, 1, 16), (2, 33, 33, 8, 32), (3, 20, 5, 5, 24), (37, 5, 1, 3, 40),
+                                            (2, 7, 7, 10, 64), (1, 9, 4, 16, 64)])
+def test_focused_features(B, N, Nk, heads, d, dtype):
+    torch.manual_seed(N * heads)
+    C = heads * d
+    values = lambda *shape: torch.randn(shape, device="cuda").to(dtype).requires_grad_()  # noqa: E731
+    q, kv, pe = values(B, N, C), values(B, Nk, 2 * C), values(1, Nk, C)
+    scale = (0.5 + torch.rand(1, 1, C, device="cuda")).to(dtype).requires_grad_()
+    assert features._takes(heads, C, 1, q, kv, pe, scale)
+    _check(lambda *a: features.focused_features(*a, 3), features.focus_formula, (q, kv, pe, scale, heads), dtype)
+    for a, b in zip(features.focused_features(q, kv, pe, scale, heads, 2.5),
+                    features.focus_formula(q, kv, pe, scale, heads, 2.5)):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
 def test_not_a_number_and_infinity_pass_through():
     """A NaN reaches both parts, an infinity its own, as relu and pow give them."""
     x = torch.randn(1, 1, 64, device="cuda")
