@@ -3,7 +3,7 @@
 //
 // The contraction runs over the tokens (1e4 .. 1e5), the result is a few hundred on a side: a GEMM that tiles the result
 // alone leaves the GPU to a dozen workgroups (the library's, bf16: 128 x 64 over 200704 tokens 419 us, 512 x 256 over
-// 50176 tokens 188 us, plus 32 us of column sums each for the bias; here, with the bias, 23 and 43 us).  So the
+// 50176 tokens 188 us, plus 32 us of column sums each for the bias; here, with the bias, 23 and 35 us).  So the
 // tokens are split: a workgroup owns a 128 x 128 tile of the result and one chunk of the tokens, the chunks' fp32 sums
 // are added in chunk order by a second kernel and rounded once.
 //
@@ -24,6 +24,7 @@ namespace {
 constexpr int kThreads = 256;
 constexpr int kTile = 128;               // rows and columns of the result per workgroup
 constexpr int kStepTokens = 64;
+constexpr int kLeastChunk = 4 * kStepTokens;
 constexpr int kRowBytes = kTile * 2;
 constexpr int kStepBytes = kStepTokens * kRowBytes;
 
@@ -58,7 +59,17 @@ __global__ __launch_bounds__(kThreads, 2) void wgrad_kernel(const T* __restrict_
                                                             int tiles_n, float* __restrict__ partial,
                                                             float* __restrict__ bias_partial) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];  // 2 x (g step, x step)
-  const int tile = blockIdx.x, c = blockIdx.y;
+  // The tiles of a chunk read the same rows: they run on one XCD (workgroup i is on XCD i % 8), whose L2 then fetches them
+  // once.  Chunks beyond the last multiple of eight keep the plain order, and so do chunks of the shortest length, which end
+  // before that pays (with / without, bf16 with bias: 512 x 256 over 50176 tokens, chunks of 832, 34.5 / 42.6 us; 640 x 640
+  // over 8192, chunks of 448, 24.9 / 29.6; over 4096, chunks of 256, 23.3 / 20.9).
+  int tile, c;
+  {
+    const int tiles = gridDim.x, i = blockIdx.x + tiles * blockIdx.y;
+    const int together = chunk > kLeastChunk ? (int)gridDim.y / 8 * 8 * tiles : 0;
+    c = i < together ? i / (8 * tiles) * 8 + i % 8 : i / tiles;
+    tile = i < together ? i / 8 % tiles : i % tiles;
+  }
   const int m0 = tile / tiles_n * kTile, n0 = tile % tiles_n * kTile;
   const int64_t t_begin = (int64_t)c * chunk;
   const int len = (int)min((int64_t)chunk, tokens - t_begin);  // >= 1: the host counts the chunks
@@ -217,7 +228,7 @@ int tiles(int n) { return (n + kTile - 1) / kTile; }
 int chunk_for(int64_t tokens, int M, int N) {
   const int64_t slots = 2 * 256 / ((int64_t)tiles(M) * tiles(N));
   int64_t chunk = cdiv64(tokens, slots < 1 ? 1 : slots);
-  if (chunk < 4 * kStepTokens) chunk = 4 * kStepTokens;
+  if (chunk < kLeastChunk) chunk = kLeastChunk;
   return (int)(cdiv64(chunk, kStepTokens) * kStepTokens);
 }
 
