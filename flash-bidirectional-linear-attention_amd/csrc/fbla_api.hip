@@ -1006,4 +1006,37 @@ int fbla_focus_bwd(const void* q, const void* kv, const void* pe, const void* sc
   return check_launch(what);
 }
 
+static int check_turn(const char* what, blocks::Shape& s, int64_t B, int64_t N, int heads, int d, int dtype) {
+  const int rc = check_blocks(what, s, B, N, N, heads, d, 1, dtype);
+  const int pieces = rc == kOk ? d / blocks::vec_of(dtype) : 1;
+  if (pieces > 64 || (pieces & (pieces - 1))) {
+    set_error("%s: a head must be a power of two of at most 64 16-byte pieces (d=%d)", what, d);
+    return kErrUnsupported;
+  }
+  return rc;
+}
+
+int fbla_turn_fwd(const void* q, const void* k, const void* weight, const float* rot, void* k_out, void* q_rot, void* k_rot,
+                  int64_t B, int64_t N, int heads, int d, int dtype, void* stream) {
+  const char* what = "fbla_turn_fwd";
+  blocks::Shape s;
+  int rc = check_turn(what, s, B, N, heads, d, dtype);
+  if (rc == kOk) rc = check_tensors(what, {q, k, weight, rot, k_out, q_rot, k_rot});
+  if (rc != kOk) return rc;
+  blocks::turn_fwd(s, q, k, weight, rot, k_out, q_rot, k_rot, dtype, (hipStream_t)stream);
+  return check_launch(what);
+}
+
+int fbla_turn_bwd(const void* k, const void* weight, const float* rot, const void* dk_out, const void* dq_rot,
+                  const void* dk_rot, void* dq, void* dk, void* dweight, int64_t B, int64_t N, int heads, int d, int dtype,
+                  void* stream) {
+  const char* what = "fbla_turn_bwd";
+  blocks::Shape s;
+  int rc = check_turn(what, s, B, N, heads, d, dtype);
+  if (rc == kOk) rc = check_tensors(what, {k, weight, rot, dk_out, dq_rot, dk_rot, dq, dk, dweight});
+  if (rc != kOk) return rc;
+  blocks::turn_bwd(s, k, weight, rot, dk_out, dq_rot, dk_rot, dq, dk, dweight, dtype, (hipStream_t)stream);
+  return check_launch(what);
+}
+
 }  // extern "C"

@@ -278,6 +278,11 @@ void rotary_fwd(const Shape& s, const void* qk, const void* x, const float* rot,
                 void* q_rot, void* k_rot, void* v, int dtype, hipStream_t st);
 void rotary_bwd(const Shape& s, const void* qk, const float* rot, int rot_channels, const RotaryGrads<const void>& g,
                 void* dqk, void* dx, int dtype, hipStream_t st);
+// on heads of d; weight [B, heads, N]; rot fp32 [N, d / 2, 2]
+void turn_fwd(const Shape& s, const void* q, const void* k, const void* weight, const float* rot, void* k_out, void* q_rot,
+              void* k_rot, int dtype, hipStream_t st);
+void turn_bwd(const Shape& s, const void* k, const void* weight, const float* rot, const void* dk_out, const void* dq_rot,
+              const void* dk_rot, void* dq, void* dk, void* dweight, int dtype, hipStream_t st);
 void merge_fwd(const Shape& s, const Merge<const void>& a, void* out, int dtype, hipStream_t st);
 void merge_bwd(const Shape& s, const Merge<const void>& a, const void* dout, void* d_o, void* d_o2, void* dlocal, void* dgate,
                int dtype, hipStream_t st);

@@ -61,6 +61,8 @@ _SIGNATURES = {
     "fbla_rotary_bwd": (_i32, [_vp] * 2 + [_i32] + [_vp] * 8 + [_i64] * 2 + [_i32] * 3 + [_vp]),
     "fbla_merge_fwd": (_i32, [_vp] * 4 + [_i64, _vp] + [_i64] * 2 + [_i32] * 3 + [_vp]),
     "fbla_merge_bwd": (_i32, [_vp] * 5 + [_i64] + [_vp] * 4 + [_i64] * 2 + [_i32] * 3 + [_vp]),
+    "fbla_turn_fwd": (_i32, [_vp] * 7 + [_i64] * 2 + [_i32] * 3 + [_vp]),
+    "fbla_turn_bwd": (_i32, [_vp] * 9 + [_i64] * 2 + [_i32] * 3 + [_vp]),
     "fbla_focus_fwd": (_i32, [_vp] * 7 + [_i64] * 3 + [_i32] * 3 + [_vp]),
     "fbla_focus_bwd_workspace_bytes": (_sz, [_i64] * 3 + [_i32] * 3),
     "fbla_focus_bwd": (_i32, [_vp] * 13 + [_sz] + [_i64] * 3 + [_i32] * 3 + [_vp]),
@@ -670,3 +672,31 @@ def focus_bwd(q, kv, pe, scale, heads, dq_heads, dk_heads, dv_heads, dv_rows):
 def most_row_channels(t):
     """The widest row of t's type that focus_fwd takes."""
     return 4096 // t.element_size()
+
+
+def turn_fwd(q, k, weight, rotations):
+    """(k * weight, q turned, k * weight turned) of heads [B, heads, N, d]; weight [B, heads, N, 1], rotations fp32
+    [..., d / 2, 2] over the N tokens."""
+    _require_gpu(q, k, weight, rotations)
+    q, k, weight, rotations = _whole(q, k, weight, rotations)
+    B, heads, N, d = q.shape
+    out = tuple(torch.empty_like(q) for _ in range(3))
+    with _on(q.device):
+        rc = lib().fbla_turn_fwd(_ptr(q), _ptr(k), _ptr(weight), _ptr(rotations), *(_ptr(t) for t in out), B, N, heads, d,
+                                 dtype_code(q), _stream(q.device))
+    _check(rc, "fbla_turn_fwd")
+    return out
+
+
+def turn_bwd(k, weight, rotations, dk_out, dq_rot, dk_rot):
+    """Gradients (dq, dk, dweight) of turn_fwd."""
+    tensors = k, weight, rotations, dk_out, dq_rot, dk_rot
+    _require_gpu(*tensors)
+    tensors = _whole(*tensors)
+    k, weight = tensors[:2]
+    B, heads, N, d = k.shape
+    grads = torch.empty_like(k), torch.empty_like(k), torch.empty_like(weight)
+    with _on(k.device):
+        rc = lib().fbla_turn_bwd(*(_ptr(t) for t in tensors + grads), B, N, heads, d, dtype_code(k), _stream(k.device))
+    _check(rc, "fbla_turn_bwd")
+    return grads

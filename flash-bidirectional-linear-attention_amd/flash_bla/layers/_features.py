@@ -148,6 +148,40 @@ def rotary_features(qk, x, rotations, side, heads):
     return rotary_formula(qk, x, rotations, side, heads, elu_plus_one)
 
 
+def turn_formula(q, k, weight, rotations):
+    b, heads, n, d = q.shape
+    k = k * weight
+    grid = (b, heads, *rotations.shape[:-2], d)
+    return (k, *(rotate(t.reshape(grid), rotations).reshape(t.shape).to(q.dtype) for t in (q, k)))
+
+
+class TurnedHeadsFunction(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, q, k, weight, rotations):
+        ctx.save_for_backward(q, k, weight, rotations)
+        return _hip.turn_fwd(q, k, weight, rotations)
+
+    @staticmethod
+    def backward(ctx, *grads):
+        q, k, weight, rotations = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            return differentiable_gradients(turn_formula, (q, k, weight, rotations), grads)
+        return (*_hip.turn_bwd(k, weight, rotations, *grads), None)
+
+
+def turned_heads(q, k, weight, rotations):
+    """q, k [B, heads, N, d], weight [B, heads, N, 1], rotations [H, W, d / 2, 2] over the N tokens.  Returns (k * weight, q
+    turned, k * weight turned)."""
+    N, d = q.shape[-2:]
+    pieces = d * q.element_size() // 16
+    if (_takes(1, d, 1, q, k, weight) and pieces <= 64 and pieces & (pieces - 1) == 0 and plain_tensors(rotations) and
+            rotations.dtype == torch.float32 and rotations.device == q.device and not rotations.requires_grad and
+            rotations.ndim == 4 and rotations.shape[0] * rotations.shape[1] == N and rotations.shape[2:] == (d // 2, 2) and
+            k.shape == q.shape and weight.shape == (*q.shape[:-1], 1)):
+        return TurnedHeadsFunction.apply(q, k, weight, rotations)
+    return turn_formula(q, k, weight, rotations)
+
+
 def merge_formula(o, o2, local, gate):
     out = merge_heads(o if o2 is None else torch.cat((o, o2), dim=-1)) + local
     return (out if gate is None else out * gate,)

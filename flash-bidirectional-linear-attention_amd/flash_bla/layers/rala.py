@@ -4,8 +4,9 @@ import torch
 import torch.nn as nn
 
 from flash_bla.layers._common import check_mode, merge_heads, split_heads, torch_linear_attention
-from flash_bla.layers._features import merge_heads_with
+from flash_bla.layers._features import merge_heads_with, turned_heads
 from flash_bla.layers.mlla import RoPE
+from flash_bla.ops._check import untouched
 from flash_bla.ops.depthwise import depthwise_conv_tokens
 from flash_bla.ops.linear_attn.decoupled import decoupled_la
 from flash_bla.ops.projection import TokenLinear
@@ -35,10 +36,13 @@ class RALALinearAttention(nn.Module):
         q, k, v = (split_heads(t, self.num_heads) for t in (self.elu(q) + 1.0, self.elu(k) + 1.0, v))
         # efficiency reweighting: softmax over tokens of scale * mean(q) . k_j, times n
         eff = torch.softmax(self.scale * q.mean(dim=-2, keepdim=True) @ k.transpose(-1, -2), dim=-1)
-        k = k * eff.transpose(-1, -2) * n
-        grid = (b, self.num_heads, side, side, self.head_dim)
-        q_rope = self.rope(q.reshape(grid)).reshape(q.shape).to(x.dtype).contiguous()
-        k_rope = self.rope(k.reshape(grid)).reshape(k.shape).to(x.dtype).contiguous()
+        if fast and untouched(self.rope, RoPE) and self.rope.rotations.shape[:2] == (side, side):
+            k, q_rope, k_rope = turned_heads(q, k, eff.transpose(-1, -2) * n, self.rope.rotations)
+        else:
+            k = k * eff.transpose(-1, -2) * n
+            grid = (b, self.num_heads, side, side, self.head_dim)
+            q_rope = self.rope(q.reshape(grid)).reshape(q.shape).to(x.dtype).contiguous()
+            k_rope = self.rope(k.reshape(grid)).reshape(k.shape).to(x.dtype).contiguous()
         if fast:
             out = decoupled_la(q, k.contiguous(), q_rope, k_rope, v, scale=n ** -1.0)
             return self.proj(merge_heads_with(out, None, lepe, gate))

@@ -343,6 +343,16 @@ int fbla_focus_bwd(const void* q, const void* kv, const void* pe, const void* sc
                    void* dscale, void* workspace, size_t workspace_bytes, int64_t B, int64_t N, int64_t Nk, int heads, int d,
                    int dtype, void* stream);
 
+/* Weighted and turned heads (flash_bla/layers/rala.py:60-69): k_out = k * weight, q_rot and k_rot = the channel pairs of q and
+ * of k_out (before its rounding) turned by rot (fp32 [N, d / 2, 2]: cos, sin).  All heads are [B, heads, N, d], weight
+ * [B, heads, N]; d a power of two of at most 64 16-byte pieces.  The backward gives the gradients through these outputs
+ * alone (dq: through q_rot). */
+int fbla_turn_fwd(const void* q, const void* k, const void* weight, const float* rot, void* k_out, void* q_rot, void* k_rot,
+                  int64_t B, int64_t N, int heads, int d, int dtype, void* stream);
+int fbla_turn_bwd(const void* k, const void* weight, const float* rot, const void* dk_out, const void* dq_rot,
+                  const void* dk_rot, void* dq, void* dk, void* dweight, int64_t B, int64_t N, int heads, int d, int dtype,
+                  void* stream);
+
 #ifdef __cplusplus
 }
 #endif

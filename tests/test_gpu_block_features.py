@@ -77,6 +77,24 @@ def test_rotary_features(B, side, heads, d, dtype):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("B,side,heads,d", [(1, 1, 1, 8), (3, 5, 3, 32), (2, 7, 2, 64), (1, 2, 2, 128)])
+def test_turned_heads(B, side, heads, d, dtype):
+    torch.manual_seed(side)
+    q, k = (torch.randn(B, heads, side * side, d, device="cuda").to(dtype).requires_grad_() for _ in range(2))
+    weight = torch.rand(B, heads, side * side, 1, device="cuda").to(dtype).requires_grad_()
+    angles = torch.randn(side, side, d // 2, device="cuda")
+    rotations = torch.stack([angles.cos(), angles.sin()], dim=-1)
+
+    def exact(q, k, weight):
+        cos, sin = rotations.double().reshape(side * side, d // 2, 2).unbind(-1)
+        turn = lambda t: torch.stack([t[..., ::2] * cos - t[..., 1::2] * sin,  # noqa: E731
+                                      t[..., ::2] * sin + t[..., 1::2] * cos], dim=-1).flatten(-2)
+        return k * weight, turn(q), turn(k * weight)
+    _check(lambda *t: features.turned_heads(*t, rotations), exact, (q, k, weight), dtype)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("halves", [False, True])
 @pytest.mark.parametrize("gated", [False, True])
 @pytest.mark.parametrize("B,N,heads,d", [(1, 1, 1, 16), (3, 21, 5, 48), (2, 50, 10, 64)])
