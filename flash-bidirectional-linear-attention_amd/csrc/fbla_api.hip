@@ -759,8 +759,9 @@ static int check_linear(const char* what, int64_t tokens, int M, int N, int dtyp
     return kErrBadArg;
   }
   // the bound on the product keeps the result's indexes in 31 bits, the one on the tokens the chunks' lengths
-  if (dtype == kF32 || M % 8 || N % 8 || (int64_t)M * N > (1 << 28) || tokens > (1LL << 30)) {
-    set_error("%s: needs 16-bit elements, rows of whole 16-byte pieces and at most 2^28 weights and 2^30 tokens "
+  const int vec = dtype == kF32 ? 4 : 8;
+  if (M % vec || N % vec || (int64_t)M * N > (1 << 28) || tokens > (1LL << 30)) {
+    set_error("%s: needs rows of whole 16-byte pieces and at most 2^28 weights and 2^30 tokens "
               "(tokens=%lld M=%d N=%d dtype=%d)", what, (long long)tokens, M, N, dtype);
     return kErrUnsupported;
   }

@@ -227,7 +227,7 @@ void grad(const Conv& a, const void* g, int64_t g_batch, int64_t g_row, void* dw
           int dtype, hipStream_t st);
 }  // namespace dwconv
 
-// Weight and bias gradient of a projection over 16-bit token rows (fbla_linear.hip): dw [M, N] and db [M] (or null) from
+// Weight and bias gradient of a projection over token rows (fbla_linear.hip): dw [M, N] and db [M] (or null) from
 // the output's gradient g (rows of M) and the input x (rows of N), row strides in elements.
 namespace linear {
 size_t wgrad_workspace_bytes(int64_t tokens, int M, int N);

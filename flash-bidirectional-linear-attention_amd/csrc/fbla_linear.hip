@@ -1,5 +1,5 @@
 // Weight and bias gradient of a projection over token rows: dW[m][n] = sum_t g[t][m] x[t][n], db[m] = sum_t g[t][m],
-// for 16-bit rows (the blocks' nn.Linear layers: layers/mlla.py:56, rala.py:31, focused_la.py:26-27, polaformer.py:24-25).
+// (the blocks' nn.Linear layers: layers/mlla.py:56, rala.py:31, focused_la.py:26-27, polaformer.py:24-25).
 //
 // The contraction runs over the tokens (1e4 .. 1e5), the result is a few hundred on a side: a GEMM that tiles the result
 // alone leaves the GPU to a dozen workgroups (the library's, bf16: 128 x 64 over 200704 tokens 419 us, 512 x 256 over
@@ -7,11 +7,12 @@
 // tokens are split: a workgroup owns a 128 x 128 tile of the result and one chunk of the tokens, the chunks' fp32 sums
 // are added in chunk order by a second kernel and rounded once.
 //
-// Tile: four waves, each a 64 x 64 quarter.  Steps of 64 tokens arrive flat (16 bytes per lane, whole rows) and are staged
+// Tile: four waves, each a 64 x 64 quarter.  16 bits: steps of 64 tokens arrive flat (16 bytes per lane, whole rows) and are staged
 // in LDS row-major; both operands are read out of it with the transposing read.  Per step a wave reads 16 KiB of LDS for
 // 16 MFMAs of 32x32x16, which take about as long: bound by LDS and matrix cores together where the result has many
 // tiles, by HBM where it has one or two.  The next step's rows are in registers meanwhile; two LDS buffers, one barrier per
-// step.
+// step.  fp32: steps of 32 tokens, the fp32 matrix instruction takes its operands from the rows as they lie;
+// bound by it where there are tiles enough (512 x 256 over 50176 tokens 558 + 32 -> 136 us, 104 TFLOP/s of 153).
 #include <hip/hip_runtime.h>
 
 #include "fbla_mfma_shared.h"
@@ -23,10 +24,12 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kTile = 128;               // rows and columns of the result per workgroup
-constexpr int kStepTokens = 64;
-constexpr int kLeastChunk = 4 * kStepTokens;
-constexpr int kRowBytes = kTile * 2;
-constexpr int kStepBytes = kStepTokens * kRowBytes;
+constexpr int kStepBytes = 64 * 128 * 2; // one operand's rows of a step: 64 tokens of 16 bits, 32 of fp32
+constexpr int kLeastChunk = 256;
+template <typename T> struct Step {
+  static constexpr int kVec = 16 / sizeof(T), kRowBytes = kTile * sizeof(T), kTokens = kStepBytes / kRowBytes;
+  static constexpr int kRowPieces = kTile / kVec, kRows = kThreads / kRowPieces;  // rows that the threads move at a time
+};
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
@@ -52,6 +55,61 @@ __device__ __forceinline__ u32x4 tr_fragment(const unsigned char* tile, int off0
   return u32x4{a[0], a[1], b[0], b[1]};
 }
 
+// One step's products for a wave's 64 x 64 quarter (wm, wn).
+template <typename T> struct Multiply {
+  static constexpr int kRowBytes = Step<T>::kRowBytes;
+  // transposing reads: this lane addresses, for element half h, token 4 (s / 4) + 2 (g / 2) + h (+ 16 ks) and the four
+  // features 16 (g % 2) + 4 (s % 4) .. + 3 of a fragment of 32 (g = lane / 16, s = lane % 16)
+  int goff[2][2], xoff[2][2];
+  __device__ __forceinline__ Multiply(int lane, int wm, int wn) {
+    const int g16 = lane >> 4, s16 = lane & 15;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int a = 0; a < 2; ++a) {
+        const int tok = 4 * (s16 >> 2) + 2 * (g16 >> 1) + h, f = 32 * a + 16 * (g16 & 1) + 4 * (s16 & 3);
+        const int fg = 64 * wm + f, fx = 64 * wn + f;
+        goff[a][h] = mfma::swz<kRowBytes>(tok, fg >> 3) + ((fg >> 2) & 1) * 8;
+        xoff[a][h] = mfma::swz<kRowBytes>(tok, fx >> 3) + ((fx >> 2) & 1) * 8;
+      }
+  }
+  static __device__ __forceinline__ int place(int row, int piece) { return mfma::swz<kRowBytes>(row, piece); }
+  __device__ __forceinline__ void operator()(const unsigned char* gt, const unsigned char* xt, f32x16 (&acc)[2][2]) const {
+#pragma unroll
+    for (int ks = 0; ks < Step<T>::kTokens / 16; ++ks) {
+      u32x4 ga[2], xb[2];
+#pragma unroll
+      for (int a = 0; a < 2; ++a) {
+        ga[a] = tr_fragment(gt + ks * 16 * kRowBytes, goff[a][0], goff[a][1]);
+        xb[a] = tr_fragment(xt + ks * 16 * kRowBytes, xoff[a][0], xoff[a][1]);
+      }
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) acc[a][b] = mma<T>(ga[a], xb[b], acc[a][b]);
+    }
+  }
+};
+// fp32: the operand of 32x32x2 is one feature per lane and a token per half wave, which is a row of the tile as it lies
+template <> struct Multiply<float> {
+  int goff, xoff;
+  __device__ __forceinline__ Multiply(int lane, int wm, int wn)
+      : goff((lane >> 5) * kTile + 64 * wm + (lane & 31)), xoff((lane >> 5) * kTile + 64 * wn + (lane & 31)) {}
+  static __device__ __forceinline__ int place(int row, int piece) { return row * Step<float>::kRowBytes + piece * 16; }
+  __device__ __forceinline__ void operator()(const unsigned char* gt, const unsigned char* xt, f32x16 (&acc)[2][2]) const {
+    const float* g = reinterpret_cast<const float*>(gt) + goff;
+    const float* x = reinterpret_cast<const float*>(xt) + xoff;
+#pragma unroll
+    for (int ks = 0; ks < Step<float>::kTokens / 2; ++ks)
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+          acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(g[2 * ks * kTile + 32 * a], x[2 * ks * kTile + 32 * b], acc[a][b],
+                                                           0, 0, 0);
+  }
+};
+
 // partial [chunk][M][N], bias_partial [chunk][M] (null: no bias)
 template <typename T>
 __global__ __launch_bounds__(kThreads, 2) void wgrad_kernel(const T* __restrict__ g, int64_t g_row, const T* __restrict__ x,
@@ -76,39 +134,25 @@ __global__ __launch_bounds__(kThreads, 2) void wgrad_kernel(const T* __restrict_
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1;
 
-  // thread t moves pieces t % 16 of rows t / 16 + 16 i of a step; what lies outside the matrices or the chunk is zero
-  const int prow = tid >> 4, pch = tid & 15;
-  const bool g_piece = m0 + 8 * pch < M, x_piece = n0 + 8 * pch < N;
-  const T* gp = g + (t_begin + prow) * g_row + m0 + 8 * pch;
-  const T* xp = x + (t_begin + prow) * x_row + n0 + 8 * pch;
+  // thread t moves one piece of rows t / kRowPieces + kRows i of a step; what lies outside the matrices or the chunk is zero
+  constexpr int V = Step<T>::kVec, kRows = Step<T>::kRows, kTokens = Step<T>::kTokens;
+  const int prow = tid / Step<T>::kRowPieces, pch = tid % Step<T>::kRowPieces;
+  const bool g_piece = m0 + V * pch < M, x_piece = n0 + V * pch < N;
+  const T* gp = g + (t_begin + prow) * g_row + m0 + V * pch;
+  const T* xp = x + (t_begin + prow) * x_row + n0 + V * pch;
   auto load_step = [&](u32x4(&dst)[4], const T* src, int64_t row, int base, bool has) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       dst[i] = u32x4{0u, 0u, 0u, 0u};
-      if (has && base + prow + 16 * i < len) dst[i] = *reinterpret_cast<const u32x4*>(src + (base + 16 * i) * row);
+      if (has && base + prow + kRows * i < len) dst[i] = *reinterpret_cast<const u32x4*>(src + (base + kRows * i) * row);
     }
   };
   auto stash = [&](const u32x4(&src)[4], unsigned char* to) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) *reinterpret_cast<u32x4*>(to + mfma::swz<kRowBytes>(prow + 16 * i, pch)) = src[i];
+    for (int i = 0; i < 4; ++i) *reinterpret_cast<u32x4*>(to + Multiply<T>::place(prow + kRows * i, pch)) = src[i];
   };
 
-  // transposing reads: this lane addresses, for element half h, token 4 (s / 4) + 2 (g / 2) + h (+ 16 ks) and the four
-  // features 16 (g % 2) + 4 (s % 4) .. + 3 of a fragment of 32 (g = lane / 16, s = lane % 16)
-  int goff[2][2], xoff[2][2];
-  {
-    const int g16 = lane >> 4, s16 = lane & 15;
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-      for (int a = 0; a < 2; ++a) {
-        const int tok = 4 * (s16 >> 2) + 2 * (g16 >> 1) + h, f = 32 * a + 16 * (g16 & 1) + 4 * (s16 & 3);
-        const int fg = 64 * wm + f, fx = 64 * wn + f;
-        goff[a][h] = mfma::swz<kRowBytes>(tok, fg >> 3) + ((fg >> 2) & 1) * 8;
-        xoff[a][h] = mfma::swz<kRowBytes>(tok, fx >> 3) + ((fx >> 2) & 1) * 8;
-      }
-  }
-
+  const Multiply<T> multiply(lane, wm, wn);
   f32x16 acc[2][2];
 #pragma unroll
   for (int a = 0; a < 2; ++a)
@@ -117,13 +161,15 @@ __global__ __launch_bounds__(kThreads, 2) void wgrad_kernel(const T* __restrict_
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.f;
   const bool with_bias = bias_partial != nullptr && n0 == 0;
-  float bias[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  float bias[V];
+#pragma unroll
+  for (int j = 0; j < V; ++j) bias[j] = 0.f;
 
   u32x4 grow[4], xrow[4];
   load_step(grow, gp, g_row, 0, g_piece);
   load_step(xrow, xp, x_row, 0, x_piece);
   int buf = 0;
-  for (int base = 0; base < len; base += kStepTokens) {
+  for (int base = 0; base < len; base += kTokens) {
     unsigned char* gt = smem + buf * 2 * kStepBytes;
     unsigned char* xt = gt + kStepBytes;
     stash(grow, gt);
@@ -131,28 +177,16 @@ __global__ __launch_bounds__(kThreads, 2) void wgrad_kernel(const T* __restrict_
     if (with_bias) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        union { u32x4 w; T e[8]; } p;
+        union { u32x4 w; T e[V]; } p;
         p.w = grow[i];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) bias[j] += (float)p.e[j];
+        for (int j = 0; j < V; ++j) bias[j] += (float)p.e[j];
       }
     }
-    load_step(grow, gp, g_row, base + kStepTokens, g_piece);
-    load_step(xrow, xp, x_row, base + kStepTokens, x_piece);
+    load_step(grow, gp, g_row, base + kTokens, g_piece);
+    load_step(xrow, xp, x_row, base + kTokens, x_piece);
     __syncthreads();  // the step is in LDS; every wave is done with the step before it, whose buffer is written next
-#pragma unroll
-    for (int ks = 0; ks < kStepTokens / 16; ++ks) {
-      u32x4 ga[2], xb[2];
-#pragma unroll
-      for (int a = 0; a < 2; ++a) {
-        ga[a] = tr_fragment(gt + ks * 16 * kRowBytes, goff[a][0], goff[a][1]);
-        xb[a] = tr_fragment(xt + ks * 16 * kRowBytes, xoff[a][0], xoff[a][1]);
-      }
-#pragma unroll
-      for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b) acc[a][b] = mma<T>(ga[a], xb[b], acc[a][b]);
-    }
+    multiply(gt, xt, acc);
     buf ^= 1;
   }
 
@@ -169,14 +203,14 @@ __global__ __launch_bounds__(kThreads, 2) void wgrad_kernel(const T* __restrict_
       }
   if (with_bias) {
     __syncthreads();  // all waves have read their last step
-    float* sums = reinterpret_cast<float*>(smem);  // [16 row groups][128]
+    float* sums = reinterpret_cast<float*>(smem);  // [kRows][128]
 #pragma unroll
-    for (int j = 0; j < 8; ++j) sums[prow * kTile + 8 * pch + j] = bias[j];
+    for (int j = 0; j < V; ++j) sums[prow * kTile + V * pch + j] = bias[j];
     __syncthreads();
     if (tid < kTile && m0 + tid < M) {
       float v = 0.f;
 #pragma unroll
-      for (int i = 0; i < 16; ++i) v += sums[i * kTile + tid];
+      for (int i = 0; i < kRows; ++i) v += sums[i * kTile + tid];
       bias_partial[(int64_t)c * M + m0 + tid] = v;
     }
   }
@@ -199,7 +233,7 @@ __global__ __launch_bounds__(kThreads) void wgrad_finish_kernel(const float* __r
     out = bias_out;
   }
   const int lane = threadIdx.x % kLanes, part = threadIdx.x / kLanes;
-  const int at = (wg * kLanes + lane) * 4;  // counts are multiples of 8
+  const int at = (wg * kLanes + lane) * 4;  // counts are multiples of 4
   f32x4 sum = {0.f, 0.f, 0.f, 0.f};
   if (at < count) {
     const float* p = partial + at;
@@ -229,7 +263,7 @@ int chunk_for(int64_t tokens, int M, int N) {
   const int64_t slots = 2 * 256 / ((int64_t)tiles(M) * tiles(N));
   int64_t chunk = cdiv64(tokens, slots < 1 ? 1 : slots);
   if (chunk < kLeastChunk) chunk = kLeastChunk;
-  return (int)(cdiv64(chunk, kStepTokens) * kStepTokens);
+  return (int)(cdiv64(chunk, 64) * 64);
 }
 
 template <typename T>
@@ -253,6 +287,7 @@ size_t wgrad_workspace_bytes(int64_t tokens, int M, int N) {
 void wgrad(const void* g, int64_t g_row, const void* x, int64_t x_row, int64_t tokens, int M, int N, void* dw, void* db,
            float* workspace, int dtype, hipStream_t st) {
   if (dtype == kF16) launch<_Float16>(g, g_row, x, x_row, tokens, M, N, dw, db, workspace, st);
+  else if (dtype == kF32) launch<float>(g, g_row, x, x_row, tokens, M, N, dw, db, workspace, st);
   else launch<__bf16>(g, g_row, x, x_row, tokens, M, N, dw, db, workspace, st);
 }
 

@@ -479,13 +479,13 @@ def _token_rows(t):
     """(tensor, row stride) of t [..., C] as rows the projection kernels can read in place: channels adjacent, whole
     16-byte pieces between the rows; anything else is copied to contiguous memory."""
     rows = t.reshape(-1, t.shape[-1])
-    if rows.stride(1) != 1 or rows.stride(0) % 8 or rows.stride(0) < rows.shape[1] or rows.data_ptr() % 16:
+    if rows.stride(1) != 1 or rows.stride(0) * rows.element_size() % 16 or rows.stride(0) < rows.shape[1] or rows.data_ptr() % 16:
         rows = rows.clone(memory_format=torch.contiguous_format)
     return rows, rows.stride(0)
 
 
 def linear_wgrad(g, x, with_bias):
-    """(dw [M, N], db [M] or None) of y = x W^T + b from the output's gradient g [..., M] and x [..., N] (16-bit)."""
+    """(dw [M, N], db [M] or None) of y = x W^T + b from the output's gradient g [..., M] and x [..., N]."""
     _require_gpu(g, x)
     g, g_row = _token_rows(g)
     x, x_row = _token_rows(x)

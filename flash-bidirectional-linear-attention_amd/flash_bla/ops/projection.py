@@ -41,24 +41,27 @@ def plain_tensors(*tensors):
                 torch._C._are_functorch_transforms_active())
 
 
-# Results beyond these are enough tiles for the library's GEMM.  Measured in bf16, library's gradient + bias sum against the
-# kernel: 1280 x 1280 over 1024 / 4096 tokens 22 + 13 against 26, 37 + 22 against 40 us; 1024 x 1024 over 2048 tokens 21 + 13
-# against 24 us; 640 x 640 over 4096 tokens 29 + 19 against 21 us, 512 x 512 over 512 tokens 21 + 9 against 17 us.
-MOST_WEIGHTS, MOST_WEIGHTS_WITH_BIAS = 1 << 19, 1 << 21
-
-
-def splits_tokens(M, N, with_bias):
-    """Whether the kernel beats the library's gradient of an M x N weight (and its bias)."""
-    return M * N <= (MOST_WEIGHTS_WITH_BIAS if with_bias else MOST_WEIGHTS)
+def splits_tokens(tokens, M, N, with_bias, fp32):
+    """Whether the kernel beats the library's gradient of an M x N weight (and its column sums for the bias).  Results with
+    many tiles fill the GPU by themselves.  Measured, library + bias sum against the kernel, us:
+    bf16: 1280 x 1280 over 1024 / 4096 tokens 22 + 13 / 26, 37 + 22 / 40; 1024 x 1024 over 2048 21 + 13 / 24; 640 x 640 over
+    4096 29 + 19 / 21; 512 x 512 over 512 21 + 9 / 17.
+    fp32: 512 x 256 over 50176 558 + 32 / 136; 320 x 320 over 8192 50 + 17 / 46; 640 x 640 over 4096 38 + 18 / 51; 1024 x 256
+    over 3136 25 + 17 / 32; 1024 x 1024 over 2048 39 + 13 / 55; 256 x 128 over 1024 22 + 11 / 28."""
+    if fp32:
+        return M * N <= 1 << 19 if with_bias else M * N <= 1 << 17 and tokens >= 8192
+    return M * N <= (1 << 21 if with_bias else 1 << 19)
 
 
 def runs_on_rows(x, weight, bias):
     """Whether the weight gradient of F.linear(x, weight, bias) is left to the kernel."""
-    return (torch.is_grad_enabled() and weight.requires_grad and x.is_cuda and
-            x.dtype in (torch.float16, torch.bfloat16) and weight.dtype == x.dtype and weight.device == x.device and
-            (bias is None or bias.dtype == x.dtype) and x.ndim >= 2 and x.numel() > 0 and
-            x.shape[-1] == weight.shape[1] and weight.shape[0] % 8 == 0 and weight.shape[1] % 8 == 0 and
-            splits_tokens(*weight.shape, bias is not None) and x.numel() // x.shape[-1] <= 1 << 30 and plain_tensors(x, weight, bias))
+    if not (weight.requires_grad and x.is_cuda and torch.is_grad_enabled() and x.ndim >= 2 and x.numel() > 0 and
+            x.dtype in (torch.float16, torch.bfloat16, torch.float32) and x.shape[-1] == weight.shape[1]):
+        return False
+    (M, N), piece, tokens = weight.shape, 16 // x.element_size(), x.numel() // x.shape[-1]
+    return (weight.dtype == x.dtype and weight.device == x.device and (bias is None or bias.dtype == x.dtype) and
+            M % piece == 0 and N % piece == 0 and tokens <= 1 << 30 and
+            splits_tokens(tokens, M, N, bias is not None, x.dtype == torch.float32) and plain_tensors(x, weight, bias))
 
 
 class TokenLinear(nn.Linear):
@@ -66,6 +69,7 @@ class TokenLinear(nn.Linear):
     faster of the two; otherwise, and on the CPU, nn.Linear itself."""
 
     def forward(self, x):
-        if runs_on_rows(x, self.weight, self.bias):
-            return TokenLinearFunction.apply(x, self.weight, self.bias)
-        return super().forward(x)
+        weight, bias = self.weight, self.bias
+        if torch.is_grad_enabled() and runs_on_rows(x, weight, bias):
+            return TokenLinearFunction.apply(x, weight, bias)
+        return F.linear(x, weight, bias)

@@ -282,7 +282,7 @@ int fbla_dwconv_grad(const void* x, int64_t x_batch, int64_t x_row, const void* 
 /* Gradients of a projection y = x W^T + b over token rows: dw [M, N] = sum over the tokens of g[t]^T x[t], db [M] (or NULL) =
  * the sum of g, in fp32 in a fixed order, rounded once.  What autograd computes for the blocks' nn.Linear layers
  * (flash_bla/layers/mlla.py:56, rala.py:31, focused_la.py:26-27, polaformer.py:24-25).  g: rows of M elements g_row
- * apart, x: rows of N elements x_row apart (whole 16-byte pieces); fp16 / bf16, M and N multiples of 8.
+ * apart, x: rows of N elements x_row apart (whole 16-byte pieces); M and N multiples of 8 (16-bit) or 4 (fp32).
  * workspace: fbla_linear_wgrad_workspace_bytes bytes of device memory. */
 size_t fbla_linear_wgrad_workspace_bytes(int64_t tokens, int M, int N, int dtype);
 int fbla_linear_wgrad(const void* g, int64_t g_row, const void* x, int64_t x_row, void* dw, void* db, void* workspace,
