@@ -716,6 +716,12 @@ int fbla_dwconv_fwd(const void* x, int64_t x_batch, int64_t x_row, const void* w
   }
   if (check_aligned(what, {x, y}) != kOk || check_row_strides(what, C, dtype, {x_batch, x_row, y_batch, y_row}) != kOk)
     return kErrBadArg;
+  // the rows of y are written by different workgroups: batches one after the other, or interleaved by tokens
+  if (B > 1 && y_batch < (H * W - 1) * y_row + C && y_row < (B - 1) * y_batch + C) {
+    set_error("%s: the batches of y overlap (y_batch=%lld y_row=%lld for %lld x %lld tokens)", what, (long long)y_batch,
+              (long long)y_row, (long long)H, (long long)W);
+    return kErrBadArg;
+  }
   dwconv::forward(c, K, dtype, flip != 0, (hipStream_t)stream);
   return check_launch(what);
 }

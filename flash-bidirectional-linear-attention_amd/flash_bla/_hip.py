@@ -444,8 +444,15 @@ def _rows(t):
     return t, t.stride(0), t.stride(1)
 
 
+def _check_grid(what, x, H, W):
+    """The kernels walk the H x W grid: it has to be the tokens'."""
+    if x.ndim != 3 or H < 1 or W < 1 or x.shape[1] != H * W:
+        raise ValueError(f"{what}: rows [B, H * W, C] needed, got {tuple(x.shape)} for H = {H}, W = {W}")
+
+
 def dwconv_fwd(x, w, bias, H, W, flip=False):
     """Depth-wise convolution of token rows x [B, H*W, C] with w [Cw, 1, K, K]; returns contiguous [B, H*W, C]."""
+    _check_grid("dwconv_fwd", x, H, W)
     _require_gpu(x, w, bias)
     x, x_batch, x_row = _rows(x)
     B, N, C = x.shape
@@ -459,6 +466,9 @@ def dwconv_fwd(x, w, bias, H, W, flip=False):
 
 def dwconv_grad(x, g, w, H, W, with_bias):
     """(dw, db or None) of dwconv_fwd from its input and its output's gradient, both [B, H*W, C]."""
+    _check_grid("dwconv_grad", x, H, W)
+    if g.shape != x.shape:
+        raise ValueError(f"dwconv_grad: x and g must have one shape, got {tuple(x.shape)} and {tuple(g.shape)}")
     _require_gpu(x, g, w)
     x, x_batch, x_row = _rows(x)
     g, g_batch, g_row = _rows(g)

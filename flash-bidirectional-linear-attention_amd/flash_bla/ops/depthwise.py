@@ -56,9 +56,9 @@ def runs_on_tokens(x, conv):
 def depthwise_conv_tokens(x, conv, H, W):
     """The depth-wise convolution `conv` (an nn.Conv2d over Cw channels) of token rows x [B, H*W, C], C a multiple of
     Cw: channel c is convolved with filter c % Cw.  Returns [B, H*W, C].  What the kernels do not take (CPU tensors,
-    other filter shapes) runs as the torch convolution of the transposed tokens."""
-    B, N, C = x.shape
-    if runs_on_tokens(x, conv):
+    other filter shapes, an H or W that the tokens do not fill: the reshape there refuses it) runs as the torch
+    convolution of the transposed tokens."""
+    if x.shape[1] == H * W and runs_on_tokens(x, conv):
         return DepthwiseConvTokensFunction.apply(x, conv.weight, conv.bias, H, W)
     return _convolution_of_images(x, H, W, conv.weight.shape[0], conv)
 

@@ -266,7 +266,8 @@ int fbla_elu1_bwd(const void* x, const void* dy, void* dx, int64_t n, int dtype,
  * nn.Conv2d on a transposed view of the tokens (flash_bla/layers/mlla.py:92, rala.py:58, focused_la.py:88-93,
  * polaformer.py:97-101), which reads and writes the tokens where they are.  Token t of batch b is the C elements at
  * x + b * x_batch + t * x_row (strides in elements: whole 16-byte pieces, at least C; likewise y and g); w [Cw, K, K] and
- * bias [Cw] (or NULL) have the element type of x.  K is 3, 5 or 7, C a multiple of Cw and of 8 (16-bit) or 4 (fp32).
+ * bias [Cw] (or NULL) have the element type of x.  x, y and g hold B batches of H * W tokens (the batches of y may not
+ * overlap).  K is 3, 5 or 7, C a multiple of Cw and of 8 (16-bit) or 4 (fp32).
  * flip != 0 applies the taps in reverse order: with the output's gradient as x and no bias, the gradient of x. */
 int fbla_dwconv_fwd(const void* x, int64_t x_batch, int64_t x_row, const void* w, const void* bias, void* y,
                     int64_t y_batch, int64_t y_row, int64_t B, int64_t H, int64_t W, int C, int Cw, int K, int flip,

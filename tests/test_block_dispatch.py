@@ -1,0 +1,32 @@
+"""What the blocks' fused steps take and what they leave to the torch compositions, decided on the host: nothing here
+launches a kernel.  A call that torch's operators refuse stays refused, one that they run stays theirs."""
+import pytest
+import torch
+import torch.nn as nn
+
+from flash_bla import _hip
+from flash_bla.ops import depthwise
+
+
+@pytest.mark.parametrize("H,W", [(5, 4), (4, 3), (8, 8), (2, 2), (16, 2)])
+def test_token_convolution_refuses_a_grid_that_is_not_the_tokens(H, W, monkeypatch):
+    """16 tokens: the reshape of the torch composition raises, and no kernel sees the call."""
+    monkeypatch.setattr(depthwise, "runs_on_tokens", lambda *a: True)
+    monkeypatch.setattr(depthwise.DepthwiseConvTokensFunction, "apply", lambda *a: pytest.fail("reached the kernel"))
+    conv, x = nn.Conv2d(8, 8, 3, padding=1, groups=8), torch.randn(2, 16, 16)
+    with pytest.raises(RuntimeError):
+        depthwise.depthwise_conv_tokens(x, conv, H, W)
+    with pytest.raises(ValueError, match="H \\* W"):
+        _hip.dwconv_fwd(x, conv.weight, conv.bias, H, W)
+    with pytest.raises(ValueError, match="H \\* W"):
+        _hip.dwconv_grad(x, x, conv.weight, H, W, True)
+    with pytest.raises(ValueError, match="one shape"):
+        _hip.dwconv_grad(x, x[:, :-1], conv.weight, 4, 4, True)
+
+
+def test_token_convolution_entry_point_refuses_overlapping_output_batches():
+    L, at = _hip.lib(), 4096  # an aligned address that is never looked at
+    args = (at, 16 * 8, 8, at, None, at)
+    for y_batch, y_row in ((8 * 15, 8), (8, 8), (16, 8)):
+        assert L.fbla_dwconv_fwd(*args, y_batch, y_row, 2, 4, 4, 8, 8, 3, 0, _hip.F16, None) == -1
+        assert b"overlap" in L.fbla_last_error()
