@@ -144,9 +144,12 @@ static bool widen(const Prob& p, int dtype) {
 }
 // 16-bit rows of the plain operator need no copies: the kernels move the last piece of a row back to its end and take
 // the true row lengths (Prob::RK, RV) next to the widened shape of the state, of which only S and km (a few MB) are
-// resized.  B8-H16-T4093, D=100 bf16, forward + backward: copies of eleven tensors 419 of 796 us before.
+// resized.  B8-H16-T4093, D=100 bf16, forward + backward: copies of eleven tensors 419 of 796 us before.  The backward
+// knows the true lengths in the one-kernel pass A only: shapes without it (wide packed heads beyond its 32-bit lane
+// offsets) keep the copies.
 static bool ragged(const Prob& p, int dtype) {
-  return dtype != kF32 && !(p.flags & (kDecoupled | kElu1 | kElu1Grad)) && p.DK >= 8 && p.DV >= 8 && widen(p, dtype);
+  return dtype != kF32 && !(p.flags & (kDecoupled | kElu1 | kElu1Grad)) && p.DK >= 8 && p.DV >= 8 && widen(p, dtype) &&
+         mfma::bwd_a_supported(widened(p, dtype), dtype);
 }
 static Prob ragged_problem(const Prob& p, int dtype) {
   Prob w = widened(p, dtype);

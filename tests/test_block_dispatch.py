@@ -30,3 +30,17 @@ def test_token_convolution_entry_point_refuses_overlapping_output_batches():
     for y_batch, y_row in ((8 * 15, 8), (8, 8), (16, 8)):
         assert L.fbla_dwconv_fwd(*args, y_batch, y_row, 2, 4, 4, 8, 8, 3, 0, _hip.F16, None) == -1
         assert b"overlap" in L.fbla_last_error()
+
+
+@pytest.mark.parametrize("dims", [(100, 100), (65, 9), (9, 121)])
+def test_ragged_heads_without_the_one_kernel_pass_a_keep_the_widened_copies(dims):
+    """More packed heads than that kernel addresses: the two kernels that replace it read rows of whole pieces, so the
+    workspace grows with the tokens by widened copies of q, k, v, dO and of the gradients; one head fewer: in place, it
+    does not grow.  (One side is 64 wide or more throughout.)"""
+    L, (DK, DV), T = _hip.lib(), dims, 64
+
+    def growth(H):
+        need = [L.fbla_varlen_workspace_bytes(1, t, 2, H, 32, DK, DV, _hip.BF16, _hip.NORMALIZE) for t in (T, 2 * T)]
+        return need[1] - need[0]
+    assert growth(65537) >= 2 * T * 65537 * (4 * ((DK + 7) // 8 * 8) + 3 * ((DV + 7) // 8 * 8))
+    assert growth(65536) == 0
