@@ -201,26 +201,29 @@ static size_t bwd_used_bytes(const Prob& pc, int dtype) {
          tokscal_bytes(p, dtype);
 }
 
+// Head dims between the row lengths: never less than the shape-generic kernels use, which take over while the phases are
+// timed one by one (phase_mask).
+
 // partials | walking order
 size_t fwd_workspace_bytes(const Prob& pc, int dtype) {
+  const size_t plain = fwd_used_bytes(pc, dtype) + perm_bytes(pc);
   if (ragged(pc, dtype)) {
     const Prob w = ragged_problem(pc, dtype);
-    // (never less than the copies' form of the same shape asks for: callers size one workspace per shape from this
+    // (nor less than the copies' form of the same shape asks for: callers size one workspace per shape from this
     // query, whichever of the two forms a flag then selects)
-    return std::max(state_bytes(w) + vec_bytes(w) + fwd_workspace_bytes(w, dtype), widened_fwd_bytes(pc, dtype));
+    return std::max({plain, state_bytes(w) + vec_bytes(w) + fwd_workspace_bytes(w, dtype), widened_fwd_bytes(pc, dtype)});
   }
-  if (widen(pc, dtype)) return widened_fwd_bytes(pc, dtype);
-  return fwd_used_bytes(pc, dtype) + perm_bytes(pc);
+  return widen(pc, dtype) ? std::max(plain, widened_fwd_bytes(pc, dtype)) : plain;
 }
 
 // partials | S^T | s*dS | (s*dS)^T | dkm/L | per-row scalars | walking order
 size_t bwd_workspace_bytes(const Prob& pc, int dtype) {
+  const size_t plain = bwd_used_bytes(pc, dtype) + perm_bytes(pc);
   if (ragged(pc, dtype)) {
     const Prob w = ragged_problem(pc, dtype);
-    return state_bytes(w) + vec_bytes(w) + bwd_workspace_bytes(w, dtype);
+    return std::max(plain, state_bytes(w) + vec_bytes(w) + bwd_workspace_bytes(w, dtype));
   }
-  if (widen(pc, dtype)) return widened_bwd_bytes(pc, dtype);
-  return bwd_used_bytes(pc, dtype) + perm_bytes(pc);
+  return widen(pc, dtype) ? std::max(plain, widened_bwd_bytes(pc, dtype)) : plain;
 }
 
 // Different numbers of queries and keys work for every operator family (the decoupled one too:

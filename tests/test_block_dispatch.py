@@ -44,3 +44,21 @@ def test_ragged_heads_without_the_one_kernel_pass_a_keep_the_widened_copies(dims
         return need[1] - need[0]
     assert growth(65537) >= 2 * T * 65537 * (4 * ((DK + 7) // 8 * 8) + 3 * ((DV + 7) // 8 * 8))
     assert growth(65536) == 0
+
+
+@pytest.mark.parametrize("L,DK,DV", [(257, 8, 13), (257, 8, 60), (4093, 100, 100), (1000, 66, 9)])
+def test_backward_workspace_of_ragged_heads_holds_the_generic_kernels(L, DK, DV):
+    """They take over while single phases are timed: one state partial and mean key per chunk of 64 tokens (the shortest
+    chunk, taken by a single head of up to 65536 tokens), S^T, s dS, (s dS)^T, dkm, each rounded up to 256 bytes."""
+    up = lambda n: (n + 255) // 256 * 256  # noqa: E731
+    need = up((L + 63) // 64 * (DK * DV + DK) * 4) + 3 * up(DK * DV * 4) + up(DK * 4)
+    for dtype in (_hip.F16, _hip.BF16):
+        assert _hip.lib().fbla_la_workspace_bytes(1, 1, 1, L, DK, DV, dtype, _hip.NORMALIZE) >= need
+
+
+def test_forward_workspace_of_ragged_heads_holds_the_generic_kernels():
+    """The same with three times as many keys as queries, where the partials outgrow the widened copies: chunks of 64
+    keys."""
+    up = lambda n: (n + 255) // 256 * 256  # noqa: E731
+    need = _hip.lib().fbla_la_cross_workspace_bytes(0, 1, 1, 1000, 3000, 127, 126, _hip.BF16, _hip.NORMALIZE)
+    assert need >= up((3000 + 63) // 64 * (127 * 126 + 127) * 4)
