@@ -453,6 +453,8 @@ def _check_grid(what, x, H, W):
 def dwconv_fwd(x, w, bias, H, W, flip=False):
     """Depth-wise convolution of token rows x [B, H*W, C] with w [Cw, 1, K, K]; returns contiguous [B, H*W, C]."""
     _check_grid("dwconv_fwd", x, H, W)
+    if w.dtype != x.dtype or (bias is not None and bias.dtype != x.dtype):
+        raise ValueError("dwconv_fwd: x, w and bias must have one dtype")
     _require_gpu(x, w, bias)
     x, x_batch, x_row = _rows(x)
     B, N, C = x.shape
@@ -469,6 +471,8 @@ def dwconv_grad(x, g, w, H, W, with_bias):
     _check_grid("dwconv_grad", x, H, W)
     if g.shape != x.shape:
         raise ValueError(f"dwconv_grad: x and g must have one shape, got {tuple(x.shape)} and {tuple(g.shape)}")
+    if w.dtype != x.dtype or g.dtype != x.dtype:
+        raise ValueError("dwconv_grad: x, g and w must have one dtype")
     _require_gpu(x, g, w)
     x, x_batch, x_row = _rows(x)
     g, g_batch, g_row = _rows(g)

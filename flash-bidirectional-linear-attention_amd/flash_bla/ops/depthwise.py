@@ -45,9 +45,11 @@ def runs_on_tokens(x, conv):
     square filters of 3 to 7 taps a side, stride 1, "same" zero padding, whole 16-byte pieces of channels; a module
     without hooks."""
     K = conv.kernel_size[0]
-    w = conv.weight
-    return (untouched(conv, nn.Conv2d) and plain_tensors(x, w, conv.bias) and x.is_cuda and x.numel() > 0 and
-            x.dtype in (torch.float16, torch.bfloat16, torch.float32) and w.dtype == x.dtype and w.device == x.device and conv.kernel_size == (K, K) and K in (3, 5, 7) and
+    w, bias = conv.weight, conv.bias
+    return (untouched(conv, nn.Conv2d) and plain_tensors(x, w, bias) and x.is_cuda and x.numel() > 0 and
+            x.dtype in (torch.float16, torch.bfloat16, torch.float32) and w.dtype == x.dtype and w.device == x.device and
+            (bias is None or bias.dtype == x.dtype and bias.device == x.device and bias.shape == w.shape[:1]) and
+            conv.kernel_size == (K, K) and w.shape[2:] == (K, K) and K in (3, 5, 7) and
             conv.padding == (K // 2, K // 2) and conv.padding_mode == 'zeros' and conv.stride == (1, 1) and
             conv.dilation == (1, 1) and conv.groups == w.shape[0] and w.shape[1] == 1 and
             x.shape[-1] % w.shape[0] == 0 and x.shape[-1] % (16 // x.element_size()) == 0)

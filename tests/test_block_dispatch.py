@@ -62,3 +62,31 @@ def test_forward_workspace_of_ragged_heads_holds_the_generic_kernels():
     up = lambda n: (n + 255) // 256 * 256  # noqa: E731
     need = _hip.lib().fbla_la_cross_workspace_bytes(0, 1, 1, 1000, 3000, 127, 126, _hip.BF16, _hip.NORMALIZE)
     assert need >= up((3000 + 63) // 64 * (127 * 126 + 127) * 4)
+
+
+class _Described(torch.Tensor):
+    is_cuda = True
+
+
+def _on_gpu(x):
+    """x with the properties of a GPU tensor, for rules that look at no more than those."""
+    return x.as_subclass(_Described)
+
+
+@pytest.mark.parametrize("types", [(torch.bfloat16, torch.float32), (torch.float32, torch.float16), None])
+def test_token_convolution_leaves_a_bias_of_another_type_to_torch(types, monkeypatch):
+    """nn.Conv2d refuses it; the kernel would read its bytes as x's type."""
+    monkeypatch.setattr(depthwise, "plain_tensors", lambda *a: True)
+    for bias in (True, False):
+        conv = nn.Conv2d(8, 8, 3, padding=1, groups=8, bias=bias)
+        x = _on_gpu(torch.randn(2, 16, 16))
+        assert depthwise.runs_on_tokens(x, conv)
+        if types:
+            conv, x = conv.to(types[0]), _on_gpu(x.to(types[0]))
+            assert depthwise.runs_on_tokens(x, conv)
+        if bias:
+            conv.bias = nn.Parameter(conv.bias.detach().to(types[1]) if types else torch.zeros(8, device="meta"))
+            assert not depthwise.runs_on_tokens(x, conv)
+    for w, b in ((torch.half, torch.float), (torch.float, torch.half)):
+        with pytest.raises(ValueError, match="dtype"):
+            _hip.dwconv_fwd(torch.randn(2, 16, 16).to(w), torch.randn(8, 1, 3, 3).to(w), torch.zeros(8, dtype=b), 4, 4)
