@@ -1,5 +1,6 @@
 """Argument validation shared by the dense operators."""
 import torch
+from torch.nn.modules.module import _has_any_global_hook
 
 
 def check_dense(name, q, k, v, extra=()):
@@ -36,6 +37,8 @@ def check_dense(name, q, k, v, extra=()):
 
 
 def untouched(module, kind):
-    """Whether `module` is a plain `kind` that a fused path may stand in for: no subclass, no hooks of its own."""
-    return type(module) is kind and not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or
-                                         module._backward_pre_hooks)
+    """Whether `module` is a plain `kind` that a fused path may stand in for: no subclass, nothing that runs around its
+    forward (hooks of its own or of all modules) or in its place (a forward set on the instance, Module.compile)."""
+    return (type(module) is kind and not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or
+                                          module._backward_pre_hooks or _has_any_global_hook()) and
+            "forward" not in module.__dict__ and module._compiled_call_impl is None)

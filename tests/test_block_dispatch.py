@@ -5,7 +5,9 @@ import torch
 import torch.nn as nn
 
 from flash_bla import _hip
+from flash_bla.layers.mlla import RoPE
 from flash_bla.ops import depthwise
+from flash_bla.ops._check import untouched
 
 
 @pytest.mark.parametrize("H,W", [(5, 4), (4, 3), (8, 8), (2, 2), (16, 2)])
@@ -90,3 +92,24 @@ def test_token_convolution_leaves_a_bias_of_another_type_to_torch(types, monkeyp
     for w, b in ((torch.half, torch.float), (torch.float, torch.half)):
         with pytest.raises(ValueError, match="dtype"):
             _hip.dwconv_fwd(torch.randn(2, 16, 16).to(w), torch.randn(8, 1, 3, 3).to(w), torch.zeros(8, dtype=b), 4, 4)
+
+
+@pytest.mark.parametrize("make", [lambda: nn.Conv2d(8, 8, 3, padding=1, groups=8), lambda: RoPE((4, 4, 8))])
+def test_modules_that_do_more_than_their_class_are_not_stood_in_for(make):
+    module = make()
+    kind, nothing = type(module), lambda *a: None
+    assert untouched(module, kind) and not untouched(module, nn.Module)
+    for register in (module.register_forward_hook, module.register_forward_pre_hook, module.register_full_backward_hook,
+                     module.register_full_backward_pre_hook, nn.modules.module.register_module_forward_hook,
+                     nn.modules.module.register_module_forward_pre_hook,
+                     nn.modules.module.register_module_full_backward_hook,
+                     nn.modules.module.register_module_full_backward_pre_hook):
+        hook = register(nothing)
+        assert not untouched(module, kind)
+        hook.remove()
+        assert untouched(module, kind)
+    module.forward = nothing
+    assert not untouched(module, kind)
+    del module.forward
+    module.compile(backend="eager")
+    assert not untouched(module, kind)
