@@ -7,7 +7,7 @@ import torch.nn.functional as F
 
 from flash_bla.layers._features import interpolate_tokens
 from flash_bla.ops.depthwise import depthwise_conv_tokens
-from flash_bla.ops.projection import TokenLinear
+from flash_bla.ops.projection import project
 
 
 class PvtLinearAttentionBase(nn.Module):
@@ -15,9 +15,9 @@ class PvtLinearAttentionBase(nn.Module):
         assert dim % num_heads == 0, f"dim {dim} should be divided by num_heads {num_heads}."
         self.dim, self.num_heads, self.sr_ratio = dim, num_heads, sr_ratio
         head_dim = dim // num_heads
-        self.kv = TokenLinear(dim, dim * 2, bias=qkv_bias)
+        self.kv = nn.Linear(dim, dim * 2, bias=qkv_bias)
         self.attn_drop = nn.Dropout(attn_drop)
-        self.proj = TokenLinear(dim, dim)
+        self.proj = nn.Linear(dim, dim)
         self.proj_drop = nn.Dropout(proj_drop)
         if sr_ratio > 1:
             self.sr = nn.Conv2d(dim, dim, kernel_size=sr_ratio, stride=sr_ratio)
@@ -31,7 +31,7 @@ class PvtLinearAttentionBase(nn.Module):
         B, N, C = x.shape
         if self.sr_ratio > 1:
             x = self.norm(self.sr(x.transpose(1, 2).reshape(B, C, H, W)).flatten(2).transpose(1, 2))
-        return self.kv(x)
+        return project(self.kv, x)
 
     def _value_conv(self, v, N, H, W):
         """v: (B, heads, n, d) -> depth-wise conv on the H x W grid -> (B, N, C)."""

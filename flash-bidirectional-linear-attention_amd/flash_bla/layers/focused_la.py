@@ -6,7 +6,7 @@ from flash_bla.layers._common import check_mode, merge_heads, torch_linear_atten
 from flash_bla.layers._features import focus_formula, focused_features, merge_heads_with
 from flash_bla.layers._pvt import PvtLinearAttentionBase
 from flash_bla.ops.linear_attn.fused import linear_attention
-from flash_bla.ops.projection import TokenLinear
+from flash_bla.ops.projection import project
 
 
 class FocusedLinearAttention(PvtLinearAttentionBase):
@@ -14,7 +14,7 @@ class FocusedLinearAttention(PvtLinearAttentionBase):
                  sr_ratio=1, focusing_factor=3, kernel_size=5):
         super().__init__()
         self._init_common(dim, num_patches, num_heads, qkv_bias, attn_drop, proj_drop, sr_ratio, kernel_size)
-        self.q = TokenLinear(dim, dim, bias=qkv_bias)
+        self.q = nn.Linear(dim, dim, bias=qkv_bias)
         self.focusing_factor = focusing_factor
 
     def forward(self, x, H, W, mode='triton'):
@@ -22,10 +22,10 @@ class FocusedLinearAttention(PvtLinearAttentionBase):
         N = x.shape[1]
         kv = self._joint_keys_values(x, H, W)
         features = focused_features if fast else focus_formula
-        q, k, v, v_rows = features(self.q(x), kv, self.positional_encoding, F.softplus(self.scale), self.num_heads,
-                                   self.focusing_factor)
+        q, k, v, v_rows = features(project(self.q, x), kv, self.positional_encoding, F.softplus(self.scale),
+                                   self.num_heads, self.focusing_factor)
         if fast:
             out = merge_heads_with(linear_attention(q, k, v), None, self._value_conv_tokens(v_rows, N, H, W))
         else:
             out = merge_heads(torch_linear_attention(q, k, v)) + self._value_conv(v, N, H, W)
-        return self.proj_drop(self.proj(out))
+        return self.proj_drop(project(self.proj, out))

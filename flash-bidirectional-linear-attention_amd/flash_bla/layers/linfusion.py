@@ -11,9 +11,10 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from flash_bla.layers._common import check_mode, torch_linear_attention
+from flash_bla.ops._check import untouched
 from flash_bla.ops.linear_attn.fused import linear_attention
 from flash_bla.ops.linear_attn.varlen import varlen_linear_attention
-from flash_bla.ops.projection import TokenLinear
+from flash_bla.ops.projection import project
 
 
 _CU_CACHE = {}
@@ -35,8 +36,17 @@ def get_none_linear_projection(query_dim, mid_dim=None):
     if mid_dim == -1:
         return nn.Identity()
     width = mid_dim or query_dim
-    return nn.Sequential(TokenLinear(query_dim, width), nn.LayerNorm(width), nn.LeakyReLU(inplace=True),
-                         TokenLinear(width, query_dim))
+    return nn.Sequential(nn.Linear(query_dim, width), nn.LayerNorm(width), nn.LeakyReLU(inplace=True),
+                         nn.Linear(width, query_dim))
+
+
+def project_through(layers, x):
+    """layers(x) with the projections of a plain nn.Sequential as `project` runs them."""
+    if torch.is_grad_enabled() and untouched(layers, nn.Sequential):
+        for layer in layers:
+            x = project(layer, x)
+        return x
+    return layers(x)
 
 
 class GeneralizedLinearAttention(nn.Module):
@@ -45,10 +55,10 @@ class GeneralizedLinearAttention(nn.Module):
         super().__init__()
         inner = out_dim if out_dim is not None else dim_head * heads
         self.heads = out_dim // dim_head if out_dim is not None else heads
-        self.to_q = TokenLinear(query_dim, inner, bias=bias)
-        self.to_k = TokenLinear(query_dim, inner, bias=bias)
-        self.to_v = TokenLinear(query_dim, inner, bias=bias)
-        self.to_out = nn.ModuleList([TokenLinear(inner, out_dim or query_dim, bias=out_bias), nn.Dropout(dropout)])
+        self.to_q = nn.Linear(query_dim, inner, bias=bias)
+        self.to_k = nn.Linear(query_dim, inner, bias=bias)
+        self.to_v = nn.Linear(query_dim, inner, bias=bias)
+        self.to_out = nn.ModuleList([nn.Linear(inner, out_dim or query_dim, bias=out_bias), nn.Dropout(dropout)])
         self.add_non_linear_model(projection_mid_dim)
 
     def add_non_linear_model(self, mid_dim=None):
@@ -67,9 +77,9 @@ class GeneralizedLinearAttention(nn.Module):
     def forward(self, hidden_states, encoder_hidden_states=None, attention_mask=None, mode='triton', **kwargs):
         fast = check_mode(mode)
         context = hidden_states if encoder_hidden_states is None else encoder_hidden_states
-        q = self.to_q(hidden_states + self.to_q_(hidden_states))
-        k = self.to_k(context + self.to_k_(context))
-        v = self.to_v(context)
+        q = project(self.to_q, hidden_states + project_through(self.to_q_, hidden_states))
+        k = project(self.to_k, context + project_through(self.to_k_, context))
+        v = project(self.to_v, context)
         if fast and q.shape[1] == k.shape[1]:
             # The projections come out token-major, (batch, tokens, heads * dim): that is the
             # packed layout of the variable-length operator with equal lengths, so the head
@@ -80,7 +90,7 @@ class GeneralizedLinearAttention(nn.Module):
             packed = [t.reshape(b * n, self.heads, -1) for t in (q, k, v)]
             out = varlen_linear_attention(*packed, _equal_cu_seqlens(b, n, q.device), n, eps=1e-4,
                                           feature_map="elu+1")
-            return self.to_out[1](self.to_out[0](out.reshape(b, n, -1)))
+            return self.to_out[1](project(self.to_out[0], out.reshape(b, n, -1)))
         q, k, v = (self.head_to_batch_dim(t) for t in (q, k, v))
         if fast:
             b = hidden_states.shape[0]
@@ -90,4 +100,4 @@ class GeneralizedLinearAttention(nn.Module):
             q, k = F.elu(q) + 1.0, F.elu(k) + 1.0
             out = torch_linear_attention(q, k, v, eps=1e-4)
         out = self.batch_to_head_dim(out)
-        return self.to_out[1](self.to_out[0](out))
+        return self.to_out[1](project(self.to_out[0], out))

@@ -9,7 +9,7 @@ from flash_bla.ops._check import untouched
 from flash_bla.ops.depthwise import depthwise_conv_tokens
 from flash_bla.ops.feature_map import elu_plus_one
 from flash_bla.ops.linear_attn.decoupled import decoupled_la
-from flash_bla.ops.projection import TokenLinear
+from flash_bla.ops.projection import project
 
 
 class RoPE(nn.Module):
@@ -34,7 +34,7 @@ class MambaLikeLinearAttention(nn.Module):
     def __init__(self, dim, input_resolution, num_heads, qkv_bias=True, **kwargs):
         super().__init__()
         self.dim, self.input_resolution, self.num_heads = dim, input_resolution, num_heads
-        self.qk = TokenLinear(dim, dim * 2, bias=qkv_bias)
+        self.qk = nn.Linear(dim, dim * 2, bias=qkv_bias)
         self.elu = nn.ELU()
         self.lepe = nn.Conv2d(dim, dim, 3, padding=1, groups=dim)
         self.rope = RoPE(shape=(input_resolution[0], input_resolution[1], dim))
@@ -43,7 +43,7 @@ class MambaLikeLinearAttention(nn.Module):
         fast = check_mode(mode)
         b, n, c = x.shape
         side = int(n ** 0.5)
-        qk = self.qk(x)
+        qk = project(self.qk, x)
         if fast and untouched(self.rope, RoPE):
             q, k, q_rope, k_rope, v, x_rows = rotary_features(qk, x, self.rope.rotations, side, self.num_heads)
         else:

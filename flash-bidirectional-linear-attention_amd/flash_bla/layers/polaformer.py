@@ -10,7 +10,7 @@ from flash_bla.layers._common import check_mode, merge_heads, torch_linear_atten
 from flash_bla.layers._features import merge_heads_with, polarity_features, polarity_formula
 from flash_bla.layers._pvt import PvtLinearAttentionBase
 from flash_bla.ops.linear_attn.paired import paired_linear_attention
-from flash_bla.ops.projection import TokenLinear
+from flash_bla.ops.projection import project
 
 
 class PolaLinearAttention(PvtLinearAttentionBase):
@@ -19,7 +19,7 @@ class PolaLinearAttention(PvtLinearAttentionBase):
         super().__init__()
         self.head_dim = self._init_common(dim, num_patches, num_heads, qkv_bias, attn_drop, proj_drop, sr_ratio,
                                           kernel_size)
-        self.qg = TokenLinear(dim, 2 * dim, bias=qkv_bias)
+        self.qg = nn.Linear(dim, 2 * dim, bias=qkv_bias)
         self.power = nn.Parameter(torch.zeros(1, num_heads, 1, self.head_dim))
         self.alpha = alpha
 
@@ -29,7 +29,7 @@ class PolaLinearAttention(PvtLinearAttentionBase):
         scale = F.softplus(self.scale)
         power = 1 + self.alpha * torch.sigmoid(self.power)
         features = polarity_features if fast else polarity_formula
-        q_same, q_opp, k_both, v, v_rows, gate = features(self.qg(x), self._joint_keys_values(x, H, W),
+        q_same, q_opp, k_both, v, v_rows, gate = features(project(self.qg, x), self._joint_keys_values(x, H, W),
                                                           self.positional_encoding, scale, power, self.num_heads)
         if fast:  # both pairings on one state pass over the shared keys and values
             o_same, o_opp = paired_linear_attention(q_same, q_opp, k_both, v)
@@ -39,4 +39,4 @@ class PolaLinearAttention(PvtLinearAttentionBase):
             out = torch.cat([torch_linear_attention(q_same, k_both, v_same),
                              torch_linear_attention(q_opp, k_both, v_opp)], dim=-1)
             out = (merge_heads(out) + self._value_conv(v, N, H, W)) * gate
-        return self.proj_drop(self.proj(out))
+        return self.proj_drop(project(self.proj, out))

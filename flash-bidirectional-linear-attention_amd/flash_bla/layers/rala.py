@@ -9,7 +9,7 @@ from flash_bla.layers.mlla import RoPE
 from flash_bla.ops._check import untouched
 from flash_bla.ops.depthwise import depthwise_conv_tokens
 from flash_bla.ops.linear_attn.decoupled import decoupled_la
-from flash_bla.ops.projection import TokenLinear
+from flash_bla.ops.projection import project
 
 
 class RALALinearAttention(nn.Module):
@@ -18,17 +18,17 @@ class RALALinearAttention(nn.Module):
         self.dim, self.input_resolution, self.num_heads = dim, input_resolution, num_heads
         self.head_dim = dim // num_heads
         self.scale = self.head_dim ** -0.5
-        self.qkvo = TokenLinear(dim, dim * 4, bias=qkv_bias)
+        self.qkvo = nn.Linear(dim, dim * 4, bias=qkv_bias)
         self.elu = nn.ELU()
         self.lepe = nn.Conv2d(dim, dim, 5, padding=2, groups=dim)
         self.rope = RoPE(shape=(input_resolution[0], input_resolution[1], self.head_dim))
-        self.proj = TokenLinear(dim, dim)
+        self.proj = nn.Linear(dim, dim)
 
     def forward(self, x, mode='triton'):
         fast = check_mode(mode)
         b, n, c = x.shape
         side = int(n ** 0.5)
-        q, k, v, gate = self.qkvo(x).chunk(4, dim=-1)
+        q, k, v, gate = project(self.qkvo, x).chunk(4, dim=-1)
         if fast:
             lepe = depthwise_conv_tokens(v, self.lepe, side, side)
         else:
@@ -45,9 +45,9 @@ class RALALinearAttention(nn.Module):
             k_rope = self.rope(k.reshape(grid)).reshape(k.shape).to(x.dtype).contiguous()
         if fast:
             out = decoupled_la(q, k.contiguous(), q_rope, k_rope, v, scale=n ** -1.0)
-            return self.proj(merge_heads_with(out, None, lepe, gate))
+            return project(self.proj, merge_heads_with(out, None, lepe, gate))
         out = torch_linear_attention(q, k, v, q_num=q_rope, k_num=k_rope)
-        return self.proj((merge_heads(out) + lepe) * gate)
+        return project(self.proj, (merge_heads(out) + lepe) * gate)
 
     def extra_repr(self):
         return f'dim={self.dim}, num_heads={self.num_heads}'

@@ -10,6 +10,7 @@ import torch.nn.functional as F
 from torch.autograd import forward_ad
 
 from flash_bla import _hip
+from flash_bla.ops._check import untouched
 
 
 class TokenLinearFunction(torch.autograd.Function):
@@ -64,12 +65,24 @@ def runs_on_rows(x, weight, bias):
             splits_tokens(tokens, M, N, bias is not None, x.dtype == torch.float32) and plain_tensors(x, weight, bias))
 
 
+def token_linear(x, weight, bias):
+    """F.linear whose backward takes the weight and bias gradients from the token-splitting kernel where that is the
+    faster of the two."""
+    if torch.is_grad_enabled() and runs_on_rows(x, weight, bias):
+        return TokenLinearFunction.apply(x, weight, bias)
+    return F.linear(x, weight, bias)
+
+
+def project(module, x):
+    """module(x), a plain nn.Linear as token_linear.  The blocks hold plain nn.Linear modules and call them through this:
+    what replaces, wraps or looks for modules by their type finds them as they always were."""
+    if torch.is_grad_enabled() and untouched(module, nn.Linear):
+        return token_linear(x, module.weight, module.bias)
+    return module(x)
+
+
 class TokenLinear(nn.Linear):
-    """nn.Linear whose backward takes the weight and bias gradients from the token-splitting kernel where that is the
-    faster of the two; otherwise, and on the CPU, nn.Linear itself."""
+    """token_linear as a module of its own."""
 
     def forward(self, x):
-        weight, bias = self.weight, self.bias
-        if torch.is_grad_enabled() and runs_on_rows(x, weight, bias):
-            return TokenLinearFunction.apply(x, weight, bias)
-        return F.linear(x, weight, bias)
+        return token_linear(x, self.weight, self.bias)

@@ -5,8 +5,10 @@ import torch
 import torch.nn as nn
 
 from flash_bla import _hip
+from flash_bla.layers import (FocusedLinearAttention, GeneralizedLinearAttention, MambaLikeLinearAttention,
+                              PolaLinearAttention, RALALinearAttention)
 from flash_bla.layers.mlla import RoPE
-from flash_bla.ops import depthwise
+from flash_bla.ops import depthwise, projection
 from flash_bla.ops._check import untouched
 
 
@@ -113,3 +115,37 @@ def test_modules_that_do_more_than_their_class_are_not_stood_in_for(make):
     del module.forward
     module.compile(backend="eager")
     assert not untouched(module, kind)
+
+
+BLOCKS = {
+    "linfusion": (lambda: GeneralizedLinearAttention(16, heads=2, dim_head=8), ()),
+    "mlla": (lambda: MambaLikeLinearAttention(16, (4, 4), 2), ()),
+    "rala": (lambda: RALALinearAttention(16, (4, 4), 2), ()),
+    "focused": (lambda: FocusedLinearAttention(16, 16, num_heads=2, sr_ratio=2), (4, 4)),
+    "pola": (lambda: PolaLinearAttention(16, 16, num_heads=2), (4, 4)),
+}
+
+
+@pytest.mark.parametrize("name", sorted(BLOCKS))
+def test_blocks_hold_plain_linear_modules_and_project_through_the_kernel_function(name, monkeypatch):
+    """By type they are nn.Linear, every one of them is offered to the token-splitting function, and one that is hooked or
+    replaced runs as the module that it is."""
+    make, extra = BLOCKS[name]
+    block, x = make(), torch.randn(2, 16, 16)
+    layers = [m for m in block.modules() if isinstance(m, nn.Linear)]
+    assert len(layers) >= 1 and all(type(m) is nn.Linear for m in layers)
+    want = block(x, *extra, mode="torch")
+
+    weights = []
+    monkeypatch.setattr(projection, "runs_on_rows", lambda x, weight, bias: True)
+    monkeypatch.setattr(projection.TokenLinearFunction, "apply",
+                        lambda x, weight, bias: weights.append(weight) or nn.functional.linear(x, weight, bias))
+    assert torch.equal(block(x, *extra, mode="torch"), want)
+    assert {id(w) for w in weights} == {id(m.weight) for m in layers}
+
+    seen = []
+    for m in layers:
+        m.register_forward_hook(lambda m, args, out: seen.append(m))
+    del weights[:]
+    assert torch.equal(block(x, *extra, mode="torch"), want) and not weights
+    assert {id(m) for m in seen} == {id(m) for m in layers}
