@@ -21,6 +21,7 @@ namespace dwconv {
 namespace {
 
 constexpr int kThreads = 256;
+constexpr float kLargest = 3.40282347e38f;  // of fp32
 constexpr int kFinishParts = 32;    // threads that share the terms of one filter's gradient
 constexpr int kBlockChannels = 64;  // channels of a workgroup: 128-byte (16-bit) or 256-byte (fp32) pieces of a row
 
@@ -59,12 +60,18 @@ template <typename T, int K, int STRIP>
 __global__ __launch_bounds__(kThreads) void conv_kernel(Conv a, int strips_per_row, int nstrips, int flip) {
   constexpr int V = Lane<T>::kVec, P = K / 2, IN = STRIP + K - 1;
   __shared__ float taps[K * K][kBlockChannels];
+  __shared__ int endless_of[kThreads / 64];  // a wave staged a tap that is infinite or NaN
   const int c0 = blockIdx.y * kBlockChannels;
+  int endless = 0;
   for (int i = threadIdx.x; i < K * K * kBlockChannels; i += kThreads) {
     const int tap = i / kBlockChannels, c = c0 + i % kBlockChannels;
     const T* w = static_cast<const T*>(a.w) + (int64_t)(c % a.Cw) * (K * K);
-    taps[tap][i % kBlockChannels] = c < a.C ? (float)w[flip ? K * K - 1 - tap : tap] : 0.f;
+    const float v = c < a.C ? (float)w[flip ? K * K - 1 - tap : tap] : 0.f;
+    taps[tap][i % kBlockChannels] = v;
+    endless |= !(fabsf(v) <= kLargest);
   }
+  endless = __ballot(endless) != 0;
+  if (threadIdx.x % 64 == 0) endless_of[threadIdx.x / 64] = endless;
   __syncthreads();
   const int lane = threadIdx.x % Lane<T>::kLanes, worker = threadIdx.x / Lane<T>::kLanes;
   const int cl = lane * V, c = c0 + cl;
@@ -109,6 +116,31 @@ __global__ __launch_bounds__(kThreads) void conv_kernel(Conv a, int strips_per_r
   }
 
   T* yo = static_cast<T*>(a.y) + (int64_t)b * a.y_batch + ((int64_t)y * a.W + x0) * a.y_row + c;
+  endless = 0;
+#pragma unroll
+  for (int i = 0; i < kThreads / 64; ++i) endless |= endless_of[i];
+  if (endless) {  // 0 times such a tap is not 0: once more, the columns around the grid left out
+#pragma unroll 1
+    for (int t = 0; t < STRIP && x0 + t < a.W; ++t) {
+      float sum[V];
+#pragma unroll
+      for (int j = 0; j < V; ++j) sum[j] = a.bias ? (float)static_cast<const T*>(a.bias)[(c + j) % a.Cw] : 0.f;
+#pragma unroll 1
+      for (int tap = 0; tap < K * K; ++tap) {
+        const int yy = y + tap / K - P, xx = x0 + t + tap % K - P;
+        if (yy < 0 || yy >= a.H || xx < 0 || xx >= a.W) continue;
+        Piece<T> in;
+        in.w = *reinterpret_cast<const u32x4*>(xb + ((int64_t)yy * a.W + xx) * a.x_row);
+#pragma unroll
+        for (int j = 0; j < V; ++j) sum[j] = fmaf(taps[tap][cl + j], (float)in.e[j], sum[j]);
+      }
+      Piece<T> out;
+#pragma unroll
+      for (int j = 0; j < V; ++j) out.e[j] = (T)sum[j];
+      *reinterpret_cast<u32x4*>(yo + t * a.y_row) = out.w;
+    }
+    return;
+  }
 #pragma unroll
   for (int t = 0; t < STRIP; ++t) {
     if (x0 + t < a.W) {
@@ -159,6 +191,39 @@ __global__ __launch_bounds__(kThreads) void grad_kernel(Conv a, const T* __restr
           for (int t = 0; t < STRIP; ++t)
 #pragma unroll
             for (int j = 0; j < V; ++j) acc[kx][j] = fmaf((float)gv[t].e[j], (float)in[t + kx].e[j], acc[kx][j]);
+      }
+    }
+  }
+  // The products above include zeros around the grid, which is wrong where the other factor is infinite or NaN: a lane whose
+  // sums are no numbers adds the products inside the grid again, alone.
+  float unbounded = 0.f;
+#pragma unroll
+  for (int k = 0; k < K; ++k)
+#pragma unroll
+    for (int j = 0; j < V; ++j) unbounded = fmaf(acc[k][j], 0.f, unbounded);
+  if (unbounded != 0.f) {
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+#pragma unroll
+      for (int j = 0; j < V; ++j) acc[k][j] = 0.f;
+    for (int strip = blockIdx.x * Lane<T>::kWorkers + worker; strip < nstrips; strip += gridDim.x * Lane<T>::kWorkers) {
+      const int yb = strip / strips_per_row, y = yb % a.H, b = yb / a.H, yy = y + ky - P;
+      if (yy < 0 || yy >= a.H) continue;
+      const T* gs = g + (int64_t)b * g_batch + (int64_t)y * a.W * g_row + c;
+      const T* xs = static_cast<const T*>(a.x) + (int64_t)b * a.x_batch + (int64_t)yy * a.W * a.x_row + c;
+      const int end = min(strip % strips_per_row * STRIP + STRIP, a.W);
+#pragma unroll 1
+      for (int t = strip % strips_per_row * STRIP; t < end; ++t) {
+        Piece<T> gv, in;
+        gv.w = *reinterpret_cast<const u32x4*>(gs + t * g_row);
+#pragma unroll
+        for (int kx = 0; kx < K; ++kx) {
+          const int xx = t + kx - P;
+          if (xx < 0 || xx >= a.W) continue;
+          in.w = *reinterpret_cast<const u32x4*>(xs + xx * a.x_row);
+#pragma unroll
+          for (int j = 0; j < V; ++j) acc[kx][j] = fmaf((float)gv.e[j], (float)in.e[j], acc[kx][j]);
+        }
       }
     }
   }

@@ -84,3 +84,42 @@ def test_hooks_run_and_the_gradient_has_a_gradient():
     assert seen
     for a, b in zip(ours, want):  # fp32 sums of 9 products, twice: a few 2^-24 of the largest
         assert (a - b).abs().max() <= 2.0 ** -18 * b.abs().max()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("where", ["input", "gradient", "filters"])
+@pytest.mark.parametrize("H,W,K", [(3, 9, 3), (4, 20, 5), (2, 3, 7), (3, 14, 3), (2, 16, 5), (2, 1, 3)])
+def test_infinities_and_nan_meet_what_lies_on_the_grid_alone(H, W, K, where, dtype):
+    """What surrounds the grid has no products, not zeros: infinities in the first and last columns (or in the outer taps of
+    a filter) and a NaN, whether the last strip of a row ends with the row or behind it, against the products of the
+    overlapping parts in float64 (which is what torch's convolutions in 16 and 32 bits give).  Whole numbers small enough to
+    be exact in every type."""
+    torch.manual_seed(W)
+    numbers = lambda *shape: torch.randint(-2, 3, shape, device="cuda").to(dtype)  # noqa: E731
+    x, g, w = numbers(2, H, W, 16), numbers(2, H, W, 16), numbers(8, 1, K, K)
+    inf, nan = float("inf"), float("nan")
+    if where == "filters":
+        w[:3, :, :, 0], w[2:4, :, :, -1], w[4, 0, 0, K // 2], w[5, 0, K // 2, 0] = inf, -inf, inf, nan
+    else:
+        t = x if where == "input" else g
+        t[:, :, -1, :6], t[:, :, 0, 4:8], t[:, 0, :, 9], t[1, -1, -1, 10] = inf, -inf, inf, nan
+    conv = nn.Conv2d(8, 8, K, padding=K // 2, groups=8, bias=False).cuda().to(dtype)
+    conv.weight.data.copy_(w)
+    rows = x.reshape(2, H * W, 16).requires_grad_()
+    assert runs_on_tokens(rows, conv)
+    y = depthwise_conv_tokens(rows, conv, H, W)
+    y.backward(g.reshape(2, H * W, 16))
+
+    x64, w64, P = x.double().requires_grad_(), w.double().requires_grad_(), K // 2
+    want = torch.zeros_like(x64)
+    for ky in range(K):
+        for kx in range(K):  # output rows and columns whose neighbour at this tap lies on the grid
+            rows_out, columns_out = (slice(max(0, P - k), min(n, n + P - k)) for k, n in ((ky, H), (kx, W)))
+            rows_in, columns_in = (slice(max(0, k - P), min(n, n + k - P)) for k, n in ((ky, H), (kx, W)))
+            want = want.clone()
+            if rows_out.start < rows_out.stop and columns_out.start < columns_out.stop:
+                want[:, rows_out, columns_out] += x64[:, rows_in, columns_in] * w64[:, 0, ky, kx].repeat(2)
+    want.backward(g.double())
+    for name, a, b in (("y", y, want), ("dx", rows.grad, x64.grad), ("dw", conv.weight.grad, w64.grad)):
+        b = b.detach().reshape(a.shape).to(dtype)
+        torch.testing.assert_close(a.detach(), b, rtol=0, atol=0, equal_nan=True, msg=lambda m: f"{name}: {m}")
