@@ -44,15 +44,23 @@ template <typename T> __device__ __forceinline__ void store(T* p, const Piece<T>
   *reinterpret_cast<u32x4*>(p) = v.w;
 }
 
-// a^p for a >= 0 (0 for a = 0, p > 0).  16-bit results: the hardware's exp2 and log2, whose error (2^-22 of p log2 a) is far
-// below the result's rounding.
+// a^p for a >= 0, p >= 1.  16-bit results: the hardware's exp2 and log2, whose error (2^-22 of p log2 a) is far below the
+// result's rounding; a result below 2^-126 is 0.
 template <typename T> __device__ __forceinline__ float power_of(float a, float p) {
   if constexpr (sizeof(T) == 4) return powf(a, p);
   else return __builtin_amdgcn_exp2f(p * __builtin_amdgcn_logf(a));
 }
-template <typename T> __device__ __forceinline__ float log_of(float a) {
-  if constexpr (sizeof(T) == 4) return logf(a);
-  else return __builtin_amdgcn_logf(a) * 0.693147180559945309f;
+// What the gradients of a^power need: slope = a^p for p = power - 1 >= 0, which is 1 for p = 0 whatever a is, and log = ln a.
+// log2f, not the bare instruction: that takes a denormal for 0, whose logarithm would make a gradient NaN.
+template <typename T> __device__ __forceinline__ void power_slope(float a, float p, float& slope, float& log) {
+  if constexpr (sizeof(T) == 4) {
+    slope = powf(a, p);
+    log = logf(a);
+  } else {
+    const float l = log2f(a);
+    slope = p == 0.f ? 1.f : __builtin_amdgcn_exp2f(p * l);
+    log = l * 0.693147180559945309f;
+  }
 }
 template <typename T> __device__ __forceinline__ float exp_of(float x) {
   if constexpr (sizeof(T) == 4) return expf(x);
@@ -128,13 +136,14 @@ __device__ __forceinline__ void polarity_piece_bwd(const float (&x)[Piece<T>::kV
 #pragma unroll
   for (int j = 0; j < Piece<T>::kVec; ++j) {
     const float y = x[j] * inv[j], a = fabsf(y);
-    const float g = y < 0.f ? gneg[j] : gpos[j];
-    const float w = power_of<T>(a, power[j] - 1.f);
+    const float gp = y < 0.f ? 0.f : gpos[j], gn = y > 0.f ? 0.f : gneg[j];  // (NaN is in both parts)
+    float slope, log;
+    power_slope<T>(a, power[j] - 1.f, slope, log);
     const bool zero = a == 0.f;  // both parts are cut off there: no gradient
-    const float dy = zero ? 0.f : (y < 0.f ? -g : g) * power[j] * w;
+    const float dy = zero ? 0.f : (gp - gn) * power[j] * slope;
     dx[j] = dy * inv[j];
     dscale[j] += dy * x[j];
-    dpower[j] += zero ? 0.f : g * (w * a) * log_of<T>(a);
+    dpower[j] += zero ? 0.f : (gp + gn) * (slope * a) * log;
   }
 }
 

@@ -150,6 +150,25 @@ def test_not_a_number_and_infinity_pass_through():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("power", [1.0, 1.5, 3.0])
+def test_gradients_at_infinities_denormals_and_a_power_of_one(power, dtype):
+    """One channel each, so that nothing is added to them: as relu and pow give them, in float64 and rounded."""
+    x = torch.tensor([float("inf"), -float("inf"), 1e-40, -1e-40, 0.0, 3.0, -3.0, float("nan")], device="cuda")
+    zero, one = torch.zeros(1, 1, 8, device="cuda"), torch.ones(1, 1, 8, device="cuda")
+    inputs = [t.to(dtype).requires_grad_() for t in (torch.cat([x, x])[None, None], torch.cat([x, x])[None, None], zero, one,
+                                                     power * one.reshape(1, 1, 1, 8))]
+    exact = [t.detach().double().requires_grad_() for t in inputs]
+    out, want = features.polarity_features(*inputs, 1), features.polarity_formula(*exact, 1)
+    for a, b in zip(out, want):
+        torch.testing.assert_close(a, b.to(dtype), equal_nan=True)
+    got = torch.autograd.grad(sum(o.float().sum((0, 1)).sum() for o in out[:3]), inputs)
+    ref = torch.autograd.grad(sum(o.sum((0, 1)).sum() for o in want[:3]), exact)
+    for name, a, b in zip(("qg", "kv", "pe", "scale", "power"), got, ref):
+        torch.testing.assert_close(a, b.to(dtype), equal_nan=True, msg=lambda m: f"{name}: {m}")
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("make,extra", [(lambda: PolaLinearAttention(24, 4, num_heads=2), (2, 2)),
                                         (lambda: MambaLikeLinearAttention(24, (2, 2), 2), ())])
 def test_heads_that_are_no_whole_pieces_run_as_torch_operators(make, extra):
