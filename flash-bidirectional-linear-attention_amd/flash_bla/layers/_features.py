@@ -18,7 +18,7 @@ def _takes(heads, channels, unit, *tensors):
     """Ordinary GPU tensors of one supported type whose heads (or their `unit` parts) are whole 16-byte pieces."""
     x = tensors[0]
     dtype, device = x.dtype, x.device
-    if not x.is_cuda or dtype not in _TYPES or channels // heads % (unit * 16 // x.element_size()):
+    if not x.is_cuda or dtype not in _TYPES or channels % heads or channels // heads % (unit * 16 // x.element_size()):
         return False
     for t in tensors:
         if t is not None and (t.dtype != dtype or t.device != device or not 0 < t.numel() < 1 << 31):
@@ -66,7 +66,9 @@ def polarity_features(qg, kv, pe, scale, power, heads):
     (at least 1).  Returns (q_same, q_opp [B, heads, N, 2d], k_both [B, heads, n, 2d], v [B, heads, n, d], the values as rows
     [B, n, C], the gate [B, N, C])."""
     C = qg.shape[-1] // 2
-    if _takes(heads, C, 1, qg, kv, pe, scale, power) and pe.shape == (1, kv.shape[1], C) and scale.shape == (1, 1, C):
+    if (_takes(heads, C, 1, qg, kv, pe, scale, power) and qg.ndim == 3 and kv.ndim == 3 and qg.shape[2] == 2 * C and
+            kv.shape == (qg.shape[0], kv.shape[1], 2 * C) and pe.shape == (1, kv.shape[1], C) and
+            scale.shape == (1, 1, C) and power.shape == (1, heads, 1, C // heads)):
         return PolarityFeaturesFunction.apply(qg, kv, pe, scale, power, heads)
     return polarity_formula(qg, kv, pe, scale, power, heads)
 
@@ -104,8 +106,8 @@ def focused_features(q, kv, pe, scale, heads, factor):
     """q [B, N, C], kv [B, n, 2C] (keys | values), pe [1, n, C], scale [1, 1, C].  Returns (q, k, v [B, heads, tokens, d],
     the values as rows [B, n, C]).  The kernels know the cube."""
     C = q.shape[-1]
-    if (factor == 3 and _takes(heads, C, 1, q, kv, pe, scale) and C <= _hip.most_row_channels(q) and
-            pe.shape == (1, kv.shape[1], C) and scale.shape == (1, 1, C)):
+    if (factor == 3 and _takes(heads, C, 1, q, kv, pe, scale) and C <= _hip.most_row_channels(q) and q.ndim == 3 and
+            kv.ndim == 3 and kv.shape == (q.shape[0], kv.shape[1], 2 * C) and pe.shape == (1, kv.shape[1], C) and scale.shape == (1, 1, C)):
         return FocusedFeaturesFunction.apply(q, kv, pe, scale, heads)
     return focus_formula(q, kv, pe, scale, heads, factor)
 
@@ -141,7 +143,8 @@ class RotaryFeaturesFunction(torch.autograd.Function):
 def rotary_features(qk, x, rotations, side, heads):
     """qk [B, N, 2C] (queries | keys before elu + 1), x [B, N, C] (the values), N = side * side, rotations
     [side, side, C / 2, 2].  Returns (q, k, q_rot, k_rot, v [B, heads, N, d], the values as rows)."""
-    if (_takes(heads, x.shape[-1], 1, x, qk) and plain_tensors(rotations) and rotations.dtype == torch.float32 and
+    if (_takes(heads, x.shape[-1], 1, x, qk) and x.ndim == 3 and qk.shape == (*x.shape[:2], 2 * x.shape[2]) and
+            plain_tensors(rotations) and rotations.dtype == torch.float32 and
             rotations.device == x.device and not rotations.requires_grad and
             rotations.shape == (side, side, x.shape[2] // 2, 2) and x.shape[1] == side * side):
         return RotaryFeaturesFunction.apply(qk, x, rotations, side, heads)
@@ -176,7 +179,7 @@ def turned_heads(q, k, weight, rotations):
     pieces = d * q.element_size() // 16
     if (_takes(1, d, 1, q, k, weight) and pieces <= 64 and pieces & (pieces - 1) == 0 and plain_tensors(rotations) and
             rotations.dtype == torch.float32 and rotations.device == q.device and not rotations.requires_grad and
-            rotations.ndim == 4 and rotations.shape[0] * rotations.shape[1] == N and rotations.shape[2:] == (d // 2, 2) and
+            q.ndim == 4 and rotations.ndim == 4 and rotations.shape[0] * rotations.shape[1] == N and rotations.shape[2:] == (d // 2, 2) and
             k.shape == q.shape and weight.shape == (*q.shape[:-1], 1)):
         return TurnedHeadsFunction.apply(q, k, weight, rotations)
     return turn_formula(q, k, weight, rotations)
@@ -208,8 +211,9 @@ class MergeHeadsFunction(torch.autograd.Function):
 def merge_heads_with(o, o2, local, gate=None):
     """(heads + local) * gate as rows [B, N, C]: o [B, heads, N, d], or the halves o, o2 [B, heads, N, d / 2] of each head;
     local [B, N, C]; gate [B, N, C] or None."""
-    heads, C = o.shape[1], local.shape[-1]
-    if _takes(heads, C, 1 if o2 is None else 2, o, o2, local, gate):
+    heads, C, halves = o.shape[1], local.shape[-1], 1 if o2 is None else 2
+    if (_takes(heads, C, halves, o, o2, local, gate) and local.shape == (o.shape[0], o.shape[2], heads * o.shape[3] * halves) and
+            (o2 is None or o2.shape == o.shape) and (gate is None or gate.shape == local.shape)):
         return MergeHeadsFunction.apply(o, o2, local, gate)
     return merge_formula(o, o2, local, gate)[0]
 
@@ -234,7 +238,7 @@ class InterpolateTokensFunction(torch.autograd.Function):
 
 def interpolate_tokens(rows, tokens):
     """Token rows [B, n, C] linearly interpolated to [B, tokens, C] (corners not aligned)."""
-    if (_takes(1, rows.shape[-1], 1, rows) and tokens > 0 and rows.shape[1] * tokens < 1 << 28 and
+    if (_takes(1, rows.shape[-1], 1, rows) and rows.ndim == 3 and tokens > 0 and rows.shape[1] * tokens < 1 << 28 and
             rows.shape[0] * tokens * rows.shape[2] < 1 << 31):
         return InterpolateTokensFunction.apply(rows, tokens)
     return interpolate_formula(rows, tokens)[0]

@@ -7,6 +7,7 @@ import torch.nn as nn
 from flash_bla import _hip
 from flash_bla.layers import (FocusedLinearAttention, GeneralizedLinearAttention, MambaLikeLinearAttention,
                               PolaLinearAttention, RALALinearAttention)
+from flash_bla.layers import _features as features
 from flash_bla.layers.mlla import RoPE
 from flash_bla.ops import depthwise, projection
 from flash_bla.ops._check import untouched
@@ -149,3 +150,86 @@ def test_blocks_hold_plain_linear_modules_and_project_through_the_kernel_functio
     del weights[:]
     assert torch.equal(block(x, *extra, mode="torch"), want) and not weights
     assert {id(m) for m in seen} == {id(m) for m in layers}
+
+
+FUSED = (features.PolarityFeaturesFunction, features.FocusedFeaturesFunction, features.RotaryFeaturesFunction,
+         features.TurnedHeadsFunction, features.MergeHeadsFunction, features.InterpolateTokensFunction)
+
+
+@pytest.fixture
+def only_shapes_decide(monkeypatch):
+    """Every tensor counts as one that the kernels could read; a call that reaches them is reported."""
+    class Reached(Exception):
+        pass
+
+    def reached(*args):
+        raise Reached
+    monkeypatch.setattr(features, "_takes", lambda *a: True)
+    monkeypatch.setattr(features, "elu_plus_one", lambda t: nn.functional.elu(t) + 1)
+    for function in FUSED:
+        monkeypatch.setattr(function, "apply", reached)
+    return Reached
+
+
+# 2 batches of 9 queries and 4 keys, 2 heads of 8 channels
+ROWS, KEYS, HEADS, DIM = 9, 4, 2, 16
+
+
+def _features_call(name, **shapes):
+    t = {k: torch.rand(v) for k, v in shapes.items()}
+    if name == "polarity":
+        args = (t["qg"], t["kv"], t["pe"], t["scale"], t["power"], HEADS)
+        return features.polarity_features(*args), features.polarity_formula(*args)
+    if name == "focused":
+        args = (t["q"], t["kv"], t["pe"], t["scale"], HEADS, 3)
+        return features.focused_features(*args), features.focus_formula(*args)
+    if name == "rotary":
+        args = (t["qk"], t["x"], t["rotations"], 3, HEADS)
+        return features.rotary_features(*args), features.rotary_formula(*args)
+    args = t["o"], t.get("o2"), t["local"], t.get("gate")
+    return (features.merge_heads_with(*args),), features.merge_formula(*args)
+
+
+FULL = {
+    "polarity": dict(qg=(2, ROWS, 2 * DIM), kv=(2, KEYS, 2 * DIM), pe=(1, KEYS, DIM), scale=(1, 1, DIM),
+                     power=(1, HEADS, 1, DIM // HEADS)),
+    "focused": dict(q=(2, ROWS, DIM), kv=(2, KEYS, 2 * DIM), pe=(1, KEYS, DIM), scale=(1, 1, DIM)),
+    "rotary": dict(qk=(2, ROWS, 2 * DIM), x=(2, ROWS, DIM), rotations=(3, 3, DIM // 2, 2)),
+    "merge": dict(o=(2, HEADS, ROWS, DIM // HEADS), local=(2, ROWS, DIM)),
+    "merge halves": dict(o=(2, HEADS, ROWS, DIM // 4), o2=(2, HEADS, ROWS, DIM // 4), local=(2, ROWS, DIM),
+                         gate=(2, ROWS, DIM)),
+}
+
+
+@pytest.mark.parametrize("name", sorted(FULL))
+def test_full_shapes_reach_the_kernels(name, only_shapes_decide):
+    with pytest.raises(only_shapes_decide):
+        _features_call(name, **FULL[name])
+
+
+@pytest.mark.parametrize("name,other", [
+    ("polarity", dict(power=(1, 1, 1, 1))), ("polarity", dict(power=(1, 1, 1, DIM // HEADS))),
+    ("polarity", dict(power=(1, HEADS, 1, 1))), ("polarity", dict(pe=(1, 1, DIM))), ("polarity", dict(scale=(1, 1, 1))),
+    ("polarity", dict(kv=(1, KEYS, 2 * DIM))), ("focused", dict(kv=(1, KEYS, 2 * DIM))), ("focused", dict(scale=(1,))),
+    ("focused", dict(pe=(2, KEYS, DIM))), ("merge", dict(local=(1, ROWS, DIM))), ("merge", dict(gate=(1, 1, DIM))),
+    ("merge halves", dict(gate=(2, ROWS, 1)))])
+def test_shapes_that_torch_broadcasts_run_as_torch_operators(name, other, only_shapes_decide):
+    """A replaced parameter of fewer elements: the kernels would read past it."""
+    got, want = _features_call(name, **{**FULL[name], **other})
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("name,other", [
+    ("polarity", dict(power=(1, HEADS, ROWS, DIM))), ("polarity", dict(kv=(2, KEYS, 2 * DIM + 16))),
+    ("focused", dict(kv=(2, KEYS, 4 * DIM))), ("rotary", dict(qk=(2, ROWS, 4 * DIM))), ("rotary", dict(qk=(2, 4, 2 * DIM))),
+    ("merge", dict(local=(2, ROWS - 1, DIM))), ("merge", dict(gate=(2, ROWS, DIM // 2))),
+    ("merge halves", dict(o2=(2, HEADS, ROWS - 1, DIM // 4)))])
+def test_shapes_that_torch_refuses_stay_refused(name, other, only_shapes_decide):
+    with pytest.raises(RuntimeError):
+        _features_call(name, **{**FULL[name], **other})
+
+
+def test_heads_that_do_not_divide_the_channels_are_not_taken(monkeypatch):
+    monkeypatch.setattr(features, "plain_tensors", lambda *a: True)
+    x = _on_gpu(torch.zeros(1, 1, 136).half())
+    assert features._takes(17, 136, 1, x) and not features._takes(16, 136, 1, x)  # 136 // 16 is one whole piece
