@@ -14,7 +14,7 @@ from flash_bla.layers._common import check_mode, torch_linear_attention
 from flash_bla.ops._check import untouched
 from flash_bla.ops.linear_attn.fused import linear_attention
 from flash_bla.ops.linear_attn.varlen import varlen_linear_attention
-from flash_bla.ops.projection import project
+from flash_bla.ops.projection import project, trains
 
 
 _CU_CACHE = {}
@@ -42,7 +42,7 @@ def get_none_linear_projection(query_dim, mid_dim=None):
 
 def project_through(layers, x):
     """layers(x) with the projections of a plain nn.Sequential as `project` runs them."""
-    if torch.is_grad_enabled() and untouched(layers, nn.Sequential):
+    if trains(x) and untouched(layers, nn.Sequential):
         for layer in layers:
             x = project(layer, x)
         return x

@@ -33,13 +33,14 @@ class TokenLinearFunction(torch.autograd.Function):
 
 
 def plain_tensors(*tensors):
-    """Whether these are ordinary tensors in an ordinary eager call: nothing that traces, maps, casts or carries a tangent
-    through torch's own operators."""
+    """Whether these are ordinary tensors in an ordinary eager call: nothing that traces, maps, watches, casts or carries a
+    tangent through torch's own operators."""
     for t in tensors:
         if t is not None and type(t) is not torch.Tensor and type(t) is not nn.Parameter:
             return False
-    return not (torch.is_autocast_enabled() or torch.compiler.is_compiling() or forward_ad._current_level >= 0 or
-                torch._C._are_functorch_transforms_active())
+    return not (torch.is_autocast_enabled() or torch.compiler.is_compiling() or torch.jit.is_tracing() or
+                forward_ad._current_level >= 0 or torch._C._are_functorch_transforms_active() or
+                torch._C._len_torch_dispatch_stack())
 
 
 def splits_tokens(tokens, M, N, with_bias, fp32):
@@ -68,16 +69,21 @@ def runs_on_rows(x, weight, bias):
 def token_linear(x, weight, bias):
     """F.linear whose backward takes the weight and bias gradients from the token-splitting kernel where that is the
     faster of the two."""
-    if torch.is_grad_enabled() and runs_on_rows(x, weight, bias):
+    if runs_on_rows(x, weight, bias):
         return TokenLinearFunction.apply(x, weight, bias)
     return F.linear(x, weight, bias)
 
 
+def trains(x):
+    """Whether a call on x can need the gradients at all: a tensor (no proxy of one), grad mode, no trace."""
+    return type(x) is torch.Tensor and torch.is_grad_enabled() and not torch.jit.is_tracing()
+
+
 def project(module, x):
     """module(x), a plain nn.Linear as token_linear.  The blocks hold plain nn.Linear modules and call them through this:
-    what replaces, wraps or looks for modules by their type finds them as they always were."""
-    if torch.is_grad_enabled() and untouched(module, nn.Linear):
-        return token_linear(x, module.weight, module.bias)
+    what replaces, wraps, traces or looks for modules by their type finds them as they always were."""
+    if trains(x) and untouched(module, nn.Linear) and runs_on_rows(x, module.weight, module.bias):
+        return TokenLinearFunction.apply(x, module.weight, module.bias)
     return module(x)
 
 

@@ -2,7 +2,9 @@
 launches a kernel.  A call that torch's operators refuse stays refused, one that they run stays theirs."""
 import pytest
 import torch
+import torch.fx
 import torch.nn as nn
+from torch.utils.flop_counter import FlopCounterMode
 
 from flash_bla import _hip
 from flash_bla.layers import (FocusedLinearAttention, GeneralizedLinearAttention, MambaLikeLinearAttention,
@@ -233,3 +235,36 @@ def test_heads_that_do_not_divide_the_channels_are_not_taken(monkeypatch):
     monkeypatch.setattr(features, "plain_tensors", lambda *a: True)
     x = _on_gpu(torch.zeros(1, 1, 136).half())
     assert features._takes(17, 136, 1, x) and not features._takes(16, 136, 1, x)  # 136 // 16 is one whole piece
+
+
+@pytest.mark.parametrize("name", sorted(BLOCKS))
+def test_blocks_in_torch_mode_can_be_traced(name):
+    """torch.jit.trace of a block that trains, and torch.fx where the block's own code allows it, see the projections as the
+    modules that they are."""
+    make, extra = BLOCKS[name]
+    block, x = make(), torch.randn(2, 16, 16)
+
+    class TorchMode(nn.Module):
+        def __init__(self):
+            super().__init__()
+            self.block = block
+
+        def forward(self, x):
+            return self.block(x, *extra, mode="torch")
+    layers = {n for n, m in block.named_modules() if type(m) is nn.Linear}
+    traced = torch.jit.trace(TorchMode(), x)
+    torch.testing.assert_close(traced(x), block(x, *extra, mode="torch"))
+    assert {n for n in layers if n.count(".") == 0} <= {n.removeprefix("block.") for n, _ in traced.named_modules()}
+    if name not in ("mlla", "rala"):  # (int() of the number of tokens)
+        fixed = {"H": 4, "W": 4} if extra else {"encoder_hidden_states": None, "attention_mask": None}
+        graph = torch.fx.symbolic_trace(block, concrete_args={"mode": "torch", **fixed}).graph
+        assert layers <= {n.target for n in graph.nodes if n.op == "call_module"}
+
+
+def test_traced_and_watched_calls_are_not_plain():
+    x = torch.randn(2, 3)
+    seen = []
+    torch.jit.trace(lambda t: seen.append(projection.plain_tensors(t)) or t + 1, x, check_trace=False)
+    assert projection.plain_tensors(x) and seen and not any(seen)
+    with FlopCounterMode(display=False):
+        assert not projection.plain_tensors(x)
