@@ -9,7 +9,7 @@ import torch.nn.functional as F
 from flash_bla import _hip
 from flash_bla.layers._common import merge_heads, split_heads
 from flash_bla.ops.feature_map import elu_plus_one
-from flash_bla.ops.projection import plain_tensors
+from flash_bla.ops.projection import composes_gradient, plain_tensors
 
 _TYPES = (torch.float16, torch.bfloat16, torch.float32)
 
@@ -27,13 +27,13 @@ def _takes(heads, channels, unit, *tensors):
 
 
 def differentiable_gradients(formula, inputs, grads):
-    """Gradients of formula(*inputs) that can be differentiated again."""
+    """Gradients of formula(*inputs) by torch's operators, which can be differentiated again where that is wanted."""
     wanted = [t for t in inputs if torch.is_tensor(t) and t.requires_grad]
     with torch.enable_grad():
         out = formula(*inputs)
         pairs = [(o, g) for o, g in zip(out, grads) if o is not None and o.requires_grad]
-        got = iter(torch.autograd.grad([o for o, _ in pairs], wanted, [g for _, g in pairs], create_graph=True,
-                                       allow_unused=True))
+    got = iter(torch.autograd.grad([o for o, _ in pairs], wanted, [g for _, g in pairs],
+                                   create_graph=torch.is_grad_enabled(), allow_unused=True))
     return tuple(next(got) if torch.is_tensor(t) and t.requires_grad else None for t in inputs)
 
 
@@ -56,7 +56,7 @@ class PolarityFeaturesFunction(torch.autograd.Function):
     @staticmethod
     def backward(ctx, *grads):
         inputs = ctx.saved_tensors
-        if torch.is_grad_enabled():
+        if composes_gradient(*grads):
             return differentiable_gradients(polarity_formula, (*inputs, ctx.heads), grads)
         return (*_hip.polarity_bwd(*inputs, ctx.heads, *grads), None)
 
@@ -97,7 +97,7 @@ class FocusedFeaturesFunction(torch.autograd.Function):
     @staticmethod
     def backward(ctx, *grads):
         inputs = ctx.saved_tensors
-        if torch.is_grad_enabled():
+        if composes_gradient(*grads):
             return differentiable_gradients(focus_formula, (*inputs, ctx.heads), grads)
         return (*_hip.focus_bwd(*inputs, ctx.heads, *grads), None)
 
@@ -135,7 +135,7 @@ class RotaryFeaturesFunction(torch.autograd.Function):
     @staticmethod
     def backward(ctx, *grads):
         qk, x, rotations = ctx.saved_tensors
-        if torch.is_grad_enabled():
+        if composes_gradient(*grads):
             return differentiable_gradients(rotary_formula, (qk, x, rotations, ctx.side, ctx.heads), grads)
         return (*_hip.rotary_bwd(qk, rotations, ctx.heads, *grads), None, None, None)
 
@@ -167,7 +167,7 @@ class TurnedHeadsFunction(torch.autograd.Function):
     @staticmethod
     def backward(ctx, *grads):
         q, k, weight, rotations = ctx.saved_tensors
-        if torch.is_grad_enabled():
+        if composes_gradient(*grads):
             return differentiable_gradients(turn_formula, (q, k, weight, rotations), grads)
         return (*_hip.turn_bwd(k, weight, rotations, *grads), None)
 
@@ -200,7 +200,7 @@ class MergeHeadsFunction(torch.autograd.Function):
     @staticmethod
     def backward(ctx, g):
         o, o2, local, gate = ctx.saved_tensors
-        if torch.is_grad_enabled():
+        if composes_gradient(g):
             if gate is not None:
                 return differentiable_gradients(merge_formula, (o, o2, local, gate), (g,))
             do = split_heads(g, ctx.heads)
@@ -230,7 +230,7 @@ class InterpolateTokensFunction(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, g):
-        if torch.is_grad_enabled():  # linear in the rows: the gradient is that of any rows
+        if composes_gradient(g):  # linear in the rows: the gradient is that of any rows
             rows = torch.zeros(g.shape[0], ctx.n, g.shape[2], dtype=g.dtype, device=g.device, requires_grad=True)
             return differentiable_gradients(interpolate_formula, (rows, g.shape[1]), (g,))
         return _hip.interpolate_bwd(g, ctx.n), None

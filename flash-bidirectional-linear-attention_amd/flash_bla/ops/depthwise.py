@@ -10,7 +10,7 @@ import torch.nn.functional as F
 
 from flash_bla import _hip
 from flash_bla.ops._check import untouched
-from flash_bla.ops.projection import plain_tensors
+from flash_bla.ops.projection import composes_gradient, plain_tensors
 
 
 class DepthwiseConvTokensFunction(torch.autograd.Function):
@@ -24,13 +24,13 @@ class DepthwiseConvTokensFunction(torch.autograd.Function):
     def backward(ctx, g):
         x, weight = ctx.saved_tensors
         dx = dw = db = None
-        if torch.is_grad_enabled():  # the gradient is to be differentiated again: of torch's convolution
+        if composes_gradient(g):  # of torch's convolution
             bias = torch.zeros(weight.shape[0], dtype=g.dtype, device=g.device, requires_grad=True)
             with torch.enable_grad():
                 y = _convolution_of_images(x, *ctx.grid, weight.shape[0], lambda images: F.conv2d(
                     images, weight, bias, padding=weight.shape[-1] // 2, groups=weight.shape[0]))
-                leaves = [t for t in (x, weight, bias) if t.requires_grad]
-                got = iter(torch.autograd.grad(y, leaves, g, create_graph=True))
+            leaves = [t for t in (x, weight, bias) if t.requires_grad]
+            got = iter(torch.autograd.grad(y, leaves, g, create_graph=torch.is_grad_enabled()))
             dx, dw, db = (next(got) if t.requires_grad else None for t in (x, weight, bias))
             return dx, dw, db if ctx.with_bias else None, None, None
         if ctx.needs_input_grad[0]:

@@ -7,6 +7,7 @@ forward and the input's gradient stay plain library GEMMs.
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch._C._functorch import is_legacy_batchedtensor as _is_batched  # what is_grads_batched makes of gradients
 from torch.autograd import forward_ad
 
 from flash_bla import _hip
@@ -25,22 +26,32 @@ class TokenLinearFunction(torch.autograd.Function):
         x, weight = ctx.saved_tensors
         dx = g @ weight if ctx.needs_input_grad[0] else None
         with_bias = ctx.with_bias and ctx.needs_input_grad[2]
-        if torch.is_grad_enabled():  # the gradient is to be differentiated again
+        if composes_gradient(g):
             rows = g.reshape(-1, g.shape[-1])
             return dx, rows.t() @ x.reshape(-1, x.shape[-1]), rows.sum(0) if with_bias else None
         dw, db = _hip.linear_wgrad(g, x, with_bias)
         return dx, dw, db
 
 
-def plain_tensors(*tensors):
-    """Whether these are ordinary tensors in an ordinary eager call: nothing that traces, maps, watches, casts or carries a
-    tangent through torch's own operators."""
+def eager_tensors(*tensors):
+    """Whether these are ordinary tensors in an ordinary eager call: nothing that traces, maps, watches or carries a tangent
+    through torch's own operators."""
     for t in tensors:
-        if t is not None and type(t) is not torch.Tensor and type(t) is not nn.Parameter:
+        if t is not None and (type(t) is not torch.Tensor and type(t) is not nn.Parameter or _is_batched(t)):
             return False
-    return not (torch.is_autocast_enabled() or torch.compiler.is_compiling() or torch.jit.is_tracing() or
-                forward_ad._current_level >= 0 or torch._C._are_functorch_transforms_active() or
-                torch._C._len_torch_dispatch_stack())
+    return not (torch.compiler.is_compiling() or torch.jit.is_tracing() or forward_ad._current_level >= 0 or
+                torch._C._are_functorch_transforms_active() or torch._C._len_torch_dispatch_stack())
+
+
+def plain_tensors(*tensors):
+    """eager_tensors in a call that casts nothing."""
+    return not torch.is_autocast_enabled() and eager_tensors(*tensors)
+
+
+def composes_gradient(*grads):
+    """Whether a backward has to be made of torch's operators: it is to be differentiated again, or the gradients it is
+    given are batches of gradients, carry tangents or are traced."""
+    return torch.is_grad_enabled() or not eager_tensors(*grads)
 
 
 def splits_tokens(tokens, M, N, with_bias, fp32):

@@ -4,6 +4,7 @@ import pytest
 import torch
 import torch.fx
 import torch.nn as nn
+from torch.autograd import forward_ad
 from torch.utils.flop_counter import FlopCounterMode
 
 from flash_bla import _hip
@@ -268,3 +269,79 @@ def test_traced_and_watched_calls_are_not_plain():
     assert projection.plain_tensors(x) and seen and not any(seen)
     with FlopCounterMode(display=False):
         assert not projection.plain_tensors(x)
+
+
+def _cpu_kernels(monkeypatch):
+    """The forward kernels by their formulas; a gradient kernel fails the test."""
+    F, n = nn.functional, features
+    for name, formula in (("polarity_fwd", lambda *a: n.polarity_formula(*a)[:4]), ("focus_fwd", lambda *a: n.focus_formula(*a)[:3]),
+                          ("rotary_fwd", lambda qk, x, rot, heads: n.rotary_formula(qk, x, rot, rot.shape[0], heads)[:5]),
+                          ("turn_fwd", n.turn_formula), ("merge_fwd", lambda *a: n.merge_formula(*a)[0]),
+                          ("interpolate_fwd", lambda *a: n.interpolate_formula(*a)[0]),
+                          ("dwconv_fwd", lambda x, w, b, H, W: depthwise._convolution_of_images(
+                              x, H, W, w.shape[0], lambda i: F.conv2d(i, w, b, padding=1, groups=w.shape[0])))):
+        monkeypatch.setattr(_hip, name, formula)
+    for name in ("polarity_bwd", "focus_bwd", "rotary_bwd", "turn_bwd", "merge_bwd", "interpolate_bwd", "dwconv_grad",
+                 "linear_wgrad"):
+        monkeypatch.setattr(_hip, name, lambda *a: pytest.fail("a kernel was given what it cannot read"))
+
+
+def _conv_formula(x, w, b, H, W):
+    return depthwise._convolution_of_images(x, H, W, w.shape[0], lambda i: nn.functional.conv2d(
+        i, w, b, padding=1, groups=w.shape[0]))
+
+
+_ANGLES = torch.arange(9 * 8.0).reshape(3, 3, 8)
+ROTATIONS = torch.stack([_ANGLES.cos(), _ANGLES.sin()], dim=-1)
+NODES = {  # function, the same by torch's operators, shapes of the inputs, what follows them
+    "polarity": (features.PolarityFeaturesFunction, features.polarity_formula, tuple(FULL["polarity"].values()), (HEADS,)),
+    "focused": (features.FocusedFeaturesFunction, features.focus_formula, tuple(FULL["focused"].values()), (HEADS,)),
+    "rotary": (features.RotaryFeaturesFunction, features.rotary_formula, tuple(FULL["rotary"].values())[:2],
+               (ROTATIONS, 3, HEADS)),
+    "turned": (features.TurnedHeadsFunction, features.turn_formula, ((2, HEADS, 9, 8),) * 2 + ((2, HEADS, 9, 1),),
+               (ROTATIONS[:, :, :4].contiguous(),)),
+    "merge": (features.MergeHeadsFunction, lambda o, local, *rest: features.merge_formula(o, None, local, None),
+              tuple(FULL["merge"].values()), ()),
+    "merge halves": (features.MergeHeadsFunction, features.merge_formula, tuple(FULL["merge halves"].values()), ()),
+    "interpolate": (features.InterpolateTokensFunction, features.interpolate_formula, ((2, 4, 8),), (9,)),
+    "convolution": (depthwise.DepthwiseConvTokensFunction, _conv_formula, ((2, 9, 16), (8, 1, 3, 3), (8,)), (3, 3)),
+    "projection": (projection.TokenLinearFunction, nn.functional.linear, ((2, 9, 16), (24, 16), (24,)), ()),
+}
+
+
+@pytest.mark.parametrize("how", ["batches", "tangents", "mapped", "twice"])
+@pytest.mark.parametrize("name", sorted(NODES))
+def test_gradients_that_kernels_cannot_read_are_composed(name, how, monkeypatch):
+    """Batches of gradients (is_grads_batched), gradients that carry tangents, gradients inside torch.func.vmap and
+    gradients of gradients give what torch's operators give."""
+    _cpu_kernels(monkeypatch)
+    function, formula, shapes, rest = NODES[name]
+    torch.manual_seed(0)
+    inputs = [(torch.rand(s) + 0.5).requires_grad_() for s in shapes]
+    if name == "merge":
+        out = function.apply(inputs[0], None, inputs[1], None)
+    else:
+        out = function.apply(*inputs, *rest)
+    results = []
+    for o in (out, formula(*inputs, *rest)):
+        o = (o,) if torch.is_tensor(o) else tuple(o)
+        gen = torch.Generator().manual_seed(1)
+        g, t = ([torch.randn(3, *x.shape, generator=gen) for x in o] for _ in range(2))
+        if how == "batches":
+            got = torch.autograd.grad(o, inputs, g, is_grads_batched=True)
+        elif how == "mapped":
+            got = torch.func.vmap(lambda *g: torch.autograd.grad(o, inputs, g, retain_graph=True))(*g)
+        elif how == "tangents":
+            with forward_ad.dual_level():
+                dual = [forward_ad.make_dual(a[0], b[0]) for a, b in zip(g, t)]
+                got = [x for d in torch.autograd.grad(o, inputs, dual) for x in forward_ad.unpack_dual(d)]
+        else:
+            first = torch.autograd.grad(o, inputs, [a[0] for a in g], create_graph=True)
+            got = torch.autograd.grad(sum(x.square().sum() for x in first if x.requires_grad), inputs, allow_unused=True) \
+                if any(x.requires_grad for x in first) else []
+        results.append([x for x in got if x is not None])
+    assert len(results[0]) == len(results[1])
+    for a, b in zip(*results):
+        assert not a.requires_grad
+        # fp32 sums of at most 36 products in another order; NaN: the power's second derivative at 0
+        torch.testing.assert_close(a, b, rtol=1e-4, atol=1e-4, equal_nan=True)
