@@ -28,7 +28,9 @@ class PolaLinearAttention(PvtLinearAttentionBase):
         N = x.shape[1]
         scale = F.softplus(self.scale)
         power = 1 + self.alpha * torch.sigmoid(self.power)
-        features = polarity_features if fast else polarity_formula
+        # (the kernels know powers of at least 1)
+        rising = isinstance(self.alpha, (int, float)) and self.alpha >= 0
+        features = polarity_features if fast and rising else polarity_formula
         q_same, q_opp, k_both, v, v_rows, gate = features(project(self.qg, x), self._joint_keys_values(x, H, W),
                                                           self.positional_encoding, scale, power, self.num_heads)
         if fast:  # both pairings on one state pass over the shared keys and values

@@ -11,6 +11,7 @@ from flash_bla import _hip
 from flash_bla.layers import (FocusedLinearAttention, GeneralizedLinearAttention, MambaLikeLinearAttention,
                               PolaLinearAttention, RALALinearAttention)
 from flash_bla.layers import _features as features
+from flash_bla.layers import polaformer
 from flash_bla.layers.mlla import RoPE
 from flash_bla.ops import depthwise, projection
 from flash_bla.ops._check import untouched
@@ -345,3 +346,17 @@ def test_gradients_that_kernels_cannot_read_are_composed(name, how, monkeypatch)
         assert not a.requires_grad
         # fp32 sums of at most 36 products in another order; NaN: the power's second derivative at 0
         torch.testing.assert_close(a, b, rtol=1e-4, atol=1e-4, equal_nan=True)
+
+
+@pytest.mark.parametrize("alpha,fused", [(4, True), (0.0, True), (-0.5, False), (torch.tensor(4.0), False)])
+def test_powers_below_one_run_as_torch_operators(alpha, fused, monkeypatch):
+    """0 to a power below 1 has an infinite slope: the kernels take the gradient there for zero, as it is from 1 on."""
+    class Reached(Exception):
+        pass
+
+    def reached(*args):
+        raise Reached
+    monkeypatch.setattr(polaformer, "polarity_features" if fused else "polarity_formula", reached)
+    block = PolaLinearAttention(16, 16, num_heads=2, alpha=alpha)
+    with pytest.raises(Reached):
+        block(torch.randn(2, 16, 16), 4, 4)
