@@ -36,7 +36,9 @@ class RALALinearAttention(nn.Module):
         q, k, v = (split_heads(t, self.num_heads) for t in (self.elu(q) + 1.0, self.elu(k) + 1.0, v))
         # efficiency reweighting: softmax over tokens of scale * mean(q) . k_j, times n
         eff = torch.softmax(self.scale * q.mean(dim=-2, keepdim=True) @ k.transpose(-1, -2), dim=-1)
-        if fast and untouched(self.rope, RoPE) and self.rope.rotations.shape[:2] == (side, side):
+        # (a score is at most 1: times n it has to stay a number of its type)
+        if (fast and untouched(self.rope, RoPE) and self.rope.rotations.shape[:2] == (side, side) and
+                n <= torch.finfo(eff.dtype).max):
             k, q_rope, k_rope = turned_heads(q, k, eff.transpose(-1, -2) * n, self.rope.rotations)
         else:
             k = k * eff.transpose(-1, -2) * n

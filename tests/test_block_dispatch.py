@@ -11,7 +11,7 @@ from flash_bla import _hip
 from flash_bla.layers import (FocusedLinearAttention, GeneralizedLinearAttention, MambaLikeLinearAttention,
                               PolaLinearAttention, RALALinearAttention)
 from flash_bla.layers import _features as features
-from flash_bla.layers import polaformer
+from flash_bla.layers import polaformer, rala
 from flash_bla.layers.mlla import RoPE
 from flash_bla.ops import depthwise, projection
 from flash_bla.ops._check import untouched
@@ -360,3 +360,18 @@ def test_powers_below_one_run_as_torch_operators(alpha, fused, monkeypatch):
     block = PolaLinearAttention(16, 16, num_heads=2, alpha=alpha)
     with pytest.raises(Reached):
         block(torch.randn(2, 16, 16), 4, 4)
+
+
+@pytest.mark.parametrize("side,dtype,fused", [(16, torch.half, True), (256, torch.half, False), (256, torch.bfloat16, True)])
+def test_rala_scores_times_tokens_that_overflow_are_not_formed(side, dtype, fused, monkeypatch):
+    """65536 tokens in fp16: a score of 1 times n is infinite, and a key of 0 times that is NaN; (k * score) * n is not."""
+    class Reached(Exception):
+        pass
+
+    def reached(*args):
+        raise Reached
+    monkeypatch.setattr(rala, "turned_heads", reached)
+    block = RALALinearAttention(8, (side, side), 1).to(dtype)
+    block.rope.float()
+    with pytest.raises(Reached if fused else ValueError, match=None if fused else "GPU"), torch.no_grad():
+        block(torch.zeros(1, side * side, 8, dtype=dtype))
