@@ -52,6 +52,18 @@ def test_weight_gradient(tokens, N, M, bias, layout, dtype, monkeypatch):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("tokens,N,M,bias", [
+    (8192, 640, 640, False),  # 25 tiles, 19 chunks of 448: two groups of eight on one XCD each, three in plain order
+    (40001, 136, 264, True),  # 6 tiles, 79 chunks of 512, the last of 65: nine groups and seven
+    (50176, 256, 512, True),  # 8 tiles, 61 chunks of 832: seven groups and five
+    (131072, 64, 128, True),  # one tile, 512 chunks of 256: plain order throughout
+    (200704, 64, 128, True)])  # one tile, 448 chunks of 448: groups throughout
+def test_weight_gradient_of_chunks_that_share_an_xcd(tokens, N, M, bias, dtype, monkeypatch):
+    test_weight_gradient(tokens, N, M, bias, "plain", dtype, monkeypatch)
+
+
+@pytest.mark.gpu
 def test_gradient_of_the_gradient(monkeypatch):
     monkeypatch.setattr(projection, "splits_tokens", lambda *a: True)
     torch.manual_seed(0)

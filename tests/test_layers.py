@@ -3,6 +3,7 @@
 input gradient, with the acceptance rule of the reference layers' self-tests
 (flash_bla/utils.py:55-67 with ratio 0.06; layers/linfusion.py:116-141 etc.)."""
 import ast
+import copy
 import os
 
 import numpy as np
@@ -181,3 +182,29 @@ def test_captured_forward_replays_the_block_bit_for_bit():
             torch.cuda.synchronize()
             got = graphed(xi).clone()
         assert torch.equal(got, eager), f"replay {i}"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16], ids=str)
+@pytest.mark.parametrize("name", sorted(GPU_CASES))
+def test_parameter_gradients_of_the_fast_mode(name, dtype):
+    """Every parameter's gradient against the block in float64 (mode='torch').  Measured at these sizes: at most 2.0e-6
+    (fp32) and 2.4e-3 (fp16) of the gradient's length; the bounds are four times that."""
+    torch.manual_seed(2)
+    make, shape, extra = GPU_CASES[name]
+    layer = make()
+    with torch.no_grad():  # parameters that start at zero have moved away from it in a trained block
+        for p in layer.parameters():
+            if not p.any():
+                p.add_(0.02 * torch.randn(p.shape))
+    layer = layer.to("cuda", dtype)
+    exact = copy.deepcopy(layer).double()
+    for block in (layer, exact):
+        if hasattr(block, "rope"):
+            block.rope.float()
+    x, do = (torch.randn(shape, device="cuda").to(dtype) for _ in range(2))
+    layer(x, *extra).backward(do)
+    exact(x.double(), *extra, mode="torch").backward(do.double())
+    for (key, ours), want in zip(layer.named_parameters(), exact.parameters()):
+        error = (ours.grad.double() - want.grad).norm() / want.grad.norm()
+        assert error <= {torch.float32: 8e-6, torch.float16: 1e-2}[dtype], (key, error)
