@@ -33,25 +33,29 @@ class TokenLinearFunction(torch.autograd.Function):
         return dx, dw, db
 
 
-def eager_tensors(*tensors):
-    """Whether these are ordinary tensors in an ordinary eager call: nothing that traces, maps, watches or carries a tangent
-    through torch's own operators."""
-    for t in tensors:
-        if t is not None and (type(t) is not torch.Tensor and type(t) is not nn.Parameter or _is_batched(t)):
-            return False
-    return not (torch.compiler.is_compiling() or torch.jit.is_tracing() or forward_ad._current_level >= 0 or
+def _eager_call():
+    """Whether nothing traces, maps, watches or carries a tangent through torch's own operators here."""
+    return not (torch.compiler.is_compiling() or torch._C._is_tracing() or forward_ad._current_level >= 0 or
                 torch._C._are_functorch_transforms_active() or torch._C._len_torch_dispatch_stack())
 
 
 def plain_tensors(*tensors):
-    """eager_tensors in a call that casts nothing."""
-    return not torch.is_autocast_enabled() and eager_tensors(*tensors)
+    """Whether these are ordinary tensors in an ordinary eager call that casts nothing."""
+    for t in tensors:
+        if t is not None and type(t) is not torch.Tensor and type(t) is not nn.Parameter:
+            return False
+    return not torch.is_autocast_enabled() and _eager_call()
 
 
 def composes_gradient(*grads):
     """Whether a backward has to be made of torch's operators: it is to be differentiated again, or the gradients it is
     given are batches of gradients, carry tangents or are traced."""
-    return torch.is_grad_enabled() or not eager_tensors(*grads)
+    if torch.is_grad_enabled() or not _eager_call():
+        return True
+    for g in grads:
+        if type(g) is not torch.Tensor or _is_batched(g):
+            return True
+    return False
 
 
 def splits_tokens(tokens, M, N, with_bias, fp32):
@@ -87,7 +91,7 @@ def token_linear(x, weight, bias):
 
 def trains(x):
     """Whether a call on x can need the gradients at all: a tensor (no proxy of one), grad mode, no trace."""
-    return type(x) is torch.Tensor and torch.is_grad_enabled() and not torch.jit.is_tracing()
+    return type(x) is torch.Tensor and torch.is_grad_enabled() and not torch._C._is_tracing()
 
 
 def project(module, x):
