@@ -444,20 +444,15 @@ def _rows(t):
     return t, t.stride(0), t.stride(1)
 
 
-def _check_grid(what, x, H, W):
-    """The kernels walk the H x W grid: it has to be the tokens'."""
-    if x.ndim != 3 or H < 1 or W < 1 or x.shape[1] != H * W:
-        raise ValueError(f"{what}: rows [B, H * W, C] needed, got {tuple(x.shape)} for H = {H}, W = {W}")
-
-
 def dwconv_fwd(x, w, bias, H, W, flip=False):
     """Depth-wise convolution of token rows x [B, H*W, C] with w [Cw, 1, K, K]; returns contiguous [B, H*W, C]."""
-    _check_grid("dwconv_fwd", x, H, W)
+    B, N, C = x.shape
+    if N != H * W or H < 1:
+        raise ValueError(f"dwconv_fwd: x must be rows of H * W tokens, got {tuple(x.shape)} for H = {H}, W = {W}")
     if w.dtype != x.dtype or (bias is not None and bias.dtype != x.dtype):
         raise ValueError("dwconv_fwd: x, w and bias must have one dtype")
     _require_gpu(x, w, bias)
     x, x_batch, x_row = _rows(x)
-    B, N, C = x.shape
     y = torch.empty(B, N, C, dtype=x.dtype, device=x.device)
     with _on(x.device):
         rc = lib().fbla_dwconv_fwd(_ptr(x), x_batch, x_row, _ptr(w), _ptr(bias), _ptr(y), N * C, C, B, H, W, C,
@@ -468,7 +463,9 @@ def dwconv_fwd(x, w, bias, H, W, flip=False):
 
 def dwconv_grad(x, g, w, H, W, with_bias):
     """(dw, db or None) of dwconv_fwd from its input and its output's gradient, both [B, H*W, C]."""
-    _check_grid("dwconv_grad", x, H, W)
+    B, N, C = x.shape
+    if N != H * W or H < 1:
+        raise ValueError(f"dwconv_grad: x must be rows of H * W tokens, got {tuple(x.shape)} for H = {H}, W = {W}")
     if g.shape != x.shape:
         raise ValueError(f"dwconv_grad: x and g must have one shape, got {tuple(x.shape)} and {tuple(g.shape)}")
     if w.dtype != x.dtype or g.dtype != x.dtype:
@@ -476,7 +473,6 @@ def dwconv_grad(x, g, w, H, W, with_bias):
     _require_gpu(x, g, w)
     x, x_batch, x_row = _rows(x)
     g, g_batch, g_row = _rows(g)
-    B, _, C = x.shape
     Cw, K, code = w.shape[0], w.shape[-1], dtype_code(x)
     L = lib()
     dw = torch.empty_like(w, memory_format=torch.contiguous_format)

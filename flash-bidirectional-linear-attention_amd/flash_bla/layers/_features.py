@@ -144,7 +144,7 @@ def rotary_features(qk, x, rotations, side, heads):
     """qk [B, N, 2C] (queries | keys before elu + 1), x [B, N, C] (the values), N = side * side, rotations
     [side, side, C / 2, 2].  Returns (q, k, q_rot, k_rot, v [B, heads, N, d], the values as rows)."""
     if (_takes(heads, x.shape[-1], 1, x, qk) and x.ndim == 3 and qk.shape == (*x.shape[:2], 2 * x.shape[2]) and
-            plain_tensors(rotations) and rotations.dtype == torch.float32 and
+            type(rotations) is torch.Tensor and rotations.dtype == torch.float32 and
             rotations.device == x.device and not rotations.requires_grad and
             rotations.shape == (side, side, x.shape[2] // 2, 2) and x.shape[1] == side * side):
         return RotaryFeaturesFunction.apply(qk, x, rotations, side, heads)
@@ -177,7 +177,7 @@ def turned_heads(q, k, weight, rotations):
     turned, k * weight turned)."""
     N, d = q.shape[-2:]
     pieces = d * q.element_size() // 16
-    if (_takes(1, d, 1, q, k, weight) and pieces <= 64 and pieces & (pieces - 1) == 0 and plain_tensors(rotations) and
+    if (_takes(1, d, 1, q, k, weight) and pieces <= 64 and pieces & (pieces - 1) == 0 and type(rotations) is torch.Tensor and
             rotations.dtype == torch.float32 and rotations.device == q.device and not rotations.requires_grad and
             q.ndim == 4 and rotations.ndim == 4 and rotations.shape[0] * rotations.shape[1] == N and rotations.shape[2:] == (d // 2, 2) and
             k.shape == q.shape and weight.shape == (*q.shape[:-1], 1)):
