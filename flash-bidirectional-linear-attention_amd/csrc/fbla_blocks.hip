@@ -11,8 +11,9 @@
 // All of it is elementwise on token rows and bound by HBM: a lane owns 16 bytes of channels of one token (the next lanes the
 // next channels), everything is computed from them in fp32 and rounded once, and nothing between the projection's rows and the
 // operator's heads is written.  Training steps with torch operators in their place and with these: polarity (64 x 28x28 x
-// 256, bf16) 2.77 -> 0.83 ms, of it here 51 us features (231 MB, 4.6 TB/s), 77 + 9 us their gradients (385 MB), 19 + 32 us the
-// merge; rotary (64 x 56x56 x 64) 0.83 -> 0.48 ms, of it 33 us features (205 MB, 6.2 TB/s), 44 us gradients (308 MB, 7 TB/s).
+// 256, bf16) 2.77 -> 0.83 ms, of it here 50 us features (257 MB, 5.1 TB/s), 77 + 9 us their gradients (385 MB, 5.0 TB/s), 19 + 33
+// us the merge; rotary (64 x 56x56 x 64) 0.83 -> 0.48 ms, of it 33 us features (205 MB, 6.2 TB/s), 45 us gradients (283 MB, 6.3
+// TB/s).
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -382,8 +383,8 @@ __global__ __launch_bounds__(kThreads) void rotary_bwd_kernel(Shape s, const T* 
 }
 
 // Keys weighted per token and both sides turned, on heads (layers/rala.py:60-69): k_out = k * weight, q_rot = R q,
-// k_rot = R k_out; weight [B, heads, N].  32 x 28x28 x 256 in bf16: 12 us forward, 15 us backward, torch's products,
-// complex products in fp32 and copies 0.25 ms.
+// k_rot = R k_out; weight [B, heads, N].  32 x 28x28 x 256 in bf16: 12 us forward, 15 us backward; torch's products,
+// complex products in fp32 and copies 58 and 150 us.
 template <typename T>
 __device__ __forceinline__ void turn(const float (&x)[Piece<T>::kVec], const float (&cs)[Piece<T>::kVec], float sign,
                                      float (&out)[Piece<T>::kVec]) {
@@ -606,7 +607,7 @@ __device__ __forceinline__ float row_max(float v, int lanes) {
 // t = (relu(x) + 1e-6) / scale; the feature is t^3 brought to t's length over all channels of the token.  With s = t / max t
 // (nothing under- or overflows) and n = |s|, m = |s^3|: feature = s^3 |t| / m, and for its gradient g, G = sum g s^3:
 // dt = 3 n s^2 g / m + G (s / (n m) - 3 n s^5 / m^3).
-// 64 x 28x28 x 256, bf16: 39 us (154 MB, 4 TB/s) and 83 + 9 us (231 MB), torch's operators 1.0 ms together.
+// 64 x 28x28 x 256, bf16: 38 us (154 MB, 4 TB/s) and 83 + 9 us (231 MB, 2.8 TB/s); torch's operators 279 and 851 us.
 // Rows of workgroup [0, q_wgs): the queries, the others the keys with the values beside them.
 template <typename T> __device__ __forceinline__ float focus_input(float x, float scale) {
   return ((x < 0.f ? 0.f : x) + 1e-6f) / scale;

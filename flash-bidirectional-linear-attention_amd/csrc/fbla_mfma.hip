@@ -151,7 +151,9 @@ template <typename T> __device__ __forceinline__ uint32_t phi_pair(uint32_t w) {
 
 // Rows whose length is no multiple of eight elements (PAD = 2: Prob::RK / RV elements in memory, inside operands of the
 // next multiple of eight).  Their 16-byte pieces start on any element.  The last piece of a row is moved back to end with
-// the row, so that no access leaves the row, and its elements are moved to their places in registers.
+// the row, so that no access leaves the row, and its elements are moved to their places in registers.  The moves cost
+// registers: bwd_a128_kernel spills 25 to 26 VGPRs a lane, part of them in its token loop (PAD = 1: 20 to 22, whole rows:
+// none), rows_kernel at 64 x 64 18; rows128_kernel spills 72 to 73 in the operand build with either PAD.
 typedef u32x4 u32x4_any __attribute__((aligned(2)));
 typedef uint32_t u32_any __attribute__((aligned(2)));
 // first element of piece `ch` of a row of `len` (>= 8) elements, and how far back it was moved

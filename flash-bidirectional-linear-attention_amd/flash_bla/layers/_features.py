@@ -1,7 +1,9 @@
 """What the vision blocks do between their projections and the attention operators, one HIP launch a direction: polarity
-features (layers/polaformer.py:63-84), focused features (layers/focused_la.py:56-74), rotary
-features (layers/mlla.py:74-81) and heads merged back to rows (polaformer.py:92-104, mlla.py:88-92).  The reference composes them of torch operators; the compositions here are what runs
-when the kernels do not take a call, and what a gradient of the gradient is made of.
+features (layers/polaformer.py:63-84), focused features (layers/focused_la.py:56-74), rotary features
+(layers/mlla.py:74-81), weighted and turned heads (layers/rala.py:60-69), interpolated tokens (focused_la.py:88-91) and
+heads merged back to rows (polaformer.py:92-104, mlla.py:88-92).  The reference composes them of torch operators; the
+compositions here are what runs when the kernels do not take a call, and what a gradient is made of that is differentiated
+again or that the kernels cannot read.
 """
 import torch
 import torch.nn.functional as F

@@ -1,4 +1,4 @@
-"""nn.Linear over token rows with the weight gradient on this package's kernel.
+"""Projections of token rows (nn.Linear) with the weight gradient on this package's kernel.
 
 The blocks' projections contract 1e4 to 1e5 tokens into a weight gradient of a few hundred on a side, a shape for which
 the library's GEMM fills a dozen CUs; `_hip.linear_wgrad` splits the tokens and takes the bias's gradient along.  The
