@@ -375,3 +375,16 @@ def test_rala_scores_times_tokens_that_overflow_are_not_formed(side, dtype, fuse
     block.rope.float()
     with pytest.raises(Reached if fused else ValueError, match=None if fused else "GPU"), torch.no_grad():
         block(torch.zeros(1, side * side, 8, dtype=dtype))
+
+
+@pytest.mark.parametrize("factor", [2.5, nn.Parameter(torch.tensor(3.0)), torch.tensor(3.0)])
+def test_focusing_factors_that_are_not_the_number_three_run_as_torch_operators(factor, only_shapes_decide):
+    """A learned factor of exactly 3 has a gradient, which the cube's kernel does not give."""
+    q, kv, pe, scale = (torch.rand(s) + 0.5 for s in FULL["focused"].values())
+    out = features.focused_features(q, kv, pe, scale, HEADS, factor)
+    for a, b in zip(out, features.focus_formula(q, kv, pe, scale, HEADS, factor)):
+        assert torch.equal(a, b)
+    if isinstance(factor, nn.Parameter):
+        assert torch.autograd.grad(out[0].sum(), factor)[0] != 0
+    with pytest.raises(only_shapes_decide):
+        features.focused_features(q, kv, pe, scale, HEADS, 3.0)
