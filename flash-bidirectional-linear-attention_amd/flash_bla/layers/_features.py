@@ -108,8 +108,9 @@ def focused_features(q, kv, pe, scale, heads, factor):
     """q [B, N, C], kv [B, n, 2C] (keys | values), pe [1, n, C], scale [1, 1, C].  Returns (q, k, v [B, heads, tokens, d],
     the values as rows [B, n, C]).  The kernels know the cube (a factor that is a tensor may want a gradient)."""
     C = q.shape[-1]
-    if (isinstance(factor, (int, float)) and factor == 3 and _takes(heads, C, 1, q, kv, pe, scale) and C <= _hip.most_row_channels(q) and q.ndim == 3 and
-            kv.ndim == 3 and kv.shape == (q.shape[0], kv.shape[1], 2 * C) and pe.shape == (1, kv.shape[1], C) and scale.shape == (1, 1, C)):
+    if (isinstance(factor, (int, float)) and factor == 3 and _takes(heads, C, 1, q, kv, pe, scale) and
+            C <= _hip.most_row_channels(q) and q.ndim == 3 and kv.ndim == 3 and
+            kv.shape == (q.shape[0], kv.shape[1], 2 * C) and pe.shape == (1, kv.shape[1], C) and scale.shape == (1, 1, C)):
         return FocusedFeaturesFunction.apply(q, kv, pe, scale, heads)
     return focus_formula(q, kv, pe, scale, heads, factor)
 
