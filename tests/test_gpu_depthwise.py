@@ -123,3 +123,23 @@ def test_infinities_and_nan_meet_what_lies_on_the_grid_alone(H, W, K, where, dty
     for name, a, b in (("y", y, want), ("dx", rows.grad, x64.grad), ("dw", conv.weight.grad, w64.grad)):
         b = b.detach().reshape(a.shape).to(dtype)
         torch.testing.assert_close(a.detach(), b, rtol=0, atol=0, equal_nan=True, msg=lambda m: f"{name}: {m}")
+
+
+@pytest.mark.parametrize("shape", [(2, 9, 7, 1, 64, 3), (4, 28, 28, 8, 32, 5), (2, 17, 23, 1, 136, 7)])
+def test_fp32_sums_are_rounded_once(shape):
+    """As torch's convolution in fp32: products and sums in 64 bits, one rounding (2^-24 of the value; the sums themselves
+    are off by less than 50 x 2^-53 of the magnitudes)."""
+    B, H, W, heads, Cw, K = shape
+    torch.manual_seed(K)
+    conv = nn.Conv2d(Cw, Cw, K, padding=K // 2, groups=Cw).cuda()
+    x, g = (torch.randn(B, H * W, heads * Cw, device="cuda") for _ in range(2))
+    x.requires_grad_()
+    y = depthwise_conv_tokens(x, conv, H, W)
+    dx, = torch.autograd.grad(y, x, g)
+    rows = x.detach().double().requires_grad_()
+    image = rows.transpose(1, 2).reshape(B, heads * Cw, H, W)
+    want = F.conv2d(image, conv.weight.double().repeat(heads, 1, 1, 1), conv.bias.double().repeat(heads), padding=K // 2,
+                    groups=heads * Cw).reshape(B, heads * Cw, H * W).transpose(1, 2)
+    exact_dx, = torch.autograd.grad(want, rows, g.double())
+    for a, b in ((y, want), (dx, exact_dx)):
+        assert ((a.double() - b).abs() <= 2.0 ** -24 * b.abs() + 2.0 ** -46).all()
