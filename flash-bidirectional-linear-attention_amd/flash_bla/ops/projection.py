@@ -97,8 +97,10 @@ def trains(x):
 def project(module, x):
     """module(x), a plain nn.Linear as token_linear.  The blocks hold plain nn.Linear modules and call them through this:
     what replaces, wraps, traces or looks for modules by their type finds them as they always were."""
-    if trains(x) and untouched(module, nn.Linear) and runs_on_rows(x, module.weight, module.bias):
-        return TokenLinearFunction.apply(x, module.weight, module.bias)
+    if trains(x) and untouched(module, nn.Linear):
+        weight, bias = module.weight, module.bias
+        if runs_on_rows(x, weight, bias):
+            return TokenLinearFunction.apply(x, weight, bias)
     return module(x)
 
 
