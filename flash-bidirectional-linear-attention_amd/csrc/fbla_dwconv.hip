@@ -162,7 +162,8 @@ __global__ __launch_bounds__(kThreads) void conv_kernel(Conv a, int strips_per_r
 
 // Weight and bias gradient: partial[chunk][ky][kx][C] = sum over the chunk's strips of g[y, x] * x[y + ky - P,
 // x + kx - P], the bias gradient in row K of ky = 0.  One tap row per workgroup (blockIdx.z): K * V accumulators per
-// lane, kept over all strips of the chunk, added over the workgroup's strips at the end in a fixed order.  46 us for the 51 MB
+// lane, kept over all strips of the chunk, added over the workgroup's strips at the end in a fixed order (fp32: sums of g alone
+// and sums over chunks in 64 bits, so that the bias gradient is no further from exact than column sums in a tree).  46 us for the 51 MB
 // of 64 x 28x28 x 256 in bf16, 5x5: the K workgroups of a chunk fetch the same rows, and at 170 to 206 VGPRs two waves fit a
 // SIMD (3x3: three).
 template <typename T, int K, int STRIP>
@@ -173,11 +174,15 @@ __global__ __launch_bounds__(kThreads) void grad_kernel(Conv a, const T* __restr
   const int ky = blockIdx.z, c0 = blockIdx.y * kBlockChannels;
   const int lane = threadIdx.x % Lane<T>::kLanes, worker = threadIdx.x / Lane<T>::kLanes;
   const int cl = lane * V, c = c0 + cl;
-  float acc[K + 1][V];
+  using A = Sum<T>;
+  float acc[K][V];
+  A total[V];  // of g
 #pragma unroll
-  for (int k = 0; k <= K; ++k)
+  for (int j = 0; j < V; ++j) {
+    total[j] = 0;
 #pragma unroll
-    for (int j = 0; j < V; ++j) acc[k][j] = 0.f;
+    for (int k = 0; k < K; ++k) acc[k][j] = 0.f;
+  }
 
   if (c < a.C) {
     const T* xc = static_cast<const T*>(a.x) + c;
@@ -193,7 +198,7 @@ __global__ __launch_bounds__(kThreads) void grad_kernel(Conv a, const T* __restr
 #pragma unroll
       for (int t = 0; t < STRIP; ++t)
 #pragma unroll
-        for (int j = 0; j < V; ++j) acc[K][j] += (float)gv[t].e[j];
+        for (int j = 0; j < V; ++j) total[j] += (A)gv[t].e[j];
       if (inside) {
 #pragma unroll
         for (int kx = 0; kx < K; ++kx)
@@ -238,25 +243,31 @@ __global__ __launch_bounds__(kThreads) void grad_kernel(Conv a, const T* __restr
     }
   }
   // the strips of a wave (lanes of equal channel), then the waves, both in a fixed order
-  __shared__ float sums[kWaves][K + 1][kBlockChannels];
+  __shared__ float sums[kWaves][K][kBlockChannels];
+  __shared__ A totals[kWaves][kBlockChannels];
+  const bool first = (threadIdx.x & 63) < Lane<T>::kLanes;
 #pragma unroll
-  for (int k = 0; k <= K; ++k)
+  for (int j = 0; j < V; ++j) {
 #pragma unroll
-    for (int j = 0; j < V; ++j) {
+    for (int k = 0; k < K; ++k) {
       float v = acc[k][j];
 #pragma unroll
       for (int m = Lane<T>::kLanes; m < 64; m *= 2) v += __shfl_xor(v, m);
-      if ((threadIdx.x & 63) < Lane<T>::kLanes) sums[threadIdx.x / 64][k][cl + j] = v;
+      if (first) sums[threadIdx.x / 64][k][cl + j] = v;
     }
+#pragma unroll
+    for (int m = Lane<T>::kLanes; m < 64; m *= 2) total[j] += __shfl_xor(total[j], m);
+    if (first) totals[threadIdx.x / 64][cl + j] = total[j];
+  }
   __syncthreads();
   float* out = partial + ((int64_t)blockIdx.x * K + ky) * (K + 1) * a.C;
   for (int i = threadIdx.x; i < (K + 1) * kBlockChannels; i += kThreads) {
     const int k = i / kBlockChannels, j = i % kBlockChannels;
     if (c0 + j < a.C) {
-      float v = 0.f;
+      A v = 0;
 #pragma unroll
-      for (int w = 0; w < kWaves; ++w) v += sums[w][k][j];
-      out[k * a.C + c0 + j] = v;
+      for (int w = 0; w < kWaves; ++w) v += k < K ? sums[w][k][j] : totals[w][j];
+      out[k * a.C + c0 + j] = (float)v;
     }
   }
 }
@@ -272,18 +283,19 @@ __global__ __launch_bounds__(kThreads) void grad_finish_kernel(const float* __re
   const int cw = blockIdx.y * (kThreads / kParts) + threadIdx.x % (kThreads / kParts);
   const int part = threadIdx.x / (kThreads / kParts);
   const int ky = row == K * K ? 0 : row / K, kx = row == K * K ? K : row % K;
-  float sum = 0.f;
+  using A = Sum<T>;
+  A sum = 0;
   if (cw < Cw) {
     const int groups = C / Cw, terms = nchunks * groups;
 #pragma unroll 4
     for (int i = part; i < terms; i += kParts)
       sum += partial[(((int64_t)(i / groups) * K + ky) * (K + 1) + kx) * C + (i % groups) * Cw + cw];
   }
-  __shared__ float sums[kParts][kThreads / kParts];
+  __shared__ A sums[kParts][kThreads / kParts];
   sums[part][threadIdx.x % (kThreads / kParts)] = sum;
   __syncthreads();
   if (part == 0 && cw < Cw) {
-    float v = 0.f;
+    A v = 0;
     for (int i = 0; i < kParts; ++i) v += sums[i][threadIdx.x];
     if (row == K * K) { if (db) db[cw] = (T)v; }
     else if (dw) dw[(int64_t)cw * K * K + row] = (T)v;
