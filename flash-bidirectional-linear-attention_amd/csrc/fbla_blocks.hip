@@ -51,21 +51,33 @@ template <typename T> __device__ __forceinline__ float power_of(float a, float p
   if constexpr (sizeof(T) == 4) return powf(a, p);
   else return __builtin_amdgcn_exp2f(p * __builtin_amdgcn_logf(a));
 }
-// What the gradients of a^power need: slope = a^p for p = power - 1 >= 0, which is 1 for p = 0 whatever a is, and log = ln a.
-// log2f, not the bare instruction: that takes a denormal for 0, whose logarithm would make a gradient NaN.
-template <typename T> __device__ __forceinline__ void power_slope(float a, float p, float& slope, float& log) {
-  if constexpr (sizeof(T) == 4) {
-    slope = powf(a, p);
-    log = logf(a);
-  } else {
-    const float l = log2f(a);
-    slope = p == 0.f ? 1.f : __builtin_amdgcn_exp2f(p * l);
-    log = l * 0.693147180559945309f;
-  }
-}
 template <typename T> __device__ __forceinline__ float exp_of(float x) {
   if constexpr (sizeof(T) == 4) return expf(x);
   else return __builtin_amdgcn_exp2f(x * 1.44269504088896341f);
+}
+
+// fp32 gradients are as far from exact as torch's operators leave them and no further: quotients are divided out there, and
+// what torch rounds product by product and sums in a tree is kept and summed in 64 bits.  16-bit types, whose results' rounding
+// is thousands of times that, multiply by reciprocals and sum in 32 bits.
+template <typename T> using Sum = std::conditional_t<sizeof(T) == 4, double, float>;
+template <typename T> __device__ __forceinline__ float divisor(T scale) { return sizeof(T) == 4 ? (float)scale : 1.f / (float)scale; }
+template <typename T> __device__ __forceinline__ float over(float x, float divisor) {
+  return sizeof(T) == 4 ? x / divisor : x * divisor;
+}
+
+// What the gradients of a^power need: slope = a^(power - 1), which is 1 for a power of 1 whatever a is, and rise = a^power
+// ln a.  log2f, not the bare instruction: that takes a denormal for 0, whose logarithm would make a gradient NaN.  fp32:
+// powf(a, power - 1) times a, the product unrounded, is as far from a^power as powf(a, power) (3.34e-8 and 3.48e-8 root mean
+// square over a in (0, 3), powers 1 to 5), and a second powf costs 80 us at 64 x 28x28 x 256.
+template <typename T> __device__ __forceinline__ void power_slope(float a, float power, float& slope, Sum<T>& rise) {
+  if constexpr (sizeof(T) == 4) {
+    slope = powf(a, power - 1.f);
+    rise = (double)slope * a * logf(a);
+  } else {
+    const float l = log2f(a), p = power - 1.f;
+    slope = p == 0.f ? 1.f : __builtin_amdgcn_exp2f(p * l);
+    rise = slope * a * (l * 0.693147180559945309f);
+  }
 }
 
 // first element of head row (b, h, t) of a [B, heads, n, width] tensor
@@ -130,21 +142,23 @@ __global__ __launch_bounds__(kThreads) void polarity_fwd_kernel(Shape s, Polarit
 // One piece's gradients: dx = the gradient of x (q, or k and its positional term alike), added to `dscale` the gradient of
 // -scale * scale, to `dpower` that of the power.
 template <typename T>
-__device__ __forceinline__ void polarity_piece_bwd(const float (&x)[Piece<T>::kVec], const float (&inv)[Piece<T>::kVec],
+__device__ __forceinline__ void polarity_piece_bwd(const float (&x)[Piece<T>::kVec], const float (&scale)[Piece<T>::kVec],
                                                    const float (&power)[Piece<T>::kVec], const float (&gpos)[Piece<T>::kVec],
                                                    const float (&gneg)[Piece<T>::kVec], float (&dx)[Piece<T>::kVec],
-                                                   float (&dscale)[Piece<T>::kVec], float (&dpower)[Piece<T>::kVec]) {
+                                                   Sum<T> (&dscale)[Piece<T>::kVec], Sum<T> (&dpower)[Piece<T>::kVec]) {
+  using A = Sum<T>;
 #pragma unroll
   for (int j = 0; j < Piece<T>::kVec; ++j) {
-    const float y = x[j] * inv[j], a = fabsf(y);
+    const float y = over<T>(x[j], scale[j]), a = fabsf(y);
     const float gp = y < 0.f ? 0.f : gpos[j], gn = y > 0.f ? 0.f : gneg[j];  // (NaN is in both parts)
-    float slope, log;
-    power_slope<T>(a, power[j] - 1.f, slope, log);
+    float slope;
+    A rise;
+    power_slope<T>(a, power[j], slope, rise);
     const bool zero = a == 0.f;  // both parts are cut off there: no gradient
-    const float dy = zero ? 0.f : (gp - gn) * power[j] * slope;
-    dx[j] = dy * inv[j];
+    const A dy = zero ? A(0) : (A)(gp - gn) * power[j] * slope;
+    dx[j] = over<T>((float)dy, scale[j]);
     dscale[j] += dy * x[j];
-    dpower[j] += zero ? 0.f : (gp + gn) * (slope * a) * log;
+    dpower[j] += zero ? A(0) : (A)(gp + gn) * rise;
   }
 }
 
@@ -164,13 +178,14 @@ __global__ __launch_bounds__(kThreads) void polarity_bwd_kernel(Shape s, Polarit
   const bool keys = (int)blockIdx.x >= q_wgs;
   const uint32_t wg = keys ? blockIdx.x - q_wgs : blockIdx.x, wgs = keys ? gridDim.x - q_wgs : q_wgs;
   const int c = (blockIdx.y * 64 + lane) * V, h = c / s.d, j0 = c % s.d;
-  float dscale[V], dpower[V], inv[V], power[V];
+  Sum<T> dscale[V], dpower[V];
+  float scale[V], power[V];
   {
     const Piece<T> sc = load(a.scale + c), pw = load(a.power + c);
 #pragma unroll
     for (int j = 0; j < V; ++j) {
-      dscale[j] = dpower[j] = 0.f;
-      inv[j] = 1.f / (float)sc.e[j];
+      dscale[j] = dpower[j] = 0;
+      scale[j] = divisor<T>(sc.e[j]);
       power[j] = (float)pw.e[j];
     }
   }
@@ -189,7 +204,7 @@ __global__ __launch_bounds__(kThreads) void polarity_bwd_kernel(Shape s, Polarit
         gpos[j] = (float)s0.e[j] + (float)o1.e[j];
         gneg[j] = (float)s1.e[j] + (float)o0.e[j];
       }
-      polarity_piece_bwd<T>(xf, inv, power, gpos, gneg, dx, dscale, dpower);
+      polarity_piece_bwd<T>(xf, scale, power, gpos, gneg, dx, dscale, dpower);
       Piece<T> out;
 #pragma unroll
       for (int j = 0; j < V; ++j) out.e[j] = (T)dx[j];
@@ -218,7 +233,7 @@ __global__ __launch_bounds__(kThreads) void polarity_bwd_kernel(Shape s, Polarit
           gpos[j] = (float)g0.e[j];
           gneg[j] = (float)g1.e[j];
         }
-        polarity_piece_bwd<T>(xf, inv, power, gpos, gneg, dx, dscale, dpower);
+        polarity_piece_bwd<T>(xf, scale, power, gpos, gneg, dx, dscale, dpower);
         Piece<T> out, v;
 #pragma unroll
         for (int j = 0; j < V; ++j) {
@@ -236,7 +251,7 @@ __global__ __launch_bounds__(kThreads) void polarity_bwd_kernel(Shape s, Polarit
     }
   }
   // the rows of the workgroup, in order
-  __shared__ float sums[kThreads * V];
+  __shared__ Sum<T> sums[kThreads * V];
   float* out = partial + (int64_t)blockIdx.x * 2 * C;
 #pragma unroll
   for (int which = 0; which < 2; ++which) {
@@ -246,31 +261,32 @@ __global__ __launch_bounds__(kThreads) void polarity_bwd_kernel(Shape s, Polarit
       for (int j = 0; j < V; ++j) sums[(r * lanes + lane) * V + j] = which ? dpower[j] : dscale[j];
     __syncthreads();
     for (int i = threadIdx.x; i < lanes * V; i += kThreads) {
-      float v = 0.f;
+      Sum<T> v = 0;
       for (int q = 0; q < rows; ++q) v += sums[q * lanes * V + i];
-      out[which * C + blockIdx.y * 64 * V + i] = v;
+      out[which * C + blockIdx.y * 64 * V + i] = (float)v;
     }
   }
 }
 
 // Sums over the partials in order, four neighbouring results per lane, 16 lanes of a column; workgroups [0, stat_wgs): the
-// `stats` C sums of the scale (times its reciprocal square or, `over` 1, its reciprocal) and the power, the others the Nk C
+// `stats` C sums of the scale (times its reciprocal square or, `by` 1, its reciprocal) and the power, the others the Nk C
 // sums of the positional term.
 template <typename T>
-__global__ __launch_bounds__(kThreads) void features_finish_kernel(int C, int stats_of, int over, int wgs, const float* __restrict__ partial,
+__global__ __launch_bounds__(kThreads) void features_finish_kernel(int C, int stats_of, int by, int wgs, const float* __restrict__ partial,
                                                                    const T* __restrict__ scale, T* __restrict__ dscale,
                                                                    T* __restrict__ dpower, int stat_wgs, int groups,
                                                                    int64_t pe_count, const float* __restrict__ pe_partial,
                                                                    T* __restrict__ dpe) {
   constexpr int kParts = 16, kLanes = kThreads / kParts;
-  __shared__ f32x4 sums[kParts][kLanes];
+  using A = Sum<T>;
+  __shared__ A sums[kParts][kLanes][4];
   const bool stats = (int)blockIdx.x < stat_wgs;
   const int lane = threadIdx.x % kLanes, part = threadIdx.x / kLanes;
   const int64_t at = ((int64_t)(stats ? blockIdx.x : blockIdx.x - stat_wgs) * kLanes + lane) * 4;
   const int64_t count = stats ? (int64_t)stats_of * C : pe_count;
   const int terms = stats ? wgs : groups;
   const float* src = stats ? partial : pe_partial;
-  f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+  A sum[4] = {0, 0, 0, 0};
   if (at < count)
 #pragma unroll 4
     for (int i = part; i < terms; i += kParts) {
@@ -278,7 +294,8 @@ __global__ __launch_bounds__(kThreads) void features_finish_kernel(int C, int st
 #pragma unroll
       for (int j = 0; j < 4; ++j) sum[j] += v[j];
     }
-  sums[part][lane] = sum;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) sums[part][lane][j] = sum[j];
   __syncthreads();
   if (part != 0 || at >= count) return;
   for (int i = 1; i < kParts; ++i)
@@ -290,8 +307,8 @@ __global__ __launch_bounds__(kThreads) void features_finish_kernel(int C, int st
     if (!stats) dpe[c] = (T)sum[j];
     else if (c >= C) dpower[c - C] = (T)sum[j];
     else {
-      const float inv = 1.f / (float)scale[c];
-      dscale[c] = (T)(over == 1 ? -sum[j] * inv : -sum[j] * inv * inv);
+      const A inv = A(1) / (A)scale[c];
+      dscale[c] = (T)(by == 1 ? -sum[j] * inv : -sum[j] * inv * inv);
     }
   }
 }
@@ -604,14 +621,16 @@ __device__ __forceinline__ float row_max(float v, int lanes) {
 // ---------------------------------------------------------------------------------------------------------------
 // focused features (layers/focused_la.py:56-74)
 // ---------------------------------------------------------------------------------------------------------------
-// t = (relu(x) + 1e-6) / scale; the feature is t^3 brought to t's length over all channels of the token.  With s = t / max t
-// (nothing under- or overflows) and n = |s|, m = |s^3|: feature = s^3 |t| / m, and for its gradient g, G = sum g s^3:
+// t = (relu(x) + 1e-6) / scale; the feature is t^3 brought to t's length over all channels of the token.  With s = t times
+// the power of two that brings max t to [0.5, 1) (exact, and nothing under- or overflows) and n = |s|, m = |s^3|: feature = s^3 |t| / m, and for its gradient g, G = sum g s^3:
 // dt = 3 n s^2 g / m + G (s / (n m) - 3 n s^5 / m^3).
 // 64 x 28x28 x 256, bf16: 38 us (154 MB, 4 TB/s) and 83 + 9 us (231 MB, 2.8 TB/s); torch's operators 279 and 851 us.
 // Rows of workgroup [0, q_wgs): the queries, the others the keys with the values beside them.
 template <typename T> __device__ __forceinline__ float focus_input(float x, float scale) {
   return ((x < 0.f ? 0.f : x) + 1e-6f) / scale;
 }
+// exponent of the largest t, such that 2^-exponent and 2^exponent are numbers
+__device__ __forceinline__ int focus_exponent(float top) { return min(max(__builtin_amdgcn_frexp_expf(top), -126), 126); }
 
 template <typename T, int PER>
 __global__ __launch_bounds__(kThreads) void focus_fwd_kernel(Shape s, Focus<const T> a, int lanes, unsigned q_wgs,
@@ -645,7 +664,8 @@ __global__ __launch_bounds__(kThreads) void focus_fwd_kernel(Shape s, Focus<cons
     }
   }
   top = row_max(top, lanes);
-  const float down = 1.f / top;
+  const int exponent = focus_exponent(top);
+  const float down = ldexpf(1.f, -exponent);
   float n2 = 0.f, m2 = 0.f;
 #pragma unroll
   for (int p = 0; p < PER; ++p)
@@ -656,7 +676,7 @@ __global__ __launch_bounds__(kThreads) void focus_fwd_kernel(Shape s, Focus<cons
       m2 = fmaf(cube, cube, m2);
       t[p][j] = cube;
     }
-  const float r = top * sqrtf(row_sum(n2, lanes) / row_sum(m2, lanes));
+  const float r = ldexpf(sqrtf(row_sum(n2, lanes) / row_sum(m2, lanes)), exponent);
 #pragma unroll
   for (int p = 0; p < PER; ++p) {
     const int c = (p * lanes + lane) * V;
@@ -681,7 +701,8 @@ __global__ __launch_bounds__(kThreads) void focus_bwd_kernel(Shape s, Focus<cons
   const uint32_t n = keys ? s.Nk : s.N;
   // queries: items are rows, one "batch" each; keys: items are (token, batch group)
   const uint32_t items = keys ? n * groups : (uint32_t)s.B * n;
-  float inv[PER][V], dscale[PER][V];
+  float scale[PER][V];
+  Sum<T> dscale[PER][V];
 #pragma unroll
   for (int p = 0; p < PER; ++p) {
     const int c = (p * lanes + lane) * V;
@@ -690,8 +711,8 @@ __global__ __launch_bounds__(kThreads) void focus_bwd_kernel(Shape s, Focus<cons
     if (c < C) sc = load(a.scale + c);
 #pragma unroll
     for (int j = 0; j < V; ++j) {
-      inv[p][j] = c < C ? 1.f / (float)sc.e[j] : 0.f;
-      dscale[p][j] = 0.f;
+      scale[p][j] = c < C ? divisor<T>(sc.e[j]) : 1.f;
+      dscale[p][j] = 0;
     }
   }
   // every group of lanes makes the same number of trips, so that all lanes of a wave reach the shuffles
@@ -735,13 +756,13 @@ __global__ __launch_bounds__(kThreads) void focus_bwd_kernel(Shape s, Focus<cons
         for (int j = 0; j < V; ++j) {
           const float xf = (float)x.e[j] + (float)pe.e[j];
           if (!(xf <= 0.f)) positive[p] |= 1u << j;
-          t[p][j] = ((xf < 0.f ? 0.f : xf) + 1e-6f) * inv[p][j];
+          t[p][j] = over<T>((xf < 0.f ? 0.f : xf) + 1e-6f, scale[p][j]);
           top = fmaxf(top, t[p][j]);
           gf[p][j] = (float)gi.e[j];
         }
       }
       top = row_max(top, lanes);
-      const float down = 1.f / top;
+      const float down = ldexpf(1.f, -focus_exponent(top));
       float n2 = 0.f, m2 = 0.f, G = 0.f;
 #pragma unroll
       for (int p = 0; p < PER; ++p)
@@ -766,8 +787,8 @@ __global__ __launch_bounds__(kThreads) void focus_bwd_kernel(Shape s, Focus<cons
         for (int j = 0; j < V; ++j) {
           const float v = t[p][j] * down, v2 = v * v;
           const float dt = c2 * v2 * gf[p][j] + c1 * v - c5 * v2 * v2 * v;
-          dscale[p][j] = fmaf(dt, t[p][j], dscale[p][j]);
-          const float dx = (positive[p] >> j & 1) ? dt * inv[p][j] : 0.f;
+          dscale[p][j] += (Sum<T>)dt * t[p][j];
+          const float dx = (positive[p] >> j & 1) ? over<T>(dt, scale[p][j]) : 0.f;
           dpe[p][j] += dx;
           out.e[j] = (T)dx;
         }
@@ -786,7 +807,7 @@ __global__ __launch_bounds__(kThreads) void focus_bwd_kernel(Shape s, Focus<cons
       }
     }
   }
-  __shared__ float sums[kThreads * V];
+  __shared__ Sum<T> sums[kThreads * V];
 #pragma unroll
   for (int p = 0; p < PER; ++p) {
     __syncthreads();
@@ -795,9 +816,9 @@ __global__ __launch_bounds__(kThreads) void focus_bwd_kernel(Shape s, Focus<cons
     __syncthreads();
     for (int i = threadIdx.x; i < lanes * V; i += kThreads) {
       const int c = p * lanes * V + i;
-      float v = 0.f;
+      Sum<T> v = 0;
       for (int q = 0; q < per_wg; ++q) v += sums[q * lanes * V + i];
-      if (c < C) partial[(int64_t)blockIdx.x * C + c] = v;
+      if (c < C) partial[(int64_t)blockIdx.x * C + c] = (float)v;
     }
   }
 }
