@@ -6,12 +6,13 @@ compositions here are what runs when the kernels do not take a call, and what a 
 again or that the kernels cannot read.
 """
 import torch
+import torch.nn as nn
 import torch.nn.functional as F
 
 from flash_bla import _hip
 from flash_bla.layers._common import merge_heads, split_heads
 from flash_bla.ops.feature_map import elu_plus_one
-from flash_bla.ops.projection import composes_gradient, plain_tensors
+from flash_bla.ops.projection import eager_call, gradient_of
 
 _TYPES = (torch.float16, torch.bfloat16, torch.float32)
 
@@ -19,21 +20,24 @@ _TYPES = (torch.float16, torch.bfloat16, torch.float32)
 def _takes(heads, channels, unit, *tensors):
     """Ordinary GPU tensors of one supported type whose heads (or their `unit` parts) are whole 16-byte pieces."""
     x = tensors[0]
-    dtype, device = x.dtype, x.device
+    dtype, device = x.dtype, x.get_device()
     if not x.is_cuda or dtype not in _TYPES or channels % heads or channels // heads % (unit * 16 // x.element_size()):
         return False
     for t in tensors:
-        if t is not None and (t.dtype != dtype or t.device != device or not 0 < t.numel() < 1 << 31):
+        if t is not None and (type(t) is not torch.Tensor and type(t) is not nn.Parameter or t.dtype != dtype or
+                              t.get_device() != device or not 0 < t.numel() < 1 << 31):
             return False
-    return plain_tensors(*tensors)
+    return not torch.is_autocast_enabled() and eager_call()
 
 
 def differentiable_gradients(formula, inputs, grads):
     """Gradients of formula(*inputs) by torch's operators, which can be differentiated again where that is wanted."""
-    wanted = [t for t in inputs if torch.is_tensor(t) and t.requires_grad]
     with torch.enable_grad():
+        # (through aliases: the inputs may depend on one another, and the engine would walk from one to the other)
+        inputs = [t.view_as(t) if torch.is_tensor(t) and t.requires_grad else t for t in inputs]
         out = formula(*inputs)
-        pairs = [(o, g) for o, g in zip(out, grads) if o is not None and o.requires_grad]
+    wanted = [t for t in inputs if torch.is_tensor(t) and t.requires_grad]
+    pairs = [(o, g) for o, g in zip(out, grads) if o is not None and o.requires_grad]
     got = iter(torch.autograd.grad([o for o, _ in pairs], wanted, [g for _, g in pairs],
                                    create_graph=torch.is_grad_enabled(), allow_unused=True))
     return tuple(next(got) if torch.is_tensor(t) and t.requires_grad else None for t in inputs)
@@ -57,10 +61,9 @@ class PolarityFeaturesFunction(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, *grads):
-        inputs = ctx.saved_tensors
-        if composes_gradient(*grads):
-            return differentiable_gradients(polarity_formula, (*inputs, ctx.heads), grads)
-        return (*_hip.polarity_bwd(*inputs, ctx.heads, *grads), None)
+        inputs = (*ctx.saved_tensors, ctx.heads)
+        return gradient_of(lambda *g: (*_hip.polarity_bwd(*inputs, *g), None),
+                           lambda *g: differentiable_gradients(polarity_formula, inputs, g), *grads)
 
 
 def polarity_features(qg, kv, pe, scale, power, heads):
@@ -98,10 +101,9 @@ class FocusedFeaturesFunction(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, *grads):
-        inputs = ctx.saved_tensors
-        if composes_gradient(*grads):
-            return differentiable_gradients(focus_formula, (*inputs, ctx.heads), grads)
-        return (*_hip.focus_bwd(*inputs, ctx.heads, *grads), None)
+        inputs = (*ctx.saved_tensors, ctx.heads)
+        return gradient_of(lambda *g: (*_hip.focus_bwd(*inputs, *g), None),
+                           lambda *g: differentiable_gradients(focus_formula, inputs, g), *grads)
 
 
 def focused_features(q, kv, pe, scale, heads, factor):
@@ -138,9 +140,9 @@ class RotaryFeaturesFunction(torch.autograd.Function):
     @staticmethod
     def backward(ctx, *grads):
         qk, x, rotations = ctx.saved_tensors
-        if composes_gradient(*grads):
-            return differentiable_gradients(rotary_formula, (qk, x, rotations, ctx.side, ctx.heads), grads)
-        return (*_hip.rotary_bwd(qk, rotations, ctx.heads, *grads), None, None, None)
+        inputs = qk, x, rotations, ctx.side, ctx.heads
+        return gradient_of(lambda *g: (*_hip.rotary_bwd(qk, rotations, ctx.heads, *g), None, None, None),
+                           lambda *g: differentiable_gradients(rotary_formula, inputs, g), *grads)
 
 
 def rotary_features(qk, x, rotations, side, heads):
@@ -169,10 +171,9 @@ class TurnedHeadsFunction(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, *grads):
-        q, k, weight, rotations = ctx.saved_tensors
-        if composes_gradient(*grads):
-            return differentiable_gradients(turn_formula, (q, k, weight, rotations), grads)
-        return (*_hip.turn_bwd(k, weight, rotations, *grads), None)
+        inputs = ctx.saved_tensors
+        return gradient_of(lambda *g: (*_hip.turn_bwd(*inputs[1:], *g), None),
+                           lambda *g: differentiable_gradients(turn_formula, inputs, g), *grads)
 
 
 def turned_heads(q, k, weight, rotations):
@@ -202,13 +203,14 @@ class MergeHeadsFunction(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, g):
-        o, o2, local, gate = ctx.saved_tensors
-        if composes_gradient(g):
-            if gate is not None:
-                return differentiable_gradients(merge_formula, (o, o2, local, gate), (g,))
+        inputs = ctx.saved_tensors  # o, o2, local, gate, or nothing without a gate
+
+        def composed(g):
+            if inputs[3] is not None:
+                return differentiable_gradients(merge_formula, inputs, (g,))
             do = split_heads(g, ctx.heads)
             return (*(do.chunk(2, dim=-1) if ctx.halves else (do, None)), g, None)
-        return _hip.merge_bwd(g, ctx.heads, ctx.halves, o, o2, local, gate)
+        return gradient_of(lambda g: _hip.merge_bwd(g, ctx.heads, ctx.halves, *inputs), composed, g)
 
 
 def merge_heads_with(o, o2, local, gate=None):
@@ -233,10 +235,10 @@ class InterpolateTokensFunction(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, g):
-        if composes_gradient(g):  # linear in the rows: the gradient is that of any rows
+        def composed(g):  # linear in the rows: the gradient is that of any rows
             rows = torch.zeros(g.shape[0], ctx.n, g.shape[2], dtype=g.dtype, device=g.device, requires_grad=True)
             return differentiable_gradients(interpolate_formula, (rows, g.shape[1]), (g,))
-        return _hip.interpolate_bwd(g, ctx.n), None
+        return gradient_of(lambda g: (_hip.interpolate_bwd(g, ctx.n), None), composed, g)
 
 
 def interpolate_tokens(rows, tokens):

@@ -10,7 +10,7 @@ import torch.nn.functional as F
 
 from flash_bla import _hip
 from flash_bla.ops._check import untouched
-from flash_bla.ops.projection import composes_gradient, plain_tensors
+from flash_bla.ops.projection import gradient_of, plain_tensors
 
 
 class DepthwiseConvTokensFunction(torch.autograd.Function):
@@ -23,21 +23,25 @@ class DepthwiseConvTokensFunction(torch.autograd.Function):
     @staticmethod
     def backward(ctx, g):
         x, weight = ctx.saved_tensors
-        dx = dw = db = None
-        if composes_gradient(g):  # of torch's convolution
+
+        def kernels(g):
+            dx = dw = db = None
+            if ctx.needs_input_grad[0]:
+                dx = _hip.dwconv_fwd(g, weight.contiguous(), None, *ctx.grid, flip=True)
+            if ctx.needs_input_grad[1] or (ctx.with_bias and ctx.needs_input_grad[2]):
+                dw, db = _hip.dwconv_grad(x, g, weight, *ctx.grid, ctx.with_bias)
+            return dx, dw, db, None, None
+
+        def composed(g):  # of torch's convolution
             bias = torch.zeros(weight.shape[0], dtype=g.dtype, device=g.device, requires_grad=True)
             with torch.enable_grad():
-                y = _convolution_of_images(x, *ctx.grid, weight.shape[0], lambda images: F.conv2d(
-                    images, weight, bias, padding=weight.shape[-1] // 2, groups=weight.shape[0]))
-            leaves = [t for t in (x, weight, bias) if t.requires_grad]
-            got = iter(torch.autograd.grad(y, leaves, g, create_graph=torch.is_grad_enabled()))
-            dx, dw, db = (next(got) if t.requires_grad else None for t in (x, weight, bias))
+                inputs = [t.view_as(t) if t.requires_grad else t for t in (x, weight, bias)]
+                y = _convolution_of_images(inputs[0], *ctx.grid, weight.shape[0], lambda images: F.conv2d(
+                    images, *inputs[1:], padding=weight.shape[-1] // 2, groups=weight.shape[0]))
+            got = iter(torch.autograd.grad(y, [t for t in inputs if t.requires_grad], g, create_graph=torch.is_grad_enabled()))
+            dx, dw, db = (next(got) if t.requires_grad else None for t in inputs)
             return dx, dw, db if ctx.with_bias else None, None, None
-        if ctx.needs_input_grad[0]:
-            dx = _hip.dwconv_fwd(g, weight.contiguous(), None, *ctx.grid, flip=True)
-        if ctx.needs_input_grad[1] or (ctx.with_bias and ctx.needs_input_grad[2]):
-            dw, db = _hip.dwconv_grad(x, g, weight, *ctx.grid, ctx.with_bias)
-        return dx, dw, db, None, None
+        return gradient_of(kernels, composed, g)
 
 
 def runs_on_tokens(x, conv):

@@ -26,14 +26,14 @@ class TokenLinearFunction(torch.autograd.Function):
         x, weight = ctx.saved_tensors
         dx = g @ weight if ctx.needs_input_grad[0] else None
         with_bias = ctx.with_bias and ctx.needs_input_grad[2]
-        if composes_gradient(g):
+
+        def composed(g):
             rows = g.reshape(-1, g.shape[-1])
-            return dx, rows.t() @ x.reshape(-1, x.shape[-1]), rows.sum(0) if with_bias else None
-        dw, db = _hip.linear_wgrad(g, x, with_bias)
-        return dx, dw, db
+            return rows.t() @ x.reshape(-1, x.shape[-1]), rows.sum(0) if with_bias else None
+        return (dx, *gradient_of(lambda g: _hip.linear_wgrad(g, x, with_bias), composed, g))
 
 
-def _eager_call():
+def eager_call():
     """Whether nothing traces, maps, watches or carries a tangent through torch's own operators here."""
     return not (torch.compiler.is_compiling() or torch._C._is_tracing() or forward_ad._current_level >= 0 or
                 torch._C._are_functorch_transforms_active() or torch._C._len_torch_dispatch_stack())
@@ -44,18 +44,21 @@ def plain_tensors(*tensors):
     for t in tensors:
         if t is not None and type(t) is not torch.Tensor and type(t) is not nn.Parameter:
             return False
-    return not torch.is_autocast_enabled() and _eager_call()
+    return not torch.is_autocast_enabled() and eager_call()
 
 
-def composes_gradient(*grads):
-    """Whether a backward has to be made of torch's operators: it is to be differentiated again, or the gradients it is
-    given are batches of gradients, carry tangents or are traced."""
-    if torch.is_grad_enabled() or not _eager_call():
-        return True
-    for g in grads:
-        if type(g) is not torch.Tensor or _is_batched(g):
-            return True
-    return False
+def gradient_of(kernel, composition, *grads):
+    """kernel(*grads), or composition(*grads) by torch's operators where the gradient is to be differentiated again, carries
+    a tangent or is traced, and where the kernel cannot read the gradients: batches of gradients (is_grads_batched) and
+    other tensors without memory of their own, whose address the kernel's binding asks for before it launches anything."""
+    if torch.is_grad_enabled() or not eager_call():
+        return composition(*grads)
+    try:
+        return kernel(*grads)
+    except RuntimeError:
+        if all(type(g) is torch.Tensor and not _is_batched(g) for g in grads):
+            raise
+    return composition(*grads)
 
 
 def splits_tokens(tokens, M, N, with_bias, fp32):

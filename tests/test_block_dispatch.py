@@ -233,12 +233,6 @@ def test_shapes_that_torch_refuses_stay_refused(name, other, only_shapes_decide)
         _features_call(name, **{**FULL[name], **other})
 
 
-def test_heads_that_do_not_divide_the_channels_are_not_taken(monkeypatch):
-    monkeypatch.setattr(features, "plain_tensors", lambda *a: True)
-    x = _on_gpu(torch.zeros(1, 1, 136).half())
-    assert features._takes(17, 136, 1, x) and not features._takes(16, 136, 1, x)  # 136 // 16 is one whole piece
-
-
 @pytest.mark.parametrize("name", sorted(BLOCKS))
 def test_blocks_in_torch_mode_can_be_traced(name):
     """torch.jit.trace of a block that trains, and torch.fx where the block's own code allows it, see the projections as the
@@ -273,18 +267,21 @@ def test_traced_and_watched_calls_are_not_plain():
 
 
 def _cpu_kernels(monkeypatch):
-    """The forward kernels by their formulas; a gradient kernel fails the test."""
-    F, n = nn.functional, features
+    """The forward kernels by their formulas; a gradient kernel asks for its tensors' addresses and fails the test."""
+    n = features
+
+    def read(*args):
+        addresses = [t.data_ptr() for t in args if torch.is_tensor(t)]
+        pytest.fail(f"a kernel read what it cannot: {addresses}")
     for name, formula in (("polarity_fwd", lambda *a: n.polarity_formula(*a)[:4]), ("focus_fwd", lambda *a: n.focus_formula(*a)[:3]),
                           ("rotary_fwd", lambda qk, x, rot, heads: n.rotary_formula(qk, x, rot, rot.shape[0], heads)[:5]),
                           ("turn_fwd", n.turn_formula), ("merge_fwd", lambda *a: n.merge_formula(*a)[0]),
                           ("interpolate_fwd", lambda *a: n.interpolate_formula(*a)[0]),
-                          ("dwconv_fwd", lambda x, w, b, H, W: depthwise._convolution_of_images(
-                              x, H, W, w.shape[0], lambda i: F.conv2d(i, w, b, padding=1, groups=w.shape[0])))):
+                          ("dwconv_fwd", lambda x, w, b, H, W, flip=False: read(x) if flip else _conv_formula(x, w, b, H, W))):
         monkeypatch.setattr(_hip, name, formula)
     for name in ("polarity_bwd", "focus_bwd", "rotary_bwd", "turn_bwd", "merge_bwd", "interpolate_bwd", "dwconv_grad",
                  "linear_wgrad"):
-        monkeypatch.setattr(_hip, name, lambda *a: pytest.fail("a kernel was given what it cannot read"))
+        monkeypatch.setattr(_hip, name, read)
 
 
 def _conv_formula(x, w, b, H, W):
@@ -388,3 +385,17 @@ def test_focusing_factors_that_are_not_the_number_three_run_as_torch_operators(f
         assert torch.autograd.grad(out[0].sum(), factor)[0] != 0
     with pytest.raises(only_shapes_decide):
         features.focused_features(q, kv, pe, scale, HEADS, 3.0)
+
+
+def test_composed_gradients_stop_at_their_inputs():
+    """One input made of another: the gradient of the step is composed without walking from one to the other (whose
+    nodes would run twice)."""
+    seen = []
+    a = torch.rand(2, HEADS, ROWS, 8, requires_grad=True)
+    o = a * 1
+    o.register_hook(lambda g: seen.append(1))
+    local = torch.rand(2, ROWS, DIM, requires_grad=True)
+    gate = (o * 2).transpose(1, 2).reshape(2, ROWS, DIM)
+    grads = features.differentiable_gradients(features.merge_formula, (o, None, local, gate), (torch.ones(2, ROWS, DIM),))
+    assert not seen and [g is None for g in grads] == [False, True, False, False]
+    assert torch.equal(grads[0], features.split_heads(gate, HEADS).detach())

@@ -10,7 +10,7 @@ import pytest
 import torch
 
 from helpers import UNIT_ROUNDOFF
-from flash_bla.layers import MambaLikeLinearAttention, PolaLinearAttention
+from flash_bla.layers import FocusedLinearAttention, MambaLikeLinearAttention, PolaLinearAttention
 from flash_bla.layers import _features as features
 
 DTYPES = [torch.float16, torch.bfloat16, torch.float32]
@@ -227,3 +227,28 @@ def test_gradient_of_the_gradient():
         results.append(torch.autograd.grad(sum(x.square().sum() for x in g), t))
     for a, b in zip(*results):
         torch.testing.assert_close(a, b)
+
+
+@pytest.mark.gpu
+def test_heads_that_do_not_divide_the_channels_are_not_taken():
+    x = torch.zeros(1, 1, 136, device="cuda").half()
+    assert features._takes(17, 136, 1, x) and not features._takes(16, 136, 1, x)  # 136 // 16 is one whole piece
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["mlla", "pola", "focused"])
+def test_batches_of_gradients(name):
+    """is_grads_batched through what follows the attention, where the kernels find no addresses: as one by one."""
+    torch.manual_seed(0)
+    block, extra = {"mlla": (MambaLikeLinearAttention(64, (4, 4), 2), ()), "pola": (PolaLinearAttention(64, 16, num_heads=2), (4, 4)),
+                    "focused": (FocusedLinearAttention(64, 16, num_heads=2), (4, 4))}[name]
+    block = block.cuda()
+    x = torch.randn(2, 16, 64, device="cuda")
+    wanted = [p for n, p in block.named_parameters() if n.startswith(("proj", "dwc", "lepe"))]
+    y = block(x, *extra)
+    g = torch.randn(3, *y.shape, device="cuda")
+    batched = torch.autograd.grad(y, wanted, g, is_grads_batched=True, retain_graph=True)
+    for i in range(3):
+        for a, b in zip(batched, torch.autograd.grad(y, wanted, g[i], retain_graph=True)):
+            # fp32 sums of 32 products in another order
+            assert (a[i] - b).abs().max() <= 2.0 ** -20 * b.abs().max()
