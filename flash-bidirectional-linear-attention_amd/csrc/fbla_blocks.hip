@@ -11,7 +11,7 @@
 // All of it is elementwise on token rows and bound by HBM: a lane owns 16 bytes of channels of one token (the next lanes the
 // next channels), everything is computed from them in fp32 and rounded once, and nothing between the projection's rows and the
 // operator's heads is written.  Training steps with torch operators in their place and with these: polarity (64 x 28x28 x
-// 256, bf16) 2.77 -> 0.83 ms, of it here 50 us features (257 MB, 5.1 TB/s), 77 + 9 us their gradients (385 MB, 5.0 TB/s), 19 + 33
+// 256, bf16) 2.77 -> 0.83 ms, of it here 50 us features (257 MB, 5.1 TB/s), 75 + 9 us their gradients (385 MB, 5.1 TB/s), 19 + 33
 // us the merge; rotary (64 x 56x56 x 64) 0.83 -> 0.48 ms, of it 33 us features (205 MB, 6.2 TB/s), 45 us gradients (283 MB, 6.3
 // TB/s).
 #include <hip/hip_runtime.h>
@@ -622,7 +622,8 @@ __device__ __forceinline__ float row_max(float v, int lanes) {
 // focused features (layers/focused_la.py:56-74)
 // ---------------------------------------------------------------------------------------------------------------
 // t = (relu(x) + 1e-6) / scale; the feature is t^3 brought to t's length over all channels of the token.  With s = t times
-// the power of two that brings max t to [0.5, 1) (exact, and nothing under- or overflows) and n = |s|, m = |s^3|: feature = s^3 |t| / m, and for its gradient g, G = sum g s^3:
+// the power of two that brings max t to [0.5, 1) (exact, and nothing under- or overflows) and n = |s|, m = |s^3|:
+// feature = s^3 |t| / m, and for its gradient g, G = sum g s^3:
 // dt = 3 n s^2 g / m + G (s / (n m) - 3 n s^5 / m^3).
 // 64 x 28x28 x 256, bf16: 38 us (154 MB, 4 TB/s) and 83 + 9 us (231 MB, 2.8 TB/s); torch's operators 279 and 851 us.
 // Rows of workgroup [0, q_wgs): the queries, the others the keys with the values beside them.

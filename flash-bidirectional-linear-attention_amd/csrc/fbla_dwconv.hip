@@ -35,7 +35,7 @@ template <typename T> struct Lane {
 };
 
 // What the products of one output are added in: 64 bits for fp32 (as torch's convolution adds them; in 32 bits a result is
-// 9.1e-8 from exact at 5x5, so it is 2.5e-8), 32 for 16-bit types.
+// 9.1e-8 from exact at 5x5, so it is 2.5e-8; 64 x 28x28 x 256 32 and 39 us), 32 for 16-bit types.
 template <typename T> using Sum = std::conditional_t<sizeof(T) == 4, double, float>;
 __device__ __forceinline__ float mul_add(float a, float b, float c) { return fmaf(a, b, c); }
 __device__ __forceinline__ double mul_add(double a, double b, double c) { return fma(a, b, c); }
