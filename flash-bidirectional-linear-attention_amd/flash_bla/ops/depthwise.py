@@ -50,13 +50,14 @@ def runs_on_tokens(x, conv):
     without hooks."""
     K = conv.kernel_size[0]
     w, bias = conv.weight, conv.bias
+    Cw = w.shape[0]
     return (untouched(conv, nn.Conv2d) and plain_tensors(x, w, bias) and x.is_cuda and x.numel() > 0 and
             x.dtype in (torch.float16, torch.bfloat16, torch.float32) and w.dtype == x.dtype and w.device == x.device and
-            (bias is None or bias.dtype == x.dtype and bias.device == x.device and bias.shape == w.shape[:1]) and
-            conv.kernel_size == (K, K) and w.shape[2:] == (K, K) and K in (3, 5, 7) and
+            (bias is None or bias.dtype == x.dtype and bias.device == x.device and bias.numel() == Cw) and
+            K in (3, 5, 7) and conv.kernel_size == (K, K) and w.shape == (Cw, 1, K, K) and
             conv.padding == (K // 2, K // 2) and conv.padding_mode == 'zeros' and conv.stride == (1, 1) and
-            conv.dilation == (1, 1) and conv.groups == w.shape[0] and w.shape[1] == 1 and
-            x.shape[-1] % w.shape[0] == 0 and x.shape[-1] % (16 // x.element_size()) == 0)
+            conv.dilation == (1, 1) and conv.groups == Cw and
+            x.shape[-1] % Cw == 0 and x.shape[-1] % (16 // x.element_size()) == 0)
 
 
 def depthwise_conv_tokens(x, conv, H, W):
