@@ -2496,13 +2496,28 @@ static int chunk_for(const Prob& p, int wgs_per_cu, int rounds, int min_chunk, i
   return (int)chunk;
 }
 
+// Shortest chunk of a reduction kernel (`chunk` tokens, halved down to `least`): a problem of few heads that would leave
+// most CUs without a workgroup is cut finer, since a workgroup's time is then its own chain of loads.  Up to 64 workgroups
+// are halved: 128 gained nothing more (B4-H8-T1024-D64 fp16 17.6 us either way).  The partials stay below 8 MiB.  Forward /
+// backward, us: B2-H4-T1024-D64 fp32 19.0 / 28.3 -> 17.3 / 25.8, fp16 14.1 / 18.3 -> 13.0 / 16.2 (partials summed by the reduce
+// kernel, see fold_reduce), B1-H2-T1024-D128 fp32 42.7 / 64.3 -> 30.9 / 50.1, fp16 25.2 / 45.1 -> 22.3 / 27.7.
+static int least_chunk(const Prob& p, int chunk, int least) {
+  static const int few = knob("FBLA_LEAST_WGS", 64);
+  const int64_t nh = (int64_t)p.N * p.H, slot = ((int64_t)p.DK * p.DV + p.DK) * (int64_t)sizeof(float);
+  while (chunk / 2 >= least && nh * cdiv64(p.L, chunk) < few && nh * cdiv64(p.L, chunk / 2) * slot <= 8 << 20) chunk /= 2;
+  return chunk;
+}
+// (one chunk a head stays one: the kernel then stores the finished state itself, B2-H4-T256-D64 fp16 forward 10.4 us, with
+// two chunks and a reduce launch 12.8)
+static int least_state_chunk(const Prob& p) { return p.L > 256 ? least_chunk(p, 256, 64) : 256; }
+
 // Reduction kernels (state, backward pass A): one round of resident workgroups.
 // 128 x 128 states of the plain operator: state128_kernel, two workgroups per CU.
 static int whole_state_chunk(const Prob& p) {
   static const int on = knob("FBLA_STATE128", 1);  // 2 = off (A/B comparisons)
   if (on != 1 || tiled_dim(p.DK) != 128 || tiled_dim(p.DV) != 128 || (p.flags & kDecoupled)) return 0;
   if (p.cu && p.H > 65536) return 0;  // 32-bit lane offsets
-  return chunk_for(p, 2, 1, 256, 64, true);
+  return chunk_for(p, 2, 1, least_state_chunk(p), 64, true);
 }
 
 // Dense heads short enough for one workgroup each: the state kernel stores the finished sums itself (no
@@ -2522,15 +2537,15 @@ int state_chunk(const Prob& p, bool block_stats) {
     if (direct) return direct;
   }
   const int whole = block_stats && padded(p) ? 0 : whole_state_chunk(p);
-  return whole ? whole : chunk_for(p, per_cu, 1, 256, 64, true);
+  return whole ? whole : chunk_for(p, per_cu, 1, block_stats ? 256 : least_state_chunk(p), 64, true);
 }
 
 int bwd_a_chunk(const Prob& p) {
   static const int per_cu = knob("FBLA_BWDA_WGS_PER_CU", 2);
 
   // 128 x 128: two workgroups of four waves per CU, steps of 64 tokens
-  if (tiled_dim(p.DK) == 128 || tiled_dim(p.DV) == 128) return chunk_for(p, 2, 1, 512, 64, true);
-  return chunk_for(p, per_cu, 1, 256, 128, true);
+  if (tiled_dim(p.DK) == 128 || tiled_dim(p.DV) == 128) return chunk_for(p, 2, 1, least_chunk(p, 512, 128), 64, true);
+  return chunk_for(p, per_cu, 1, least_chunk(p, 256, 128), 128, true);
 }
 
 static bool use_rows128(const Prob& p);

@@ -98,7 +98,10 @@ static bool fold_reduce(const Prob& p, int reduce_nchunks, int DR, int DC) {
   const double extra = (double)p.N * p.H * (double)(rows_nchunks - 1) * reduce_nchunks *
                        ((double)p.DK * p.DV + p.DK) * sizeof(float);
   static const double limit = tuning_knob("FBLA_FOLD_MAX_MB", 16) * 1e6;
-  return extra <= limit;
+  // Nor do the partials of one head exceed what a prologue reads in less than a launch takes: four of 64 x 64 (B2-H4-T1024
+  // fp16 with eight: forward 16.8 us folded, 13.0 reduced; B1-H2-T1024-D128 with eight: 36.2, 22.3).
+  static const double each = tuning_knob("FBLA_FOLD_EACH_KB", 70) * 1024.0;
+  return extra <= limit && reduce_nchunks * ((double)p.DK * p.DV + p.DK) * sizeof(float) <= each;
 }
 
 // the walking order of a packed batch with too many sequences to rank inside every workgroup
