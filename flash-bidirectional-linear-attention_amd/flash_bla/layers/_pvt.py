@@ -27,11 +27,11 @@ class PvtLinearAttentionBase(nn.Module):
         self.positional_encoding = nn.Parameter(torch.zeros(1, num_patches // (sr_ratio * sr_ratio), dim))
         return head_dim
 
-    def _joint_keys_values(self, x, H, W):
+    def _reduced(self, x, H, W):
+        """The rows that keys and values are made of, None where they are x itself."""
         B, N, C = x.shape
         if self.sr_ratio > 1:
-            x = self.norm(self.sr(x.transpose(1, 2).reshape(B, C, H, W)).flatten(2).transpose(1, 2))
-        return project(self.kv, x)
+            return self.norm(self.sr(x.transpose(1, 2).reshape(B, C, H, W)).flatten(2).transpose(1, 2))
 
     def _value_conv(self, v, N, H, W):
         """v: (B, heads, n, d) -> depth-wise conv on the H x W grid -> (B, N, C)."""

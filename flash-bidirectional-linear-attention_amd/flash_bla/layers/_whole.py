@@ -1,0 +1,238 @@
+"""Blocks as one native call a direction (csrc/fbla_torch.cpp).
+
+Issued step by step from Python, a block's training step on few tokens is bound by the host: every projection, feature map,
+operator and merge is a node of the autograd graph with its checks, its Python calls and its bookkeeping.  Where nothing
+looks between the steps - an ordinary eager call of the block's own class on plain modules, without hooks, of the shapes that
+all its fused steps take - the block is one node instead, whose forward and backward issue the same kernels in the same
+order.  Everything else runs step by step (`_steps` of the block), and so does a gradient that is to be differentiated again or
+that the kernels cannot read: it is composed by running the steps again on the node's inputs.
+
+Host time of a forward / a training step before (steps from Python through ctypes) and here, us, on a host in whose slower
+state a node of the graph that does nothing costs 63 us (33 in the other): mlla 107 / 301 -> 55 / 229, pola 195 / 614 -> 134 /
+470, with spatial reduction 352 / 1160 -> 250 / 940, focused 159 / 600 -> 106 / 445 (2 x 14x14 x 64 bf16), linfusion 245 / 1010 ->
+234 / 815 (1 x 16x16 x 320 fp16); what is left is the library's GEMM calls (17 us each, a launch of this package 4) and the graph.
+"""
+import contextlib
+
+import torch
+import torch.nn as nn
+from torch._C import _functorch
+from torch._functorch.pyfunctorch import temporarily_clear_interpreter_stack
+from torch.func import functional_call
+from torch.nn.modules.module import _has_any_global_hook
+
+from flash_bla import _hip
+from flash_bla.ops.projection import eager_call, gradient_of, splits_tokens
+
+
+class _Steps(nn.Module):
+    """A block's steps as a module of their own, for functional_call."""
+
+    def __init__(self, block):
+        super().__init__()
+        self.block = block
+
+    def forward(self, *args):
+        return self.block._steps(*args)
+
+
+def _batch_of(g):
+    """A batch of gradients (is_grads_batched, torch.func.vmap) as an ordinary tensor with the batch first, what wraps results
+    like it, and a context in which ordinary tensors are no more than that; None for any other gradient."""
+    if _functorch.is_legacy_batchedtensor(g):
+        values = torch._remove_batch_dim(g, 1, 1, 0)  # (batched at another level, it stays a batch)
+        if not _functorch.is_legacy_batchedtensor(values):
+            return values, lambda t: torch._add_batch_dim(t, 0, 1), contextlib.nullcontext
+    elif _functorch.is_batchedtensor(g):
+        level, values = _functorch.maybe_get_level(g), _functorch.get_unwrapped(g).movedim(_functorch.maybe_get_bdim(g), 0)
+        if not _functorch.is_functorch_wrapped_tensor(values):
+            return values, lambda t: _functorch._add_batch_dim(t, 0, level), temporarily_clear_interpreter_stack
+    return None
+
+
+class WholeBlockFunction(torch.autograd.Function):
+    """call: the block's native pair (below); inputs: its rows and parameters, some of them None."""
+
+    @staticmethod
+    def forward(ctx, call, *inputs):
+        ctx.call = call
+        out, *saved = call.run(inputs)
+        ctx.save_for_backward(*inputs, *saved)
+        return out
+
+    @staticmethod
+    def backward(ctx, g):
+        call, tensors = ctx.call, ctx.saved_tensors
+        n = len(call.names)
+        inputs, saved, need = tensors[:n], tensors[n:], ctx.needs_input_grad[1:]
+
+        def composed(g):
+            batch = None if torch.is_grad_enabled() else _batch_of(g)
+            if batch is not None:  # (the node has to give all its gradients, and the operators' kernels take one at a time)
+                values, wrapped, ordinary = batch
+                with ordinary():
+                    each = [call.run_backward(e, inputs, saved, need) for e in values.unbind()]
+                    stacked = [None if t[0] is None else torch.stack(t) for t in zip(*each)]
+                return [None if t is None else wrapped(t) for t in stacked]
+            with torch.enable_grad():  # (through aliases: the inputs may depend on one another)
+                aliases = [t.view_as(t) if t is not None and t.requires_grad else t for t in inputs]
+                rows = [a for a, name in zip(aliases, call.names) if name is None]
+                state = {"block." + name: a for a, name in zip(aliases, call.names) if name is not None and a is not None}
+                out = functional_call(_Steps(call.block), state, (*rows, *call.extra))
+            wanted = [a for a, wants in zip(aliases, need) if wants]
+            got = iter(torch.autograd.grad(out, wanted, g, create_graph=torch.is_grad_enabled(), allow_unused=True))
+            return [next(got) if wants else None for wants in need]
+        return (None, *gradient_of(lambda g: call.run_backward(g, inputs, saved, need), composed, g))
+
+
+def _run(call, inputs):
+    if torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in inputs):
+        return WholeBlockFunction.apply(call, *inputs)
+    return call.run(inputs)[0]
+
+
+def _ordinary(block, kind, x, modules):
+    """An eager call of the block's own class on GPU rows, nothing around or in place of its modules' forwards."""
+    return (type(x) is torch.Tensor and x.is_cuda and x.ndim == 3 and type(block) is kind and not torch.is_autocast_enabled() and
+            eager_call() and not _has_any_global_hook() and _hip.untouched_modules(modules))
+
+
+def _same_convolution(conv):
+    """Stride 1 and "same" zero padding; the filter's shape is compared natively."""
+    K = conv.kernel_size[0]
+    return (conv.kernel_size == (K, K) and conv.padding == (K // 2, K // 2) and conv.padding_mode == 'zeros' and
+            conv.stride == (1, 1) and conv.dilation == (1, 1) and conv.groups == conv.in_channels)
+
+
+def _splits(rows, weight, bias):
+    """Whether a projection's weight gradient is the token-splitting kernel's."""
+    return splits_tokens(rows.numel() // rows.shape[-1], *weight.shape, bias is not None, rows.dtype == torch.float32)
+
+
+class _Mlla:
+    names = (None, "qk.weight", "qk.bias", "lepe.weight", "lepe.bias")
+
+    def __init__(self, block, rotations, side):
+        self.block, self.rotations, self.side, self.extra = block, rotations, side, (True,)
+
+    def run(self, inputs):
+        return _hip.mlla_fwd(inputs[0], inputs[1:], self.rotations, self.side, self.block.num_heads)
+
+    def run_backward(self, g, inputs, saved, need):
+        x, w, b, conv_w, _ = inputs
+        return _hip.mlla_bwd(g, x, w, conv_w, self.rotations, saved, self.side, self.block.num_heads, need, _splits(x, w, b))
+
+
+def mlla(block, kind, rope, x):
+    """The block's output, or None where it is not to run whole."""
+    if not _ordinary(block, kind, x, [(block.qk, nn.Linear), (block.lepe, nn.Conv2d), (block.rope, rope)]):
+        return None
+    side, rotations = int(x.shape[1] ** 0.5), block.rope.rotations
+    params = (block.qk.weight, block.qk.bias, block.lepe.weight, block.lepe.bias)
+    if not (type(rotations) is torch.Tensor and _hip.plain_gpu_tensors(x, *params) and _same_convolution(block.lepe) and
+            _hip.mlla_fits(x, params, rotations, side, block.num_heads)):
+        return None
+    return _run(_Mlla(block, rotations, side), (x, *params))
+
+
+class _Pvt:
+    """PolaFormer's and FLatten's blocks: x, the rows of keys and values (None: x), parameters by name."""
+    def __init__(self, block, H, W):
+        self.block, self.H, self.W, self.extra = block, H, W, (H, W, True)
+
+    def _split(self, inputs, saved):
+        x, src, *p = inputs
+        q_w, q_b, kv_w, kv_b = p[:4]
+        return _splits(x, q_w, q_b), _splits(x if src is None else src, kv_w, kv_b), _splits(x, p[-2], p[-1])
+
+
+class _Pola(_Pvt):
+    names = (None, None, "qg.weight", "qg.bias", "kv.weight", "kv.bias", "positional_encoding", "scale", "power", "dwc.weight",
+             "dwc.bias", "proj.weight", "proj.bias")
+
+    def run(self, inputs):
+        x, src, *p = inputs
+        return _hip.pola_fwd(x, x if src is None else src, p, self.block.alpha, self.H, self.W, self.block.num_heads)
+
+    def run_backward(self, g, inputs, saved, need):
+        x, src, *p = inputs
+        return _hip.pola_bwd(g, x, x if src is None else src, src is None, p, saved, self.block.alpha, self.H, self.W,
+                             self.block.num_heads, need, self._split(inputs, saved))
+
+
+class _Focused(_Pvt):
+    names = (None, None, "q.weight", "q.bias", "kv.weight", "kv.bias", "positional_encoding", "scale", "dwc.weight", "dwc.bias",
+             "proj.weight", "proj.bias")
+
+    def run(self, inputs):
+        x, src, *p = inputs
+        return _hip.focused_fwd(x, x if src is None else src, p, self.H, self.W, self.block.num_heads)
+
+    def run_backward(self, g, inputs, saved, need):
+        x, src, *p = inputs
+        return _hip.focused_bwd(g, x, x if src is None else src, src is None, p, saved, self.H, self.W, self.block.num_heads, need,
+                                self._split(inputs, saved))
+
+
+def _pvt(call, fits, query, params, x, src):
+    block, H, W = call.block, call.H, call.W
+    if not (type(H) is int and type(W) is int and (src is None or type(src) is torch.Tensor) and
+            _hip.plain_gpu_tensors(x, src, *params) and _same_convolution(block.dwc) and
+            fits(x, x if src is None else src, params, H, W, block.num_heads)):
+        return None
+    return _run(call, (x, src, *params))
+
+
+def pola(block, kind, x, src, H, W):
+    if not (type(block.alpha) in (int, float) and block.alpha >= 0 and _ordinary(block, kind, x, [
+            (block.qg, nn.Linear), (block.kv, nn.Linear), (block.proj, nn.Linear), (block.dwc, nn.Conv2d)])):
+        return None
+    return _pvt(_Pola(block, H, W), _hip.pola_fits, block.qg, (
+        block.qg.weight, block.qg.bias, block.kv.weight, block.kv.bias, block.positional_encoding, block.scale, block.power,
+        block.dwc.weight, block.dwc.bias, block.proj.weight, block.proj.bias), x, src)
+
+
+def focused(block, kind, x, src, H, W):
+    factor = block.focusing_factor
+    if not (type(factor) in (int, float) and factor == 3 and _ordinary(block, kind, x, [
+            (block.q, nn.Linear), (block.kv, nn.Linear), (block.proj, nn.Linear), (block.dwc, nn.Conv2d)])):
+        return None
+    return _pvt(_Focused(block, H, W), _hip.focused_fits, block.q, (
+        block.q.weight, block.q.bias, block.kv.weight, block.kv.bias, block.positional_encoding, block.scale, block.dwc.weight,
+        block.dwc.bias, block.proj.weight, block.proj.bias), x, src)
+
+
+class _LinFusion:
+    names = (None, *(f"to_{p}_.{layer}.{n}" for p in "qk" for layer in (0, 1, 3) for n in ("weight", "bias")),
+             *(f"to_{p}.{n}" for p in "qkv" for n in ("weight", "bias")), "to_out.0.weight", "to_out.0.bias")
+
+    def __init__(self, block, cu):
+        self.block, self.cu, self.extra = block, cu, ()
+        self.slope = tuple(path[2].negative_slope for path in (block.to_q_, block.to_k_))
+
+    def run(self, inputs):
+        eps = tuple(path[1].eps for path in (self.block.to_q_, self.block.to_k_))
+        return _hip.linfusion_fwd(inputs[0], self.cu, inputs[1:], eps, self.slope, self.block.heads)
+
+    def run_backward(self, g, inputs, saved, need):
+        x, *p = inputs
+        split = [_splits(x, p[i], p[i + 1]) for i in (0, 4, 6, 10, 12, 14, 16, 18)]
+        return _hip.linfusion_bwd(g, x, self.cu, p, saved, self.slope, need, split)
+
+
+def linfusion(block, kind, x, cu):
+    """cu(): the packed batch's offsets."""
+    paths = (block.to_q_, block.to_k_)
+    if type(x) is not torch.Tensor or not x.is_cuda or not all(type(p) is nn.Sequential and len(p) == 4 for p in paths):
+        return None
+    projections = (block.to_q, block.to_k, block.to_v, block.to_out[0])
+    kinds = (nn.Linear, nn.LayerNorm, nn.LeakyReLU, nn.Linear)
+    if not _ordinary(block, kind, x, [(p, nn.Sequential) for p in paths] + [m for p in paths for m in zip(p, kinds)] +
+                     [(m, nn.Linear) for m in projections]):
+        return None
+    params = [t for p in paths for i in (0, 1, 3) for t in (p[i].weight, p[i].bias)]
+    params += [t for m in projections for t in (m.weight, m.bias)]
+    if not (_hip.plain_gpu_tensors(x, *params) and all(len(p[1].normalized_shape) == 1 and p[1].normalized_shape[0] == p[0].out_features
+                                                       for p in paths) and _hip.linfusion_fits(x, params, block.heads)):
+        return None
+    return _run(_LinFusion(block, cu()), (x, *params))

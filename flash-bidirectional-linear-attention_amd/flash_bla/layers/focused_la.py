@@ -2,6 +2,7 @@
 import torch.nn as nn
 import torch.nn.functional as F
 
+from flash_bla.layers import _whole
 from flash_bla.layers._common import check_mode, merge_heads, torch_linear_attention
 from flash_bla.layers._features import focus_formula, focused_features, merge_heads_with
 from flash_bla.layers._pvt import PvtLinearAttentionBase
@@ -19,8 +20,13 @@ class FocusedLinearAttention(PvtLinearAttentionBase):
 
     def forward(self, x, H, W, mode='triton'):
         fast = check_mode(mode)
+        src = self._reduced(x, H, W)
+        out = _whole.focused(self, FocusedLinearAttention, x, src, H, W) if fast else None
+        return self.proj_drop(self._steps(x, src, H, W, fast) if out is None else out)
+
+    def _steps(self, x, src, H, W, fast):
         N = x.shape[1]
-        kv = self._joint_keys_values(x, H, W)
+        kv = project(self.kv, x if src is None else src)
         features = focused_features if fast else focus_formula
         q, k, v, v_rows = features(project(self.q, x), kv, self.positional_encoding, F.softplus(self.scale),
                                    self.num_heads, self.focusing_factor)
@@ -28,4 +34,4 @@ class FocusedLinearAttention(PvtLinearAttentionBase):
             out = merge_heads_with(linear_attention(q, k, v), None, self._value_conv_tokens(v_rows, N, H, W))
         else:
             out = merge_heads(torch_linear_attention(q, k, v)) + self._value_conv(v, N, H, W)
-        return self.proj_drop(project(self.proj, out))
+        return project(self.proj, out)

@@ -10,6 +10,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from flash_bla.layers import _whole
 from flash_bla.layers._common import check_mode, torch_linear_attention
 from flash_bla.ops._check import untouched
 from flash_bla.ops.linear_attn.fused import linear_attention
@@ -76,6 +77,14 @@ class GeneralizedLinearAttention(nn.Module):
 
     def forward(self, hidden_states, encoder_hidden_states=None, attention_mask=None, mode='triton', **kwargs):
         fast = check_mode(mode)
+        if fast and encoder_hidden_states is None:
+            out = _whole.linfusion(self, GeneralizedLinearAttention, hidden_states,
+                                   lambda: _equal_cu_seqlens(*hidden_states.shape[:2], hidden_states.device))
+            if out is not None:
+                return self.to_out[1](out)
+        return self.to_out[1](self._steps(hidden_states, encoder_hidden_states, fast))
+
+    def _steps(self, hidden_states, encoder_hidden_states=None, fast=True):
         context = hidden_states if encoder_hidden_states is None else encoder_hidden_states
         q = project(self.to_q, hidden_states + project_through(self.to_q_, hidden_states))
         k = project(self.to_k, context + project_through(self.to_k_, context))
@@ -90,7 +99,7 @@ class GeneralizedLinearAttention(nn.Module):
             packed = [t.reshape(b * n, self.heads, -1) for t in (q, k, v)]
             out = varlen_linear_attention(*packed, _equal_cu_seqlens(b, n, q.device), n, eps=1e-4,
                                           feature_map="elu+1")
-            return self.to_out[1](project(self.to_out[0], out.reshape(b, n, -1)))
+            return project(self.to_out[0], out.reshape(b, n, -1))
         q, k, v = (self.head_to_batch_dim(t) for t in (q, k, v))
         if fast:
             b = hidden_states.shape[0]
@@ -100,4 +109,4 @@ class GeneralizedLinearAttention(nn.Module):
             q, k = F.elu(q) + 1.0, F.elu(k) + 1.0
             out = torch_linear_attention(q, k, v, eps=1e-4)
         out = self.batch_to_head_dim(out)
-        return self.to_out[1](project(self.to_out[0], out))
+        return project(self.to_out[0], out)

@@ -3,6 +3,7 @@ elu+1 features, 2-D rotary numerator features, depth-wise conv positional term."
 import torch
 import torch.nn as nn
 
+from flash_bla.layers import _whole
 from flash_bla.layers._common import check_mode, merge_heads, split_heads, torch_linear_attention
 from flash_bla.layers._features import merge_heads_with, rotary_features, rotate
 from flash_bla.ops._check import untouched
@@ -41,6 +42,10 @@ class MambaLikeLinearAttention(nn.Module):
 
     def forward(self, x, mode='triton'):
         fast = check_mode(mode)
+        out = _whole.mlla(self, MambaLikeLinearAttention, RoPE, x) if fast else None
+        return self._steps(x, fast) if out is None else out
+
+    def _steps(self, x, fast):
         b, n, c = x.shape
         side = int(n ** 0.5)
         qk = project(self.qk, x)

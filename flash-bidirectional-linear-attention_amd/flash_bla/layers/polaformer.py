@@ -6,6 +6,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from flash_bla.layers import _whole
 from flash_bla.layers._common import check_mode, merge_heads, torch_linear_attention
 from flash_bla.layers._features import merge_heads_with, polarity_features, polarity_formula
 from flash_bla.layers._pvt import PvtLinearAttentionBase
@@ -25,13 +26,18 @@ class PolaLinearAttention(PvtLinearAttentionBase):
 
     def forward(self, x, H, W, mode='triton'):
         fast = check_mode(mode)
+        src = self._reduced(x, H, W)
+        out = _whole.pola(self, PolaLinearAttention, x, src, H, W) if fast else None
+        return self.proj_drop(self._steps(x, src, H, W, fast) if out is None else out)
+
+    def _steps(self, x, src, H, W, fast):
         N = x.shape[1]
         scale = F.softplus(self.scale)
         power = 1 + self.alpha * torch.sigmoid(self.power)
         # (the kernels know powers of at least 1)
         rising = isinstance(self.alpha, (int, float)) and self.alpha >= 0
         features = polarity_features if fast and rising else polarity_formula
-        q_same, q_opp, k_both, v, v_rows, gate = features(project(self.qg, x), self._joint_keys_values(x, H, W),
+        q_same, q_opp, k_both, v, v_rows, gate = features(project(self.qg, x), project(self.kv, x if src is None else src),
                                                           self.positional_encoding, scale, power, self.num_heads)
         if fast:  # both pairings on one state pass over the shared keys and values
             o_same, o_opp = paired_linear_attention(q_same, q_opp, k_both, v)
@@ -41,4 +47,4 @@ class PolaLinearAttention(PvtLinearAttentionBase):
             out = torch.cat([torch_linear_attention(q_same, k_both, v_same),
                              torch_linear_attention(q_opp, k_both, v_opp)], dim=-1)
             out = (merge_heads(out) + self._value_conv(v, N, H, W)) * gate
-        return self.proj_drop(project(self.proj, out))
+        return project(self.proj, out)

@@ -2,10 +2,14 @@
 import torch
 from torch.nn.modules.module import _has_any_global_hook
 
+from flash_bla import _hip
+
 
 def check_dense(name, q, k, v, extra=()):
     """The reference's dense wrappers validate nothing (linear_attn/fused.py:456-480);
-    the HIP kernels index raw memory, so shapes, dtypes and devices are checked here."""
+    the HIP kernels index raw memory, so shapes, dtypes and devices are checked here (one native look, then what is wrong)."""
+    if len(extra) in (0, 2) and _hip.dense_operands(q, k, v, *(extra or (None, None))):
+        return
     tensors = (q, k, v) + tuple(extra)
     for t in tensors:
         if not isinstance(t, torch.Tensor) or t.ndim != 4:
