@@ -800,6 +800,73 @@ int fbla_linear_wgrad(const void* g, int64_t g_row, const void* x, int64_t x_row
   return check_launch(what);
 }
 
+int fbla_project(const fbla_projection* jobs, int count, int64_t tokens, int rows_of_w, int dtype, void* stream) {
+  const char* what = "fbla_project";
+  if (!jobs || count < 1 || count > gemm::kMostJobs || tokens < 0) {
+    set_error("%s: bad sizes (count=%d tokens=%lld)", what, count, (long long)tokens);
+    return kErrBadArg;
+  }
+  if (dtype != kF16 && dtype != kBF16) {
+    set_error("%s: fp16 and bf16 only (dtype=%d)", what, dtype);
+    return kErrUnsupported;
+  }
+  if (tokens == 0) return kOk;
+  gemm::Job js[gemm::kMostJobs];
+  int64_t tiles = 0;
+  for (int i = 0; i < count; ++i) {
+    const fbla_projection& j = jobs[i];
+    const int K2 = j.a2 ? j.K2 : 0;
+    // (32-bit offsets into W and into the rows of a tile)
+    if (j.N > 1 << 16 || j.K > 1 << 16 || K2 > 1 << 16 || (int64_t)j.N * (j.K > K2 ? j.K : K2) > 1 << 29 || j.a_row > 1 << 22 ||
+        (j.a2 && j.a2_row > 1 << 22)) {
+      set_error("%s: too many channels (N=%d K=%d K2=%d)", what, j.N, j.K, K2);
+      return kErrUnsupported;
+    }
+    if (!j.a || !j.w || !j.out || (j.a2 && !j.w2) || j.N < 8 || j.K < 8 || (j.a2 && j.K2 < 8) || j.N % 8 || j.K % 8 || K2 % 8) {
+      set_error("%s: null pointers, or channels that are no multiples of 8 (N=%d K=%d K2=%d)", what, j.N, j.K, K2);
+      return kErrBadArg;
+    }
+    if (check_aligned(what, {j.a, j.w, j.a2, j.w2, j.bias, j.add, j.out}) != kOk || check_row_strides(what, j.K, dtype, {j.a_row}) != kOk ||
+        check_row_strides(what, j.N, dtype, {j.out_row}) != kOk || (j.a2 && check_row_strides(what, j.K2, dtype, {j.a2_row}) != kOk) ||
+        (j.add && check_row_strides(what, j.N, dtype, {j.add_row}) != kOk))
+      return kErrBadArg;
+    js[i] = {{j.a, j.a2}, {j.a_row, j.a2_row}, {j.w, j.w2}, {j.K, K2}, j.N, j.bias, j.add, j.add_row, j.out, j.out_row};
+    tiles += (j.N + 63) / 64;
+  }
+  if (tokens > (1LL << 31) || cdiv64(tokens, 64) * tiles > 0x7fffffffLL) {
+    set_error("%s: too many tokens (%lld)", what, (long long)tokens);
+    return kErrUnsupported;
+  }
+  gemm::project(js, count, tokens, rows_of_w != 0, dtype, (hipStream_t)stream);
+  return check_launch(what);
+}
+
+int fbla_norm_leaky(const fbla_norm* jobs, int count, int64_t tokens, int C, int dtype, void* stream) {
+  const char* what = "fbla_norm_leaky";
+  if (!jobs || count < 1 || count > 2 || tokens < 0 || C < 8) {
+    set_error("%s: bad sizes (count=%d tokens=%lld C=%d)", what, count, (long long)tokens, C);
+    return kErrBadArg;
+  }
+  if ((dtype != kF16 && dtype != kBF16) || C % 8 || C > 2048 || tokens > 1LL << 30) {
+    set_error("%s: fp16 and bf16 rows of whole 16-byte pieces, at most 2048 channels (dtype=%d C=%d tokens=%lld)", what, dtype, C,
+              (long long)tokens);
+    return kErrUnsupported;
+  }
+  if (tokens == 0) return kOk;
+  gemm::NormJob js[2];
+  for (int i = 0; i < count; ++i) {
+    const fbla_norm& j = jobs[i];
+    if (!j.x || !j.out || !j.mean != !j.rstd) {
+      set_error("%s: null tensor pointer", what);
+      return kErrBadArg;
+    }
+    if (check_aligned(what, {j.x, j.weight, j.bias, j.out}) != kOk) return kErrBadArg;
+    js[i] = {j.x, j.weight, j.bias, j.out, j.mean, j.rstd, j.eps, j.slope};
+  }
+  gemm::norm_leaky(js, count, tokens, C, dtype, (hipStream_t)stream);
+  return check_launch(what);
+}
+
 static int check_blocks(const char* what, blocks::Shape& s, int64_t B, int64_t N, int64_t Nk, int heads, int d, int unit,
                         int dtype) {
   if (B < 1 || N < 1 || Nk < 1 || heads < 1 || d < 1 || (dtype != kF16 && dtype != kBF16 && dtype != kF32)) {

@@ -235,6 +235,36 @@ void wgrad(const void* g, int64_t g_row, const void* x, int64_t x_row, int64_t t
            float* workspace, int dtype, hipStream_t st);
 }  // namespace linear
 
+// Projections of token rows, 16-bit types (fbla_gemm.hip).
+namespace gemm {
+constexpr int kMostJobs = 3;
+struct Job {
+  // out [tokens][N] = a[0] W[0] + a[1] W[1] (K[1] = 0: the first alone) + bias [N] (or null) + add [tokens][N] (or null);
+  // W as [N][K] or [K][N] rows without gaps; rows of a, add and out a_row, add_row, out_row elements apart.  K, N and the
+  // distances are multiples of 8, all pointers of 16 bytes.
+  const void* a[2];
+  int64_t a_row[2];
+  const void* w[2];
+  int K[2];
+  int N;
+  const void* bias;
+  const void* add;
+  int64_t add_row;
+  void* out;
+  int64_t out_row;
+};
+// rows_of_w: the contraction runs over W's rows ([K][N])
+void project(const Job* jobs, int count, int64_t tokens, bool rows_of_w, int dtype, hipStream_t st);
+// LayerNorm over rows of C channels (a multiple of 8, at most 2048) and LeakyReLU; one or two jobs
+struct NormJob {
+  const void *x, *weight, *bias;  // weight, bias [C] or null
+  void* out;
+  float *mean, *rstd;  // [tokens] or null
+  float eps, slope;
+};
+void norm_leaky(const NormJob* jobs, int count, int64_t tokens, int C, int dtype, hipStream_t st);
+}  // namespace gemm
+
 // Elementwise work of the vision blocks around the attention operators (fbla_blocks.hip).  Rows are [B, N, C] with
 // C = heads * d, joint projections [B, N, 2 C], heads [B, heads, N, width]; all contiguous, d in whole 16-byte pieces.
 namespace blocks {

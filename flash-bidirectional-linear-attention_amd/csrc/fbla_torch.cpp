@@ -33,7 +33,8 @@ using Maybe = std::optional<Tensor>;
   X(fbla_dwconv_grad_workspace_bytes) X(fbla_dwconv_grad) X(fbla_linear_wgrad_workspace_bytes) X(fbla_linear_wgrad)    \
   X(fbla_polarity_fwd) X(fbla_polarity_bwd_workspace_bytes) X(fbla_polarity_bwd) X(fbla_rotary_fwd) X(fbla_rotary_bwd) \
   X(fbla_merge_fwd) X(fbla_merge_bwd) X(fbla_turn_fwd) X(fbla_turn_bwd) X(fbla_focus_fwd)                              \
-  X(fbla_focus_bwd_workspace_bytes) X(fbla_focus_bwd) X(fbla_interpolate_fwd) X(fbla_interpolate_bwd)
+  X(fbla_focus_bwd_workspace_bytes) X(fbla_focus_bwd) X(fbla_interpolate_fwd) X(fbla_interpolate_bwd)                   \
+  X(fbla_project) X(fbla_norm_leaky)
 
 struct Api {
 #define FBLA_MEMBER(f) decltype(&::f) f = nullptr;
@@ -390,6 +391,68 @@ std::pair<Tensor, Tensor> linear_wgrad(const Tensor& g_, const Tensor& x_, bool 
   return {dw, db};
 }
 
+// Projections of rows with one number of tokens, 16-bit types: out = a W^T + bias + add, or (rows_of_w) a W + a2 W2 + add.
+struct Projection {
+  Tensor a, w, bias, add, a2, w2;
+};
+std::vector<Tensor> project(const std::vector<Projection>& p, bool rows_of_w) {
+  TORCH_CHECK(!p.empty() && p.size() <= 3);
+  std::array<fbla_projection, 3> jobs{};
+  std::vector<Tensor> keep, out;
+  auto ready = [&](const Tensor& t) {
+    if (!t.defined()) return t;
+    const Tensor r = token_rows(t);
+    keep.push_back(r);
+    return r;
+  };
+  int64_t tokens = -1;
+  for (size_t i = 0; i < p.size(); ++i) {
+    const Tensor a = ready(p[i].a), a2 = ready(p[i].a2), add = ready(p[i].add), w = whole(p[i].w), w2 = whole(p[i].w2),
+                 bias = whole(p[i].bias);
+    keep.insert(keep.end(), {w, w2, bias});
+    const int64_t N = rows_of_w ? w.size(1) : w.size(0), K = rows_of_w ? w.size(0) : w.size(1);
+    if (tokens < 0) tokens = a.size(0);
+    TORCH_CHECK(a.size(0) == tokens && a.size(1) == K && (!a2.defined() || (a2.size(0) == tokens && a2.size(1) == w2.size(0))) &&
+                (!add.defined() || (add.size(0) == tokens && add.size(1) == N)));
+    std::vector<int64_t> shape = p[i].a.sizes().vec();
+    shape.back() = N;
+    out.push_back(like(a, shape));
+    jobs[i] = {ptr(a), a.stride(0), ptr(w), ptr(a2), a2.defined() ? a2.stride(0) : 0, ptr(w2), ptr(bias), ptr(add),
+               add.defined() ? add.stride(0) : 0, ptr(out[i]), N, (int32_t)N, (int32_t)K, a2.defined() ? (int32_t)a2.size(1) : 0};
+  }
+  const On on(p[0].a);
+  check(api.fbla_project(jobs.data(), p.size(), tokens, rows_of_w, code_of(p[0].a), on.stream), "fbla_project");
+  return out;
+}
+
+// LeakyReLU of LayerNorm over rows, one or two sets of one shape; mean and rstd as torch's LayerNorm saves them
+struct Norm {
+  Tensor x, weight, bias;
+  double eps, slope;
+};
+struct Normed {
+  Tensor y, mean, rstd;
+};
+std::vector<Normed> norm_leaky(const std::vector<Norm>& p, bool with_stats) {
+  TORCH_CHECK(!p.empty() && p.size() <= 2);
+  std::array<fbla_norm, 2> jobs{};
+  std::vector<Tensor> keep;
+  std::vector<Normed> r;
+  const int64_t C = p[0].x.size(-1), tokens = p[0].x.numel() / C;
+  for (size_t i = 0; i < p.size(); ++i) {
+    TORCH_CHECK(p[i].x.sizes() == p[0].x.sizes());
+    const Tensor x = whole(p[i].x), weight = whole(p[i].weight), bias = whole(p[i].bias);
+    keep.insert(keep.end(), {x, weight, bias});
+    std::vector<int64_t> shape = x.sizes().vec();
+    shape.back() = 1;
+    r.push_back({like(x), with_stats ? like_f32(x, shape) : Tensor(), with_stats ? like_f32(x, shape) : Tensor()});
+    jobs[i] = {ptr(x), ptr(weight), ptr(bias), ptr(r[i].y), f32(r[i].mean), f32(r[i].rstd), (float)p[i].eps, (float)p[i].slope};
+  }
+  const On on(p[0].x);
+  check(api.fbla_norm_leaky(jobs.data(), p.size(), tokens, C, code_of(p[0].x), on.stream), "fbla_norm_leaky");
+  return r;
+}
+
 // qg [B,N,2C], kv [B,n,2C], pe [1,n,C], scale [1,1,C], power [1,heads,1,d] -> q_same, q_opp, k_both [B,heads,.,2d], v [B,heads,n,d]
 std::array<Tensor, 4> polarity_fwd(const Tensor& qg_, const Tensor& kv_, const Tensor& pe_, const Tensor& scale_, const Tensor& power_,
                                    int64_t heads) {
@@ -559,11 +622,48 @@ std::array<Tensor, 3> turn_bwd(const Tensor& k_, const Tensor& weight_, const Te
 // Python call and their checks between them.  The gradient of a tensor that two steps read is accumulated by the second
 // step's GEMM instead of a launch of its own (12 us at 200704 x 64 and 50176 x 256 in bf16).
 Tensor flat(const Tensor& t) { return t.reshape({-1, t.size(-1)}); }
-// gradient of x in y = x W^T
-Tensor input_grad(const Tensor& g, const Tensor& w) {
+// Whether `project` takes a projection of these rows rather than torch's GEMM: 16-bit types, unless the product is large enough
+// for the library's deeper pipeline to count.  GPU us of the library / here (bf16, with bias; a call of the library takes the
+// host 17 us, one of ours 4): 200704 x 64 -> 128 24.1 / 21.4, its input gradient 45.9 / 15.8; 50176 x 256 -> 512 33.5 / 31.3; 50176 x
+// 256 -> 256 14.7 / 19.6; 8192 x 640 -> 640 13.4 / 17.4, three of them 40 / 36; 1024 x 1280 -> 1280 11.3 / 14.6; 4096 x 1280 -> 1280 19.9 /
+// 28.8.
+bool projects(const Tensor& x, const Tensor& w) {
+  const double work = (double)(x.numel() / x.size(-1)) * w.numel();
+  return x.element_size() == 2 && (w.size(0) < 512 || w.size(1) < 512 || work <= 4e9);
+}
+// y = x W^T + b (+ add) for one or more projections
+struct Linear {
+  Tensor x, w, b, add;
+};
+std::vector<Tensor> linears(const std::vector<Linear>& p) {
+  bool own = p.size() <= 3;
+  for (const Linear& l : p) own = own && projects(l.x, l.w) && l.x.numel() / l.x.size(-1) == p[0].x.numel() / p[0].x.size(-1);
+  std::vector<Tensor> r;
+  if (own) {
+    std::vector<Projection> jobs;
+    for (const Linear& l : p) jobs.push_back({l.x, l.w, l.b, l.add, Tensor(), Tensor()});
+    return project(jobs, false);
+  }
+  for (const Linear& l : p) {
+    r.push_back(at::linear(l.x, l.w, l.b));
+    if (l.add.defined()) r.back().add_(l.add);
+  }
+  return r;
+}
+std::pair<Tensor, Tensor> two_linears(const Linear& a, const Linear& b) {
+  if (a.x.numel() != b.x.numel()) return {linears({a})[0], linears({b})[0]};
+  const std::vector<Tensor> r = linears({a, b});
+  return {r[0], r[1]};
+}
+Tensor linear(const Tensor& x, const Tensor& w, const Tensor& b) { return linears({{x, w, b, Tensor()}})[0]; }
+// gradient of x in y = x W^T, of x in y = x W^T and y2 = x W2^T, plus `add`
+Tensor input_grad(const Tensor& g, const Tensor& w, const Tensor& g2 = Tensor(), const Tensor& w2 = Tensor(), const Tensor& add = Tensor()) {
+  if (projects(g, w) && (!g2.defined() || projects(g2, w2))) return project({{g, w, Tensor(), add, g2, w2}}, true)[0];
   std::vector<int64_t> shape = g.sizes().vec();
   shape.back() = w.size(1);
-  return at::mm(flat(g), w).view(shape);
+  Tensor r = add.defined() ? at::addmm(flat(add), flat(g), w) : at::mm(flat(g), w);
+  if (g2.defined()) r.addmm_(flat(g2), w2);
+  return r.view(shape);
 }
 // gradients of W and b; kernel: by the token-splitting kernel, else torch's GEMM and column sums
 std::pair<Tensor, Tensor> weight_grad(const Tensor& g, const Tensor& x, bool weight, bool bias, bool kernel) {
@@ -580,7 +680,7 @@ struct NoGraph {  // (called inside an autograd function or without gradients: n
 std::vector<Tensor> mlla_fwd(const Tensor& x, const Tensor& w, const Tensor& b, const Tensor& conv_w, const Tensor& conv_b,
                              const Tensor& rotations, int64_t side, int64_t heads) {
   const NoGraph none;
-  const Tensor qk = at::linear(x, w, b);
+  const Tensor qk = linear(x, w, b);
   const auto [q, k, qr, kr, v] = rotary_fwd(qk, x, rotations, heads);
   const Attended a = la_fwd(q, k, v, qr, kr, 1.0 / x.size(1), 1e-6, FBLA_NORMALIZE | FBLA_DECOUPLED);
   const Tensor local = dwconv_fwd(x, conv_w, conv_b, side, side, false);
@@ -601,7 +701,7 @@ std::vector<Tensor> mlla_bwd(const Tensor& g, const Tensor& x, const Tensor& w, 
     Tensor dqk;
     std::tie(dqk, dx) = rotary_bwd(qk, rotations, heads, d.q, d.k, d.q_rope, d.k_rope, d.v, dlocal);
     std::tie(dw, db) = weight_grad(dqk, x, need[1], need[2], kernel);
-    if (need[0]) flat(dx).addmm_(flat(dqk), w);
+    if (need[0]) dx = input_grad(dqk, w, Tensor(), Tensor(), dx);
   }
   return {need[0] ? dx : Tensor(), dw, db, dconv_w, dconv_b};
 }
@@ -622,10 +722,7 @@ Tensor local_values_grad(const Tensor& dlocal, int64_t n, const Tensor& conv_w, 
 std::pair<Tensor, Tensor> two_input_grads(const Tensor& dq, const Tensor& q_w, bool need_x, const Tensor& dkv, const Tensor& kv_w, bool same,
                                           bool need_src) {
   if (same) {
-    if (!need_x) return {};
-    Tensor dx = input_grad(dq, q_w);
-    flat(dx).addmm_(flat(dkv), kv_w);
-    return {dx, Tensor()};
+    return {need_x ? input_grad(dq, q_w, dkv, kv_w) : Tensor(), Tensor()};
   }
   return {need_x ? input_grad(dq, q_w) : Tensor(), need_src ? input_grad(dkv, kv_w) : Tensor()};
 }
@@ -647,7 +744,7 @@ std::vector<Tensor> pola_fwd(const Tensor& x, const Tensor& src, const std::vect
   const PolaWeights p = pola_weights(params);
   const int64_t N = x.size(1), n = src.size(1), C = x.size(2);
   const Tensor scale = at::softplus(p.scale), sigmoid = at::sigmoid(p.power), power = at::add(at::mul(sigmoid, alpha), 1);
-  const Tensor qg = at::linear(x, p.q_w, p.q_b), kv = at::linear(src, p.kv_w, p.kv_b);
+  const auto [qg, kv] = two_linears({x, p.q_w, p.q_b, Tensor()}, {src, p.kv_w, p.kv_b, Tensor()});
   const auto [q_same, q_opp, k, v] = polarity_fwd(qg, kv, p.pe, scale, power, heads);
   const LocalValues l = local_values(kv.narrow(2, C, C), N, p.conv_w, p.conv_b, H, W);
   Tensor o1, o2, s, km, s2, km2, v1, v2;
@@ -662,7 +759,7 @@ std::vector<Tensor> pola_fwd(const Tensor& x, const Tensor& src, const std::vect
     o1 = a.o, s = a.s, km = a.km, o2 = b.o, s2 = b.s, km2 = b.km;
   }
   const Tensor merged = merge_fwd(o1, o2, l.local, qg.narrow(2, C, C));
-  return {at::linear(merged, p.proj_w, p.proj_b), scale, sigmoid, power, qg, kv, q_same, q_opp, k, v, l.grid, l.local, o1, o2, s, km, s2,
+  return {linear(merged, p.proj_w, p.proj_b), scale, sigmoid, power, qg, kv, q_same, q_opp, k, v, l.grid, l.local, o1, o2, s, km, s2,
           km2, v1, v2, merged};
 }
 
@@ -717,12 +814,13 @@ std::vector<Tensor> focused_fwd(const Tensor& x, const Tensor& src, const std::v
   const NoGraph none;
   const FocusedWeights p = focused_weights(params);
   const int64_t N = x.size(1), n = src.size(1), C = x.size(2);
-  const Tensor scale = at::softplus(p.scale), q_rows = at::linear(x, p.q_w, p.q_b), kv = at::linear(src, p.kv_w, p.kv_b);
+  const Tensor scale = at::softplus(p.scale);
+  const auto [q_rows, kv] = two_linears({x, p.q_w, p.q_b, Tensor()}, {src, p.kv_w, p.kv_b, Tensor()});
   const auto [q, k, v] = focus_fwd(q_rows, kv, p.pe, scale, heads);
   const Attended a = la_fwd(q, k, v, Tensor(), Tensor(), 1.0 / n, 1e-6, FBLA_NORMALIZE);
   const LocalValues l = local_values(kv.narrow(2, C, C), N, p.conv_w, p.conv_b, H, W);
   const Tensor merged = merge_fwd(a.o, Tensor(), l.local, Tensor());
-  return {at::linear(merged, p.proj_w, p.proj_b), scale, q_rows, kv, q, k, v, l.grid, a.s, a.km, merged};
+  return {linear(merged, p.proj_w, p.proj_b), scale, q_rows, kv, q, k, v, l.grid, a.s, a.km, merged};
 }
 
 std::vector<Tensor> focused_bwd(const Tensor& g, const Tensor& x, const Tensor& src, bool same, const std::vector<Maybe>& params,
@@ -770,27 +868,27 @@ LinFusionWeights linfusion_weights(const std::vector<Maybe>& p) {
 }
 
 std::vector<Tensor> linfusion_fwd(const Tensor& x, const Tensor& cu, const std::vector<Maybe>& params, const std::array<double, 2>& eps,
-                                  const std::array<double, 2>& slope, int64_t heads) {
+                                  const std::array<double, 2>& slope, int64_t heads, bool trains) {
   const NoGraph none;
   const LinFusionWeights p = linfusion_weights(params);
   const int64_t B = x.size(0), N = x.size(1);
-  std::vector<Tensor> r(1);
-  Tensor packed[3];
-  for (int i = 0; i < 3; ++i) {
-    Tensor in = x;
-    if (i < 2) {
-      const auto& path = p.path[i];
-      const Tensor hidden = at::linear(x, path.in_w, path.in_b);
-      auto [normed, mean, rstd] = at::native_layer_norm(hidden, {hidden.size(-1)}, path.norm_w, path.norm_b, eps[i]);
-      at::leaky_relu_(normed, slope[i]);
-      in = at::add(x, at::linear(normed, path.out_w, path.out_b));
-      r.insert(r.end(), {hidden, mean, rstd, normed, in});
-    }
-    packed[i] = at::linear(in, p.w[i], p.b[i]).view({B * N, heads, -1});
+  const auto &pq = p.path[0], &pk = p.path[1];
+  const auto first = linears({{x, pq.in_w, pq.in_b, Tensor()}, {x, pk.in_w, pk.in_b, Tensor()}, {x, p.w[2], p.b[2], Tensor()}});
+  std::vector<Normed> normed;
+  const Norm norms[2] = {{first[0], pq.norm_w, pq.norm_b, eps[0], slope[0]}, {first[1], pk.norm_w, pk.norm_b, eps[1], slope[1]}};
+  if (first[0].sizes() == first[1].sizes()) {
+    normed = norm_leaky({norms[0], norms[1]}, trains);
+  } else {
+    for (const Norm& n : norms) normed.push_back(norm_leaky({n}, trains)[0]);
   }
+  const auto in = linears({{normed[0].y, pq.out_w, pq.out_b, x}, {normed[1].y, pk.out_w, pk.out_b, x}});
+  const auto qk = linears({{in[0], p.w[0], p.b[0], Tensor()}, {in[1], p.w[1], p.b[1], Tensor()}});
+  Tensor packed[3] = {qk[0], qk[1], first[2]};
+  for (Tensor& t : packed) t = t.view({B * N, heads, -1});
   const Attended a = varlen_fwd(packed[0], packed[1], packed[2], cu, N, std::nullopt, 1e-4, FBLA_ELU1_QK);
   const Tensor o = a.o.view({B, N, -1});
-  r[0] = at::linear(o, p.proj_w, p.proj_b);
+  std::vector<Tensor> r{linear(o, p.proj_w, p.proj_b)};
+  for (int i = 0; i < 2; ++i) r.insert(r.end(), {first[i], normed[i].mean, normed[i].rstd, normed[i].y, in[i]});
   r.insert(r.end(), {packed[0], packed[1], packed[2], a.s, a.km, o});
   return r;
 }
@@ -810,25 +908,22 @@ std::vector<Tensor> linfusion_bwd(const Tensor& g, const Tensor& x, const Tensor
   const auto [dq, dk, dv] = varlen_bwd(qp, kp, vp, cu, N, input_grad(g, p.proj_w).view(vp.sizes()), at_(13), at_(14), std::nullopt, 1e-4,
                                        FBLA_ELU1_QK | FBLA_ELU1_GRAD);
   const Tensor d[3] = {flat(dq.view({-1, p.w[0].size(0)})), flat(dk.view({-1, p.w[1].size(0)})), flat(dv.view({-1, p.w[2].size(0)}))};
-  Tensor dx = need[0] ? at::mm(d[2], p.w[2]) : Tensor();
   std::tie(r[17], r[18]) = weight_grad(d[2], x, need[17], need[18], kernel[6]);
+  Tensor dx = need[0] ? input_grad(d[2], p.w[2]) : Tensor();
   for (int i = 0; i < 2; ++i) {
     const auto& path = p.path[i];
     const Tensor hidden = at_(5 * i), mean = at_(5 * i + 1), rstd = at_(5 * i + 2), normed = at_(5 * i + 3), in = at_(5 * i + 4);
     const int at0 = 1 + 6 * i;
     std::tie(r[13 + 2 * i], r[14 + 2 * i]) = weight_grad(d[i], in, need[13 + 2 * i], need[14 + 2 * i], kernel[4 + i]);
-    const Tensor din = at::mm(d[i], p.w[i]);  // of x + residual
+    const Tensor din = input_grad(d[i], p.w[i]);  // of x + residual
     std::tie(r[at0 + 4], r[at0 + 5]) = weight_grad(din, normed, need[at0 + 4], need[at0 + 5], kernel[2 * i + 1]);
-    const Tensor dnormed = at::leaky_relu_backward(at::mm(din, path.out_w), flat(normed), slope[i], true);
+    const Tensor dnormed = at::leaky_relu_backward(input_grad(din, path.out_w), flat(normed), slope[i], true);
     Tensor dhidden;
     std::tie(dhidden, r[at0 + 2], r[at0 + 3]) =
         at::native_layer_norm_backward(dnormed.view(hidden.sizes()), hidden, {hidden.size(-1)}, mean, rstd, path.norm_w, path.norm_b,
                                        {true, need[at0 + 2], need[at0 + 3]});
     std::tie(r[at0], r[at0 + 1]) = weight_grad(dhidden, x, need[at0], need[at0 + 1], kernel[2 * i]);
-    if (need[0]) {
-      dx.add_(din);
-      dx.addmm_(flat(dhidden), path.in_w);
-    }
+    if (need[0]) dx = input_grad(flat(dhidden), path.in_w, Tensor(), Tensor(), dx.add_(din));
   }
   if (need[0]) r[0] = dx.view(x.sizes());
   return r;
@@ -960,7 +1055,7 @@ bool linfusion_fits(const Tensor& x, const std::vector<Maybe>& params, int64_t h
   for (const auto& path : p.path) {
     if (!path.in_w.defined() || path.in_w.dim() != 2) return false;
     const int64_t width = path.in_w.size(0);
-    if (!linear_shapes(path.in_w, path.in_b, width, C, 8) || !shaped_or_none(path.norm_w, {width}) || !shaped_or_none(path.norm_b, {width}) ||
+    if (width > 2048 || !linear_shapes(path.in_w, path.in_b, width, C, 8) || !shaped_or_none(path.norm_w, {width}) || !shaped_or_none(path.norm_b, {width}) ||
         !linear_shapes(path.out_w, path.out_b, C, width, 8))
       return false;
   }
@@ -1034,6 +1129,18 @@ PYBIND11_MODULE(fbla_torch, m) {
     const auto r = linear_wgrad(g, x, with_bias);
     return outs(r.first, r.second);
   });
+  m.def("project", [](const std::vector<std::array<Maybe, 6>>& p, bool rows_of_w) {
+    std::vector<Projection> jobs;
+    for (const auto& t : p) jobs.push_back({given(t[0]), given(t[1]), given(t[2]), given(t[3]), given(t[4]), given(t[5])});
+    return project(jobs, rows_of_w);
+  });
+  m.def("norm_leaky", [](const std::vector<std::tuple<Tensor, Maybe, Maybe, double, double>>& p, bool with_stats) {
+    std::vector<Norm> jobs;
+    for (const auto& [x, w, b, eps, slope] : p) jobs.push_back({x, given(w), given(b), eps, slope});
+    py::list r;
+    for (const Normed& n : norm_leaky(jobs, with_stats)) r.append(outs(n.y, n.mean, n.rstd));
+    return r;
+  });
   m.def("polarity_fwd", [](const Tensor& qg, const Tensor& kv, const Tensor& pe, const Tensor& scale, const Tensor& power, int64_t heads) {
     return outs(polarity_fwd(qg, kv, pe, scale, power, heads));
   });
@@ -1092,7 +1199,9 @@ PYBIND11_MODULE(fbla_torch, m) {
                           const std::vector<Maybe>& s, int64_t H, int64_t W, int64_t heads, const std::array<bool, 12>& need,
                           const std::array<bool, 3>& kernel) { return listed(focused_bwd(g, x, src, same, p, s, H, W, heads, need, kernel)); });
   m.def("linfusion_fwd", [](const Tensor& x, const Tensor& cu, const std::vector<Maybe>& p, const std::array<double, 2>& eps,
-                            const std::array<double, 2>& slope, int64_t heads) { return listed(linfusion_fwd(x, cu, p, eps, slope, heads)); });
+                            const std::array<double, 2>& slope, int64_t heads, bool trains) {
+    return listed(linfusion_fwd(x, cu, p, eps, slope, heads, trains));
+  });
   m.def("linfusion_bwd", [](const Tensor& g, const Tensor& x, const Tensor& cu, const std::vector<Maybe>& p, const std::vector<Maybe>& s,
                             const std::array<double, 2>& slope, const std::array<bool, 21>& need, const std::array<bool, 8>& kernel) {
     return listed(linfusion_bwd(g, x, cu, p, s, slope, need, kernel));

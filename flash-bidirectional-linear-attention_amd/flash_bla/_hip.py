@@ -16,6 +16,8 @@ library.  `lib()` is the library itself through ctypes.  There is no fallback: a
     elu1_fwd(x0, x1=None) -> y0 or (y0, y1), elu1_bwd(x, dy) -> dx
     dwconv_fwd(x, w, bias, H, W, flip=False) -> y, dwconv_grad(x, g, w, H, W, with_bias) -> dw, db
     linear_wgrad(g, x, with_bias) -> dw, db
+    project([(a, w, bias, add, a2, w2), ...], rows_of_w) -> [a w^T + bias + add, ...] or (rows_of_w) [a w + a2 w2 + add, ...]
+    norm_leaky([(x, weight, bias, eps, slope), ...], with_stats) -> [(y, mean, rstd), ...]
     polarity_fwd(qg, kv, pe, scale, power, heads) -> q_same, q_opp, k_both, v
     polarity_bwd(qg, kv, pe, scale, power, heads, dq_same, dq_opp, dk_both, dv, dv_rows, dgate) -> dqg, dkv, dpe, dscale, dpower
     rotary_fwd(qk, x, rotations, heads) -> q, k, q_rot, k_rot, v
@@ -83,6 +85,8 @@ _SIGNATURES = {
     "fbla_dwconv_grad": (_i32, [_vp, _i64, _i64, _vp, _i64, _i64, _vp, _vp, _vp, _sz] + [_i64] * 3 + [_i32] * 4 + [_vp]),
     "fbla_linear_wgrad_workspace_bytes": (_sz, [_i64] + [_i32] * 3),
     "fbla_linear_wgrad": (_i32, [_vp, _i64, _vp, _i64, _vp, _vp, _vp, _sz, _i64] + [_i32] * 3 + [_vp]),
+    "fbla_project": (_i32, [_vp, _i32, _i64, _i32, _i32, _vp]),
+    "fbla_norm_leaky": (_i32, [_vp, _i32, _i64, _i32, _i32, _vp]),
     "fbla_polarity_fwd": (_i32, [_vp] * 9 + [_i64] * 3 + [_i32] * 3 + [_vp]),
     "fbla_polarity_bwd_workspace_bytes": (_sz, [_i64] * 3 + [_i32] * 3),
     "fbla_polarity_bwd": (_i32, [_vp] * 17 + [_sz] + [_i64] * 3 + [_i32] * 3 + [_vp]),
@@ -128,7 +132,7 @@ def lib():
 
 _NATIVE = frozenset((
     "la_fwd", "la_bwd", "pair_supported", "pair_fwd", "pair_bwd", "varlen_fwd", "varlen_bwd", "chunk_reduce", "select_blocks",
-    "piecewise_supported", "piecewise_fwd", "elu1_fwd", "elu1_bwd", "dwconv_fwd", "dwconv_grad", "linear_wgrad", "polarity_fwd",
+    "piecewise_supported", "piecewise_fwd", "elu1_fwd", "elu1_bwd", "dwconv_fwd", "dwconv_grad", "linear_wgrad", "project", "norm_leaky", "polarity_fwd",
     "polarity_bwd", "rotary_fwd", "rotary_bwd", "merge_fwd", "merge_bwd", "interpolate_fwd", "interpolate_bwd", "focus_fwd",
     "focus_bwd", "turn_fwd", "turn_bwd", "mlla_fwd", "mlla_bwd", "pola_fwd", "pola_bwd", "focused_fwd", "focused_bwd",
     "linfusion_fwd", "linfusion_bwd", "dense_operands", "plain_gpu_tensors", "untouched_modules", "mlla_fits", "pola_fits",

@@ -88,7 +88,7 @@ class WholeBlockFunction(torch.autograd.Function):
 def _run(call, inputs):
     if torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in inputs):
         return WholeBlockFunction.apply(call, *inputs)
-    return call.run(inputs)[0]
+    return call.run(inputs, trains=False)[0]
 
 
 def _ordinary(block, kind, x, modules):
@@ -115,7 +115,7 @@ class _Mlla:
     def __init__(self, block, rotations, side):
         self.block, self.rotations, self.side, self.extra = block, rotations, side, (True,)
 
-    def run(self, inputs):
+    def run(self, inputs, trains=True):
         return _hip.mlla_fwd(inputs[0], inputs[1:], self.rotations, self.side, self.block.num_heads)
 
     def run_backward(self, g, inputs, saved, need):
@@ -150,7 +150,7 @@ class _Pola(_Pvt):
     names = (None, None, "qg.weight", "qg.bias", "kv.weight", "kv.bias", "positional_encoding", "scale", "power", "dwc.weight",
              "dwc.bias", "proj.weight", "proj.bias")
 
-    def run(self, inputs):
+    def run(self, inputs, trains=True):
         x, src, *p = inputs
         return _hip.pola_fwd(x, x if src is None else src, p, self.block.alpha, self.H, self.W, self.block.num_heads)
 
@@ -164,7 +164,7 @@ class _Focused(_Pvt):
     names = (None, None, "q.weight", "q.bias", "kv.weight", "kv.bias", "positional_encoding", "scale", "dwc.weight", "dwc.bias",
              "proj.weight", "proj.bias")
 
-    def run(self, inputs):
+    def run(self, inputs, trains=True):
         x, src, *p = inputs
         return _hip.focused_fwd(x, x if src is None else src, p, self.H, self.W, self.block.num_heads)
 
@@ -210,9 +210,9 @@ class _LinFusion:
         self.block, self.cu, self.extra = block, cu, ()
         self.slope = tuple(path[2].negative_slope for path in (block.to_q_, block.to_k_))
 
-    def run(self, inputs):
+    def run(self, inputs, trains=True):
         eps = tuple(path[1].eps for path in (self.block.to_q_, self.block.to_k_))
-        return _hip.linfusion_fwd(inputs[0], self.cu, inputs[1:], eps, self.slope, self.block.heads)
+        return _hip.linfusion_fwd(inputs[0], self.cu, inputs[1:], eps, self.slope, self.block.heads, trains)
 
     def run_backward(self, g, inputs, saved, need):
         x, *p = inputs

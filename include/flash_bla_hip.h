@@ -289,6 +289,39 @@ size_t fbla_linear_wgrad_workspace_bytes(int64_t tokens, int M, int N, int dtype
 int fbla_linear_wgrad(const void* g, int64_t g_row, const void* x, int64_t x_row, void* dw, void* db, void* workspace,
                       size_t workspace_bytes, int64_t tokens, int M, int N, int dtype, void* stream);
 
+/* Up to three projections of the same number of token rows in one launch (fp16 / bf16): out [tokens, N] = a W + a2 W2 + bias +
+ * add, in fp32, rounded once.  rows_of_w = 0: w is [N, K] (nn.Linear's forward, a w^T; flash_bla/layers/mlla.py:56,
+ * linfusion.py:26-38,83-103, rala.py:31, focused_la.py:26-27, polaformer.py:24-25); 1: w is [K, N] (its input gradient).  a2
+ * (with w2 of K2 channels), bias [N] and add (rows) may be NULL.  Rows of a, a2, add and out lie a_row, .. elements apart
+ * (whole 16-byte pieces, at least their channels); w without gaps; N and K multiples of 8; 16-byte aligned pointers.  out may
+ * be add. */
+typedef struct {
+  const void* a;
+  int64_t a_row;
+  const void* w;
+  const void* a2;
+  int64_t a2_row;
+  const void* w2;
+  const void* bias;
+  const void* add;
+  int64_t add_row;
+  void* out;
+  int64_t out_row;
+  int32_t N, K, K2;
+} fbla_projection;
+int fbla_project(const fbla_projection* jobs, int count, int64_t tokens, int rows_of_w, int dtype, void* stream);
+
+/* LayerNorm over the C channels of contiguous rows and LeakyReLU (flash_bla/layers/linfusion.py:26-38), one or two sets of rows
+ * in one launch, in fp32 and rounded once.  weight and bias [C] may be NULL; mean and rstd (fp32 [tokens], for a backward) may
+ * both be NULL.  fp16 / bf16, C a multiple of 8 up to 2048. */
+typedef struct {
+  const void *x, *weight, *bias;
+  void* out;
+  float *mean, *rstd;
+  float eps, slope;
+} fbla_norm;
+int fbla_norm_leaky(const fbla_norm* jobs, int count, int64_t tokens, int C, int dtype, void* stream);
+
 /* What the vision blocks do between their projections and the attention operators.  Rows are [B, N, C], C = heads * d,
  * joint projections [B, N, 2 C], heads [B, heads, N, width]; contiguous, one element type, d in whole 16-byte pieces.
  *
