@@ -10,13 +10,16 @@
 // into LDS, or by the transposing read where the contraction runs over W's rows); results leave through LDS as whole rows.
 // Sums are fp32 and rounded once, bias, `add` and the second product included.
 //
-// GPU us, the library / here (bf16, with bias; in brackets the input gradient): 200704 x 64 -> 128 24.1 / 21.4 (45.9 / 15.8), 50176 x 256
-// -> 512 33.5 / 31.3 (22.2 / 26.0), 3136 x 256 -> 512 6.2 / 5.7 (7.5 / 6.1), 1024 x 640 -> 640 6.4 / 7.5 (7.3 / 6.9), 8192 x 640 -> 640
-// 13.4 / 17.4, three of them in one launch 40.5 / 36.1.  Where the library's GEMM is faster by itself (contractions of 512 and more over
-// many tokens) the blocks keep it (`projects` in fbla_torch.cpp); elsewhere what counts beside the GPU's time is that a launch here
-// costs the host 4 us and a GEMM call of torch 17.  Blocks: LinFusion forward 8192 x 640 243 -> 147 us (with norm_leaky below,
-// residual sums in the products), MLLA step 64 x 56x56 x 64 414 -> 373, PolaFormer step 64 x 28x28 x 256 781 -> 747.
+// GPU us, the library / here (bf16, with bias; in brackets the input gradient): 200704 x 64 -> 128 24.1 / 16.9 (46 / 16.4), 50176 x 256
+// -> 512 33.2 / 30.6 (22.2 / 24.8), -> 256 14.6 / 16.8 (16.4 / 16.5), 3136 x 256 -> 512 6.2 / 5.6 (7.5 / 5.5), 1024 x 640 -> 640 6.4 / 6.4
+// (7.3 / 5.9), 8192 x 640 -> 640 13.2 / 14.5 (16.4 / 14.5), three of them in one launch 40 / 30.3.  Where the library's GEMM is faster by
+// itself (contractions of 512 and more over many tokens) the blocks keep it (`projects` in fbla_torch.cpp); elsewhere what
+// counts beside the GPU's time is that a launch here costs the host 4 us and a GEMM call of torch 17.  A first form with
+// branches around its loads waited for every step's rows (and looped over lanes for descriptors the compiler could not see to
+// be uniform): 15 % more throughout.  Blocks: LinFusion forward 8192 x 640 243 -> 142 us (with norm_leaky below, residual sums in
+// the products), MLLA step 64 x 56x56 x 64 414 -> 371, PolaFormer step 64 x 28x28 x 256 781 -> 750.
 #include <hip/hip_runtime.h>
+
 
 #include "fbla_mfma_shared.h"
 
@@ -27,6 +30,7 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kBufferFlags = 0x00020000;  // raw buffer, 32-bit words, range checked
+constexpr int kPast = 1 << 30;             // a lane offset past every buffer
 constexpr int kStep = 64;  // channels of the contraction per step: 128 bytes of a row
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -63,7 +67,7 @@ template <int TN> __device__ __forceinline__ int place_rows(int row, int ch) {
   else return row * 128 + ((ch ^ ((row & 2) << 1)) << 4);
 }
 
-template <typename T, int TM, int TN, bool ROWS>
+template <typename T, int TM, int TN, bool ROWS, bool TWO>
 __global__ __launch_bounds__(kThreads, 2) void project_kernel(Jobs jobs) {
   using V = typename Vec<T>::type;
   constexpr int kABytes = TM * kStep * 2, kWBytes = TN * kStep * 2, kBuf = kABytes + kWBytes;
@@ -72,72 +76,63 @@ __global__ __launch_bounds__(kThreads, 2) void project_kernel(Jobs jobs) {
   constexpr int kOutRow = TN * 2 + 16;  // (16 bytes apart from a multiple of the banks)
   __shared__ __attribute__((aligned(16))) unsigned char smem[2 * kBuf > TM * kOutRow ? 2 * kBuf : TM * kOutRow];
 
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 1, wn = wave & 1, kb = lane >> 5;
+
+  struct Source {
+    __amdgpu_buffer_rsrc_t a, w;
+    int a_row, w_row, K;
+  };
   // The output tiles of a block of tokens read the same rows: they run on one XCD (workgroup i is on XCD i % 8).  Blocks beyond
-  // the last multiple of eight keep the plain order.
-  const int tiles = jobs.first_tile[jobs.count];
-  const int blocks = (int)(gridDim.x / tiles), i = blockIdx.x, together = blocks / 8 * 8 * tiles;
+  // the last multiple of eight keep the plain order.  (One round of workgroups that walk the tiles, the next one's first rows
+  // requested before the results leave, was slower throughout: 50176 x 256 -> 2 x 512 57.4 us against 48.8, spilling at two
+  // workgroups a CU.)
+  const int tiles = jobs.first_tile[jobs.count], blocks = (int)((jobs.tokens + TM - 1) / TM), i = blockIdx.x;
+  const int together = blocks / 8 * 8 * tiles;
   const int block = i < together ? i / (8 * tiles) * 8 + i % 8 : i / tiles;
-  int tile = i < together ? i / 8 % tiles : i % tiles;
+  const int tile = i < together ? i / 8 % tiles : i % tiles;
   int j = 0;
-  while (j + 1 < jobs.count && tile >= jobs.first_tile[j + 1]) ++j;
+  if (jobs.count > 1 && tile >= jobs.first_tile[1]) j = 1;
+  if (jobs.count > 2 && tile >= jobs.first_tile[2]) j = 2;
   const Job& job = jobs.job[j];
   const int n0 = (tile - jobs.first_tile[j]) * TN, N = job.N;
   const int64_t t0 = (int64_t)block * TM;
   const int rows = (int)min((int64_t)TM, jobs.tokens - t0);
-
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave >> 1, wn = wave & 1, kb = lane >> 5;
-
-  // The steps of both products, one after the other.  Loads are buffer loads: one lane offset per piece for the whole loop, the
-  // step is the scalar offset, and what lies past the last token (or W's last row) comes back as zero.
-  const int steps0 = (job.K[0] + kStep - 1) / kStep, steps = steps0 + (job.K[1] + kStep - 1) / kStep;
-  struct Source {
-    __amdgpu_buffer_rsrc_t a, w;
-    int aoff[kAPieces], woff[kWPieces], wstep, K;
-  };
+  const int steps0 = (job.K[0] + kStep - 1) / kStep, steps = steps0 + (TWO ? (job.K[1] + kStep - 1) / kStep : 0);
   auto source = [&](int seg) {
     Source r;
-    const int K = job.K[seg];
-    const int a_row = (int)job.a_row[seg] * 2, w_row = (ROWS ? N : K) * 2;
-    r.K = K;
-    r.wstep = ROWS ? w_row : 2;
+    r.K = job.K[seg];
+    r.a_row = (int)job.a_row[seg] * 2;
+    r.w_row = (ROWS ? N : r.K) * 2;
     const T* a = (const T*)job.a[seg] + t0 * job.a_row[seg];
-    const T* w = (const T*)job.w[seg] + (ROWS ? (int64_t)n0 : (int64_t)n0 * K);
-    r.a = __builtin_amdgcn_make_buffer_rsrc((void*)a, 0, (rows - 1) * a_row + K * 2, kBufferFlags);
-    r.w = __builtin_amdgcn_make_buffer_rsrc((void*)w, 0, ROWS ? (int)(((int64_t)K * N - n0) * 2) : min(TN, N - n0) * w_row, kBufferFlags);
+    const T* w = (const T*)job.w[seg] + (ROWS ? (int64_t)n0 : (int64_t)n0 * r.K);
+    r.a = __builtin_amdgcn_make_buffer_rsrc((void*)a, 0, (rows - 1) * r.a_row + r.K * 2, kBufferFlags);
+    r.w = __builtin_amdgcn_make_buffer_rsrc((void*)w, 0, ROWS ? (int)(((int64_t)r.K * N - n0) * 2) : min(TN, N - n0) * r.w_row, kBufferFlags);
+    return r;
+  };
+  const Source first = source(0), other = source(TWO ? 1 : 0);
+  // The steps of both products, one after the other.  Loads are buffer loads without a branch around them (so that a wait for one
+  // step's rows leaves the next step's in flight): the step is the scalar offset, and what lies past the last token, past W's
+  // last row, past the rows' channels or past the last step comes back as zero.
+  struct Regs {
+    u32x4 a[kAPieces], w[kWPieces];
+  };
+  auto fetch = [&](Regs& r, int s) {
+    const bool second = TWO && s >= steps0;
+    const __amdgpu_buffer_rsrc_t a = second ? other.a : first.a, w = second ? other.w : first.w;
+    const int a_row = second ? other.a_row : first.a_row, w_row = second ? other.w_row : first.w_row;
+    const int K = second ? other.K : first.K, k0 = (second ? s - steps0 : s) * kStep;
+    const int past = k0 + (tid & 7) * 8 >= K ? kPast : 0;
 #pragma unroll
     for (int p = 0; p < kAPieces; ++p) {
       const int q = tid + kThreads * p;
-      r.aoff[p] = (q >> 3) * a_row + (q & 7) * 16;
+      r.a[p] = __builtin_amdgcn_raw_buffer_load_b128(a, ((q >> 3) * a_row + (q & 7) * 16) | past, k0 * 2, 0);
     }
 #pragma unroll
     for (int p = 0; p < kWPieces; ++p) {
       const int q = tid + kThreads * p;
-      r.woff[p] = ROWS ? q / (TN / 8) * w_row + q % (TN / 8) * 16 : (q >> 3) * w_row + (q & 7) * 16;
-    }
-    return r;
-  };
-  struct Regs {
-    u32x4 a[kAPieces], w[kWPieces];
-  };
-  Source from = source(0);
-  auto fetch = [&](Regs& r, int s) {
-    if (s >= steps) return;
-    if (s == steps0) from = source(1);
-    const int k0 = (s >= steps0 ? s - steps0 : s) * kStep;
-#pragma unroll
-    for (int p = 0; p < kAPieces; ++p) r.a[p] = __builtin_amdgcn_raw_buffer_load_b128(from.a, from.aoff[p], k0 * 2, 0);
-#pragma unroll
-    for (int p = 0; p < kWPieces; ++p) r.w[p] = __builtin_amdgcn_raw_buffer_load_b128(from.w, from.woff[p], k0 * from.wstep, 0);
-    if (k0 + kStep > from.K) {  // channels past the row's end are the next row's
-#pragma unroll
-      for (int p = 0; p < kAPieces; ++p)
-        if (k0 + (tid & 7) * 8 >= from.K) r.a[p] = u32x4{0u, 0u, 0u, 0u};
-      if constexpr (!ROWS) {
-#pragma unroll
-        for (int p = 0; p < kWPieces; ++p)
-          if (k0 + (tid & 7) * 8 >= from.K) r.w[p] = u32x4{0u, 0u, 0u, 0u};
-      }
+      if constexpr (ROWS) r.w[p] = __builtin_amdgcn_raw_buffer_load_b128(w, q / (TN / 8) * w_row + q % (TN / 8) * 16, k0 * w_row, 0);
+      else r.w[p] = __builtin_amdgcn_raw_buffer_load_b128(w, ((q >> 3) * w_row + (q & 7) * 16) | past, k0 * 2, 0);
     }
   };
   auto stash = [&](const Regs& r, unsigned char* at) {
@@ -169,50 +164,70 @@ __global__ __launch_bounds__(kThreads, 2) void project_kernel(Jobs jobs) {
         woff[b][h] = place_rows<TN>(8 * (g >> 1) + 4 * h + (s >> 2), 4 * (wn * NB + b) + 2 * (q & 1) + (g & 1)) + 8 * (q >> 1);
   }
   f32x16 acc[MB][NB];
+  struct Fragments {
+    V x[MB], w[NB];
+  };
+  auto fragments = [&](Fragments& f, const unsigned char* at, int ks) {
+    const unsigned char* wt = at + kABytes;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      if constexpr (ROWS) {  // (16 rows further on the swizzle is the same)
+        const u32x2 lo = transposed_read(wt + ks * 16 * TN * 2 + woff[b][0]), hi = transposed_read(wt + ks * 16 * TN * 2 + woff[b][1]);
+        f.w[b] = __builtin_bit_cast(V, u32x4{lo[0], lo[1], hi[0], hi[1]});
+      } else {
+        f.w[b] = __builtin_bit_cast(V, *reinterpret_cast<const u32x4*>(wt + mfma::swz<128>(32 * (wn * NB + b) + (lane & 31), 2 * ks + kb)));
+      }
+    }
+#pragma unroll
+    for (int a = 0; a < MB; ++a)
+      f.x[a] = __builtin_bit_cast(V, *reinterpret_cast<const u32x4*>(at + mfma::swz<128>(32 * (wm * MB + a) + (lane & 31), 2 * ks + kb)));
+  };
+  auto multiply = [&](const unsigned char* at) {  // the next fragments are requested before the products of the ones at hand
+    Fragments f[2];
+    fragments(f[0], at, 0);
+#pragma unroll
+    for (int ks = 0; ks < kStep / 16; ++ks) {
+      if (ks + 1 < kStep / 16) fragments(f[(ks + 1) & 1], at, ks + 1);
+#pragma unroll
+      for (int a = 0; a < MB; ++a)
+#pragma unroll
+        for (int b = 0; b < NB; ++b) acc[a][b] = mma(f[ks & 1].w[b], f[ks & 1].x[a], acc[a][b]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+
+  Regs r0, r1;
+  fetch(r0, 0);
+  fetch(r1, 1);
+  V bias[NB][2];  // this lane's outputs'
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int n = n0 + 32 * (wn * NB + b) + 16 * kb + 8 * h;
+      bias[b][h] = job.bias ? *reinterpret_cast<const V*>((const T*)job.bias + (n < N ? n : 0)) : V{};
+    }
 #pragma unroll
   for (int a = 0; a < MB; ++a)
 #pragma unroll
     for (int b = 0; b < NB; ++b)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.f;
-  auto multiply = [&](const unsigned char* at) {
-    const unsigned char* wt = at + kABytes;
-#pragma unroll
-    for (int ks = 0; ks < kStep / 16; ++ks) {
-      V x[MB], w[NB];
-#pragma unroll
-      for (int a = 0; a < MB; ++a)
-        x[a] = __builtin_bit_cast(V, *reinterpret_cast<const u32x4*>(at + mfma::swz<128>(32 * (wm * MB + a) + (lane & 31), 2 * ks + kb)));
-#pragma unroll
-      for (int b = 0; b < NB; ++b) {
-        if constexpr (ROWS) {  // (16 rows further on the swizzle is the same)
-          const u32x2 lo = transposed_read(wt + ks * 16 * TN * 2 + woff[b][0]), hi = transposed_read(wt + ks * 16 * TN * 2 + woff[b][1]);
-          w[b] = __builtin_bit_cast(V, u32x4{lo[0], lo[1], hi[0], hi[1]});
-        } else {
-          w[b] = __builtin_bit_cast(V, *reinterpret_cast<const u32x4*>(wt + mfma::swz<128>(32 * (wn * NB + b) + (lane & 31), 2 * ks + kb)));
-        }
-      }
-#pragma unroll
-      for (int a = 0; a < MB; ++a)
-#pragma unroll
-        for (int b = 0; b < NB; ++b) acc[a][b] = mma(w[b], x[a], acc[a][b]);
-    }
-  };
-
   // step s is in LDS buffer s % 2 while s + 1 and s + 2 are in registers or on their way there
-  Regs r0, r1;
-  fetch(r0, 0);
-  fetch(r1, 1);
-  for (int s = 0; s < steps; s += 2) {
+  for (int s = 0; s + 1 < steps; s += 2) {
     stash(r0, smem);
     fetch(r0, s + 2);
     __syncthreads();  // (every wave is done with the step before, whose buffer is written next)
     multiply(smem);
-    if (s + 1 >= steps) break;
     stash(r1, smem + kBuf);
     fetch(r1, s + 3);
     __syncthreads();
     multiply(smem + kBuf);
+  }
+  if (steps & 1) {
+    stash(r0, smem);
+    __syncthreads();
+    multiply(smem);
   }
 
   // ---- out: a lane's 16 neighbouring outputs of a token, rounded, to LDS; whole rows from there
@@ -226,16 +241,12 @@ __global__ __launch_bounds__(kThreads, 2) void project_kernel(Jobs jobs) {
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         const int n = n0 + col + 8 * h;
-        const bool in = n < N;
         f32x8 v;
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] = acc[a][b][8 * h + e];
-        if (job.bias) {
-          const V x = *reinterpret_cast<const V*>((const T*)job.bias + (in ? n : 0));
-          v += __builtin_convertvector(x, f32x8);
-        }
+        v += __builtin_convertvector(bias[b][h], f32x8);
         if (job.add) {
-          const bool has = in && row < rows;
+          const bool has = n < N && row < rows;
           const V x = *reinterpret_cast<const V*>((const T*)job.add + (has ? (t0 + row) * job.add_row + n : 0));
           v += __builtin_convertvector(x, f32x8);
         }
@@ -259,24 +270,32 @@ void launch(const Job* job, int count, int64_t tokens, hipStream_t st) {
   Jobs jobs{};
   jobs.count = count;
   jobs.tokens = tokens;
+  bool two = false;
   for (int j = 0; j < count; ++j) {
     jobs.job[j] = job[j];
     jobs.first_tile[j + 1] = jobs.first_tile[j] + (job[j].N + TN - 1) / TN;
+    two = two || job[j].K[1] > 0;
   }
-  const int64_t wgs = cdiv64(tokens, TM) * jobs.first_tile[count];
-  project_kernel<T, TM, TN, ROWS><<<dim3((unsigned)wgs), dim3(kThreads), 0, st>>>(jobs);
+  const dim3 grid((unsigned)(cdiv64(tokens, TM) * jobs.first_tile[count])), block(kThreads);
+  if (two) project_kernel<T, TM, TN, ROWS, true><<<grid, block, 0, st>>>(jobs);
+  else project_kernel<T, TM, TN, ROWS, false><<<grid, block, 0, st>>>(jobs);
 }
 
+// By the number of 128 x 128 tiles: too few for the CUs are cut to 64 x 64; large tiles need enough of them and of steps to
+// outweigh three workgroups a CU of 128 x 64.  us with 64 x 64 / 128 x 64 / 128 x 128, forward (bf16): 392 x 64 -> 128 3.8 / 4.6 / 4.6, 1024 x
+// 640 -> 3 x 640 (120 tiles) 8.5 / 8.6 / 11.3, 1024 x 1280 -> 3 x 1280 (240) 26.6 / 20.7 / 20.7, 8192 x 640 -> 640 (320) 14.6 / 14.5 / 16.3,
+// -> 3 x 640 (960) 36.4 / 32.9 / 30.3, 50176 x 256 -> 256 (784) 17.2 / 16.8 / 17.5, -> 2 x 512 (3136) 61 / 51.8 / 48.8, 200704 x 64 -> 128
+// (1568) 18.9 / 16.9 / 17.6.
 template <typename T, bool ROWS> void choose(const Job* job, int count, int64_t tokens, hipStream_t st) {
-  int64_t wide = 0, narrow = 0, most = 0;
+  int64_t wide = 0;
+  int least_k = 1 << 30;
   for (int j = 0; j < count; ++j) {
     wide += (job[j].N + 127) / 128;
-    narrow += (job[j].N + 63) / 64;
-    most = job[j].N > most ? job[j].N : most;
+    least_k = job[j].K[0] < least_k ? job[j].K[0] : least_k;
   }
-  static const int few = tuning_knob("FBLA_GEMM_FEW", 256);
-  if (cdiv64(tokens, 128) * wide < few) launch<T, 64, 64, ROWS>(job, count, tokens, st);
-  else if (most <= 64) launch<T, 128, 64, ROWS>(job, count, tokens, st);
+  const int64_t tiles = cdiv64(tokens, 128) * wide;
+  if (tiles < 200) launch<T, 64, 64, ROWS>(job, count, tokens, st);
+  else if (tiles < 900 || least_k < 256) launch<T, 128, 64, ROWS>(job, count, tokens, st);
   else launch<T, 128, 128, ROWS>(job, count, tokens, st);
 }
 

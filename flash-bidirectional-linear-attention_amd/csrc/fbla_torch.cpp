@@ -624,9 +624,8 @@ std::array<Tensor, 3> turn_bwd(const Tensor& k_, const Tensor& weight_, const Te
 Tensor flat(const Tensor& t) { return t.reshape({-1, t.size(-1)}); }
 // Whether `project` takes a projection of these rows rather than torch's GEMM: 16-bit types, unless the product is large enough
 // for the library's deeper pipeline to count.  GPU us of the library / here (bf16, with bias; a call of the library takes the
-// host 17 us, one of ours 4): 200704 x 64 -> 128 24.1 / 21.4, its input gradient 45.9 / 15.8; 50176 x 256 -> 512 33.5 / 31.3; 50176 x
-// 256 -> 256 14.7 / 19.6; 8192 x 640 -> 640 13.4 / 17.4, three of them 40 / 36; 1024 x 1280 -> 1280 11.3 / 14.6; 4096 x 1280 -> 1280 19.9 /
-// 28.8.
+// host 17 us, one of ours 4): 8192 x 640 -> 640 13.2 / 14.5, three of them 40 / 30.3; 1024 x 1280 -> 1280 11.2 / 12.5; 4096 x 1280 -> 1280
+// 20 / 26.8; see fbla_gemm.hip.
 bool projects(const Tensor& x, const Tensor& w) {
   const double work = (double)(x.numel() / x.size(-1)) * w.numel();
   return x.element_size() == 2 && (w.size(0) < 512 || w.size(1) < 512 || work <= 4e9);
