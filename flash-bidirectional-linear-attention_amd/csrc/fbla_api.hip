@@ -867,6 +867,95 @@ int fbla_norm_leaky(const fbla_norm* jobs, int count, int64_t tokens, int C, int
   return check_launch(what);
 }
 
+// what: 0 forward, 1 backward over the queries, 2 over the keys
+static int block_attn(const char* name, const fbla_block_attn* p, int what, rows::Attn& a) {
+  if (!p || (p->kind != 0 && p->kind != 1) || p->B < 1 || p->N < 1 || p->Nk < 1 || p->heads < 1) {
+    set_error("%s: bad sizes or kind", name);
+    return kErrBadArg;
+  }
+  const bool pola = p->kind == 0;
+  const int64_t n = p->N > p->Nk ? p->N : p->Nk, C = (int64_t)p->heads * 32;
+  if ((p->dtype != kF16 && p->dtype != kBF16) || p->B > 65535 || p->heads > 2048 || n > (1 << 24) || (int64_t)p->B * n * C > 1LL << 40 ||
+      (!pola && p->N != p->Nk)) {
+    set_error("%s: fp16 / bf16, at most 65535 batches, 2048 heads and 2^24 tokens, as many keys as queries for kind 1", name);
+    return kErrUnsupported;
+  }
+  auto need = [&](std::initializer_list<const void*> ptrs) -> int {
+    for (const void* q : ptrs)
+      if (!q) {
+        set_error("%s: null tensor pointer", name);
+        return kErrBadArg;
+      }
+    return check_aligned(name, ptrs);
+  };
+  int rc = need({p->q, p->k, p->v, p->state_planes, p->state_km, p->workspace});
+  if (rc == kOk && pola) rc = need({p->pe, p->scale, p->power});
+  if (rc == kOk && !pola) rc = need({p->rot});
+  if (rc == kOk && (what == 0 || pola)) rc = need({p->local});
+  if (rc == kOk && pola) rc = need({p->gate});
+  if (rc == kOk && what == 0) rc = need({p->out});
+  if (rc == kOk && what == 1) rc = need({p->dout, p->dq});
+  if (rc == kOk && what == 1 && pola) rc = need({p->dlocal, p->dgate});
+  if (rc == kOk && what == 2) rc = need({p->dk, p->dv, p->dv_more});
+  if (rc == kOk && what == 2 && pola) rc = need({p->dpe, p->dscale, p->dpower});
+  if (rc == kOk) rc = check_row_strides(name, (int)C, p->dtype, {p->q_row, p->k_row, p->v_row});
+  if (rc == kOk && pola) rc = check_row_strides(name, (int)C, p->dtype, {p->gate_row});
+  if (rc == kOk && what == 1) rc = check_row_strides(name, (int)C, p->dtype, {p->dq_row});
+  if (rc == kOk && what == 1 && pola) rc = check_row_strides(name, (int)C, p->dtype, {p->dgate_row});
+  if (rc == kOk && what == 2) rc = check_row_strides(name, (int)C, p->dtype, {p->dk_row, p->dv_row});
+  if (rc != kOk) return rc;
+  for (int64_t row : {p->q_row, p->k_row, p->v_row, p->gate_row, p->dq_row, p->dk_row, p->dv_row, p->dgate_row})
+    if (row > 1 << 22) {  // (32-bit offsets within a tile's rows)
+      set_error("%s: rows too long (%lld elements)", name, (long long)row);
+      return kErrUnsupported;
+    }
+  a = {pola, p->B, p->N, p->Nk, p->heads, p->eps, p->q, p->k, p->v, p->local, p->gate, p->q_row, p->k_row, p->v_row, p->gate_row, p->pe,
+       p->scale, p->power, p->rot, p->out, p->state_planes, p->state_km, p->dout, p->dv_more, p->dq, p->dk, p->dv, p->dlocal, p->dgate,
+       p->dq_row, p->dk_row, p->dv_row, p->dgate_row, p->dpe, p->dscale, p->dpower, p->workspace};
+  if (p->workspace_bytes < rows::workspace_bytes(a)) {
+    set_error("%s: workspace too small (%zu < %zu bytes)", name, p->workspace_bytes, rows::workspace_bytes(a));
+    return kErrWorkspace;
+  }
+  return kOk;
+}
+
+size_t fbla_block_attn_workspace_bytes(int kind, int64_t B, int64_t N, int64_t Nk, int heads) {
+  if (B < 1 || N < 1 || Nk < 1 || heads < 1 || B > 65535 || N > 1 << 24 || Nk > 1 << 24 || heads > 2048) return 0;
+  rows::Attn a{};
+  a.pola = kind == 0;
+  a.B = (int)B, a.N = (int)N, a.Nk = (int)Nk, a.heads = heads;
+  return rows::workspace_bytes(a);
+}
+size_t fbla_block_attn_state_elements(int kind, int64_t B, int heads) {
+  rows::Attn a{};
+  a.pola = kind == 0;
+  a.B = (int)B, a.heads = heads;
+  return B < 1 || heads < 1 ? 0 : rows::planes_elements(a);
+}
+int fbla_block_attn_forward(const fbla_block_attn* p, void* stream) {
+  const char* name = "fbla_block_attn_forward";
+  rows::Attn a;
+  const int rc = block_attn(name, p, 0, a);
+  if (rc != kOk) return rc;
+  rows::forward(a, p->dtype, (hipStream_t)stream);
+  return check_launch(name);
+}
+int fbla_block_attn_backward_queries(const fbla_block_attn* p, void* stream) {
+  const char* name = "fbla_block_attn_backward_queries";
+  rows::Attn a;
+  int rc = block_attn(name, p, 1, a);
+  if (rc == kOk) rc = rows::backward_queries(a, p->dtype, (hipStream_t)stream);
+  return rc != kOk ? rc : check_launch(name);
+}
+int fbla_block_attn_backward_keys(const fbla_block_attn* p, void* stream) {
+  const char* name = "fbla_block_attn_backward_keys";
+  rows::Attn a;
+  const int rc = block_attn(name, p, 2, a);
+  if (rc != kOk) return rc;
+  rows::backward_keys(a, p->dtype, (hipStream_t)stream);
+  return check_launch(name);
+}
+
 static int check_blocks(const char* what, blocks::Shape& s, int64_t B, int64_t N, int64_t Nk, int heads, int d, int unit,
                         int dtype) {
   if (B < 1 || N < 1 || Nk < 1 || heads < 1 || d < 1 || (dtype != kF16 && dtype != kBF16 && dtype != kF32)) {

@@ -10,10 +10,10 @@
 //
 // All of it is elementwise on token rows and bound by HBM: a lane owns 16 bytes of channels of one token (the next lanes the
 // next channels), everything is computed from them in fp32 and rounded once, and nothing between the projection's rows and the
-// operator's heads is written.  Training steps with torch operators in their place and with these: polarity (64 x 28x28 x
-// 256, bf16) 2.77 -> 0.83 ms, of it here 50 us features (257 MB, 5.1 TB/s), 75 + 9 us their gradients (385 MB, 5.1 TB/s), 19 + 33
-// us the merge; rotary (64 x 56x56 x 64) 0.83 -> 0.48 ms, of it 33 us features (205 MB, 6.2 TB/s), 45 us gradients (283 MB, 6.3
-// TB/s).
+// operator's heads is written.  bf16: polarity (64 x 28x28 x 256) 50 us features (257 MB, 5.1 TB/s), 75 + 9 us their gradients
+// (385 MB, 5.1 TB/s), 19 + 33 us the merge; rotary (64 x 56x56 x 64) 33 us features (205 MB, 6.2 TB/s), 45 us gradients (283 MB,
+// 6.3 TB/s).  Whole polarity and rotary blocks of 16-bit types with heads of 32 channels do not come here: fbla_rows.hip takes them
+// from rows to rows.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -882,10 +882,17 @@ void polarity_bwd(const Shape& s, const Polarity<const void>& a, const PolarityG
     float* pe_partial = workspace + (int64_t)2 * C * wgs;
     polarity_bwd_kernel<T><<<dim3((unsigned)wgs, (unsigned)w.channel_wgs), dim3(kThreads), 0, st>>>(
         s, typed<T, Polarity>(a), typed<T, PolarityGrads>(g), (T*)dqg, (T*)dkv, workspace, pe_partial, w.q_wgs, w.groups);
-    const int64_t pe_count = (int64_t)s.Nk * C;
+    features_finish(C, wgs, workspace, a.scale, dscale, dpower, w.groups, (int64_t)s.Nk * C, pe_partial, dpe, dtype, st);
+  });
+}
+
+void features_finish(int C, int terms, const float* partial, const void* scale, void* dscale, void* dpower, int groups,
+                     int64_t pe_count, const float* pe_partial, void* dpe, int dtype, hipStream_t st) {
+  by_type(dtype, [&](auto tag) {
+    using T = decltype(tag);
     const int stat_wgs = (2 * C + 63) / 64;
     features_finish_kernel<T><<<dim3((unsigned)(stat_wgs + cdiv64(pe_count, 64))), dim3(kThreads), 0, st>>>(
-        C, 2, 2, wgs, workspace, (const T*)a.scale, (T*)dscale, (T*)dpower, stat_wgs, w.groups, pe_count, pe_partial, (T*)dpe);
+        C, 2, 2, terms, partial, (const T*)scale, (T*)dscale, (T*)dpower, stat_wgs, groups, pe_count, pe_partial, (T*)dpe);
   });
 }
 

@@ -293,6 +293,9 @@ template <typename P> struct FocusGrads {
   P *q, *k, *v, *v_rows;  // heads of d; rows of C
 };
 int vec_of(int dtype);  // elements of a piece
+// sums of the partials of polarity gradients: dscale, dpower [C] from `terms` x [2][C], dpe [pe_count] from `groups` x [pe_count]
+void features_finish(int C, int terms, const float* partial, const void* scale, void* dscale, void* dpower, int groups,
+                     int64_t pe_count, const float* pe_partial, void* dpe, int dtype, hipStream_t st);
 int most_row_channels(int dtype);  // of rows that are normalised over their channels (focus_*)
 void focus_fwd(const Shape& s, const Focus<const void>& a, void* q, void* k, void* v, int dtype, hipStream_t st);
 size_t focus_bwd_workspace_bytes(const Shape& s, int dtype);
@@ -321,6 +324,33 @@ void interpolate_fwd(const void* x, int64_t x_batch, int64_t x_row, int B, int f
                      hipStream_t st);
 void interpolate_bwd(const void* g, int B, int from, int to, int C, void* dx, int dtype, hipStream_t st);
 }  // namespace blocks
+
+// Attention of the vision blocks on their projections' rows, 16-bit types, heads of 32 channels (fbla_rows.hip).
+namespace rows {
+struct Attn {
+  bool pola;  // polarity features, gate, two pairings; else rotary numerator, plain denominator
+  int B, N, Nk, heads;
+  float eps;
+  // rows of 32 * heads channels, `_row` elements apart, batches one after the other; local, dout, dlocal, dv_more, out: without gaps
+  const void *q, *k, *v, *local, *gate;
+  int64_t q_row, k_row, v_row, gate_row;
+  const void *pe, *scale, *power;  // polarity
+  const float* rot;                // rotary: fp32 [N][C / 2][2]
+  void* out;
+  void* planes;  // state, written by the forward: planes_elements of the type
+  float* km;     // [B * heads][64 or 32, and 8 more]
+  const void *dout, *dv_more;  // dv_more: added to dv
+  void *dq, *dk, *dv, *dlocal, *dgate;
+  int64_t dq_row, dk_row, dv_row, dgate_row;
+  void *dpe, *dscale, *dpower;
+  void* workspace;  // handed from backward_queries to backward_keys
+};
+size_t workspace_bytes(const Attn& a);
+size_t planes_elements(const Attn& a);
+void forward(const Attn& a, int dtype, hipStream_t st);
+int backward_queries(const Attn& a, int dtype, hipStream_t st);
+void backward_keys(const Attn& a, int dtype, hipStream_t st);
+}  // namespace rows
 
 // Piecewise (PISA) attention, forward only (fbla_piecewise.hip).
 namespace piecewise {

@@ -34,7 +34,8 @@ using Maybe = std::optional<Tensor>;
   X(fbla_polarity_fwd) X(fbla_polarity_bwd_workspace_bytes) X(fbla_polarity_bwd) X(fbla_rotary_fwd) X(fbla_rotary_bwd) \
   X(fbla_merge_fwd) X(fbla_merge_bwd) X(fbla_turn_fwd) X(fbla_turn_bwd) X(fbla_focus_fwd)                              \
   X(fbla_focus_bwd_workspace_bytes) X(fbla_focus_bwd) X(fbla_interpolate_fwd) X(fbla_interpolate_bwd)                   \
-  X(fbla_project) X(fbla_norm_leaky)
+  X(fbla_project) X(fbla_norm_leaky) X(fbla_block_attn_workspace_bytes) X(fbla_block_attn_state_elements)              \
+  X(fbla_block_attn_forward) X(fbla_block_attn_backward_queries) X(fbla_block_attn_backward_keys)
 
 struct Api {
 #define FBLA_MEMBER(f) decltype(&::f) f = nullptr;
@@ -675,30 +676,78 @@ struct NoGraph {  // (called inside an autograd function or without gradients: n
   at::AutoDispatchBelowADInplaceOrView guard;
 };
 
+// The attention between the projections' rows and the block's, where the kernels of fbla_rows.hip take it: 16-bit types, heads of
+// 32 channels.  `rows` are the projections with queries (and keys) first in a row.
+constexpr int kPolarity = 0, kRotary = 1;
+bool on_rows(const Tensor& x, int64_t heads) { return x.element_size() == 2 && x.size(2) == 32 * heads && x.size(0) <= 65535 && heads <= 2048; }
+struct RowState {
+  Tensor planes, km;
+};
+fbla_block_attn row_args(int kind, const Tensor& q, int64_t q_offset, const Tensor& k, int64_t k_offset, const Tensor& v, int64_t v_offset,
+                         int64_t heads, const RowState& state) {
+  fbla_block_attn a{};
+  auto at = [](const Tensor& t, int64_t offset) { return static_cast<char*>(ptr(t)) + offset * t.element_size(); };
+  a.kind = kind, a.dtype = code_of(q), a.B = q.size(0), a.N = q.size(1), a.Nk = k.size(1), a.heads = heads, a.eps = 1e-6f;
+  a.q = at(q, q_offset), a.k = at(k, k_offset), a.v = at(v, v_offset);
+  a.q_row = q.size(2), a.k_row = k.size(2), a.v_row = v.size(2);
+  a.state_planes = ptr(state.planes), a.state_km = f32(state.km);
+  return a;
+}
+RowState new_row_state(int kind, const Tensor& x, int64_t heads) {
+  return {like(x, {(int64_t)api.fbla_block_attn_state_elements(kind, x.size(0), heads)}),
+          like_f32(x, {x.size(0), heads, kind == kPolarity ? 72 : 40})};
+}
+Tensor row_workspace(const fbla_block_attn& a, const Tensor& x) {
+  return scratch(api.fbla_block_attn_workspace_bytes(a.kind, a.B, a.N, a.Nk, a.heads), x);
+}
+
 // layers/mlla.py: qk projection, rotary features, decoupled attention, positional convolution of the input
 std::vector<Tensor> mlla_fwd(const Tensor& x, const Tensor& w, const Tensor& b, const Tensor& conv_w, const Tensor& conv_b,
                              const Tensor& rotations, int64_t side, int64_t heads) {
   const NoGraph none;
-  const Tensor qk = linear(x, w, b);
+  const Tensor qk = linear(x, w, b), local = dwconv_fwd(x, conv_w, conv_b, side, side, false);
+  if (on_rows(x, heads)) {
+    const Tensor xs = whole(x), rot = whole(rotations), out = like(local);
+    const RowState state = new_row_state(kRotary, x, heads);
+    fbla_block_attn a = row_args(kRotary, qk, 0, qk, x.size(2), xs, 0, heads, state);
+    const Tensor ws = row_workspace(a, x);
+    a.local = ptr(local), a.rot = f32(rot), a.out = ptr(out), a.workspace = ptr(ws), a.workspace_bytes = ws.numel();
+    const On on(x);
+    check(api.fbla_block_attn_forward(&a, on.stream), "fbla_block_attn_forward");
+    return {out, qk, state.planes, state.km};
+  }
   const auto [q, k, qr, kr, v] = rotary_fwd(qk, x, rotations, heads);
   const Attended a = la_fwd(q, k, v, qr, kr, 1.0 / x.size(1), 1e-6, FBLA_NORMALIZE | FBLA_DECOUPLED);
-  const Tensor local = dwconv_fwd(x, conv_w, conv_b, side, side, false);
   return {merge_fwd(a.o, Tensor(), local, Tensor()), qk, q, k, qr, kr, v, a.s, a.km};
 }
 
-// need: x, w, b, conv_w, conv_b
+// saved: what mlla_fwd returned after its output.  need: x, w, b, conv_w, conv_b
 std::vector<Tensor> mlla_bwd(const Tensor& g, const Tensor& x, const Tensor& w, const Tensor& conv_w, const Tensor& rotations,
-                             const Tensor& qk, const Tensor& q, const Tensor& k, const Tensor& qr, const Tensor& kr, const Tensor& v,
-                             const Tensor& s, const Tensor& km, int64_t side, int64_t heads, const std::array<bool, 5>& need, bool kernel) {
+                             const std::vector<Tensor>& saved, int64_t side, int64_t heads, const std::array<bool, 5>& need, bool kernel) {
   const NoGraph none;
   Tensor dx, dw, db, dconv_w, dconv_b;
-  const MergeGrads m = merge_bwd(g, heads, false, Tensor(), Tensor(), Tensor(), Tensor());
-  if (need[3] || need[4]) std::tie(dconv_w, dconv_b) = dwconv_grad(x, m.local, conv_w, side, side, need[4]);
+  if (need[3] || need[4]) std::tie(dconv_w, dconv_b) = dwconv_grad(x, g, conv_w, side, side, need[4]);
   if (need[0] || need[1] || need[2]) {
-    const AttendedGrads d = la_bwd(q, k, v, qr, kr, m.o, s, km, 1.0 / x.size(1), 1e-6, FBLA_NORMALIZE | FBLA_DECOUPLED);
-    const Tensor dlocal = dwconv_fwd(m.local, conv_w, Tensor(), side, side, true);
+    const Tensor qk = saved.at(0), dlocal = dwconv_fwd(g, conv_w, Tensor(), side, side, true);
     Tensor dqk;
-    std::tie(dqk, dx) = rotary_bwd(qk, rotations, heads, d.q, d.k, d.q_rope, d.k_rope, d.v, dlocal);
+    if (saved.size() == 3) {
+      const Tensor xs = whole(x), gs = whole(g), rot = whole(rotations);
+      dqk = like(qk), dx = like(gs);
+      const int64_t C = x.size(2);
+      fbla_block_attn a = row_args(kRotary, qk, 0, qk, C, xs, 0, heads, {saved[1], saved[2]});
+      const Tensor ws = row_workspace(a, x);
+      a.rot = f32(rot), a.workspace = ptr(ws), a.workspace_bytes = ws.numel(), a.dout = ptr(gs), a.dv_more = ptr(dlocal);
+      a.dq = ptr(dqk), a.dk = static_cast<char*>(ptr(dqk)) + C * dqk.element_size(), a.dv = ptr(dx);
+      a.dq_row = a.dk_row = 2 * C, a.dv_row = C;
+      const On on(x);
+      check(api.fbla_block_attn_backward_queries(&a, on.stream), "fbla_block_attn_backward_queries");
+      check(api.fbla_block_attn_backward_keys(&a, on.stream), "fbla_block_attn_backward_keys");
+    } else {
+      const Tensor q = saved.at(1), k = saved.at(2), qr = saved.at(3), kr = saved.at(4), v = saved.at(5);
+      const MergeGrads m = merge_bwd(g, heads, false, Tensor(), Tensor(), Tensor(), Tensor());
+      const AttendedGrads d = la_bwd(q, k, v, qr, kr, m.o, saved.at(6), saved.at(7), 1.0 / x.size(1), 1e-6, FBLA_NORMALIZE | FBLA_DECOUPLED);
+      std::tie(dqk, dx) = rotary_bwd(qk, rotations, heads, d.q, d.k, d.q_rope, d.k_rope, d.v, dlocal);
+    }
     std::tie(dw, db) = weight_grad(dqk, x, need[1], need[2], kernel);
     if (need[0]) dx = input_grad(dqk, w, Tensor(), Tensor(), dx);
   }
@@ -744,8 +793,21 @@ std::vector<Tensor> pola_fwd(const Tensor& x, const Tensor& src, const std::vect
   const int64_t N = x.size(1), n = src.size(1), C = x.size(2);
   const Tensor scale = at::softplus(p.scale), sigmoid = at::sigmoid(p.power), power = at::add(at::mul(sigmoid, alpha), 1);
   const auto [qg, kv] = two_linears({x, p.q_w, p.q_b, Tensor()}, {src, p.kv_w, p.kv_b, Tensor()});
-  const auto [q_same, q_opp, k, v] = polarity_fwd(qg, kv, p.pe, scale, power, heads);
   const LocalValues l = local_values(kv.narrow(2, C, C), N, p.conv_w, p.conv_b, H, W);
+  if (on_rows(x, heads)) {
+    const Tensor merged = like(l.local), pe = whole(p.pe);
+    const RowState state = new_row_state(kPolarity, x, heads);
+    fbla_block_attn a = row_args(kPolarity, qg, 0, kv, 0, kv, C, heads, state);
+    const Tensor ws = row_workspace(a, x);
+    a.local = ptr(l.local), a.gate = static_cast<char*>(ptr(qg)) + C * qg.element_size(), a.gate_row = 2 * C, a.out = ptr(merged);
+    a.pe = ptr(pe), a.scale = ptr(scale), a.power = ptr(power), a.workspace = ptr(ws), a.workspace_bytes = ws.numel();
+    {
+      const On on(x);
+      check(api.fbla_block_attn_forward(&a, on.stream), "fbla_block_attn_forward");
+    }
+    return {linear(merged, p.proj_w, p.proj_b), scale, sigmoid, power, qg, kv, l.grid, l.local, state.planes, state.km, merged};
+  }
+  const auto [q_same, q_opp, k, v] = polarity_fwd(qg, kv, p.pe, scale, power, heads);
   Tensor o1, o2, s, km, s2, km2, v1, v2;
   if (n == N && pair_supported(q_same, v)) {
     const Paired a = pair_fwd(q_same, q_opp, k, v, 1.0 / n, 1e-6);
@@ -768,34 +830,57 @@ std::vector<Tensor> pola_bwd(const Tensor& g, const Tensor& x, const Tensor& src
                              const std::array<bool, 2 + kPola>& need, const std::array<bool, 3>& kernel) {
   const NoGraph none;
   const PolaWeights p = pola_weights(params);
-  TORCH_CHECK(saved.size() == 20);
-  auto at_ = [&](int i) { return given(saved[i]); };
-  const Tensor scale = at_(0), sigmoid = at_(1), power = at_(2), qg = at_(3), kv = at_(4), q_same = at_(5), q_opp = at_(6), k = at_(7),
-               v = at_(8), grid = at_(9), local = at_(10), o1 = at_(11), o2 = at_(12), s = at_(13), km = at_(14), s2 = at_(15), km2 = at_(16),
-               v1 = at_(17), v2 = at_(18), merged = at_(19);
+  auto at_ = [&](int i) { return given(saved.at(i)); };
+  const bool rows_ = saved.size() == 10;
+  const Tensor scale = at_(0), sigmoid = at_(1), power = at_(2), qg = at_(3), kv = at_(4), merged = at_(rows_ ? 9 : 19);
   const int64_t n = src.size(1), C = x.size(2);
   std::vector<Tensor> r(2 + kPola);
   std::tie(r[11], r[12]) = weight_grad(g, merged, need[11], need[12], kernel[2]);
   if (std::none_of(need.begin(), need.begin() + 11, [](bool b) { return b; })) return r;
-  const MergeGrads m = merge_bwd(input_grad(g, p.proj_w), heads, true, o1, o2, local, qg.narrow(2, C, C));
-  if (need[9] || need[10]) std::tie(r[9], r[10]) = dwconv_grad(grid, m.local, p.conv_w, H, W, need[10]);
-  if (std::none_of(need.begin(), need.begin() + 9, [](bool b) { return b; })) return r;
-  const Tensor dv_rows = local_values_grad(m.local, n, p.conv_w, H, W);
-  PairedGrads d;
-  if (!s2.defined()) {
-    d = pair_bwd(q_same, q_opp, k, v, m.o, m.o2, s, km, 1.0 / n, 1e-6);
+  const Tensor dmerged = input_grad(g, p.proj_w);
+  std::array<Tensor, 5> d;  // of qg, kv, pe, scale, power
+  if (rows_) {
+    const Tensor grid = at_(5), local = at_(6), pe = whole(p.pe), dlocal = like(dmerged);
+    d = {like(qg), like(kv), like(pe), like(scale), like(power)};
+    fbla_block_attn a = row_args(kPolarity, qg, 0, kv, 0, kv, C, heads, {at_(7), at_(8)});
+    const Tensor ws = row_workspace(a, x);
+    auto half = [&](const Tensor& t) { return static_cast<char*>(ptr(t)) + C * t.element_size(); };
+    a.local = ptr(local), a.gate = half(qg), a.gate_row = 2 * C, a.dout = ptr(dmerged), a.pe = ptr(pe), a.scale = ptr(scale);
+    a.power = ptr(power), a.workspace = ptr(ws), a.workspace_bytes = ws.numel(), a.dq = ptr(d[0]), a.dgate = half(d[0]), a.dlocal = ptr(dlocal);
+    a.dk = ptr(d[1]), a.dv = half(d[1]), a.dq_row = a.dgate_row = a.dk_row = a.dv_row = 2 * C;
+    a.dpe = ptr(d[2]), a.dscale = ptr(d[3]), a.dpower = ptr(d[4]);
+    {
+      const On on(x);
+      check(api.fbla_block_attn_backward_queries(&a, on.stream), "fbla_block_attn_backward_queries");
+    }
+    if (need[9] || need[10]) std::tie(r[9], r[10]) = dwconv_grad(grid, dlocal, p.conv_w, H, W, need[10]);
+    if (std::none_of(need.begin(), need.begin() + 9, [](bool b) { return b; })) return r;
+    const Tensor dv_rows = local_values_grad(dlocal, n, p.conv_w, H, W);
+    a.dv_more = ptr(dv_rows);
+    const On on(x);
+    check(api.fbla_block_attn_backward_keys(&a, on.stream), "fbla_block_attn_backward_keys");
   } else {
-    const AttendedGrads a = la_bwd(q_same, k, v1, Tensor(), Tensor(), m.o, s, km, 1.0 / n, 1e-6, FBLA_NORMALIZE);
-    const AttendedGrads b = la_bwd(q_opp, k, v2, Tensor(), Tensor(), m.o2, s2, km2, 1.0 / n, 1e-6, FBLA_NORMALIZE);
-    d = {a.q, b.q, at::add(a.k, b.k), at::cat({a.v, b.v}, -1)};
+    const Tensor q_same = at_(5), q_opp = at_(6), k = at_(7), v = at_(8), grid = at_(9), s = at_(13), km = at_(14), s2 = at_(15);
+    const MergeGrads m = merge_bwd(dmerged, heads, true, at_(11), at_(12), at_(10), qg.narrow(2, C, C));
+    if (need[9] || need[10]) std::tie(r[9], r[10]) = dwconv_grad(grid, m.local, p.conv_w, H, W, need[10]);
+    if (std::none_of(need.begin(), need.begin() + 9, [](bool b) { return b; })) return r;
+    const Tensor dv_rows = local_values_grad(m.local, n, p.conv_w, H, W);
+    PairedGrads pd;
+    if (!s2.defined()) {
+      pd = pair_bwd(q_same, q_opp, k, v, m.o, m.o2, s, km, 1.0 / n, 1e-6);
+    } else {
+      const AttendedGrads a = la_bwd(q_same, k, at_(17), Tensor(), Tensor(), m.o, s, km, 1.0 / n, 1e-6, FBLA_NORMALIZE);
+      const AttendedGrads b = la_bwd(q_opp, k, at_(18), Tensor(), Tensor(), m.o2, s2, at_(16), 1.0 / n, 1e-6, FBLA_NORMALIZE);
+      pd = {a.q, b.q, at::add(a.k, b.k), at::cat({a.v, b.v}, -1)};
+    }
+    d = polarity_bwd(qg, kv, p.pe, scale, power, heads, pd.q1, pd.q2, pd.k, pd.v, dv_rows, m.gate);
   }
-  const auto [dqg, dkv, dpe, dscale, dpower] = polarity_bwd(qg, kv, p.pe, scale, power, heads, d.q1, d.q2, d.k, d.v, dv_rows, m.gate);
-  std::tie(r[0], r[1]) = two_input_grads(dqg, p.q_w, need[0], dkv, p.kv_w, same, need[1]);
-  std::tie(r[2], r[3]) = weight_grad(dqg, x, need[2], need[3], kernel[0]);
-  std::tie(r[4], r[5]) = weight_grad(dkv, src, need[4], need[5], kernel[1]);
-  if (need[6]) r[6] = dpe;
-  if (need[7]) r[7] = at::softplus_backward(dscale, p.scale, 1, 20);
-  if (need[8]) r[8] = at::sigmoid_backward(at::mul(dpower, alpha), sigmoid);
+  std::tie(r[0], r[1]) = two_input_grads(d[0], p.q_w, need[0], d[1], p.kv_w, same, need[1]);
+  std::tie(r[2], r[3]) = weight_grad(d[0], x, need[2], need[3], kernel[0]);
+  std::tie(r[4], r[5]) = weight_grad(d[1], src, need[4], need[5], kernel[1]);
+  if (need[6]) r[6] = d[2];
+  if (need[7]) r[7] = at::softplus_backward(d[3], p.scale, 1, 20);
+  if (need[8]) r[8] = at::sigmoid_backward(at::mul(d[4], alpha), sigmoid);
   return r;
 }
 
@@ -1182,8 +1267,7 @@ PYBIND11_MODULE(fbla_torch, m) {
   });
   m.def("mlla_bwd", [](const Tensor& g, const Tensor& x, const Tensor& w, const Tensor& conv_w, const Tensor& rotations,
                        const std::vector<Tensor>& s, int64_t side, int64_t heads, const std::array<bool, 5>& need, bool kernel) {
-    return listed(mlla_bwd(g, x, w, conv_w, rotations, s.at(0), s.at(1), s.at(2), s.at(3), s.at(4), s.at(5), s.at(6), s.at(7), side, heads,
-                           need, kernel));
+    return listed(mlla_bwd(g, x, w, conv_w, rotations, s, side, heads, need, kernel));
   });
   m.def("pola_fwd", [](const Tensor& x, const Tensor& src, const std::vector<Maybe>& p, double alpha, int64_t H, int64_t W, int64_t heads) {
     return listed(pola_fwd(x, src, p, alpha, H, W, heads));

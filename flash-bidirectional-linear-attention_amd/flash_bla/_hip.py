@@ -94,6 +94,11 @@ _SIGNATURES = {
     "fbla_rotary_bwd": (_i32, [_vp] * 2 + [_i32] + [_vp] * 8 + [_i64] * 2 + [_i32] * 3 + [_vp]),
     "fbla_merge_fwd": (_i32, [_vp] * 4 + [_i64, _vp] + [_i64] * 2 + [_i32] * 3 + [_vp]),
     "fbla_merge_bwd": (_i32, [_vp] * 5 + [_i64] + [_vp] * 4 + [_i64] * 2 + [_i32] * 3 + [_vp]),
+    "fbla_block_attn_workspace_bytes": (_sz, [_i32] + [_i64] * 3 + [_i32]),
+    "fbla_block_attn_state_elements": (_sz, [_i32, _i64, _i32]),
+    "fbla_block_attn_forward": (_i32, [_vp, _vp]),
+    "fbla_block_attn_backward_queries": (_i32, [_vp, _vp]),
+    "fbla_block_attn_backward_keys": (_i32, [_vp, _vp]),
     "fbla_turn_fwd": (_i32, [_vp] * 7 + [_i64] * 2 + [_i32] * 3 + [_vp]),
     "fbla_turn_bwd": (_i32, [_vp] * 9 + [_i64] * 2 + [_i32] * 3 + [_vp]),
     "fbla_focus_fwd": (_i32, [_vp] * 7 + [_i64] * 3 + [_i32] * 3 + [_vp]),

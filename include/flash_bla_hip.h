@@ -377,6 +377,39 @@ int fbla_focus_bwd(const void* q, const void* kv, const void* pe, const void* sc
                    void* dscale, void* workspace, size_t workspace_bytes, int64_t B, int64_t N, int64_t Nk, int heads, int d,
                    int dtype, void* stream);
 
+/* The attention of two vision blocks on their projections' rows, heads of 32 channels, fp16 / bf16 (C = 32 * heads): with
+ * features, state, output, merge and gate of flash_bla/layers/polaformer.py:63-104 (kind 0: polarity features of q and k, values v,
+ * local values, gate; pe [Nk, C], scale [C], power [C] at least 1) or flash_bla/layers/mlla.py:74-92 (kind 1: rotary features of q
+ * and k before elu + 1, values v, local values; N = Nk, rot fp32 [N, C / 2, 2]).  Rows of q, k, v, gate, dq, dk, dv, dgate lie
+ * *_row elements apart (whole 16-byte pieces, at least C; batches one after the other); local, out, dout, dlocal, dv_more are
+ * contiguous rows of C.
+ *
+ * forward: out = (attention + local) * gate (kind 1: no gate); state_planes (fbla_block_attn_state_elements of the type) and
+ * state_km (fp32 [B, heads, 72] or [.., 40]) are written for the backward.  backward_queries: dout -> dq, kind 0 also dgate and
+ * dlocal (kind 1: dlocal is dout).  backward_keys, after it with the same workspace: dk, dv = its gradient + dv_more, kind 0 also
+ * dpe, dscale, dpower.  workspace: fbla_block_attn_workspace_bytes, any contents before forward and backward_queries. */
+typedef struct {
+  int32_t kind, dtype, B, N, Nk, heads;
+  float eps;
+  const void *q, *k, *v, *local, *gate;
+  int64_t q_row, k_row, v_row, gate_row;
+  const void *pe, *scale, *power;
+  const float* rot;
+  void *out, *state_planes;
+  float* state_km;
+  const void *dout, *dv_more;
+  void *dq, *dk, *dv, *dlocal, *dgate;
+  int64_t dq_row, dk_row, dv_row, dgate_row;
+  void *dpe, *dscale, *dpower;
+  void* workspace;
+  size_t workspace_bytes;
+} fbla_block_attn;
+size_t fbla_block_attn_workspace_bytes(int kind, int64_t B, int64_t N, int64_t Nk, int heads);
+size_t fbla_block_attn_state_elements(int kind, int64_t B, int heads);
+int fbla_block_attn_forward(const fbla_block_attn* a, void* stream);
+int fbla_block_attn_backward_queries(const fbla_block_attn* a, void* stream);
+int fbla_block_attn_backward_keys(const fbla_block_attn* a, void* stream);
+
 /* Weighted and turned heads (flash_bla/layers/rala.py:60-69): k_out = k * weight, q_rot and k_rot = the channel pairs of q and
  * of k_out (before its rounding) turned by rot (fp32 [N, d / 2, 2]: cos, sin).  All heads are [B, heads, N, d], weight
  * [B, heads, N]; d a power of two of at most 64 16-byte pieces.  The backward gives the gradients through these outputs
