@@ -910,7 +910,7 @@ static int block_attn(const char* name, const fbla_block_attn* p, int what, rows
       return kErrUnsupported;
     }
   a = {pola, p->B, p->N, p->Nk, p->heads, p->eps, p->q, p->k, p->v, p->local, p->gate, p->q_row, p->k_row, p->v_row, p->gate_row, p->pe,
-       p->scale, p->power, p->rot, p->out, p->state_planes, p->state_km, p->dout, p->dv_more, p->dq, p->dk, p->dv, p->dlocal, p->dgate,
+       p->scale, p->power, p->alpha, p->rot, p->out, p->state_planes, p->state_km, p->dout, p->dv_more, p->dq, p->dk, p->dv, p->dlocal, p->dgate,
        p->dq_row, p->dk_row, p->dv_row, p->dgate_row, p->dpe, p->dscale, p->dpower, p->workspace};
   if (p->workspace_bytes < rows::workspace_bytes(a)) {
     set_error("%s: workspace too small (%zu < %zu bytes)", name, p->workspace_bytes, rows::workspace_bytes(a));

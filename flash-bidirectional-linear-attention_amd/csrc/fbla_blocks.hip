@@ -273,8 +273,8 @@ __global__ __launch_bounds__(kThreads) void polarity_bwd_kernel(Shape s, Polarit
 // sums of the positional term.
 template <typename T>
 __global__ __launch_bounds__(kThreads) void features_finish_kernel(int C, int stats_of, int by, int wgs, const float* __restrict__ partial,
-                                                                   const T* __restrict__ scale, T* __restrict__ dscale,
-                                                                   T* __restrict__ dpower, int stat_wgs, int groups,
+                                                                   const T* __restrict__ scale, const T* __restrict__ raw_power,
+                                                                   float alpha, T* __restrict__ dscale, T* __restrict__ dpower, int stat_wgs, int groups,
                                                                    int64_t pe_count, const float* __restrict__ pe_partial,
                                                                    T* __restrict__ dpe) {
   constexpr int kParts = 16, kLanes = kThreads / kParts;
@@ -305,10 +305,13 @@ __global__ __launch_bounds__(kThreads) void features_finish_kernel(int C, int st
   for (int j = 0; j < 4; ++j) {
     const int64_t c = at + j;
     if (!stats) dpe[c] = (T)sum[j];
-    else if (c >= C) dpower[c - C] = (T)sum[j];
-    else {
-      const A inv = A(1) / (A)scale[c];
-      dscale[c] = (T)(by == 1 ? -sum[j] * inv : -sum[j] * inv * inv);
+    else if (c >= C) {
+      const float s = raw_power ? sigmoid((float)raw_power[c - C]) : 0.f;
+      dpower[c - C] = (T)(raw_power ? sum[j] * (A)(alpha * s * (1.f - s)) : sum[j]);
+    } else {
+      const float p = (float)scale[c];
+      const A inv = A(1) / (A)(raw_power ? softplus(p) : p), d = by == 1 ? -sum[j] * inv : -sum[j] * inv * inv;
+      dscale[c] = (T)(raw_power ? d * (A)sigmoid(p) : d);
     }
   }
 }
@@ -882,17 +885,17 @@ void polarity_bwd(const Shape& s, const Polarity<const void>& a, const PolarityG
     float* pe_partial = workspace + (int64_t)2 * C * wgs;
     polarity_bwd_kernel<T><<<dim3((unsigned)wgs, (unsigned)w.channel_wgs), dim3(kThreads), 0, st>>>(
         s, typed<T, Polarity>(a), typed<T, PolarityGrads>(g), (T*)dqg, (T*)dkv, workspace, pe_partial, w.q_wgs, w.groups);
-    features_finish(C, wgs, workspace, a.scale, dscale, dpower, w.groups, (int64_t)s.Nk * C, pe_partial, dpe, dtype, st);
+    features_finish(C, wgs, workspace, a.scale, {}, dscale, dpower, w.groups, (int64_t)s.Nk * C, pe_partial, dpe, dtype, st);
   });
 }
 
-void features_finish(int C, int terms, const float* partial, const void* scale, void* dscale, void* dpower, int groups,
+void features_finish(int C, int terms, const float* partial, const void* scale, RawPower raw, void* dscale, void* dpower, int groups,
                      int64_t pe_count, const float* pe_partial, void* dpe, int dtype, hipStream_t st) {
   by_type(dtype, [&](auto tag) {
     using T = decltype(tag);
     const int stat_wgs = (2 * C + 63) / 64;
     features_finish_kernel<T><<<dim3((unsigned)(stat_wgs + cdiv64(pe_count, 64))), dim3(kThreads), 0, st>>>(
-        C, 2, 2, terms, partial, (const T*)scale, (T*)dscale, (T*)dpower, stat_wgs, groups, pe_count, pe_partial, (T*)dpe);
+        C, 2, 2, terms, partial, (const T*)scale, (const T*)raw.power, raw.alpha, (T*)dscale, (T*)dpower, stat_wgs, groups, pe_count, pe_partial, (T*)dpe);
   });
 }
 
@@ -1011,7 +1014,7 @@ void focus_bwd(const Shape& s, const Focus<const void>& a, const FocusGrads<cons
     const int64_t pe_count = (int64_t)s.Nk * C;
     const int stat_wgs = (C + 63) / 64;
     features_finish_kernel<T><<<dim3((unsigned)(stat_wgs + cdiv64(pe_count, 64))), dim3(kThreads), 0, st>>>(
-        C, 1, 1, wgs, workspace, (const T*)a.scale, (T*)dscale, nullptr, stat_wgs, w.groups, pe_count, pe_partial, (T*)dpe);
+        C, 1, 1, wgs, workspace, (const T*)a.scale, nullptr, 0.f, (T*)dscale, nullptr, stat_wgs, w.groups, pe_count, pe_partial, (T*)dpe);
   });
 }
 

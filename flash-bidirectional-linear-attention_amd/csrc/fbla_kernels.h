@@ -293,8 +293,15 @@ template <typename P> struct FocusGrads {
   P *q, *k, *v, *v_rows;  // heads of d; rows of C
 };
 int vec_of(int dtype);  // elements of a piece
+// Scale and power as a block's parameters: softplus(scale) and 1 + alpha sigmoid(power) are what the features use.
+__device__ __forceinline__ float sigmoid(float x) { return 1.f / (1.f + expf(-x)); }
+__device__ __forceinline__ float softplus(float x) { return x > 20.f ? x : log1pf(expf(x)); }
+struct RawPower {
+  const void* power;  // null: scale and power (and their gradients) are the features' own
+  float alpha;
+};
 // sums of the partials of polarity gradients: dscale, dpower [C] from `terms` x [2][C], dpe [pe_count] from `groups` x [pe_count]
-void features_finish(int C, int terms, const float* partial, const void* scale, void* dscale, void* dpower, int groups,
+void features_finish(int C, int terms, const float* partial, const void* scale, RawPower raw, void* dscale, void* dpower, int groups,
                      int64_t pe_count, const float* pe_partial, void* dpe, int dtype, hipStream_t st);
 int most_row_channels(int dtype);  // of rows that are normalised over their channels (focus_*)
 void focus_fwd(const Shape& s, const Focus<const void>& a, void* q, void* k, void* v, int dtype, hipStream_t st);
@@ -334,7 +341,8 @@ struct Attn {
   // rows of 32 * heads channels, `_row` elements apart, batches one after the other; local, dout, dlocal, dv_more, out: without gaps
   const void *q, *k, *v, *local, *gate;
   int64_t q_row, k_row, v_row, gate_row;
-  const void *pe, *scale, *power;  // polarity
+  const void *pe, *scale, *power;  // polarity: q and k + pe over softplus(scale), to 1 + alpha sigmoid(power)
+  float alpha;
   const float* rot;                // rotary: fp32 [N][C / 2][2]
   void* out;
   void* planes;  // state, written by the forward: planes_elements of the type

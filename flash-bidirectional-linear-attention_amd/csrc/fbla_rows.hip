@@ -18,9 +18,9 @@
 // (32), M = S, the denominator from the plain features.  Matrices are operands as hi + lo pairs of 16 bits.
 //
 // Measured, bf16, heads as kernels of their own (features to heads, both operators, merge and gate, and the gradients of each) ->
-// here, with what each reaches of the bytes it moves: PolaFormer's 64 x 28x28 x 256: forward 136 -> 64 us (state 20 us, 2.6 TB/s;
-// output 33 us, 3.1 TB/s), backward 270 -> 128 us (queries 61 us, 2.9 TB/s; keys 55 us, 2.6 TB/s; the two finishing launches 11 us
-// each), the whole step 750 -> 555 us.  MLLA's 64 x 56x56 x 64: forward 84 -> 48 us (state 17, output 24 us, 3.3 TB/s), backward
+// here, with what each reaches of the bytes it moves: PolaFormer's 64 x 28x28 x 256: forward 136 -> 62 us (state 21 us, 2.6 TB/s;
+// output 33 us, 3.1 TB/s), backward 270 -> 131 us (queries 61 us, 2.9 TB/s; keys 55 us, 2.6 TB/s; the two finishing launches 7 us
+// each), the whole step 750 -> 525 us.  MLLA's 64 x 56x56 x 64: forward 84 -> 48 us (state 17, output 24 us, 3.3 TB/s), backward
 // 139 -> 71 us (queries 30, keys 33 us, 3.9 TB/s), the step 371 -> 252 us.  What was tried and cost time: three waves a SIMD for
 // state and output (4 spilled registers each: 24 and 35 us), two tiles a wave for the keys (256 registers: 72 us), shuffles of each
 // sum by itself at the end of the queries' pass (86 us), LDS addresses kept over the tiles (76 spilled: 141 us).
@@ -187,14 +187,14 @@ struct Place {
     subs = kWaves / group_heads;
   }
 };
-// 1 / scale and power of the head's channels, in LDS (64 floats a wave): registers are what these kernels are short of
+// 1 / scale and power of the head's channels from their parameters, in LDS (64 floats a wave): registers are what these kernels are short of
 template <typename T, bool POLA> struct Constants {
   float* at;
   int c0;
   __device__ __forceinline__ Constants(float* to, const Attn& a, const Place& p) : at(to), c0(8 * p.kb) {
     if constexpr (POLA) {
       const int c = p.h * D + p.t;
-      at[p.lane] = p.kb ? (float)((const T*)a.power)[c] : 1.f / (float)((const T*)a.scale)[c];
+      at[p.lane] = p.kb ? 1.f + a.alpha * blocks::sigmoid((float)((const T*)a.power)[c]) : 1.f / blocks::softplus((float)((const T*)a.scale)[c]);
     }
   }
   __device__ __forceinline__ f32x8 inv(int s) const { return POLA ? load_f8(at + 16 * s + c0) : f32x8{}; }
@@ -301,13 +301,15 @@ __global__ __launch_bounds__(kThreads, 2) void state_kernel(Attn a, float* __res
 // ---------------------------------------------------------------------------------------------------------------
 // the partials' sum, in order, as operands: planes [f][v] hi, lo and [v][f] hi, lo of `scale` times the matrix, brought to a largest
 // value of 8 to 16 by a power of two (as 16-bit pairs it would lose to denormals otherwise), and `scale` times the vector, followed by
-// the factor that takes the power back.  Forward: M and the mean key; backward, from the sums of M's gradient: S's and the mean key's.
+// the factor that takes the power back.  Through LDS to 16-byte pieces of both orders (2 bytes at a time: 11 us, 512 heads, four
+// partials; so 7 us).  Forward: M and the mean key; backward, from the sums of M's gradient: S's and the mean key's.
 // ---------------------------------------------------------------------------------------------------------------
 template <typename T, bool POLA>
 __global__ __launch_bounds__(kThreads) void finish_kernel(const float* __restrict__ partial, int parts, float scale, T* __restrict__ planes,
                                                           float* __restrict__ vec) {
   constexpr int F = kFeatures<POLA>, E = F * D, kEach = E / kThreads;
-  __shared__ float largest[kWaves];
+  static_assert(E / 8 <= kThreads);
+  __shared__ float largest[kWaves], matrix[F][D + 1];
   const int64_t head = blockIdx.x;
   const float* from = partial + head * parts * kSlot<POLA>;
   float x[kEach] = {}, y = 0.f, most = 0.f;
@@ -331,17 +333,24 @@ __global__ __launch_bounds__(kThreads) void finish_kernel(const float* __restric
     frexpf(most, &e);
     norm = ldexpf(1.f, 4 - e);
   }
-  T* to = planes + head * 4 * E;
 #pragma unroll
   for (int e = 0; e < kEach; ++e) {
     const int at = threadIdx.x + kThreads * e, f = at / D, v = at % D;
-    const int g = POLA && v >= 16 ? f ^ 32 : f;  // the last value channels pair with the swapped halves
-    const float z = x[e] * norm;
-    const T hi = (T)z, lo = (T)(z - (float)hi);
-    to[g * D + v] = hi;
-    to[E + g * D + v] = lo;
-    to[2 * E + v * F + g] = hi;
-    to[3 * E + v * F + g] = lo;
+    matrix[POLA && v >= 16 ? f ^ 32 : f][v] = x[e] * norm;  // the last value channels pair with the swapped halves
+  }
+  __syncthreads();
+  T* to = planes + head * 4 * E;
+  auto write = [&](T* plane, auto at) {  // 8 values of a row of the plane, hi and lo
+    f32x8 z;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) z[e] = at(e);
+    const V8<T> hi = narrow<T>(z);
+    *reinterpret_cast<V8<T>*>(plane) = hi;
+    *reinterpret_cast<V8<T>*>(plane + E) = narrow<T>(z - wide<T>(hi));
+  };
+  if (const int q = threadIdx.x; q < E / 8) {
+    write(to + 8 * q, [&](int e) { return matrix[q / (D / 8)][8 * (q % (D / 8)) + e]; });
+    write(to + 2 * E + 8 * q, [&](int e) { return matrix[8 * (q % (F / 8)) + e][q / (F / 8)]; });
   }
   if ((int)threadIdx.x < F) vec[head * kVector<POLA> + threadIdx.x] = y * scale;
   if (threadIdx.x == 0) vec[head * kVector<POLA> + F] = 1.f / norm;
@@ -894,7 +903,7 @@ template <typename T, bool POLA> void bwd_keys_t(const Attn& a, int dtype, hipSt
   keys_kernel<T, POLA><<<dim3(w.key_tiles, a.heads / g, w.groups), dim3(kThreads), 0, st>>>(
       a, (const T*)c.planes, c.dkm, c.stats + (size_t)w.query_rows * 2 * a.heads * D, c.pe, w.groups, g);
   if (POLA)
-    blocks::features_finish(a.heads * D, w.query_rows + w.key_rows, c.stats, a.scale, a.dscale, a.dpower, w.groups, (int64_t)a.Nk * a.heads * D,
+    blocks::features_finish(a.heads * D, w.query_rows + w.key_rows, c.stats, a.scale, {a.power, a.alpha}, a.dscale, a.dpower, w.groups, (int64_t)a.Nk * a.heads * D,
                             c.pe, a.dpe, dtype, st);
 }
 

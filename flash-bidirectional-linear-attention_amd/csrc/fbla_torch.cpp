@@ -679,7 +679,7 @@ struct NoGraph {  // (called inside an autograd function or without gradients: n
 // The attention between the projections' rows and the block's, where the kernels of fbla_rows.hip take it: 16-bit types, heads of
 // 32 channels.  `rows` are the projections with queries (and keys) first in a row.
 constexpr int kPolarity = 0, kRotary = 1;
-bool on_rows(const Tensor& x, int64_t heads) { return x.element_size() == 2 && x.size(2) == 32 * heads && x.size(0) <= 65535 && heads <= 2048; }
+bool on_rows(const Tensor& x, int64_t heads) { return x.element_size() == 2 && x.size(2) == 32 * heads && x.size(0) <= 65535 && x.size(1) <= 1 << 24 && heads <= 2048; }
 struct RowState {
   Tensor planes, km;
 };
@@ -791,22 +791,22 @@ std::vector<Tensor> pola_fwd(const Tensor& x, const Tensor& src, const std::vect
   const NoGraph none;
   const PolaWeights p = pola_weights(params);
   const int64_t N = x.size(1), n = src.size(1), C = x.size(2);
-  const Tensor scale = at::softplus(p.scale), sigmoid = at::sigmoid(p.power), power = at::add(at::mul(sigmoid, alpha), 1);
   const auto [qg, kv] = two_linears({x, p.q_w, p.q_b, Tensor()}, {src, p.kv_w, p.kv_b, Tensor()});
   const LocalValues l = local_values(kv.narrow(2, C, C), N, p.conv_w, p.conv_b, H, W);
   if (on_rows(x, heads)) {
-    const Tensor merged = like(l.local), pe = whole(p.pe);
+    const Tensor merged = like(l.local), pe = whole(p.pe), scale = whole(p.scale), power = whole(p.power);
     const RowState state = new_row_state(kPolarity, x, heads);
     fbla_block_attn a = row_args(kPolarity, qg, 0, kv, 0, kv, C, heads, state);
     const Tensor ws = row_workspace(a, x);
     a.local = ptr(l.local), a.gate = static_cast<char*>(ptr(qg)) + C * qg.element_size(), a.gate_row = 2 * C, a.out = ptr(merged);
-    a.pe = ptr(pe), a.scale = ptr(scale), a.power = ptr(power), a.workspace = ptr(ws), a.workspace_bytes = ws.numel();
+    a.pe = ptr(pe), a.scale = ptr(scale), a.power = ptr(power), a.alpha = alpha, a.workspace = ptr(ws), a.workspace_bytes = ws.numel();
     {
       const On on(x);
       check(api.fbla_block_attn_forward(&a, on.stream), "fbla_block_attn_forward");
     }
-    return {linear(merged, p.proj_w, p.proj_b), scale, sigmoid, power, qg, kv, l.grid, l.local, state.planes, state.km, merged};
+    return {linear(merged, p.proj_w, p.proj_b), qg, kv, l.grid, l.local, state.planes, state.km, merged};
   }
+  const Tensor scale = at::softplus(p.scale), sigmoid = at::sigmoid(p.power), power = at::add(at::mul(sigmoid, alpha), 1);
   const auto [q_same, q_opp, k, v] = polarity_fwd(qg, kv, p.pe, scale, power, heads);
   Tensor o1, o2, s, km, s2, km2, v1, v2;
   if (n == N && pair_supported(q_same, v)) {
@@ -831,8 +831,9 @@ std::vector<Tensor> pola_bwd(const Tensor& g, const Tensor& x, const Tensor& src
   const NoGraph none;
   const PolaWeights p = pola_weights(params);
   auto at_ = [&](int i) { return given(saved.at(i)); };
-  const bool rows_ = saved.size() == 10;
-  const Tensor scale = at_(0), sigmoid = at_(1), power = at_(2), qg = at_(3), kv = at_(4), merged = at_(rows_ ? 9 : 19);
+  const bool rows_ = saved.size() == 7;
+  TORCH_CHECK(rows_ || saved.size() == 20);
+  const Tensor qg = at_(rows_ ? 0 : 3), kv = at_(rows_ ? 1 : 4), merged = at_(rows_ ? 6 : 19);
   const int64_t n = src.size(1), C = x.size(2);
   std::vector<Tensor> r(2 + kPola);
   std::tie(r[11], r[12]) = weight_grad(g, merged, need[11], need[12], kernel[2]);
@@ -840,13 +841,13 @@ std::vector<Tensor> pola_bwd(const Tensor& g, const Tensor& x, const Tensor& src
   const Tensor dmerged = input_grad(g, p.proj_w);
   std::array<Tensor, 5> d;  // of qg, kv, pe, scale, power
   if (rows_) {
-    const Tensor grid = at_(5), local = at_(6), pe = whole(p.pe), dlocal = like(dmerged);
+    const Tensor grid = at_(2), local = at_(3), pe = whole(p.pe), scale = whole(p.scale), power = whole(p.power), dlocal = like(dmerged);
     d = {like(qg), like(kv), like(pe), like(scale), like(power)};
-    fbla_block_attn a = row_args(kPolarity, qg, 0, kv, 0, kv, C, heads, {at_(7), at_(8)});
+    fbla_block_attn a = row_args(kPolarity, qg, 0, kv, 0, kv, C, heads, {at_(4), at_(5)});
     const Tensor ws = row_workspace(a, x);
     auto half = [&](const Tensor& t) { return static_cast<char*>(ptr(t)) + C * t.element_size(); };
     a.local = ptr(local), a.gate = half(qg), a.gate_row = 2 * C, a.dout = ptr(dmerged), a.pe = ptr(pe), a.scale = ptr(scale);
-    a.power = ptr(power), a.workspace = ptr(ws), a.workspace_bytes = ws.numel(), a.dq = ptr(d[0]), a.dgate = half(d[0]), a.dlocal = ptr(dlocal);
+    a.power = ptr(power), a.alpha = alpha, a.workspace = ptr(ws), a.workspace_bytes = ws.numel(), a.dq = ptr(d[0]), a.dgate = half(d[0]), a.dlocal = ptr(dlocal);
     a.dk = ptr(d[1]), a.dv = half(d[1]), a.dq_row = a.dgate_row = a.dk_row = a.dv_row = 2 * C;
     a.dpe = ptr(d[2]), a.dscale = ptr(d[3]), a.dpower = ptr(d[4]);
     {
@@ -860,7 +861,7 @@ std::vector<Tensor> pola_bwd(const Tensor& g, const Tensor& x, const Tensor& src
     const On on(x);
     check(api.fbla_block_attn_backward_keys(&a, on.stream), "fbla_block_attn_backward_keys");
   } else {
-    const Tensor q_same = at_(5), q_opp = at_(6), k = at_(7), v = at_(8), grid = at_(9), s = at_(13), km = at_(14), s2 = at_(15);
+    const Tensor scale = at_(0), power = at_(2), q_same = at_(5), q_opp = at_(6), k = at_(7), v = at_(8), grid = at_(9), s = at_(13), km = at_(14), s2 = at_(15);
     const MergeGrads m = merge_bwd(dmerged, heads, true, at_(11), at_(12), at_(10), qg.narrow(2, C, C));
     if (need[9] || need[10]) std::tie(r[9], r[10]) = dwconv_grad(grid, m.local, p.conv_w, H, W, need[10]);
     if (std::none_of(need.begin(), need.begin() + 9, [](bool b) { return b; })) return r;
@@ -879,8 +880,8 @@ std::vector<Tensor> pola_bwd(const Tensor& g, const Tensor& x, const Tensor& src
   std::tie(r[2], r[3]) = weight_grad(d[0], x, need[2], need[3], kernel[0]);
   std::tie(r[4], r[5]) = weight_grad(d[1], src, need[4], need[5], kernel[1]);
   if (need[6]) r[6] = d[2];
-  if (need[7]) r[7] = at::softplus_backward(d[3], p.scale, 1, 20);
-  if (need[8]) r[8] = at::sigmoid_backward(at::mul(d[4], alpha), sigmoid);
+  if (need[7]) r[7] = rows_ ? d[3] : at::softplus_backward(d[3], p.scale, 1, 20);
+  if (need[8]) r[8] = rows_ ? d[4] : at::sigmoid_backward(at::mul(d[4], alpha), at_(1));
   return r;
 }
 

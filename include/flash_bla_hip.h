@@ -379,7 +379,8 @@ int fbla_focus_bwd(const void* q, const void* kv, const void* pe, const void* sc
 
 /* The attention of two vision blocks on their projections' rows, heads of 32 channels, fp16 / bf16 (C = 32 * heads): with
  * features, state, output, merge and gate of flash_bla/layers/polaformer.py:63-104 (kind 0: polarity features of q and k, values v,
- * local values, gate; pe [Nk, C], scale [C], power [C] at least 1) or flash_bla/layers/mlla.py:74-92 (kind 1: rotary features of q
+ * local values, gate; pe [Nk, C], scale [C] and power [C] the parameters: over softplus(scale), to 1 + alpha sigmoid(power),
+ * alpha >= 0) or flash_bla/layers/mlla.py:74-92 (kind 1: rotary features of q
  * and k before elu + 1, values v, local values; N = Nk, rot fp32 [N, C / 2, 2]).  Rows of q, k, v, gate, dq, dk, dv, dgate lie
  * *_row elements apart (whole 16-byte pieces, at least C; batches one after the other); local, out, dout, dlocal, dv_more are
  * contiguous rows of C.
@@ -394,6 +395,7 @@ typedef struct {
   const void *q, *k, *v, *local, *gate;
   int64_t q_row, k_row, v_row, gate_row;
   const void *pe, *scale, *power;
+  float alpha;
   const float* rot;
   void *out, *state_planes;
   float* state_km;
