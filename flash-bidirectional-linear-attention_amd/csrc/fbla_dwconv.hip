@@ -24,6 +24,7 @@ namespace {
 constexpr int kThreads = 256;
 constexpr float kLargest = 3.40282347e38f;  // of fp32
 constexpr int kFinishParts = 32;    // threads that share the terms of one filter's gradient
+constexpr int kAtOnce = 2;          // channels of a lane that the gradient kernel holds as fp32 at a time
 constexpr int kBlockChannels = 64;  // channels of a workgroup: 128-byte (16-bit) or 256-byte (fp32) pieces of a row
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -163,9 +164,10 @@ __global__ __launch_bounds__(kThreads) void conv_kernel(Conv a, int strips_per_r
 // Weight and bias gradient: partial[chunk][ky][kx][C] = sum over the chunk's strips of g[y, x] * x[y + ky - P,
 // x + kx - P], the bias gradient in row K of ky = 0.  One tap row per workgroup (blockIdx.z): K * V accumulators per
 // lane, kept over all strips of the chunk, added over the workgroup's strips at the end in a fixed order (fp32: sums of g alone
-// and sums over chunks in 64 bits, so that the bias gradient is no further from exact than column sums in a tree).  46 us for the 51 MB
-// of 64 x 28x28 x 256 in bf16, 5x5: the K workgroups of a chunk fetch the same rows, and at 170 to 206 VGPRs two waves fit a
-// SIMD (3x3: three).
+// and sums over chunks in 64 bits, so that the bias gradient is no further from exact than column sums in a tree).  The K
+// workgroups of a chunk fetch the same rows (out of the caches), what bounds it is the latency of a strip's loads: two of a lane's
+// channels are fp32 at a time, so that three waves fit a SIMD (all eight: 173 VGPRs at 5x5, two waves), and the grid
+// is the three workgroups a CU that run at once.  bf16: 64 x 28x28 x 256, 5x5, 46 -> 33 us (51 MB); 64 x 56x56 x 64, 3x3, 29 -> 22 us.
 template <typename T, int K, int STRIP>
 __global__ __launch_bounds__(kThreads) void grad_kernel(Conv a, const T* __restrict__ g, int64_t g_batch, int64_t g_row,
                                                         float* __restrict__ partial, int strips_per_row, int nstrips) {
@@ -195,17 +197,23 @@ __global__ __launch_bounds__(kThreads) void grad_kernel(Conv a, const T* __restr
       Piece<T> gv[STRIP], in[IN];
       load_row<T, STRIP>(g + (int64_t)b * g_batch + (int64_t)y * a.W * g_row + c, g_row, x0, a.W, gv);
       load_row<T, IN>(xc + (int64_t)b * a.x_batch + (int64_t)(inside ? yy : y) * a.W * a.x_row, a.x_row, x0 - P, a.W, in);
+      if (ky == 0) {  // (no other workgroup's is kept)
 #pragma unroll
-      for (int t = 0; t < STRIP; ++t)
+        for (int t = 0; t < STRIP; ++t)
 #pragma unroll
-        for (int j = 0; j < V; ++j) total[j] += (A)gv[t].e[j];
+          for (int j = 0; j < V; ++j) total[j] += (A)gv[t].e[j];
+      }
       if (inside) {
 #pragma unroll
-        for (int kx = 0; kx < K; ++kx)
+        for (int j0 = 0; j0 < V; j0 += kAtOnce) {
 #pragma unroll
-          for (int t = 0; t < STRIP; ++t)
+          for (int kx = 0; kx < K; ++kx)
 #pragma unroll
-            for (int j = 0; j < V; ++j) acc[kx][j] = fmaf((float)gv[t].e[j], (float)in[t + kx].e[j], acc[kx][j]);
+            for (int t = 0; t < STRIP; ++t)
+#pragma unroll
+              for (int j = j0; j < j0 + kAtOnce; ++j) acc[kx][j] = fmaf((float)gv[t].e[j], (float)in[t + kx].e[j], acc[kx][j]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
       }
     }
   }
@@ -305,13 +313,13 @@ __global__ __launch_bounds__(kThreads) void grad_finish_kernel(const float* __re
 // outputs of one lane: the strip length that leaves fewer unused columns in the last strip of a row
 int strip_for(int W) { return ((W + 6) / 7) * 7 < ((W + 7) / 8) * 8 ? 7 : 8; }
 
-// workgroups of the gradient kernel along the strips: about four per CU over all tap rows and channel blocks, no more
-// than there are strips (each chunk costs K * (K + 1) * C partial sums)
+// workgroups of the gradient kernel along the strips: over all tap rows and channel blocks about three per CU, what its registers
+// let run at once, and no more than there are strips (each chunk costs K * (K + 1) * C partial sums)
 int grad_chunks(const Conv& a, int K, int workers) {
   const int s = strip_for(a.W);
   const int64_t nstrips = (int64_t)a.B * a.H * ((a.W + s - 1) / s);
   const int64_t share = (int64_t)K * ((a.C + kBlockChannels - 1) / kBlockChannels);
-  const int64_t want = 1024 / share < 1 ? 1 : 1024 / share;
+  const int64_t want = 768 / share < 1 ? 1 : 768 / share;
   const int64_t most = (nstrips + workers - 1) / workers;
   return (int)(want < most ? want : most);
 }
