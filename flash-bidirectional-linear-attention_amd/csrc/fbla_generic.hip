@@ -564,7 +564,7 @@ __global__ __launch_bounds__(kThreads) void resize_matrices_kernel(const E* __re
 // The same for one matrix of many rows whose number does not change (token tensors): every workgroup takes a
 // span of kResizeSpan consecutive destination elements, thread t the elements t, t + 256, ... of it (whole
 // 128-byte pieces per wave instruction), with one division per thread and the row / column carried along.
-constexpr int kResizePer = 16, kResizeSpan = kThreads * kResizePer;
+constexpr int kResizePer = 16, kResizeSpan = kThreads * kResizePer, kResizeStateSpan = 4 * kThreads;
 template <typename E>
 __global__ __launch_bounds__(kThreads) void resize_rows_kernel(const E* __restrict__ src, int cs, E* __restrict__ dst,
                                                                int cd, int64_t total) {
@@ -625,6 +625,34 @@ void resize_matrices(const void* src, int64_t rs, int cs, void* dst, int64_t rd,
   else
     resize_matrices_kernel<uint32_t><<<dim3(grid), dim3(kThreads), 0, st>>>((const uint32_t*)src, rs, cs, (uint32_t*)dst,
                                                                            rd, cd, total);
+}
+
+// The same for a state's matrices and vectors (when given) together: one launch a direction between a head's own row lengths and
+// the wider ones.  Bound by the launch (two cost 5 us each next to 3 us of bytes, 128 heads of 100 x 100); 32-bit divisions.
+__global__ __launch_bounds__(kThreads) void resize_state_kernel(const float* __restrict__ mat, const float* __restrict__ vec, int rs, int cs,
+                                                                float* __restrict__ mat_to, float* __restrict__ vec_to, int rd, int cd,
+                                                                int blocks_per_head) {
+  const int64_t head = blockIdx.x / blocks_per_head;
+  const int of_mat = rd * cd, total = of_mat + (vec ? rd : 0);
+  const int e0 = (blockIdx.x % blocks_per_head) * kResizeStateSpan + threadIdx.x;
+#pragma unroll
+  for (int u = 0; u < kResizeStateSpan / kThreads; ++u) {
+    const int e = e0 + u * kThreads;
+    if (e >= total) return;
+    if (e < of_mat) {
+      const int r = e / cd, c = e - r * cd;
+      mat_to[head * of_mat + e] = r < rs && c < cs ? mat[(head * rs + r) * cs + c] : 0.f;
+    } else {
+      const int r = e - of_mat;
+      vec_to[head * rd + r] = r < rs ? vec[head * rs + r] : 0.f;
+    }
+  }
+}
+void resize_state(const float* mat, const float* vec, int rs, int cs, float* mat_to, float* vec_to, int rd, int cd, int64_t heads,
+                  hipStream_t st) {
+  const int blocks_per_head = (rd * cd + rd + kResizeStateSpan - 1) / kResizeStateSpan;
+  resize_state_kernel<<<dim3((unsigned)(heads * blocks_per_head)), dim3(kThreads), 0, st>>>(mat, vec, rs, cs, mat_to, vec_to, rd, cd,
+                                                                                            blocks_per_head);
 }
 
 // Two queries sharing keys and values: the state's value columns [0, DV/2) serve the first query,

@@ -81,6 +81,9 @@ void transpose_state(const Prob& p, const float* mat, float* mat_t, hipStream_t 
 // the rest of the destination is zero
 void resize_matrices(const void* src, int64_t rs, int cs, void* dst, int64_t rd, int cd, int64_t count, int elem_bytes,
                      hipStream_t st);
+// the states of `heads` (sequence, head)s, matrix [rs][cs] and vector [rs] (or null), as [rd][cd] and [rd] in the same way
+void resize_state(const float* mat, const float* vec, int rs, int cs, float* mat_to, float* vec_to, int rd, int cd, int64_t heads,
+                  hipStream_t st);
 // p.DV even: the column halves of a [N*H, DK, DV] matrix as two [N*H, DK, DV/2] matrices, and back
 // (join also adds two [N*H, DK] vectors when `vec` is given)
 void split_columns(const Prob& p, const float* mat, float* lo, float* hi, hipStream_t st);

@@ -251,8 +251,7 @@ static int widened_forward(const Prob& p, int dtype, const FwdArgs& a, hipStream
   int rc = forward(w, dtype, b, st);
   if (rc != kOk) return rc;
   generic::resize_matrices(b.o, qr, w.DV, a.o, qr, p.DV, 1, elem_bytes(dtype), st);
-  generic::resize_matrices(b.s, w.DK, w.DV, a.s, p.DK, p.DV, nh, 4, st);
-  if (a.km) generic::resize_matrices(b.km, 1, w.DK, a.km, 1, p.DK, nh, 4, st);
+  generic::resize_state(b.s, a.km ? b.km : nullptr, w.DK, w.DV, a.s, a.km, p.DK, p.DV, nh, st);
   return kOk;
 }
 
@@ -270,8 +269,7 @@ static int widened_backward(const Prob& p, int dtype, const BwdArgs& a, hipStrea
   b.dout = widen_rows(a.dout, qr, p.DV, w.DV, dtype, ws, st);
   float* sw = (float*)take(ws, state_bytes(w));
   float* kmw = (float*)take(ws, vec_bytes(w));
-  generic::resize_matrices(a.s, p.DK, p.DV, sw, w.DK, w.DV, nh, 4, st);
-  if (a.km) generic::resize_matrices(a.km, 1, p.DK, kmw, 1, w.DK, nh, 4, st);
+  generic::resize_state(a.s, a.km, p.DK, p.DV, sw, kmw, w.DK, w.DV, nh, st);
   b.s = sw;
   b.km = a.km ? kmw : nullptr;
   b.dq = take(ws, rows_bytes(qr, w.DK, dtype));
@@ -305,8 +303,7 @@ static int ragged_forward(const Prob& p, int dtype, const FwdArgs& a, hipStream_
   b.workspace_bytes = a.workspace_bytes - (size_t)(ws - (char*)a.workspace);
   int rc = forward(w, dtype, b, st);
   if (rc != kOk) return rc;
-  generic::resize_matrices(b.s, w.DK, w.DV, a.s, p.DK, p.DV, nh, 4, st);
-  if (a.km) generic::resize_matrices(b.km, 1, w.DK, a.km, 1, p.DK, nh, 4, st);
+  generic::resize_state(b.s, a.km ? b.km : nullptr, w.DK, w.DV, a.s, a.km, p.DK, p.DV, nh, st);
   return kOk;
 }
 
@@ -317,8 +314,7 @@ static int ragged_backward(const Prob& p, int dtype, const BwdArgs& a, hipStream
   BwdArgs b = a;
   float* sw = (float*)take(ws, state_bytes(w));
   float* kmw = (float*)take(ws, vec_bytes(w));
-  generic::resize_matrices(a.s, p.DK, p.DV, sw, w.DK, w.DV, nh, 4, st);
-  if (a.km) generic::resize_matrices(a.km, 1, p.DK, kmw, 1, w.DK, nh, 4, st);
+  generic::resize_state(a.s, a.km, p.DK, p.DV, sw, kmw, w.DK, w.DV, nh, st);
   b.s = sw;
   b.km = a.km ? kmw : nullptr;
   b.workspace = ws;
