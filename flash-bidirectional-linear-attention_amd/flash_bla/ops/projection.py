@@ -2,7 +2,8 @@
 
 The blocks' projections contract 1e4 to 1e5 tokens into a weight gradient of a few hundred on a side, a shape for which
 the library's GEMM fills a dozen CUs; `_hip.linear_wgrad` splits the tokens and takes the bias's gradient along.  The
-forward and the input's gradient stay plain library GEMMs.
+forward and the input's gradient of a projection by itself stay plain library GEMMs (blocks that run whole: `_hip.mlla_fwd` and
+the like, 16-bit types, on `csrc/fbla_gemm.hip`).
 """
 import torch
 import torch.nn as nn
