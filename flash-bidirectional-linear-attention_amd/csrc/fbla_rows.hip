@@ -19,13 +19,14 @@
 //
 // Measured, bf16, heads as kernels of their own (features to heads, both operators, merge and gate, and the gradients of each) ->
 // here, with what each reaches of the bytes it moves: PolaFormer's 64 x 28x28 x 256: forward 136 -> 62 us (state 21 us, 2.6 TB/s;
-// output 33 us, 3.1 TB/s), backward 270 -> 131 us (queries 61 us, 2.9 TB/s; keys 55 us, 2.6 TB/s; the two finishing launches 7 us
-// each), the whole step 750 -> 525 us.  MLLA's 64 x 56x56 x 64: forward 84 -> 48 us (state 17, output 24 us, 3.3 TB/s), backward
-// 139 -> 71 us (queries 30, keys 33 us, 3.9 TB/s), the step 371 -> 252 us.  What was tried and cost time: three waves a SIMD for
+// output 33 us, 3.1 TB/s), backward 270 -> 131 us (queries 61 us, 2.9 TB/s; keys 55 us, 2.6 TB/s; the two finishing launches 5 us
+// each), the whole step 750 -> 502 us.  MLLA's 64 x 56x56 x 64: forward 84 -> 48 us (state 17, output 24 us, 3.3 TB/s), backward
+// 139 -> 71 us (queries 30, keys 33 us, 3.9 TB/s), the step 371 -> 238 us.  What was tried and cost time: three waves a SIMD for
 // state and output (4 spilled registers each: 24 and 35 us), two tiles a wave for the keys (256 registers: 72 us), shuffles of each
 // sum by itself at the end of the queries' pass (86 us), LDS addresses kept over the tiles (76 spilled: 141 us).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "fbla_mfma_shared.h"
@@ -301,32 +302,48 @@ __global__ __launch_bounds__(kThreads, 2) void state_kernel(Attn a, float* __res
 // ---------------------------------------------------------------------------------------------------------------
 // the partials' sum, in order, as operands: planes [f][v] hi, lo and [v][f] hi, lo of `scale` times the matrix, brought to a largest
 // value of 8 to 16 by a power of two (as 16-bit pairs it would lose to denormals otherwise), and `scale` times the vector, followed by
-// the factor that takes the power back.  Through LDS to 16-byte pieces of both orders (2 bytes at a time: 11 us, 512 heads, four
-// partials; so 7 us).  Forward: M and the mean key; backward, from the sums of M's gradient: S's and the mean key's.
+// the factor that takes the power back.  Forward: M and the mean key; backward, from the sums of M's gradient: S's and the mean
+// key's.  Bound by the latency of the partials' loads: four sets of threads share them (one set: 111 us for 392 partials of one head, 7
+// us for 512 heads of four), and the result leaves in 16-byte pieces of both orders through LDS (2 bytes at a time: 11 us).  Now 5 us
+// for 512 heads of four, 11 to 14 us where a head has its most, kMostParts.
 // ---------------------------------------------------------------------------------------------------------------
+constexpr int kFinishThreads = 1024, kFinishSets = 4;  // sets of threads that share a head's partials
 template <typename T, bool POLA>
-__global__ __launch_bounds__(kThreads) void finish_kernel(const float* __restrict__ partial, int parts, float scale, T* __restrict__ planes,
-                                                          float* __restrict__ vec) {
-  constexpr int F = kFeatures<POLA>, E = F * D, kEach = E / kThreads;
-  static_assert(E / 8 <= kThreads);
-  __shared__ float largest[kWaves], matrix[F][D + 1];
+__global__ __launch_bounds__(kFinishThreads) void finish_kernel(const float* __restrict__ partial, int parts, float scale, T* __restrict__ planes,
+                                                                float* __restrict__ vec) {
+  constexpr int F = kFeatures<POLA>, E = F * D, kSet = kFinishThreads / kFinishSets, kEach = E / kSet, kOwn = E / kFinishThreads;
+  static_assert(2 * (E / 8) <= kFinishThreads && F <= kSet && kSlot<POLA> == E + F);
+  __shared__ float sums[kFinishSets][kSlot<POLA>], largest[kFinishThreads / 64], matrix[F][D + 1];
   const int64_t head = blockIdx.x;
-  const float* from = partial + head * parts * kSlot<POLA>;
-  float x[kEach] = {}, y = 0.f, most = 0.f;
+  const int set = threadIdx.x / kSet, t = threadIdx.x % kSet;
+  {
+    const float* from = partial + head * parts * kSlot<POLA>;
+    float x[kEach] = {}, y = 0.f;
 #pragma unroll 4
-  for (int i = 0; i < parts; ++i) {
-    const float* at = from + (int64_t)i * kSlot<POLA>;
+    for (int i = set; i < parts; i += kFinishSets) {
+      const float* at = from + (int64_t)i * kSlot<POLA>;
 #pragma unroll
-    for (int e = 0; e < kEach; ++e) x[e] += at[threadIdx.x + kThreads * e];
-    if ((int)threadIdx.x < F) y += at[E + threadIdx.x];
+      for (int e = 0; e < kEach; ++e) x[e] += at[t + kSet * e];
+      if (t < F) y += at[E + t];
+    }
+#pragma unroll
+    for (int e = 0; e < kEach; ++e) sums[set][t + kSet * e] = x[e];
+    if (t < F) sums[set][E + t] = y;
   }
+  __syncthreads();
+  auto total = [&](int at) { return ((sums[0][at] + sums[1][at]) + (sums[2][at] + sums[3][at])) * scale; };
+  float x[kOwn], most = 0.f;
 #pragma unroll
-  for (int e = 0; e < kEach; ++e) most = fmaxf(most, fabsf(x[e] *= scale));
+  for (int e = 0; e < kOwn; ++e) {
+    x[e] = total(threadIdx.x + kFinishThreads * e);
+    most = fmaxf(most, fabsf(x[e]));
+  }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) most = fmaxf(most, __shfl_xor(most, off));
   if (threadIdx.x % 64 == 0) largest[threadIdx.x / 64] = most;
   __syncthreads();
-  most = fmaxf(fmaxf(largest[0], largest[1]), fmaxf(largest[2], largest[3]));
+#pragma unroll
+  for (int w = 0; w < kFinishThreads / 64; ++w) most = fmaxf(most, largest[w]);
   float norm = 1.f;  // also when the matrix is zero or not finite
   if (most > 1e-30f && most < 3e38f) {
     int e;
@@ -334,8 +351,8 @@ __global__ __launch_bounds__(kThreads) void finish_kernel(const float* __restric
     norm = ldexpf(1.f, 4 - e);
   }
 #pragma unroll
-  for (int e = 0; e < kEach; ++e) {
-    const int at = threadIdx.x + kThreads * e, f = at / D, v = at % D;
+  for (int e = 0; e < kOwn; ++e) {
+    const int at = threadIdx.x + kFinishThreads * e, f = at / D, v = at % D;
     matrix[POLA && v >= 16 ? f ^ 32 : f][v] = x[e] * norm;  // the last value channels pair with the swapped halves
   }
   __syncthreads();
@@ -350,9 +367,10 @@ __global__ __launch_bounds__(kThreads) void finish_kernel(const float* __restric
   };
   if (const int q = threadIdx.x; q < E / 8) {
     write(to + 8 * q, [&](int e) { return matrix[q / (D / 8)][8 * (q % (D / 8)) + e]; });
-    write(to + 2 * E + 8 * q, [&](int e) { return matrix[8 * (q % (F / 8)) + e][q / (F / 8)]; });
+  } else if (const int r = q - E / 8; r < E / 8) {
+    write(to + 2 * E + 8 * r, [&](int e) { return matrix[8 * (r % (F / 8)) + e][r / (F / 8)]; });
   }
-  if ((int)threadIdx.x < F) vec[head * kVector<POLA> + threadIdx.x] = y * scale;
+  if ((int)threadIdx.x < F) vec[head * kVector<POLA> + threadIdx.x] = total(E + threadIdx.x);
   if (threadIdx.x == 0) vec[head * kVector<POLA> + F] = 1.f / norm;
 }
 
@@ -814,15 +832,18 @@ __global__ __launch_bounds__(kThreads, POLA ? 2 : 3) void keys_kernel(Attn a, co
 // ---------------------------------------------------------------------------------------------------------------
 // heads of a workgroup: its waves' where they are whole fours or twos, otherwise the waves take tiles of one head
 int group_heads(int heads) { return heads % 4 == 0 ? 4 : heads % 2 == 0 ? 2 : 1; }
-// Tokens of a workgroup of the kernels that leave sums: two workgroups a CU over all, whole tiles of its waves.
+// Tokens of a workgroup: `per_cu` workgroups a CU over all, whole tiles of its waves, and where sums are left no more of them than
+// `most_parts` a head, which one workgroup adds up (one head, 112 x 112 tokens, rotary: 98 chunks, state 5 + finish 111 us; 25 chunks,
+// 7 + 11 us, the queries' pass 7 -> 13 us).
 struct Cut {
   int chunk, chunks, parts;
 };
-Cut cut(int64_t B, int64_t n, int heads, int per_cu) {
+constexpr int kMostParts = 128;
+Cut cut(int64_t B, int64_t n, int heads, int per_cu, int most_parts) {
   const int g = group_heads(heads), step = 32 * (kWaves / g);
   const int64_t places = B * (heads / g);
   int64_t chunks = 256 * per_cu / places;
-  const int64_t most = cdiv64(n, step);
+  const int64_t most = std::min<int64_t>(cdiv64(n, step), most_parts / (kWaves / g));
   chunks = chunks < 1 ? 1 : chunks > most ? most : chunks;
   const int64_t chunk = cdiv64(cdiv64(n, chunks), step) * step;
   chunks = cdiv64(n, chunk);
@@ -835,7 +856,7 @@ struct Work {  // floats (planes: T) of the workspace, in order
 Work work(const Attn& a) {
   const int F = a.pola ? 64 : 32, C = a.heads * D, g = group_heads(a.heads);
   const size_t heads = (size_t)a.B * a.heads;
-  const Cut s = cut(a.B, a.Nk, a.heads, 2), q = cut(a.B, a.N, a.heads, 2);
+  const Cut s = cut(a.B, a.Nk, a.heads, 2, kMostParts), q = cut(a.B, a.N, a.heads, 2, kMostParts);
   const size_t slot = F * (D + 1);
   Work w{};
   w.partial = heads * (s.parts > q.parts ? s.parts : q.parts) * slot;
@@ -854,11 +875,11 @@ Work work(const Attn& a) {
 
 template <typename T, bool POLA> void fwd_t(const Attn& a, hipStream_t st) {
   const int g = group_heads(a.heads);
-  const Cut s = cut(a.B, a.Nk, a.heads, 2), o = cut(a.B, a.N, a.heads, POLA ? 2 : 4);
+  const Cut s = cut(a.B, a.Nk, a.heads, 2, kMostParts), o = cut(a.B, a.N, a.heads, POLA ? 2 : 4, 1 << 30);
   const dim3 block(kThreads);
   float* partial = (float*)a.workspace;
   state_kernel<T, POLA><<<dim3(s.chunks, a.heads / g, a.B), block, 0, st>>>(a, partial, s.chunk, s.parts, g);
-  finish_kernel<T, POLA><<<dim3(a.B * a.heads), block, 0, st>>>(partial, s.parts, 1.f / (float)a.Nk, (T*)a.planes, a.km);
+  finish_kernel<T, POLA><<<dim3(a.B * a.heads), dim3(kFinishThreads), 0, st>>>(partial, s.parts, 1.f / (float)a.Nk, (T*)a.planes, a.km);
   output_kernel<T, POLA><<<dim3(o.chunks, a.heads / g, a.B), block, 0, st>>>(a, o.chunk, g);
 }
 
@@ -878,7 +899,7 @@ Carved carve(const Attn& a, const Work& w) {
 
 template <typename T, bool POLA> int bwd_queries_t(const Attn& a, hipStream_t st) {
   const int g = group_heads(a.heads);
-  const Cut q = cut(a.B, a.N, a.heads, 2);
+  const Cut q = cut(a.B, a.N, a.heads, 2, kMostParts);
   const Carved c = carve(a, work(a));
   constexpr int kLds = kWaves * kQueriesWave<POLA>;
   static thread_local bool configured = false;
@@ -892,7 +913,7 @@ template <typename T, bool POLA> int bwd_queries_t(const Attn& a, hipStream_t st
     configured = true;
   }
   queries_kernel<T, POLA><<<dim3(q.chunks, a.heads / g, a.B), dim3(kThreads), kLds, st>>>(a, c.partial, c.stats, q.chunk, q.parts, g);
-  finish_kernel<T, POLA><<<dim3(a.B * a.heads), dim3(kThreads), 0, st>>>(c.partial, q.parts, 1.f / (float)a.Nk, (T*)c.planes, c.dkm);
+  finish_kernel<T, POLA><<<dim3(a.B * a.heads), dim3(kFinishThreads), 0, st>>>(c.partial, q.parts, 1.f / (float)a.Nk, (T*)c.planes, c.dkm);
   return kOk;
 }
 
