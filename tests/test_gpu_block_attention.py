@@ -36,7 +36,8 @@ CASES = [("mlla", 1, 1, 1, 1, 2, 1.0), ("mlla", 3, 5, 5, 1, 3, 1.0), ("mlla", 4,
          ("mlla", 2, 9, 9, 1, 1, 2.0 ** -6), ("mlla", 4, 40, 40, 1, 9, 1.0), ("mlla", 6, 28, 28, 1, 70, 1.0),
          ("pola", 1, 3, 11, 1, 3, 1.0), ("pola", 2, 31, 1, 1, 2, 1.0), ("pola", 3, 4, 8, 1, 1, 2.0 ** -6), ("pola", 4, 1, 1, 1, 2, 1.0),
          ("pola", 8, 13, 5, 1, 3, 1.0), ("pola", 4, 14, 14, 2, 5, 1.0), ("pola", 2, 40, 40, 8, 9, 1.0), ("pola", 4, 28, 28, 1, 70, 1.0),
-         ("pola", 4, 40, 40, 1, 2, 1.0)]
+         ("pola", 4, 40, 40, 1, 2, 1.0),
+         ("mlla", 1, 72, 72, 1, 1, 1.0), ("pola", 1, 72, 72, 1, 1, 1.0)]  # (more tiles than a head may leave partials)
 
 
 @pytest.mark.parametrize("dtype", [torch.half, torch.bfloat16])
