@@ -110,7 +110,8 @@ __global__ __launch_bounds__(kThreads, 2) void project_kernel(Jobs jobs) {
     r.w = __builtin_amdgcn_make_buffer_rsrc((void*)w, 0, ROWS ? (int)(((int64_t)r.K * N - n0) * 2) : min(TN, N - n0) * r.w_row, kBufferFlags);
     return r;
   };
-  const Source first = source(0), other = source(TWO ? 1 : 0);
+  // (a job of one product next to others of two: what its last loads ask for beyond its steps is the first product's again)
+  const Source first = source(0), other = source(TWO && job.K[1] ? 1 : 0);
   // The steps of both products, one after the other.  Loads are buffer loads without a branch around them (so that a wait for one
   // step's rows leaves the next step's in flight): the step is the scalar offset, and what lies past the last token, past W's
   // last row, past the rows' channels or past the last step comes back as zero.

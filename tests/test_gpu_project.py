@@ -40,7 +40,10 @@ def test_projection(tokens, K, N, dtype):
               [(x, w.t(), None, g2.double() + b.double()), (x2, w2.t(), None, None), (x2, w.t(), None, b.double())]),
              ([(g, w, None, None, None, None), (g2, w2, None, x, None, None)], True,
               [(g, w, None, None), (g2, w2, None, x.double())]),
-             ([(g, w, None, x2, g2, w2)], True, [(g, w, (g2, w2), x2.double())])]
+             ([(g, w, None, x2, g2, w2)], True, [(g, w, (g2, w2), x2.double())]),
+             # a job of one product next to one of two: it has no second rows to look at
+             ([(g, w, None, None, g2, w2), (g2, w2, None, x, None, None)], True, [(g, w, (g2, w2), None), (g2, w2, None, x.double())]),
+             ([(g2, w2, None, x, None, None), (g, w, None, None, g2, w2)], True, [(g2, w2, None, x.double()), (g, w, (g2, w2), None)])]
     for jobs, rows_of_w, wants in cases:
         for got, (a, m, second, more) in zip(_hip.project(jobs, rows_of_w), wants):
             a, m = a.double(), m.double()
