@@ -80,8 +80,8 @@ __global__ __launch_bounds__(kThreads, 2) void project_kernel(Jobs jobs) {
   const int wm = wave >> 1, wn = wave & 1, kb = lane >> 5;
 
   struct Source {
-    __amdgpu_buffer_rsrc_t a, w;
-    int a_row, w_row, K;
+    const T *a, *w;
+    int a_row, w_row, K, a_bytes, w_bytes;  // bytes to the end of the tile's last row, and of W's last row
   };
   // The output tiles of a block of tokens read the same rows: they run on one XCD (workgroup i is on XCD i % 8).  Blocks beyond
   // the last multiple of eight keep the plain order.  (One round of workgroups that walk the tiles, the next one's first rows
@@ -104,36 +104,40 @@ __global__ __launch_bounds__(kThreads, 2) void project_kernel(Jobs jobs) {
     r.K = job.K[seg];
     r.a_row = (int)job.a_row[seg] * 2;
     r.w_row = (ROWS ? N : r.K) * 2;
-    const T* a = (const T*)job.a[seg] + t0 * job.a_row[seg];
-    const T* w = (const T*)job.w[seg] + (ROWS ? (int64_t)n0 : (int64_t)n0 * r.K);
-    r.a = __builtin_amdgcn_make_buffer_rsrc((void*)a, 0, (rows - 1) * r.a_row + r.K * 2, kBufferFlags);
-    r.w = __builtin_amdgcn_make_buffer_rsrc((void*)w, 0, ROWS ? (int)(((int64_t)r.K * N - n0) * 2) : min(TN, N - n0) * r.w_row, kBufferFlags);
+    r.a = (const T*)job.a[seg] + t0 * job.a_row[seg];
+    r.w = (const T*)job.w[seg] + (ROWS ? (int64_t)n0 : (int64_t)n0 * r.K);
+    r.a_bytes = (rows - 1) * r.a_row + r.K * 2;
+    r.w_bytes = ROWS ? (r.K * N - n0) * 2 : min(TN, N - n0) * r.w_row;
     return r;
   };
   // (a job of one product next to others of two: what its last loads ask for beyond its steps is the first product's again)
   const Source first = source(0), other = source(TWO && job.K[1] ? 1 : 0);
   // The steps of both products, one after the other.  Loads are buffer loads without a branch around them (so that a wait for one
-  // step's rows leaves the next step's in flight): the step is the scalar offset, and what lies past the last token, past W's
-  // last row, past the rows' channels or past the last step comes back as zero.
+  // step's rows leaves the next step's in flight).  Each step's buffers begin at its first channels (or W's first row) and end with
+  // the rows, so that it is the lanes' own offsets that meet the end: a scalar offset past a buffer's bytes is not sure to be seen
+  // by the bounds check.  What lies past the last token, past W's last row, past the rows' channels or past the last step comes back
+  // as zero.
   struct Regs {
     u32x4 a[kAPieces], w[kWPieces];
   };
   auto fetch = [&](Regs& r, int s) {
     const bool second = TWO && s >= steps0;
-    const __amdgpu_buffer_rsrc_t a = second ? other.a : first.a, w = second ? other.w : first.w;
-    const int a_row = second ? other.a_row : first.a_row, w_row = second ? other.w_row : first.w_row;
-    const int K = second ? other.K : first.K, k0 = (second ? s - steps0 : s) * kStep;
-    const int past = k0 + (tid & 7) * 8 >= K ? kPast : 0;
+    const Source from = second ? other : first;
+    const int k0 = (second ? s - steps0 : s) * kStep;
+    const __amdgpu_buffer_rsrc_t a = __builtin_amdgcn_make_buffer_rsrc((void*)(from.a + k0), 0, max(from.a_bytes - k0 * 2, 0), kBufferFlags);
+    const __amdgpu_buffer_rsrc_t w = __builtin_amdgcn_make_buffer_rsrc((void*)(from.w + (ROWS ? (int64_t)k0 * N : k0)), 0,
+                                                                       max(from.w_bytes - (ROWS ? k0 * from.w_row : k0 * 2), 0), kBufferFlags);
+    const int past = k0 + (tid & 7) * 8 >= from.K ? kPast : 0;
 #pragma unroll
     for (int p = 0; p < kAPieces; ++p) {
       const int q = tid + kThreads * p;
-      r.a[p] = __builtin_amdgcn_raw_buffer_load_b128(a, ((q >> 3) * a_row + (q & 7) * 16) | past, k0 * 2, 0);
+      r.a[p] = __builtin_amdgcn_raw_buffer_load_b128(a, ((q >> 3) * from.a_row + (q & 7) * 16) | past, 0, 0);
     }
 #pragma unroll
     for (int p = 0; p < kWPieces; ++p) {
       const int q = tid + kThreads * p;
-      if constexpr (ROWS) r.w[p] = __builtin_amdgcn_raw_buffer_load_b128(w, q / (TN / 8) * w_row + q % (TN / 8) * 16, k0 * w_row, 0);
-      else r.w[p] = __builtin_amdgcn_raw_buffer_load_b128(w, ((q >> 3) * w_row + (q & 7) * 16) | past, k0 * 2, 0);
+      if constexpr (ROWS) r.w[p] = __builtin_amdgcn_raw_buffer_load_b128(w, q / (TN / 8) * from.w_row + q % (TN / 8) * 16, 0, 0);
+      else r.w[p] = __builtin_amdgcn_raw_buffer_load_b128(w, ((q >> 3) * from.w_row + (q & 7) * 16) | past, 0, 0);
     }
   };
   auto stash = [&](const Regs& r, unsigned char* at) {

@@ -55,6 +55,18 @@ def test_projection(tokens, K, N, dtype):
             assert got.is_contiguous() and got.dtype == dtype
 
 
+@pytest.mark.parametrize("rows_of_w", [False, True])
+def test_weight_that_ends_with_its_memory(rows_of_w):
+    """A weight and rows that fill an allocation of their own: the loads ahead of the last step are past its end."""
+    torch.manual_seed(0)
+    K, N, tokens = 1536, 4096, 4096  # 12 MiB each
+    a, w = (torch.empty(tokens, K, device="cuda", dtype=torch.half).normal_() for _ in range(2))
+    m = w.view(K, N) if rows_of_w else w.view(N, K).t()
+    got, = _hip.project([(a, m if rows_of_w else m.t(), None, None, None, None)], rows_of_w)
+    a, m = a.double(), m.double()
+    _close(got, a @ m, (a.square() @ m.square() / K).sqrt(), K, torch.half)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("tokens,C", [(1, 8), (5, 504), (4, 512), (7, 520), (9, 640), (3, 1280), (33, 2048)])
 def test_norm_leaky(tokens, C, dtype):
