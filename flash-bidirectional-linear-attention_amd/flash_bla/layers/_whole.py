@@ -51,7 +51,8 @@ def _batch_of(g):
 
 
 class WholeBlockFunction(torch.autograd.Function):
-    """call: the block's native pair (below); inputs: its rows and parameters, some of them None."""
+    """call: the block's native pair (below), with the module's numbers as they are when it is called (a schedule may move them
+    before the backward); inputs: its rows and parameters, some of them None."""
 
     @staticmethod
     def forward(ctx, call, *inputs):
@@ -114,13 +115,14 @@ class _Mlla:
 
     def __init__(self, block, rotations, side):
         self.block, self.rotations, self.side, self.extra = block, rotations, side, (True,)
+        self.heads = block.num_heads
 
     def run(self, inputs, trains=True):
-        return _hip.mlla_fwd(inputs[0], inputs[1:], self.rotations, self.side, self.block.num_heads)
+        return _hip.mlla_fwd(inputs[0], inputs[1:], self.rotations, self.side, self.heads)
 
     def run_backward(self, g, inputs, saved, need):
         x, w, b, conv_w, _ = inputs
-        return _hip.mlla_bwd(g, x, w, conv_w, self.rotations, saved, self.side, self.block.num_heads, need, _splits(x, w, b))
+        return _hip.mlla_bwd(g, x, w, conv_w, self.rotations, saved, self.side, self.heads, need, _splits(x, w, b))
 
 
 def mlla(block, kind, rope, x):
@@ -139,6 +141,7 @@ class _Pvt:
     """PolaFormer's and FLatten's blocks: x, the rows of keys and values (None: x), parameters by name."""
     def __init__(self, block, H, W):
         self.block, self.H, self.W, self.extra = block, H, W, (H, W, True)
+        self.heads = block.num_heads
 
     def _split(self, inputs, saved):
         x, src, *p = inputs
@@ -150,14 +153,18 @@ class _Pola(_Pvt):
     names = (None, None, "qg.weight", "qg.bias", "kv.weight", "kv.bias", "positional_encoding", "scale", "power", "dwc.weight",
              "dwc.bias", "proj.weight", "proj.bias")
 
+    def __init__(self, block, H, W):
+        super().__init__(block, H, W)
+        self.alpha = block.alpha
+
     def run(self, inputs, trains=True):
         x, src, *p = inputs
-        return _hip.pola_fwd(x, x if src is None else src, p, self.block.alpha, self.H, self.W, self.block.num_heads)
+        return _hip.pola_fwd(x, x if src is None else src, p, self.alpha, self.H, self.W, self.heads)
 
     def run_backward(self, g, inputs, saved, need):
         x, src, *p = inputs
-        return _hip.pola_bwd(g, x, x if src is None else src, src is None, p, saved, self.block.alpha, self.H, self.W,
-                             self.block.num_heads, need, self._split(inputs, saved))
+        return _hip.pola_bwd(g, x, x if src is None else src, src is None, p, saved, self.alpha, self.H, self.W,
+                             self.heads, need, self._split(inputs, saved))
 
 
 class _Focused(_Pvt):
@@ -166,11 +173,11 @@ class _Focused(_Pvt):
 
     def run(self, inputs, trains=True):
         x, src, *p = inputs
-        return _hip.focused_fwd(x, x if src is None else src, p, self.H, self.W, self.block.num_heads)
+        return _hip.focused_fwd(x, x if src is None else src, p, self.H, self.W, self.heads)
 
     def run_backward(self, g, inputs, saved, need):
         x, src, *p = inputs
-        return _hip.focused_bwd(g, x, x if src is None else src, src is None, p, saved, self.H, self.W, self.block.num_heads, need,
+        return _hip.focused_bwd(g, x, x if src is None else src, src is None, p, saved, self.H, self.W, self.heads, need,
                                 self._split(inputs, saved))
 
 
@@ -178,7 +185,7 @@ def _pvt(call, fits, query, params, x, src):
     block, H, W = call.block, call.H, call.W
     if not (type(H) is int and type(W) is int and (src is None or type(src) is torch.Tensor) and
             _hip.plain_gpu_tensors(x, src, *params) and _same_convolution(block.dwc) and
-            fits(x, x if src is None else src, params, H, W, block.num_heads)):
+            fits(x, x if src is None else src, params, H, W, call.heads)):
         return None
     return _run(call, (x, src, *params))
 

@@ -11,6 +11,7 @@ from flash_bla import _hip
 from flash_bla.layers import (FocusedLinearAttention, GeneralizedLinearAttention, MambaLikeLinearAttention,
                               PolaLinearAttention, RALALinearAttention)
 from flash_bla.layers import _features as features
+from flash_bla.layers import _whole
 from flash_bla.layers import polaformer, rala
 from flash_bla.layers.mlla import RoPE
 from flash_bla.ops import depthwise, projection
@@ -399,3 +400,41 @@ def test_composed_gradients_stop_at_their_inputs():
     grads = features.differentiable_gradients(features.merge_formula, (o, None, local, gate), (torch.ones(2, ROWS, DIM),))
     assert not seen and [g is None for g in grads] == [False, True, False, False]
     assert torch.equal(grads[0], features.split_heads(gate, HEADS).detach())
+
+
+@pytest.fixture
+def native(monkeypatch):
+    """Blocks that run whole on the CPU: every call fits; the native calls note the numbers they are given and return zeros."""
+    seen = []
+
+    def numbers(args):
+        return [a for a in args if type(a) in (int, float)]
+
+    def forward(x, *args):
+        seen.append(numbers(args))
+        return [torch.zeros_like(x), x.detach()]
+
+    def backward(g, x, *args):
+        seen.append(numbers(args))
+        need = next(a for a in args if isinstance(a, (list, tuple)) and all(type(e) is bool for e in a))
+        return [torch.zeros_like(x)] + [None] * (len(need) - 1)
+    monkeypatch.setattr(_whole, "_ordinary", lambda *a: True)
+    monkeypatch.setattr(_hip, "plain_gpu_tensors", lambda *a: True)
+    for name in ("mlla", "pola", "focused"):
+        monkeypatch.setattr(_hip, name + "_fits", lambda *a: True)
+        monkeypatch.setattr(_hip, name + "_fwd", forward)
+        monkeypatch.setattr(_hip, name + "_bwd", backward)
+    return seen
+
+
+@pytest.mark.parametrize("name", ["mlla", "pola", "focused"])
+def test_numbers_of_a_whole_call_are_those_of_its_forward(name, native):
+    """A schedule moves them, two calls of different numbers share a backward: each has its own."""
+    make, extra = BLOCKS[name]
+    block, x = make(), torch.randn(2, 16, 16, requires_grad=True)
+    out = [block(x, *extra)]
+    block.alpha, block.num_heads = 1.5, 4
+    out.append(block(x, *extra))
+    block.alpha, block.num_heads = 2.5, 1
+    (out[0] + out[1]).sum().backward()
+    assert len(native) == 4 and native[0] != native[1] and sorted(native[2:]) == sorted(native[:2])
