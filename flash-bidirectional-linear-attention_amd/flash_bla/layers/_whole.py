@@ -52,7 +52,7 @@ def _batch_of(g):
 
 class WholeBlockFunction(torch.autograd.Function):
     """call: the block's native pair (below), with the module's numbers as they are when it is called (a schedule may move them
-    before the backward); inputs: its rows and parameters, some of them None."""
+    before the backward); inputs: its rows and parameters, some of them None, and what else the backward reads."""
 
     @staticmethod
     def forward(ctx, call, *inputs):
@@ -78,7 +78,7 @@ class WholeBlockFunction(torch.autograd.Function):
             with torch.enable_grad():  # (through aliases: the inputs may depend on one another)
                 aliases = [t.view_as(t) if t is not None and t.requires_grad else t for t in inputs]
                 rows = [a for a, name in zip(aliases, call.names) if name is None]
-                state = {"block." + name: a for a, name in zip(aliases, call.names) if name is not None and a is not None}
+                state = {"block." + name: a for a, name in zip(aliases, call.names) if name and a is not None}
                 out = functional_call(_Steps(call.block), state, (*rows, *call.extra))
             wanted = [a for a, wants in zip(aliases, need) if wants]
             got = iter(torch.autograd.grad(out, wanted, g, create_graph=torch.is_grad_enabled(), allow_unused=True))
@@ -111,18 +111,19 @@ def _splits(rows, weight, bias):
 
 
 class _Mlla:
-    names = (None, "qk.weight", "qk.bias", "lepe.weight", "lepe.bias")
+    names = (None, "qk.weight", "qk.bias", "lepe.weight", "lepe.bias", "rope.rotations")
 
-    def __init__(self, block, rotations, side):
-        self.block, self.rotations, self.side, self.extra = block, rotations, side, (True,)
+    def __init__(self, block, side):
+        self.block, self.side, self.extra = block, side, (True,)
         self.heads = block.num_heads
 
     def run(self, inputs, trains=True):
-        return _hip.mlla_fwd(inputs[0], inputs[1:], self.rotations, self.side, self.heads)
+        *inputs, rotations = inputs
+        return _hip.mlla_fwd(inputs[0], inputs[1:], rotations, self.side, self.heads)
 
     def run_backward(self, g, inputs, saved, need):
-        x, w, b, conv_w, _ = inputs
-        return _hip.mlla_bwd(g, x, w, conv_w, self.rotations, saved, self.side, self.heads, need, _splits(x, w, b))
+        x, w, b, conv_w, _, rotations = inputs
+        return [*_hip.mlla_bwd(g, x, w, conv_w, rotations, saved, self.side, self.heads, need[:5], _splits(x, w, b)), None]
 
 
 def mlla(block, kind, rope, x):
@@ -134,7 +135,7 @@ def mlla(block, kind, rope, x):
     if not (type(rotations) is torch.Tensor and _hip.plain_gpu_tensors(x, *params) and _same_convolution(block.lepe) and
             _hip.mlla_fits(x, params, rotations, side, block.num_heads)):
         return None
-    return _run(_Mlla(block, rotations, side), (x, *params))
+    return _run(_Mlla(block, side), (x, *params, rotations))
 
 
 class _Pvt:
@@ -211,20 +212,21 @@ def focused(block, kind, x, src, H, W):
 
 class _LinFusion:
     names = (None, *(f"to_{p}_.{layer}.{n}" for p in "qk" for layer in (0, 1, 3) for n in ("weight", "bias")),
-             *(f"to_{p}.{n}" for p in "qkv" for n in ("weight", "bias")), "to_out.0.weight", "to_out.0.bias")
+             *(f"to_{p}.{n}" for p in "qkv" for n in ("weight", "bias")), "to_out.0.weight", "to_out.0.bias", "")  # (last: the packed batch's offsets)
 
-    def __init__(self, block, cu):
-        self.block, self.cu, self.extra = block, cu, ()
+    def __init__(self, block):
+        self.block, self.extra = block, ()
         self.slope = tuple(path[2].negative_slope for path in (block.to_q_, block.to_k_))
 
     def run(self, inputs, trains=True):
         eps = tuple(path[1].eps for path in (self.block.to_q_, self.block.to_k_))
-        return _hip.linfusion_fwd(inputs[0], self.cu, inputs[1:], eps, self.slope, self.block.heads, trains)
+        x, *p, cu = inputs
+        return _hip.linfusion_fwd(x, cu, p, eps, self.slope, self.block.heads, trains)
 
     def run_backward(self, g, inputs, saved, need):
-        x, *p = inputs
+        x, *p, cu = inputs
         split = [_splits(x, p[i], p[i + 1]) for i in (0, 4, 6, 10, 12, 14, 16, 18)]
-        return _hip.linfusion_bwd(g, x, self.cu, p, saved, self.slope, need, split)
+        return [*_hip.linfusion_bwd(g, x, cu, p, saved, self.slope, need[:-1], split), None]
 
 
 def linfusion(block, kind, x, cu):
@@ -242,4 +244,4 @@ def linfusion(block, kind, x, cu):
     if not (_hip.plain_gpu_tensors(x, *params) and all(len(p[1].normalized_shape) == 1 and p[1].normalized_shape[0] == p[0].out_features
                                                        for p in paths) and _hip.linfusion_fits(x, params, block.heads)):
         return None
-    return _run(_LinFusion(block, cu()), (x, *params))
+    return _run(_LinFusion(block), (x, *params, cu()))

@@ -438,3 +438,17 @@ def test_numbers_of_a_whole_call_are_those_of_its_forward(name, native):
     block.alpha, block.num_heads = 2.5, 1
     (out[0] + out[1]).sum().backward()
     assert len(native) == 4 and native[0] != native[1] and sorted(native[2:]) == sorted(native[:2])
+
+
+def test_a_whole_call_saves_what_its_backward_reads(native):
+    """A rotation that is written between forward and backward is noticed, and saved-tensor hooks see it."""
+    make, extra = BLOCKS["mlla"]
+    block, x, packed = make(), torch.randn(2, 16, 16, requires_grad=True), []
+    out = block(x, *extra)
+    with torch.no_grad():
+        block.rope.rotations.mul_(2)
+    with pytest.raises(RuntimeError, match="inplace"):
+        out.sum().backward()
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: packed.append(t) or t, lambda t: t):
+        block(x, *extra)
+    assert any(t is block.rope.rotations or t.data_ptr() == block.rope.rotations.data_ptr() for t in packed)
