@@ -18,22 +18,30 @@ import torch
 import torch.nn as nn
 from torch._C import _functorch
 from torch._functorch.pyfunctorch import temporarily_clear_interpreter_stack
-from torch.func import functional_call
 from torch.nn.modules.module import _has_any_global_hook
 
 from flash_bla import _hip
 from flash_bla.ops.projection import eager_call, gradient_of, splits_tokens
 
 
-class _Steps(nn.Module):
-    """A block's steps as a module of their own, for functional_call."""
+def _bare(kind, **members):
+    """A module of the class that holds these and nothing else: what `_steps` of a block and `project` look at."""
+    module = kind.__new__(kind)
+    nn.Module.__init__(module)
+    for name, value in members.items():
+        setattr(module, name, value)
+    return module
 
-    def __init__(self, block):
-        super().__init__()
-        self.block = block
 
-    def forward(self, *args):
-        return self.block._steps(*args)
+def _linear(weight, bias):
+    return _bare(nn.Linear, weight=weight, bias=bias)
+
+
+def _convolution(weight, bias):
+    """As _same_convolution knows it."""
+    Cw, _, K, _ = weight.shape
+    return _bare(nn.Conv2d, weight=weight, bias=bias, in_channels=Cw, out_channels=Cw, groups=Cw, kernel_size=(K, K), stride=(1, 1),
+                 padding=(K // 2, K // 2), dilation=(1, 1), padding_mode='zeros')
 
 
 def _batch_of(g):
@@ -51,8 +59,9 @@ def _batch_of(g):
 
 
 class WholeBlockFunction(torch.autograd.Function):
-    """call: the block's native pair (below), with the module's numbers as they are when it is called (a schedule may move them
-    before the backward); inputs: its rows and parameters, some of them None, and what else the backward reads."""
+    """call: the block's native pair and the same as `_steps` of a block that holds the inputs (below), with the module's numbers
+    as they are when it is called: by the time of the backward a schedule may have moved them, or hooks and other parameters
+    taken their place.  inputs: the block's rows and parameters, some of them None, and what else the backward reads."""
 
     @staticmethod
     def forward(ctx, call, *inputs):
@@ -64,8 +73,8 @@ class WholeBlockFunction(torch.autograd.Function):
     @staticmethod
     def backward(ctx, g):
         call, tensors = ctx.call, ctx.saved_tensors
-        n = len(call.names)
-        inputs, saved, need = tensors[:n], tensors[n:], ctx.needs_input_grad[1:]
+        need = ctx.needs_input_grad[1:]
+        inputs, saved = tensors[:len(need)], tensors[len(need):]
 
         def composed(g):
             batch = None if torch.is_grad_enabled() else _batch_of(g)
@@ -75,11 +84,9 @@ class WholeBlockFunction(torch.autograd.Function):
                     each = [call.run_backward(e, inputs, saved, need) for e in values.unbind()]
                     stacked = [None if t[0] is None else torch.stack(t) for t in zip(*each)]
                 return [None if t is None else wrapped(t) for t in stacked]
-            with torch.enable_grad():  # (through aliases: the inputs may depend on one another)
+            with torch.enable_grad():  # (through aliases: the inputs may depend on one another, or be one tensor)
                 aliases = [t.view_as(t) if t is not None and t.requires_grad else t for t in inputs]
-                rows = [a for a, name in zip(aliases, call.names) if name is None]
-                state = {"block." + name: a for a, name in zip(aliases, call.names) if name and a is not None}
-                out = functional_call(_Steps(call.block), state, (*rows, *call.extra))
+                out = call.steps(*aliases)
             wanted = [a for a, wants in zip(aliases, need) if wants]
             got = iter(torch.autograd.grad(out, wanted, g, create_graph=torch.is_grad_enabled(), allow_unused=True))
             return [next(got) if wants else None for wants in need]
@@ -111,11 +118,14 @@ def _splits(rows, weight, bias):
 
 
 class _Mlla:
-    names = (None, "qk.weight", "qk.bias", "lepe.weight", "lepe.bias", "rope.rotations")
+    """inputs: x, parameters, rotations."""
 
-    def __init__(self, block, side):
-        self.block, self.side, self.extra = block, side, (True,)
-        self.heads = block.num_heads
+    def __init__(self, block, kind, rope, side):
+        self.kind, self.rope, self.side, self.heads = kind, rope, side, block.num_heads
+
+    def steps(self, x, w, b, conv_w, conv_b, rotations):
+        return _bare(self.kind, num_heads=self.heads, qk=_linear(w, b), lepe=_convolution(conv_w, conv_b),
+                     rope=_bare(self.rope, rotations=rotations))._steps(x, True)
 
     def run(self, inputs, trains=True):
         *inputs, rotations = inputs
@@ -135,14 +145,18 @@ def mlla(block, kind, rope, x):
     if not (type(rotations) is torch.Tensor and _hip.plain_gpu_tensors(x, *params) and _same_convolution(block.lepe) and
             _hip.mlla_fits(x, params, rotations, side, block.num_heads)):
         return None
-    return _run(_Mlla(block, side), (x, *params, rotations))
+    return _run(_Mlla(block, kind, rope, side), (x, *params, rotations))
 
 
 class _Pvt:
-    """PolaFormer's and FLatten's blocks: x, the rows of keys and values (None: x), parameters by name."""
-    def __init__(self, block, H, W):
-        self.block, self.H, self.W, self.extra = block, H, W, (H, W, True)
-        self.heads = block.num_heads
+    """PolaFormer's and FLatten's blocks.  inputs: x, the rows of keys and values (None: x), parameters."""
+
+    def __init__(self, block, kind, H, W):
+        self.kind, self.H, self.W, self.heads, self.sr_ratio = kind, H, W, block.num_heads, block.sr_ratio
+
+    def _block(self, kv_w, kv_b, pe, scale, conv_w, conv_b, proj_w, proj_b, **more):
+        return _bare(self.kind, num_heads=self.heads, sr_ratio=self.sr_ratio, kv=_linear(kv_w, kv_b), positional_encoding=pe,
+                     scale=scale, dwc=_convolution(conv_w, conv_b), proj=_linear(proj_w, proj_b), **more)
 
     def _split(self, inputs, saved):
         x, src, *p = inputs
@@ -151,12 +165,13 @@ class _Pvt:
 
 
 class _Pola(_Pvt):
-    names = (None, None, "qg.weight", "qg.bias", "kv.weight", "kv.bias", "positional_encoding", "scale", "power", "dwc.weight",
-             "dwc.bias", "proj.weight", "proj.bias")
-
-    def __init__(self, block, H, W):
-        super().__init__(block, H, W)
+    def __init__(self, block, kind, H, W):
+        super().__init__(block, kind, H, W)
         self.alpha = block.alpha
+
+    def steps(self, x, src, q_w, q_b, kv_w, kv_b, pe, scale, power, *more):
+        block = self._block(kv_w, kv_b, pe, scale, *more, qg=_linear(q_w, q_b), power=power, alpha=self.alpha)
+        return block._steps(x, src, self.H, self.W, True)
 
     def run(self, inputs, trains=True):
         x, src, *p = inputs
@@ -169,8 +184,8 @@ class _Pola(_Pvt):
 
 
 class _Focused(_Pvt):
-    names = (None, None, "q.weight", "q.bias", "kv.weight", "kv.bias", "positional_encoding", "scale", "dwc.weight", "dwc.bias",
-             "proj.weight", "proj.bias")
+    def steps(self, x, src, q_w, q_b, *more):
+        return self._block(*more, q=_linear(q_w, q_b), focusing_factor=3)._steps(x, src, self.H, self.W, True)
 
     def run(self, inputs, trains=True):
         x, src, *p = inputs
@@ -182,8 +197,8 @@ class _Focused(_Pvt):
                                 self._split(inputs, saved))
 
 
-def _pvt(call, fits, query, params, x, src):
-    block, H, W = call.block, call.H, call.W
+def _pvt(call, block, fits, params, x, src):
+    H, W = call.H, call.W
     if not (type(H) is int and type(W) is int and (src is None or type(src) is torch.Tensor) and
             _hip.plain_gpu_tensors(x, src, *params) and _same_convolution(block.dwc) and
             fits(x, x if src is None else src, params, H, W, call.heads)):
@@ -195,7 +210,7 @@ def pola(block, kind, x, src, H, W):
     if not (type(block.alpha) in (int, float) and block.alpha >= 0 and _ordinary(block, kind, x, [
             (block.qg, nn.Linear), (block.kv, nn.Linear), (block.proj, nn.Linear), (block.dwc, nn.Conv2d)])):
         return None
-    return _pvt(_Pola(block, H, W), _hip.pola_fits, block.qg, (
+    return _pvt(_Pola(block, kind, H, W), block, _hip.pola_fits, (
         block.qg.weight, block.qg.bias, block.kv.weight, block.kv.bias, block.positional_encoding, block.scale, block.power,
         block.dwc.weight, block.dwc.bias, block.proj.weight, block.proj.bias), x, src)
 
@@ -205,23 +220,31 @@ def focused(block, kind, x, src, H, W):
     if not (type(factor) in (int, float) and factor == 3 and _ordinary(block, kind, x, [
             (block.q, nn.Linear), (block.kv, nn.Linear), (block.proj, nn.Linear), (block.dwc, nn.Conv2d)])):
         return None
-    return _pvt(_Focused(block, H, W), _hip.focused_fits, block.q, (
+    return _pvt(_Focused(block, kind, H, W), block, _hip.focused_fits, (
         block.q.weight, block.q.bias, block.kv.weight, block.kv.bias, block.positional_encoding, block.scale, block.dwc.weight,
         block.dwc.bias, block.proj.weight, block.proj.bias), x, src)
 
 
 class _LinFusion:
-    names = (None, *(f"to_{p}_.{layer}.{n}" for p in "qk" for layer in (0, 1, 3) for n in ("weight", "bias")),
-             *(f"to_{p}.{n}" for p in "qkv" for n in ("weight", "bias")), "to_out.0.weight", "to_out.0.bias", "")  # (last: the packed batch's offsets)
+    """inputs: x, parameters (both paths' first projection, norm and second projection, then queries, keys, values, output), the
+    packed batch's offsets."""
 
-    def __init__(self, block):
-        self.block, self.extra = block, ()
-        self.slope = tuple(path[2].negative_slope for path in (block.to_q_, block.to_k_))
+    def __init__(self, block, kind):
+        paths = block.to_q_, block.to_k_
+        self.kind, self.heads = kind, block.heads
+        self.eps, self.slope = tuple(p[1].eps for p in paths), tuple(p[2].negative_slope for p in paths)
+
+    def steps(self, x, *p):
+        def path(i):
+            in_w, in_b, norm_w, norm_b, out_w, out_b = p[6 * i:6 * i + 6]
+            norm = _bare(nn.LayerNorm, normalized_shape=in_w.shape[:1], weight=norm_w, bias=norm_b, eps=self.eps[i])
+            return nn.Sequential(_linear(in_w, in_b), norm, nn.LeakyReLU(self.slope[i]), _linear(out_w, out_b))
+        q, k, v, out = (_linear(*p[i:i + 2]) for i in range(12, 20, 2))
+        return _bare(self.kind, heads=self.heads, to_q_=path(0), to_k_=path(1), to_q=q, to_k=k, to_v=v, to_out=[out])._steps(x)
 
     def run(self, inputs, trains=True):
-        eps = tuple(path[1].eps for path in (self.block.to_q_, self.block.to_k_))
         x, *p, cu = inputs
-        return _hip.linfusion_fwd(x, cu, p, eps, self.slope, self.block.heads, trains)
+        return _hip.linfusion_fwd(x, cu, p, self.eps, self.slope, self.heads, trains)
 
     def run_backward(self, g, inputs, saved, need):
         x, *p, cu = inputs
@@ -244,4 +267,4 @@ def linfusion(block, kind, x, cu):
     if not (_hip.plain_gpu_tensors(x, *params) and all(len(p[1].normalized_shape) == 1 and p[1].normalized_shape[0] == p[0].out_features
                                                        for p in paths) and _hip.linfusion_fits(x, params, block.heads)):
         return None
-    return _run(_LinFusion(block), (x, *params, cu()))
+    return _run(_LinFusion(block, kind), (x, *params, cu()))

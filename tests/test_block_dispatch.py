@@ -12,7 +12,8 @@ from flash_bla.layers import (FocusedLinearAttention, GeneralizedLinearAttention
                               PolaLinearAttention, RALALinearAttention)
 from flash_bla.layers import _features as features
 from flash_bla.layers import _whole
-from flash_bla.layers import polaformer, rala
+from flash_bla.layers import focused_la, linfusion, mlla, polaformer, rala
+from flash_bla.layers._common import torch_linear_attention
 from flash_bla.layers.mlla import RoPE
 from flash_bla.ops import depthwise, projection
 from flash_bla.ops._check import untouched
@@ -420,7 +421,7 @@ def native(monkeypatch):
         return [torch.zeros_like(x)] + [None] * (len(need) - 1)
     monkeypatch.setattr(_whole, "_ordinary", lambda *a: True)
     monkeypatch.setattr(_hip, "plain_gpu_tensors", lambda *a: True)
-    for name in ("mlla", "pola", "focused"):
+    for name in ("mlla", "pola", "focused", "linfusion"):
         monkeypatch.setattr(_hip, name + "_fits", lambda *a: True)
         monkeypatch.setattr(_hip, name + "_fwd", forward)
         monkeypatch.setattr(_hip, name + "_bwd", backward)
@@ -452,3 +453,66 @@ def test_a_whole_call_saves_what_its_backward_reads(native):
     with torch.autograd.graph.saved_tensors_hooks(lambda t: packed.append(t) or t, lambda t: t):
         block(x, *extra)
     assert any(t is block.rope.rotations or t.data_ptr() == block.rope.rotations.data_ptr() for t in packed)
+
+
+@pytest.fixture
+def torch_operators(monkeypatch):
+    """The attention operators by torch's on the CPU."""
+    def paired(q1, q2, k, v):
+        return tuple(torch_linear_attention(q, k, part) for q, part in zip((q1, q2), v.chunk(2, dim=-1)))
+
+    def packed(q, k, v, cu, n, eps, feature_map):
+        heads = [t.unflatten(0, (-1, n)).transpose(1, 2) for t in (nn.functional.elu(q) + 1, nn.functional.elu(k) + 1, v)]
+        return torch_linear_attention(*heads, eps=eps).transpose(1, 2).flatten(0, 1)
+    for module in (mlla, features):
+        monkeypatch.setattr(module, "elu_plus_one", lambda t: nn.functional.elu(t) + 1)
+    monkeypatch.setattr(mlla, "decoupled_la", lambda q, k, q_rope, k_rope, v, scale: torch_linear_attention(
+        q, k, v, q_num=q_rope, k_num=k_rope))
+    monkeypatch.setattr(polaformer, "paired_linear_attention", paired)
+    monkeypatch.setattr(focused_la, "linear_attention", torch_linear_attention)
+    monkeypatch.setattr(linfusion, "varlen_linear_attention", packed)
+
+
+@pytest.mark.parametrize("name", ["mlla", "pola", "focused", "linfusion"])
+def test_composed_gradients_of_a_whole_call_are_those_of_its_forward(name, native, torch_operators, monkeypatch):
+    """Gradients of gradients, of parameters that two projections share, after the module has got other numbers, hooks and
+    parameters; the module is not touched meanwhile."""
+    make, extra = BLOCKS[name]
+    torch.manual_seed(0)
+    block, x, g = make(), torch.randn(2, 16, 16, requires_grad=True), torch.randn(2, 16, 16)
+    with torch.no_grad():
+        for p in block.parameters():
+            p.add_(0.1 * torch.randn(p.shape))
+    if name == "linfusion":
+        block.to_k.weight = block.to_q.weight
+        block.to_q_[2].negative_slope = 0.3
+    elif name == "pola":
+        block.qg.weight = block.kv.weight
+    elif name == "focused":
+        block.proj.weight = block.q.weight
+    wanted = [x, *(p for n, p in block.named_parameters() if not n.startswith(("sr", "norm")))]
+
+    def gradients(out):
+        once = torch.autograd.grad(out, wanted, g, create_graph=True)
+        return once, torch.autograd.grad(sum(t.square().sum() for t in once), wanted, allow_unused=True)
+    want = gradients(block(x, *extra, mode="torch"))
+    if name == "linfusion":
+        call = _whole._LinFusion(block, GeneralizedLinearAttention)
+        paths, rest = (block.to_q_, block.to_k_), (block.to_q, block.to_k, block.to_v, block.to_out[0])
+        params = [t for p in paths for i in (0, 1, 3) for t in (p[i].weight, p[i].bias)] + [t for m in rest for t in (m.weight, m.bias)]
+        monkeypatch.setattr(_hip, "linfusion_fwd", lambda x, *a: [torch.zeros_like(x)])
+        out = _whole.WholeBlockFunction.apply(call, x, *params, torch.tensor([0, 16, 32], dtype=torch.int32))
+        block.to_q_[2].negative_slope = block.to_k_[1].eps = 0.7
+        block.heads = 1
+    else:
+        out = block(x, *extra)
+        block.num_heads, block.alpha, block.focusing_factor = 1, 0.5, 1
+    for m in list(block.modules())[1:]:
+        m.register_forward_hook(lambda m, args, out: pytest.fail("the module ran"))
+    for m in block.children():
+        m.weight = nn.Parameter(torch.zeros(3))
+    for got, expected in zip(gradients(out), want):
+        assert [t is None for t in got] == [t is None for t in expected]
+        for a, b in zip(got, expected):
+            if a is not None:  # fp32 sums of at most 64 products in another order; NaN: the power's second derivative at 0
+                torch.testing.assert_close(a, b, rtol=1e-3, atol=1e-4 * float(b.detach().nan_to_num().abs().max() + 1), equal_nan=True)
