@@ -252,6 +252,11 @@ class _LinFusion:
         return [*_hip.linfusion_bwd(g, x, cu, p, saved, self.slope, need[:-1], split), None]
 
 
+def _keeps_signs(activation):
+    """Whether LeakyReLU's output has its input's sign, from which the backward takes the activation's gradient."""
+    return type(activation.negative_slope) in (int, float) and activation.negative_slope >= 0
+
+
 def linfusion(block, kind, x, cu):
     """cu(): the packed batch's offsets."""
     paths = (block.to_q_, block.to_k_)
@@ -264,7 +269,7 @@ def linfusion(block, kind, x, cu):
         return None
     params = [t for p in paths for i in (0, 1, 3) for t in (p[i].weight, p[i].bias)]
     params += [t for m in projections for t in (m.weight, m.bias)]
-    if not (_hip.plain_gpu_tensors(x, *params) and all(len(p[1].normalized_shape) == 1 and p[1].normalized_shape[0] == p[0].out_features
+    if not (all(_keeps_signs(p[2]) for p in paths) and _hip.plain_gpu_tensors(x, *params) and all(len(p[1].normalized_shape) == 1 and p[1].normalized_shape[0] == p[0].out_features
                                                        for p in paths) and _hip.linfusion_fits(x, params, block.heads)):
         return None
     return _run(_LinFusion(block, kind), (x, *params, cu()))

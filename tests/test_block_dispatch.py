@@ -516,3 +516,8 @@ def test_composed_gradients_of_a_whole_call_are_those_of_its_forward(name, nativ
         for a, b in zip(got, expected):
             if a is not None:  # fp32 sums of at most 64 products in another order; NaN: the power's second derivative at 0
                 torch.testing.assert_close(a, b, rtol=1e-3, atol=1e-4 * float(b.detach().nan_to_num().abs().max() + 1), equal_nan=True)
+
+
+@pytest.mark.parametrize("slope,kept", [(0.01, True), (0, True), (-0.1, False), (float("nan"), False), (torch.tensor(0.1), False)])
+def test_slopes_that_turn_signs_run_step_by_step(slope, kept):
+    assert _whole._keeps_signs(nn.LeakyReLU(slope)) == kept

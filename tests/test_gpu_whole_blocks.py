@@ -185,3 +185,17 @@ def test_two_streams():
         torch.cuda.current_stream().wait_stream(side)
         assert torch.equal(y.detach(), want)
         block.zero_grad()
+
+
+def test_negative_slope(counted):
+    """torch takes it, and so does the block: step by step, with the gradients of torch's operators."""
+    block, x, _ = _make("linfusion", torch.half)
+    for path in (block.to_q_, block.to_k_):
+        path[2] = torch.nn.LeakyReLU(-0.5)  # (in place torch refuses the backward)
+    leaf, g = x.requires_grad_(), torch.randn_like(x)
+    out = block(leaf)
+    out.backward(g)
+    got = [out.detach(), leaf.grad] + [p.grad for p in block.parameters()]
+    assert not counted
+    for a, e in zip(got, _exact(block, x, (), g)):  # (a value whose rounding crosses the kink: 1.5 of its gradient, as in _make)
+        assert _distance(a, e) <= 0.1
