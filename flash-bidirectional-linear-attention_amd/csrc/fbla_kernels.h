@@ -138,7 +138,7 @@ bool bwd_a_supported(const Prob& p, int dtype);
 // matrices (no partial sums in their prologue)
 bool pair_mode(const Prob& p, int dtype);
 // block_stats: the launch that also writes piecewise attention's block statistics
-int state_chunk(const Prob& p, bool block_stats = false);
+int state_chunk(const Prob& p, int dtype, bool block_stats = false);
 int bwd_a_chunk(const Prob& p);
 int rows_chunk(const Prob& p, int DR, int DC);
 // Tokens per partial as a reduction must count them (`kernel_bit`: 1 the state kernel, 4 backward

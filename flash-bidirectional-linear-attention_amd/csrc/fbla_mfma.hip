@@ -2501,15 +2501,21 @@ static int chunk_for(const Prob& p, int wgs_per_cu, int rounds, int min_chunk, i
 // are halved: 128 gained nothing more (B4-H8-T1024-D64 fp16 17.6 us either way).  The partials stay below 8 MiB.  Forward /
 // backward, us: B2-H4-T1024-D64 fp32 19.0 / 28.3 -> 17.3 / 25.8, fp16 14.1 / 18.3 -> 13.0 / 16.2 (partials summed by the reduce
 // kernel, see fold_reduce), B1-H2-T1024-D128 fp32 42.7 / 64.3 -> 30.9 / 50.1, fp16 25.2 / 45.1 -> 22.3 / 27.7.
-static int least_chunk(const Prob& p, int chunk, int least) {
+// `few_long`: the same line for heads of 16 chunks and more.  From 32 workgroups on the sum over a head's partials costs more than
+// finer chunks save, in the forward (fp16, us, not halved / halved: B1-H1-T8192-D64 20.0 / 22.0, D128 31.0 / 32.6, B1-H3-T4096-D64
+// 19.6 / 20.5, B1-H1-T4096-D128 29.1 at 32 workgroups, 31.5 at 64) and in the backward of 64 x 64 (B1-H1-T8192 20.2 / 21.2); that
+// of 128 x 128 gains (B1-H1-T8192 36.1 / 33.5).
+static int least_chunk(const Prob& p, int chunk, int least, int few_long = 64) {
   static const int few = knob("FBLA_LEAST_WGS", 64);
   const int64_t nh = (int64_t)p.N * p.H, slot = ((int64_t)p.DK * p.DV + p.DK) * (int64_t)sizeof(float);
-  while (chunk / 2 >= least && nh * cdiv64(p.L, chunk) < few && nh * cdiv64(p.L, chunk / 2) * slot <= 8 << 20) chunk /= 2;
+  while (chunk / 2 >= least && nh * cdiv64(p.L, chunk) < (cdiv64(p.L, chunk) < 16 ? few : few_long) &&
+         nh * cdiv64(p.L, chunk / 2) * slot <= 8 << 20)
+    chunk /= 2;
   return chunk;
 }
 // (one chunk a head stays one: the kernel then stores the finished state itself, B2-H4-T256-D64 fp16 forward 10.4 us, with
 // two chunks and a reduce launch 12.8)
-static int least_state_chunk(const Prob& p) { return p.L > 256 ? least_chunk(p, 256, 64) : 256; }
+static int least_state_chunk(const Prob& p) { return p.L > 256 ? least_chunk(p, 256, 64, 32) : 256; }
 
 // Reduction kernels (state, backward pass A): one round of resident workgroups.
 // 128 x 128 states of the plain operator: state128_kernel, two workgroups per CU.
@@ -2530,14 +2536,17 @@ static int whole_sequence_chunk(const Prob& p, int align) {
   return (int)(cdiv64(p.L, align) * align);
 }
 
-int state_chunk(const Prob& p, bool block_stats) {
+int state_chunk(const Prob& p, int dtype, bool block_stats) {
   static const int per_cu = knob("FBLA_STATE_WGS_PER_CU", 2);
   if (!block_stats) {
     const int direct = whole_sequence_chunk(p, 64);
     if (direct) return direct;
   }
   const int whole = block_stats && padded(p) ? 0 : whole_state_chunk(p);
-  return whole ? whole : chunk_for(p, per_cu, 1, block_stats ? 256 : least_state_chunk(p), 64, true);
+  // 16-bit heads of two chunks, 32 workgroups and more: the consumers' prologues read twice the partials of chunks half as long
+  // (B1-H16-T512-D64 fp16 forward 17.6 us, 18.6 with four chunks; fp32, whose state kernel is longer, 24.1 and 21.6).
+  const bool two = dtype != kF32 && p.L <= 512 && (int64_t)p.N * p.H >= 16;
+  return whole ? whole : chunk_for(p, per_cu, 1, block_stats || two ? 256 : least_state_chunk(p), 64, true);
 }
 
 int bwd_a_chunk(const Prob& p) {
@@ -2545,7 +2554,7 @@ int bwd_a_chunk(const Prob& p) {
 
   // 128 x 128: two workgroups of four waves per CU, steps of 64 tokens
   if (tiled_dim(p.DK) == 128 || tiled_dim(p.DV) == 128) return chunk_for(p, 2, 1, least_chunk(p, 512, 128), 64, true);
-  return chunk_for(p, per_cu, 1, least_chunk(p, 256, 128), 128, true);
+  return chunk_for(p, per_cu, 1, least_chunk(p, 256, 128, 32), 128, true);
 }
 
 static bool use_rows128(const Prob& p);

@@ -77,11 +77,11 @@ static Prob with_chunk_bases(const Prob& p, int dtype, int chunk, void* workspac
   return r;
 }
 static int fwd_chunk(const Prob& p, int dtype) {
-  return mfma::supported(p, dtype) ? mfma::state_chunk(p) : generic::state_chunk(p);
+  return mfma::supported(p, dtype) ? mfma::state_chunk(p, dtype) : generic::state_chunk(p);
 }
 static int bwd_chunk(const Prob& p, int dtype) {
   if (mfma::bwd_a_supported(p, dtype)) return mfma::bwd_a_chunk(p);
-  return mfma::supported(p, dtype) ? mfma::state_chunk(p) : generic::state_chunk(p);
+  return mfma::supported(p, dtype) ? mfma::state_chunk(p, dtype) : generic::state_chunk(p);
 }
 // per-row scalars 1/z_t and dz_t of the two-kernel backward pass A
 static size_t tokscal_bytes(const Prob& p, int dtype) {
@@ -98,10 +98,11 @@ static bool fold_reduce(const Prob& p, int reduce_nchunks, int DR, int DC) {
   const double extra = (double)p.N * p.H * (double)(rows_nchunks - 1) * reduce_nchunks *
                        ((double)p.DK * p.DV + p.DK) * sizeof(float);
   static const double limit = tuning_knob("FBLA_FOLD_MAX_MB", 16) * 1e6;
-  // Nor do the partials of one head exceed what a prologue reads in less than a launch takes: four of 64 x 64 (B2-H4-T1024
-  // fp16 with eight: forward 16.8 us folded, 13.0 reduced; B1-H2-T1024-D128 with eight: 36.2, 22.3).
+  // Nor do the partials of one head, where there are more than two, exceed what a prologue reads in less than a launch takes:
+  // four of 64 x 64 (B2-H4-T1024 fp16 with eight: forward 16.8 us folded, 13.0 reduced; B1-H2-T1024-D128 with eight: 36.2, 22.3;
+  // a step of B1-H48-T640-D128 with two: 85.9 folded, 88.1 reduced).
   static const double each = tuning_knob("FBLA_FOLD_EACH_KB", 70) * 1024.0;
-  return extra <= limit && reduce_nchunks * ((double)p.DK * p.DV + p.DK) * sizeof(float) <= each;
+  return extra <= limit && (reduce_nchunks <= 2 || reduce_nchunks * ((double)p.DK * p.DV + p.DK) * sizeof(float) <= each);
 }
 
 // the walking order of a packed batch with too many sequences to rank inside every workgroup

@@ -75,6 +75,14 @@ def test_forward_workspace_of_ragged_heads_holds_the_generic_kernels():
     assert need >= up((3000 + 63) // 64 * (127 * 126 + 127) * 4)
 
 
+@pytest.mark.parametrize("H,L,D", [(1, 8192, 64), (1, 4096, 128), (3, 4096, 64), (2, 4096, 128), (16, 512, 64)])
+def test_long_heads_are_not_cut_finer_than_their_partials_are_worth(H, L, D):
+    """The forward's workspace holds one state partial a chunk: few heads are cut until 32 workgroups run, no further."""
+    slot = (D * D + D) * 4
+    need = _hip.lib().fbla_la_workspace_bytes(0, 1, H, L, D, D, _hip.F16, _hip.NORMALIZE)
+    assert need <= max(32, H * L // 256) * slot + 4096
+
+
 class _Described(torch.Tensor):
     is_cuda = True
 
