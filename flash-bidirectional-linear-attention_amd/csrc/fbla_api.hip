@@ -98,6 +98,15 @@ static size_t workspace_bytes(const Prob& p, int dtype, int pass) {
   return pass == 0 ? plan::fwd_workspace_bytes(p, dtype) : plan::bwd_workspace_bytes(p, dtype);
 }
 
+// The dense forward of fbla_la_fwd and fbla_la_fwd_static.  Finer chunks for few heads (up to 8 MiB of partials) are not taken
+// where the problem fits the built-in scratch without them only: what that entry point takes does not depend on them.
+static Prob forward_prob(const Prob& p, int dtype) {
+  if (workspace_bytes(p, dtype, 0) <= FBLA_STATIC_SCRATCH_BYTES) return p;
+  Prob coarse = p;
+  coarse.flags |= kCoarse;
+  return workspace_bytes(coarse, dtype, 0) <= FBLA_STATIC_SCRATCH_BYTES ? coarse : p;
+}
+
 static int run_fwd(const char* what, const Prob& p, int dtype, const FwdArgs& a, hipStream_t st) {
   if ((int64_t)p.N * p.H == 0 || p.L == 0) return kOk;
   if (check_aligned(what, {a.q, a.k, a.v, a.q_rope, a.k_rope, a.o, a.s, a.km, a.workspace}) != kOk)
@@ -148,7 +157,7 @@ size_t fbla_la_workspace_bytes(int pass, int64_t B, int64_t H, int64_t L, int DK
                                int flags) {
   if (check_dims("fbla_la_workspace_bytes", B, H, L, DK, DV, dtype, flags) != kOk) return 0;
   Prob p = make_prob(nullptr, B, H, L, B * L, DK, DV, flags, 1.f, 0.f);
-  return workspace_bytes(p, dtype, pass);
+  return workspace_bytes(pass == 0 ? forward_prob(p, dtype) : p, dtype, pass);
 }
 
 int fbla_la_fwd(const void* q, const void* k, const void* v, const void* q_rope,
@@ -169,7 +178,7 @@ int fbla_la_fwd(const void* q, const void* k, const void* v, const void* q_rope,
       return kErrBadArg;
     }
   }
-  Prob p = make_prob(nullptr, B, H, L, B * L, DK, DV, flags, scale, eps);
+  const Prob p = forward_prob(make_prob(nullptr, B, H, L, B * L, DK, DV, flags, scale, eps), dtype);
   FwdArgs a{q, k, v, q_rope, k_rope, o, s, km, workspace, workspace_bytes_};
   return run_fwd(what, p, dtype, a, (hipStream_t)stream);
 }
@@ -253,7 +262,7 @@ int fbla_la_fwd_static(const void* q, const void* k, const void* v, const void* 
     set_error("%s: null tensor pointer", what);
     return kErrBadArg;
   }
-  Prob p = make_prob(nullptr, B, H, L, B * L, DK, DV, flags, scale, eps);
+  const Prob p = forward_prob(make_prob(nullptr, B, H, L, B * L, DK, DV, flags, scale, eps), dtype);
   const size_t need = workspace_bytes(p, dtype, 0);
   if (need > kStaticScratchBytes) {
     set_error("%s: this problem needs %zu bytes of workspace, the built-in scratch holds %zu; "

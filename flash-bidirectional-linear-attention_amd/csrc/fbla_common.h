@@ -22,6 +22,7 @@ enum Flags : int {
                       // with respect to x: the kernels multiply them by phi'(x) = min(phi(x), 1)
   kXcdOrder = 256,    // internal (set per launch): packed batches keep a sequence's heads on one XCD
   kInterleave = 512,  // internal (set per launch): the workgroups of a head take interleaved token steps
+  kCoarse = 1024,     // internal: few heads keep the chunks of many (mfma::state_chunk), whose partials are fewer
 };
 // what a caller may pass; the per-launch bits are the plan's alone (set from outside they would change
 // how the kernels walk without changing how the partials are counted)

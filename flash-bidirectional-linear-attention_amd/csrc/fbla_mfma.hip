@@ -2507,6 +2507,7 @@ static int chunk_for(const Prob& p, int wgs_per_cu, int rounds, int min_chunk, i
 // of 128 x 128 gains (B1-H1-T8192 36.1 / 33.5).
 static int least_chunk(const Prob& p, int chunk, int least, int few_long = 64) {
   static const int few = knob("FBLA_LEAST_WGS", 64);
+  if (p.flags & kCoarse) return chunk;
   const int64_t nh = (int64_t)p.N * p.H, slot = ((int64_t)p.DK * p.DV + p.DK) * (int64_t)sizeof(float);
   while (chunk / 2 >= least && nh * cdiv64(p.L, chunk) < (cdiv64(p.L, chunk) < 16 ? few : few_long) &&
          nh * cdiv64(p.L, chunk / 2) * slot <= 8 << 20)

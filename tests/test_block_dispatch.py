@@ -83,6 +83,15 @@ def test_long_heads_are_not_cut_finer_than_their_partials_are_worth(H, L, D):
     assert need <= max(32, H * L // 256) * slot + 4096
 
 
+@pytest.mark.parametrize("B,H,L,DK,DV,dtype,flags", [
+    (3, 3, 1750, 110, 87, _hip.F16, 0), (4, 1, 1704, 126, 126, _hip.F32, 1), (8, 2, 648, 83, 114, _hip.BF16, 3),
+    (1, 16, 689, 76, 123, _hip.F16, 3), (2, 2, 3520, 121, 84, _hip.BF16, 0), (7, 1, 1140, 125, 97, _hip.F32, 1)])
+def test_finer_chunks_do_not_take_a_forward_past_the_built_in_scratch(B, H, L, DK, DV, dtype, flags):
+    """fbla_la_fwd_static took these: their chunks of 256 tokens need less than the scratch, finer ones more."""
+    need = _hip.lib().fbla_la_workspace_bytes(0, B, H, L, DK, DV, dtype, flags)
+    assert need <= _hip.lib().fbla_static_scratch_bytes()
+
+
 class _Described(torch.Tensor):
     is_cuda = True
 
