@@ -19,6 +19,8 @@ import torch.nn as nn
 from torch._C import _functorch
 from torch._functorch.pyfunctorch import temporarily_clear_interpreter_stack
 from torch.nn.modules.module import _has_any_global_hook
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 from flash_bla import _hip
 from flash_bla.ops.projection import eager_call, gradient_of, splits_tokens
@@ -99,10 +101,16 @@ def _run(call, inputs):
     return call.run(inputs, trains=False)[0]
 
 
+def _watched():
+    """Whether a torch function mode would see, or replace, the operators that the steps call (a default device is one, too, and
+    neither)."""
+    return torch._C._len_torch_function_stack() and any(type(mode) is not DeviceContext for mode in _get_current_function_mode_stack())
+
+
 def _ordinary(block, kind, x, modules):
     """An eager call of the block's own class on GPU rows, nothing around or in place of its modules' forwards."""
     return (type(x) is torch.Tensor and x.is_cuda and x.ndim == 3 and type(block) is kind and not torch.is_autocast_enabled() and
-            eager_call() and not _has_any_global_hook() and _hip.untouched_modules(modules))
+            eager_call() and not _watched() and not _has_any_global_hook() and _hip.untouched_modules(modules))
 
 
 def _same_convolution(conv):

@@ -538,3 +538,16 @@ def test_composed_gradients_of_a_whole_call_are_those_of_its_forward(name, nativ
 @pytest.mark.parametrize("slope,kept", [(0.01, True), (0, True), (-0.1, False), (float("nan"), False), (torch.tensor(0.1), False)])
 def test_slopes_that_turn_signs_run_step_by_step(slope, kept):
     assert _whole._keeps_signs(nn.LeakyReLU(slope)) == kept
+
+
+def test_function_modes_are_noticed():
+    """What watches or replaces torch's functions sees a block's steps; a default device is no such thing."""
+    class Watch(torch.overrides.TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+    assert not _whole._watched()
+    with torch.device("cpu"):
+        assert not _whole._watched()
+        with Watch():
+            assert _whole._watched()
+        assert not _whole._watched()

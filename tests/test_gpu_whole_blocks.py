@@ -199,3 +199,20 @@ def test_negative_slope(counted):
     assert not counted
     for a, e in zip(got, _exact(block, x, (), g)):  # (a value whose rounding crosses the kink: 1.5 of its gradient, as in _make)
         assert _distance(a, e) <= 0.1
+
+
+@pytest.mark.parametrize("name", ["mlla", "pola", "focused", "linfusion"])
+def test_function_modes_see_the_steps(name, counted):
+    block, x, extra = _make(name, torch.half)
+    seen = []
+
+    class Watch(torch.overrides.TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(func)
+            return func(*args, **(kwargs or {}))
+    with torch.device("cuda"):  # (a default device looks at no operator)
+        plain = block(x, *extra)
+        assert len(counted) == 1
+        with Watch():
+            _close(block(x, *extra), plain, torch.half)
+    assert len(counted) == 1 and torch.nn.functional.linear in seen
