@@ -17,7 +17,6 @@ import contextlib
 import torch
 import torch.nn as nn
 from torch._C import _functorch
-from torch._functorch.pyfunctorch import temporarily_clear_interpreter_stack
 from torch.nn.modules.module import _has_any_global_hook
 from torch.overrides import _get_current_function_mode_stack
 from torch.utils._device import DeviceContext
@@ -56,6 +55,7 @@ def _batch_of(g):
     elif _functorch.is_batchedtensor(g):
         level, values = _functorch.maybe_get_level(g), _functorch.get_unwrapped(g).movedim(_functorch.maybe_get_bdim(g), 0)
         if not _functorch.is_functorch_wrapped_tensor(values):
+            from torch._functorch.pyfunctorch import temporarily_clear_interpreter_stack  # (a private name: needed here only)
             return values, lambda t: _functorch._add_batch_dim(t, 0, level), temporarily_clear_interpreter_stack
     return None
 

@@ -1,5 +1,9 @@
 """What the blocks' fused steps take and what they leave to the torch compositions, decided on the host: nothing here
 launches a kernel.  A call that torch's operators refuse stays refused, one that they run stays theirs."""
+import os
+import subprocess
+import sys
+
 import pytest
 import torch
 import torch.fx
@@ -551,3 +555,11 @@ def test_function_modes_are_noticed():
         with Watch():
             assert _whole._watched()
         assert not _whole._watched()
+
+
+def test_layers_import_where_a_private_name_of_functorch_is_missing():
+    """A torch without it has every layer; only gradients inside torch.func.vmap ask for it."""
+    code = ("import torch, torch._functorch.pyfunctorch as p; del p.temporarily_clear_interpreter_stack; "
+            "import flash_bla.layers")
+    path = os.pathsep.join(p for p in sys.path if p)
+    subprocess.run([sys.executable, "-c", code], check=True, env={**os.environ, "PYTHONPATH": path})
