@@ -114,10 +114,10 @@ def _ordinary(block, kind, x, modules):
 
 
 def _same_convolution(conv):
-    """Stride 1 and "same" zero padding; the filter's shape is compared natively."""
-    K = conv.kernel_size[0]
+    """Stride 1 and "same" zero padding for the filters that it holds; their shape is compared natively."""
+    Cw, K = conv.weight.shape[0], conv.weight.shape[-1]
     return (conv.kernel_size == (K, K) and conv.padding == (K // 2, K // 2) and conv.padding_mode == 'zeros' and
-            conv.stride == (1, 1) and conv.dilation == (1, 1) and conv.groups == conv.in_channels)
+            conv.stride == (1, 1) and conv.dilation == (1, 1) and conv.groups == Cw)
 
 
 def _splits(rows, weight, bias):
@@ -277,7 +277,8 @@ def linfusion(block, kind, x, cu):
         return None
     params = [t for p in paths for i in (0, 1, 3) for t in (p[i].weight, p[i].bias)]
     params += [t for m in projections for t in (m.weight, m.bias)]
-    if not (all(_keeps_signs(p[2]) for p in paths) and _hip.plain_gpu_tensors(x, *params) and all(len(p[1].normalized_shape) == 1 and p[1].normalized_shape[0] == p[0].out_features
-                                                       for p in paths) and _hip.linfusion_fits(x, params, block.heads)):
+    if not (all(_keeps_signs(p[2]) for p in paths) and _hip.plain_gpu_tensors(x, *params) and
+            all(tuple(p[1].normalized_shape) == tuple(p[0].weight.shape[:1]) for p in paths) and
+            _hip.linfusion_fits(x, params, block.heads)):
         return None
     return _run(_LinFusion(block, kind), (x, *params, cu()))

@@ -563,3 +563,14 @@ def test_layers_import_where_a_private_name_of_functorch_is_missing():
             "import flash_bla.layers")
     path = os.pathsep.join(p for p in sys.path if p)
     subprocess.run([sys.executable, "-c", code], check=True, env={**os.environ, "PYTHONPATH": path})
+
+
+def test_convolutions_whose_weight_was_replaced_are_not_taken_for_what_they_were():
+    """torch reads groups and padding off the module and refuses filters that do not go with them (or leaves a smaller grid)."""
+    def conv(**more):
+        return nn.Conv2d(8, 8, 3, padding=1, groups=8, **more)
+    assert _whole._same_convolution(conv())
+    for shape in ((8, 1, 5, 5), (4, 1, 3, 3), (16, 1, 3, 3)):
+        other = conv()
+        other.weight = nn.Parameter(torch.zeros(shape))
+        assert not _whole._same_convolution(other)
