@@ -123,6 +123,11 @@ Tensor scratch(size_t bytes, const Tensor& like) {
   return at::empty({std::max<int64_t>((int64_t)bytes, 1)}, like.options().dtype(at::kByte));
 }
 
+// A number that sizes are divided by (in C++ a division by zero ends the process).
+void check_positive(const char* what, int64_t n) {
+  if (n < 1) throw py::value_error(std::string(what) + " must be positive, got " + std::to_string(n));
+}
+
 // Makes the tensor's device the current one and holds torch's current stream there.
 struct On {
   c10::DeviceGuard guard;
@@ -273,6 +278,7 @@ struct Statistics {
 };
 
 Statistics chunk_reduce(const Tensor& q_, const Tensor& k_, const Tensor& v_, int64_t chunk, bool with_norm, double p_norm) {
+  check_positive("chunk", chunk);
   require_gpu({q_, k_, v_});
   const Tensor q = whole(q_), k = whole(k_), v = whole(v_);
   const int64_t B = k.size(0), H = k.size(1), T = k.size(2), NT = (T + chunk - 1) / chunk;
@@ -439,7 +445,9 @@ std::vector<Normed> norm_leaky(const std::vector<Norm>& p, bool with_stats) {
   std::array<fbla_norm, 2> jobs{};
   std::vector<Tensor> keep;
   std::vector<Normed> r;
-  const int64_t C = p[0].x.size(-1), tokens = p[0].x.numel() / C;
+  const int64_t C = p[0].x.size(-1);
+  check_positive("channels", C);
+  const int64_t tokens = p[0].x.numel() / C;
   for (size_t i = 0; i < p.size(); ++i) {
     TORCH_CHECK(p[i].x.sizes() == p[0].x.sizes());
     const Tensor x = whole(p[i].x), weight = whole(p[i].weight), bias = whole(p[i].bias);
@@ -457,6 +465,7 @@ std::vector<Normed> norm_leaky(const std::vector<Norm>& p, bool with_stats) {
 // qg [B,N,2C], kv [B,n,2C], pe [1,n,C], scale [1,1,C], power [1,heads,1,d] -> q_same, q_opp, k_both [B,heads,.,2d], v [B,heads,n,d]
 std::array<Tensor, 4> polarity_fwd(const Tensor& qg_, const Tensor& kv_, const Tensor& pe_, const Tensor& scale_, const Tensor& power_,
                                    int64_t heads) {
+  check_positive("heads", heads);
   require_gpu({qg_, kv_, pe_, scale_, power_});
   const Tensor qg = whole(qg_), kv = whole(kv_), pe = whole(pe_), scale = whole(scale_), power = whole(power_);
   const int64_t B = qg.size(0), N = qg.size(1), n = kv.size(1), d = qg.size(2) / 2 / heads;
@@ -472,6 +481,7 @@ std::array<Tensor, 4> polarity_fwd(const Tensor& qg_, const Tensor& kv_, const T
 std::array<Tensor, 5> polarity_bwd(const Tensor& qg_, const Tensor& kv_, const Tensor& pe_, const Tensor& scale_, const Tensor& power_,
                                    int64_t heads, const Tensor& dq_same, const Tensor& dq_opp, const Tensor& dk_both, const Tensor& dv,
                                    const Tensor& dv_rows, const Tensor& dgate) {
+  check_positive("heads", heads);
   require_gpu({qg_, kv_, pe_, scale_, power_, dq_same, dq_opp, dk_both, dv, dv_rows, dgate});
   const Tensor qg = whole(qg_), kv = whole(kv_), pe = whole(pe_), scale = whole(scale_), power = whole(power_);
   const std::array<Tensor, 6> g{whole(dq_same), whole(dq_opp), whole(dk_both), whole(dv), whole(dv_rows), whole(dgate)};
@@ -488,6 +498,7 @@ std::array<Tensor, 5> polarity_bwd(const Tensor& qg_, const Tensor& kv_, const T
 
 // qk [B,N,2C], x [B,N,C], rotations fp32 [..., pairs, 2] over the N tokens -> q, k, q_rot, k_rot, v [B,heads,N,d]
 std::array<Tensor, 5> rotary_fwd(const Tensor& qk_, const Tensor& x_, const Tensor& rotations_, int64_t heads) {
+  check_positive("heads", heads);
   require_gpu({qk_, x_, rotations_});
   const Tensor qk = whole(qk_), x = whole(x_), rotations = whole(rotations_);
   const int64_t B = x.size(0), N = x.size(1), d = x.size(2) / heads;
@@ -502,6 +513,7 @@ std::array<Tensor, 5> rotary_fwd(const Tensor& qk_, const Tensor& x_, const Tens
 // gradients of qk and x; dv_rows [B,N,C] is added to the values' gradient
 std::pair<Tensor, Tensor> rotary_bwd(const Tensor& qk_, const Tensor& rotations_, int64_t heads, const Tensor& dq, const Tensor& dk,
                                      const Tensor& dq_rot, const Tensor& dk_rot, const Tensor& dv, const Tensor& dv_rows) {
+  check_positive("heads", heads);
   require_gpu({qk_, rotations_, dq, dk, dq_rot, dk_rot, dv, dv_rows});
   const Tensor qk = whole(qk_), rotations = whole(rotations_);
   const std::array<Tensor, 6> g{whole(dq), whole(dk), whole(dq_rot), whole(dk_rot), whole(dv), whole(dv_rows)};
@@ -532,6 +544,7 @@ struct MergeGrads {
 // without a gate o, o2 and local are not looked at
 MergeGrads merge_bwd(const Tensor& dout_, int64_t heads, bool halves, const Tensor& o_, const Tensor& o2_, const Tensor& local_,
                      const Tensor& gate_) {
+  check_positive("heads", heads);
   require_gpu({dout_, o_, o2_, local_, gate_});
   const Tensor dout = whole(dout_), o = whole(o_), o2 = whole(o2_), local = whole(local_), gate = rows_of_batches(gate_);
   const int64_t B = dout.size(0), N = dout.size(1), d = dout.size(2) / heads, width = halves ? d / 2 : d;
@@ -569,6 +582,7 @@ Tensor interpolate_bwd(const Tensor& g_, int64_t n) {
 
 // q [B,N,C], kv [B,n,2C], pe [1,n,C], scale [1,1,C] -> q, k, v [B,heads,tokens,d]
 std::array<Tensor, 3> focus_fwd(const Tensor& q_, const Tensor& kv_, const Tensor& pe_, const Tensor& scale_, int64_t heads) {
+  check_positive("heads", heads);
   require_gpu({q_, kv_, pe_, scale_});
   const Tensor q = whole(q_), kv = whole(kv_), pe = whole(pe_), scale = whole(scale_);
   const int64_t B = q.size(0), N = q.size(1), n = kv.size(1), d = q.size(2) / heads;
@@ -582,6 +596,7 @@ std::array<Tensor, 3> focus_fwd(const Tensor& q_, const Tensor& kv_, const Tenso
 // gradients of q, kv, pe and scale; dv_rows [B,n,C] is added to the values' gradient
 std::array<Tensor, 4> focus_bwd(const Tensor& q_, const Tensor& kv_, const Tensor& pe_, const Tensor& scale_, int64_t heads,
                                 const Tensor& dq, const Tensor& dk, const Tensor& dv, const Tensor& dv_rows) {
+  check_positive("heads", heads);
   require_gpu({q_, kv_, pe_, scale_, dq, dk, dv, dv_rows});
   const Tensor q = whole(q_), kv = whole(kv_), pe = whole(pe_), scale = whole(scale_);
   const std::array<Tensor, 4> g{whole(dq), whole(dk), whole(dv), whole(dv_rows)};
@@ -1104,7 +1119,7 @@ bool conv_shapes(const Tensor& w, const Tensor& b, int64_t Cw, int64_t C) {
 // the shapes that the steps of a block take one by one (layers/_features.py, ops/depthwise.py, ops/projection.py)
 bool mlla_fits(const Tensor& x, const std::vector<Maybe>& p, const Tensor& rotations, int64_t side, int64_t heads) {
   const Tensor w = given(p[0]), b = given(p[1]), conv_w = given(p[2]), conv_b = given(p[3]);
-  if (x.dim() != 3) return false;
+  if (x.dim() != 3 || heads < 1) return false;
   const int64_t C = x.size(2), piece = 16 / x.element_size();
   return x.size(1) == side * side && C % heads == 0 && C / heads % piece == 0 && C / heads <= 128 && linear_shapes(w, b, 2 * C, C, piece) &&
          conv_shapes(conv_w, conv_b, C, C) && rotations.scalar_type() == at::kFloat && rotations.device() == x.device() &&
@@ -1114,7 +1129,7 @@ bool mlla_fits(const Tensor& x, const std::vector<Maybe>& p, const Tensor& rotat
 bool pvt_fits(const Tensor& x, const Tensor& src, const Tensor& kv_w, const Tensor& kv_b, const Tensor& pe, const Tensor& scale,
               const Tensor& conv_w, const Tensor& conv_b, const Tensor& proj_w, const Tensor& proj_b, int64_t H, int64_t W, int64_t heads,
               int64_t unit) {
-  if (x.dim() != 3 || src.dim() != 3 || !proj_w.defined() || proj_w.dim() != 2) return false;
+  if (x.dim() != 3 || src.dim() != 3 || heads < 1 || !proj_w.defined() || proj_w.dim() != 2) return false;
   const int64_t C = x.size(2), n = src.size(1), piece = 16 / x.element_size();
   return H > 0 && x.size(1) == H * W && C % heads == 0 && C / heads % (unit * piece) == 0 && shaped(src, {x.size(0), n, C}) &&
          linear_shapes(kv_w, kv_b, 2 * C, C, piece) && shaped(pe, {1, n, C}) && shaped(scale, {1, 1, C}) &&

@@ -574,3 +574,26 @@ def test_convolutions_whose_weight_was_replaced_are_not_taken_for_what_they_were
         other = conv()
         other.weight = nn.Parameter(torch.zeros(shape))
         assert not _whole._same_convolution(other)
+
+
+@pytest.mark.parametrize("heads", [0, -2])
+def test_numbers_of_heads_that_are_none_do_not_fit(heads):
+    """Python's division by zero raises, C++'s ends the process."""
+    block, x = MambaLikeLinearAttention(64, (4, 4), 2), torch.zeros(1, 16, 64)
+    params = (block.qk.weight, block.qk.bias, block.lepe.weight, block.lepe.bias)
+    assert _hip.mlla_fits(x, params, block.rope.rotations, 4, 2) and not _hip.mlla_fits(x, params, block.rope.rotations, 4, heads)
+    for fits, block, q in ((_hip.pola_fits, PolaLinearAttention(64, 16, num_heads=2, qkv_bias=True), "qg"),
+                           (_hip.focused_fits, FocusedLinearAttention(64, 16, num_heads=2, qkv_bias=True), "q")):
+        names = [f"{q}.weight", f"{q}.bias", "kv.weight", "kv.bias", "positional_encoding", "scale", "power", "dwc.weight", "dwc.bias",
+                 "proj.weight", "proj.bias"]
+        named = dict(block.named_parameters())
+        params = [named[n] for n in names if n in named]
+        assert fits(x, x, params, 4, 4, 2) and not fits(x, x, params, 4, 4, heads)
+    rows, heads4 = torch.zeros(1, 16, 128), torch.zeros(1, 2, 16, 32)
+    for call in (lambda: _hip.polarity_fwd(rows, rows, rows, rows, rows, heads), lambda: _hip.rotary_fwd(rows, x, rows, heads),
+                 lambda: _hip.focus_fwd(x, rows, x, x, heads), lambda: _hip.merge_bwd(x, heads, False, None, None, None, None),
+                 lambda: _hip.polarity_bwd(rows, rows, rows, rows, rows, heads, *[rows] * 6),
+                 lambda: _hip.rotary_bwd(rows, rows, heads, *[x] * 6), lambda: _hip.focus_bwd(x, rows, x, x, heads, *[x] * 4),
+                 lambda: _hip.chunk_reduce(heads4, heads4, heads4, heads), lambda: _hip.norm_leaky([(x[..., :0], None, None, 1e-5, 0.1)], False)):
+        with pytest.raises(ValueError, match="positive"):
+            call()
