@@ -638,13 +638,20 @@ std::array<Tensor, 3> turn_bwd(const Tensor& k_, const Tensor& weight_, const Te
 // Python call and their checks between them.  The gradient of a tensor that two steps read is accumulated by the second
 // step's GEMM instead of a launch of its own (12 us at 200704 x 64 and 50176 x 256 in bf16).
 Tensor flat(const Tensor& t) { return t.reshape({-1, t.size(-1)}); }
-// Whether `project` takes a projection of these rows rather than torch's GEMM: 16-bit types, unless the product is large enough
-// for the library's deeper pipeline to count.  GPU us of the library / here (bf16, with bias; a call of the library takes the
-// host 17 us, one of ours 4): 8192 x 640 -> 640 13.2 / 14.5, three of them 40 / 30.3; 1024 x 1280 -> 1280 11.2 / 12.5; 4096 x 1280 -> 1280
-// 20 / 26.8; see fbla_gemm.hip.
+// Whether `project` takes a projection of these rows rather than torch's GEMM: 16-bit types within the entry point's limits
+// (fbla_project refuses others), unless both sides of the weight are 512 and more and the product is one of 4e9 multiply-adds and
+// more, where the library's deeper pipeline counts.  The line is drawn for a call by itself, host included: a call of the library
+// takes the host 17 us, one of ours 4 for up to three products.  GPU us of the library / here (bf16, with bias): 8192 x 640 -> 640
+// 14.4 / 16.8, three of them 42.6 / 37.1; 1024 x 1280 -> 1280 12.0 / 13.5; 4096 x 1280 -> 1280 21.5 / 26.1; 12544 x 512 -> 512 15.4 / 18.5,
+// -> 1024 20.7 / 28.5; 50176 x 256 -> 256 15.8 / 20.3, -> 512 41 / 38.5.  In a captured graph, which pays no host time, the products
+// below the line that the library is faster at cost up to 10 us more here (50176 x 512 -> 256 24.1 / 33.6).
 bool projects(const Tensor& x, const Tensor& w) {
+  constexpr int64_t kMostChannels = 1 << 16, kMostWeights = 1 << 29, kLongestRow = 1 << 22;  // of fbla_project
+  if (x.element_size() != 2 || w.size(0) > kMostChannels || w.size(1) > kMostChannels || w.numel() > kMostWeights ||
+      (x.dim() > 1 && x.stride(-2) > kLongestRow))
+    return false;
   const double work = (double)(x.numel() / x.size(-1)) * w.numel();
-  return x.element_size() == 2 && (w.size(0) < 512 || w.size(1) < 512 || work <= 4e9);
+  return w.size(0) < 512 || w.size(1) < 512 || work <= 4e9;
 }
 // y = x W^T + b (+ add) for one or more projections
 struct Linear {

@@ -216,3 +216,22 @@ def test_function_modes_see_the_steps(name, counted):
         with Watch():
             _close(block(x, *extra), plain, torch.half)
     assert len(counted) == 1 and torch.nn.functional.linear in seen
+
+
+@pytest.mark.parametrize("what", ["outputs", "rows"])
+def test_projections_past_the_kernels_limits_run_on_the_library(what, counted, monkeypatch):
+    """More outputs than the projections' kernel addresses, rows further apart: the library's GEMM takes them as it always did."""
+    block, x, extra = _make("focused" if what == "outputs" else "linfusion", torch.half)
+    if what == "outputs":
+        block.proj = torch.nn.Linear(64, 65544).cuda().half()
+    else:
+        row = (1 << 22) + 8
+        x = torch.empty(3 * 40 * row, device="cuda", dtype=torch.half).as_strided((3, 40, 128), (40 * row, row, 1)).copy_(x)
+    got = []
+    for whole in (True, False):
+        leaf = x.detach().requires_grad_()
+        out = block(leaf, *extra) if whole else _steps(block, monkeypatch, lambda b: b(leaf, *extra))
+        got.append([out.detach(), *torch.autograd.grad(out, [leaf, *block.parameters()], torch.ones_like(out))])
+    assert len(counted) == 1
+    for a, b in zip(*got):
+        _close(a, b, torch.half)
