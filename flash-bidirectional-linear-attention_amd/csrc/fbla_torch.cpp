@@ -743,20 +743,20 @@ std::vector<Tensor> mlla_fwd(const Tensor& x, const Tensor& w, const Tensor& b, 
   return {merge_fwd(a.o, Tensor(), local, Tensor()), qk, q, k, qr, kr, v, a.s, a.km};
 }
 
-// saved: what mlla_fwd returned after its output.  need: x, w, b, conv_w, conv_b
+// saved: what mlla_fwd returned after its output, or what saved-tensor hooks made of it (any strides).  need: x, w, b, conv_w, conv_b
 std::vector<Tensor> mlla_bwd(const Tensor& g, const Tensor& x, const Tensor& w, const Tensor& conv_w, const Tensor& rotations,
                              const std::vector<Tensor>& saved, int64_t side, int64_t heads, const std::array<bool, 5>& need, bool kernel) {
   const NoGraph none;
   Tensor dx, dw, db, dconv_w, dconv_b;
   if (need[3] || need[4]) std::tie(dconv_w, dconv_b) = dwconv_grad(x, g, conv_w, side, side, need[4]);
   if (need[0] || need[1] || need[2]) {
-    const Tensor qk = saved.at(0), dlocal = dwconv_fwd(g, conv_w, Tensor(), side, side, true);
+    const Tensor qk = whole(saved.at(0)), dlocal = dwconv_fwd(g, conv_w, Tensor(), side, side, true);
     Tensor dqk;
     if (saved.size() == 3) {
       const Tensor xs = whole(x), gs = whole(g), rot = whole(rotations);
       dqk = like(qk), dx = like(gs);
       const int64_t C = x.size(2);
-      fbla_block_attn a = row_args(kRotary, qk, 0, qk, C, xs, 0, heads, {saved[1], saved[2]});
+      fbla_block_attn a = row_args(kRotary, qk, 0, qk, C, xs, 0, heads, {whole(saved[1]), whole(saved[2])});
       const Tensor ws = row_workspace(a, x);
       a.rot = f32(rot), a.workspace = ptr(ws), a.workspace_bytes = ws.numel(), a.dout = ptr(gs), a.dv_more = ptr(dlocal);
       a.dq = ptr(dqk), a.dk = static_cast<char*>(ptr(dqk)) + C * dqk.element_size(), a.dv = ptr(dx);
@@ -855,7 +855,7 @@ std::vector<Tensor> pola_bwd(const Tensor& g, const Tensor& x, const Tensor& src
   auto at_ = [&](int i) { return given(saved.at(i)); };
   const bool rows_ = saved.size() == 7;
   TORCH_CHECK(rows_ || saved.size() == 20);
-  const Tensor qg = at_(rows_ ? 0 : 3), kv = at_(rows_ ? 1 : 4), merged = at_(rows_ ? 6 : 19);
+  const Tensor qg = whole(at_(rows_ ? 0 : 3)), kv = whole(at_(rows_ ? 1 : 4)), merged = at_(rows_ ? 6 : 19);
   const int64_t n = src.size(1), C = x.size(2);
   std::vector<Tensor> r(2 + kPola);
   std::tie(r[11], r[12]) = weight_grad(g, merged, need[11], need[12], kernel[2]);
@@ -863,9 +863,9 @@ std::vector<Tensor> pola_bwd(const Tensor& g, const Tensor& x, const Tensor& src
   const Tensor dmerged = input_grad(g, p.proj_w);
   std::array<Tensor, 5> d;  // of qg, kv, pe, scale, power
   if (rows_) {
-    const Tensor grid = at_(2), local = at_(3), pe = whole(p.pe), scale = whole(p.scale), power = whole(p.power), dlocal = like(dmerged);
+    const Tensor grid = at_(2), local = whole(at_(3)), pe = whole(p.pe), scale = whole(p.scale), power = whole(p.power), dlocal = like(dmerged);
     d = {like(qg), like(kv), like(pe), like(scale), like(power)};
-    fbla_block_attn a = row_args(kPolarity, qg, 0, kv, 0, kv, C, heads, {at_(4), at_(5)});
+    fbla_block_attn a = row_args(kPolarity, qg, 0, kv, 0, kv, C, heads, {whole(at_(4)), whole(at_(5))});
     const Tensor ws = row_workspace(a, x);
     auto half = [&](const Tensor& t) { return static_cast<char*>(ptr(t)) + C * t.element_size(); };
     a.local = ptr(local), a.gate = half(qg), a.gate_row = 2 * C, a.dout = ptr(dmerged), a.pe = ptr(pe), a.scale = ptr(scale);
@@ -1019,7 +1019,7 @@ std::vector<Tensor> linfusion_bwd(const Tensor& g, const Tensor& x, const Tensor
   Tensor dx = need[0] ? input_grad(d[2], p.w[2]) : Tensor();
   for (int i = 0; i < 2; ++i) {
     const auto& path = p.path[i];
-    const Tensor hidden = at_(5 * i), mean = at_(5 * i + 1), rstd = at_(5 * i + 2), normed = at_(5 * i + 3), in = at_(5 * i + 4);
+    const Tensor hidden = whole(at_(5 * i)), mean = whole(at_(5 * i + 1)), rstd = whole(at_(5 * i + 2)), normed = at_(5 * i + 3), in = at_(5 * i + 4);
     const int at0 = 1 + 6 * i;
     std::tie(r[13 + 2 * i], r[14 + 2 * i]) = weight_grad(d[i], in, need[13 + 2 * i], need[14 + 2 * i], kernel[4 + i]);
     const Tensor din = input_grad(d[i], p.w[i]);  // of x + residual

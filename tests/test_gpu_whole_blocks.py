@@ -235,3 +235,22 @@ def test_projections_past_the_kernels_limits_run_on_the_library(what, counted, m
     assert len(counted) == 1
     for a, b in zip(*got):
         _close(a, b, torch.half)
+
+
+@pytest.mark.parametrize("name", ["mlla", "pola", "focused", "linfusion"])  # (torch's own LayerNorm reads strided statistics wrongly)
+def test_saved_tensors_that_come_back_elsewhere(name, counted):
+    """Saved-tensor hooks may return other strides and addresses that are no multiple of 16 bytes."""
+    def unpack(t):
+        if t.ndim > 1:
+            return torch.cat([t, t + 1], dim=-1)[..., :t.shape[-1]]
+        return torch.cat([t[:1], t])[1:]
+    block, x, extra = _make(name, torch.half)
+    grads = []
+    for hooks in (False, True):
+        leaf = x.detach().requires_grad_()
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack if hooks else lambda t: t):
+            out = block(leaf, *extra)
+        grads.append(torch.autograd.grad(out, [leaf, *block.parameters()], torch.ones_like(out)))
+    assert len(counted) == 2
+    for a, b in zip(*grads):
+        _close(a, b, torch.half)
