@@ -13,6 +13,7 @@
 #include <algorithm>
 #include <array>
 #include <string>
+#include <variant>
 #include <vector>
 
 #include "../../include/flash_bla_hip.h"
@@ -1037,11 +1038,14 @@ std::vector<Tensor> linfusion_bwd(const Tensor& g, const Tensor& x, const Tensor
 }
 
 // None for a tensor that does not exist
-py::object out(const Tensor& t) { return t.defined() ? py::cast(t) : py::none(); }
-template <typename... T> py::tuple outs(const T&... t) { return py::make_tuple(out(t)...); }
-template <size_t N> py::tuple outs(const std::array<Tensor, N>& t) {
-  py::tuple r(N);
-  for (size_t i = 0; i < N; ++i) r[i] = out(t[i]);
+Maybe out(const Tensor& t) { return t.defined() ? Maybe(t) : std::nullopt; }
+template <typename... T> auto outs(const T&... t) { return std::make_tuple(out(t)...); }
+template <size_t N> auto outs(const std::array<Tensor, N>& t) {
+  return std::apply([](const auto&... e) { return std::make_tuple(out(e)...); }, t);
+}
+std::vector<Maybe> listed(const std::vector<Tensor>& t) {
+  std::vector<Maybe> r;
+  for (const Tensor& e : t) r.push_back(out(e));
   return r;
 }
 
@@ -1086,12 +1090,6 @@ bool plain_gpu_tensors(py::handle x_, py::args rest, PyObject* parameter) {
     if (!t || !ordinary(h) || !fits(*t)) return false;
   }
   return true;
-}
-
-py::list listed(const std::vector<Tensor>& t) {
-  py::list r(t.size());
-  for (size_t i = 0; i < t.size(); ++i) r[i] = out(t[i]);
-  return r;
 }
 
 // ---- which blocks run whole -----------------------------------------------------------------------------------------------
@@ -1183,132 +1181,136 @@ PYBIND11_MODULE(fbla_torch, m) {
     }
   });
   m.def("load", &load);
-  m.def("la_fwd", [](const Tensor& q, const Tensor& k, const Tensor& v, const Maybe& qr, const Maybe& kr, double scale, double eps,
+  // Without the interpreter's lock: a launch waits where the queue is full, an allocation where it frees memory, and other Python
+  // threads (those that drive other GPUs among them) run meanwhile.
+  auto op = [&m](const char* name, auto f, const auto&... more) { m.def(name, f, py::call_guard<py::gil_scoped_release>(), more...); };
+  op("la_fwd", [](const Tensor& q, const Tensor& k, const Tensor& v, const Maybe& qr, const Maybe& kr, double scale, double eps,
                      int flags) {
     const Attended r = la_fwd(q, k, v, given(qr), given(kr), scale, eps, flags);
     return outs(r.o, r.s, r.km);
   });
-  m.def("la_bwd", [](const Tensor& q, const Tensor& k, const Tensor& v, const Maybe& qr, const Maybe& kr, const Tensor& g, const Tensor& s,
+  op("la_bwd", [](const Tensor& q, const Tensor& k, const Tensor& v, const Maybe& qr, const Maybe& kr, const Tensor& g, const Tensor& s,
                      const Maybe& km, double scale, double eps, int flags) {
     const AttendedGrads d = la_bwd(q, k, v, given(qr), given(kr), g, s, given(km), scale, eps, flags);
     return outs(d.q, d.k, d.v, d.q_rope, d.k_rope);
   });
   m.def("pair_supported", &pair_supported);
-  m.def("pair_fwd", [](const Tensor& q1, const Tensor& q2, const Tensor& k, const Tensor& v, double scale, double eps) {
+  op("pair_fwd", [](const Tensor& q1, const Tensor& q2, const Tensor& k, const Tensor& v, double scale, double eps) {
     const Paired r = pair_fwd(q1, q2, k, v, scale, eps);
     return outs(r.o1, r.o2, r.s, r.km);
   });
-  m.def("pair_bwd", [](const Tensor& q1, const Tensor& q2, const Tensor& k, const Tensor& v, const Tensor& g1, const Tensor& g2,
+  op("pair_bwd", [](const Tensor& q1, const Tensor& q2, const Tensor& k, const Tensor& v, const Tensor& g1, const Tensor& g2,
                        const Tensor& s, const Tensor& km, double scale, double eps) {
     const PairedGrads d = pair_bwd(q1, q2, k, v, g1, g2, s, km, scale, eps);
     return outs(d.q1, d.q2, d.k, d.v);
   });
-  m.def("varlen_fwd", [](const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& cu, int64_t longest, std::optional<double> scale,
+  op("varlen_fwd", [](const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& cu, int64_t longest, std::optional<double> scale,
                          double eps, int extra) {
     const Attended r = varlen_fwd(q, k, v, cu, longest, scale, eps, extra);
     return outs(r.o, r.s, r.km);
   }, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("cu_seqlens"), py::arg("max_seqlen"), py::arg("scale"), py::arg("eps"),
         py::arg("extra_flags") = 0);
-  m.def("varlen_bwd", &varlen_bwd, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("cu_seqlens"), py::arg("max_seqlen"), py::arg("do"),
+  op("varlen_bwd", &varlen_bwd, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("cu_seqlens"), py::arg("max_seqlen"), py::arg("do"),
         py::arg("s"), py::arg("km"), py::arg("scale"), py::arg("eps"), py::arg("extra_flags") = 0);
-  m.def("chunk_reduce", [](const Tensor& q, const Tensor& k, const Tensor& v, int64_t chunk, bool with_norm, double p_norm) {
+  op("chunk_reduce", [](const Tensor& q, const Tensor& k, const Tensor& v, int64_t chunk, bool with_norm, double p_norm) {
     const Statistics r = chunk_reduce(q, k, v, chunk, with_norm, p_norm);
     return outs(r.qc, r.kc, r.vc, r.h, r.h_norm);
   }, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("chunk"), py::arg("with_norm") = false, py::arg("p_norm") = 2.0);
-  m.def("select_blocks", [](const Tensor& qc, const Tensor& kc, const Maybe& bias, int64_t top_k, double scale) {
+  op("select_blocks", [](const Tensor& qc, const Tensor& kc, const Maybe& bias, int64_t top_k, double scale) {
     return select_blocks(qc, kc, given(bias), top_k, scale);
   });
   m.def("piecewise_supported", &piecewise_supported);
-  m.def("piecewise_fwd", &piecewise_fwd);
-  m.def("elu1_fwd", [](const Tensor& x0, const Maybe& x1) -> py::object {
+  op("piecewise_fwd", &piecewise_fwd);
+  op("elu1_fwd", [](const Tensor& x0, const Maybe& x1) -> std::variant<Tensor, std::pair<Tensor, Tensor>> {
     const auto y = elu1_fwd(x0, given(x1));
-    return x1 ? py::object(outs(y.first, y.second)) : out(y.first);
+    if (x1) return y;
+    return y.first;
   }, py::arg("x0"), py::arg("x1") = py::none());
-  m.def("elu1_bwd", &elu1_bwd);
-  m.def("dwconv_fwd", [](const Tensor& x, const Tensor& w, const Maybe& bias, int64_t H, int64_t W, bool flip) {
+  op("elu1_bwd", &elu1_bwd);
+  op("dwconv_fwd", [](const Tensor& x, const Tensor& w, const Maybe& bias, int64_t H, int64_t W, bool flip) {
     return dwconv_fwd(x, w, given(bias), H, W, flip);
   }, py::arg("x"), py::arg("w"), py::arg("bias"), py::arg("H"), py::arg("W"), py::arg("flip") = false);
-  m.def("dwconv_grad", [](const Tensor& x, const Tensor& g, const Tensor& w, int64_t H, int64_t W, bool with_bias) {
+  op("dwconv_grad", [](const Tensor& x, const Tensor& g, const Tensor& w, int64_t H, int64_t W, bool with_bias) {
     const auto r = dwconv_grad(x, g, w, H, W, with_bias);
     return outs(r.first, r.second);
   });
-  m.def("linear_wgrad", [](const Tensor& g, const Tensor& x, bool with_bias) {
+  op("linear_wgrad", [](const Tensor& g, const Tensor& x, bool with_bias) {
     const auto r = linear_wgrad(g, x, with_bias);
     return outs(r.first, r.second);
   });
-  m.def("project", [](const std::vector<std::array<Maybe, 6>>& p, bool rows_of_w) {
+  op("project", [](const std::vector<std::array<Maybe, 6>>& p, bool rows_of_w) {
     std::vector<Projection> jobs;
     for (const auto& t : p) jobs.push_back({given(t[0]), given(t[1]), given(t[2]), given(t[3]), given(t[4]), given(t[5])});
     return project(jobs, rows_of_w);
   });
-  m.def("norm_leaky", [](const std::vector<std::tuple<Tensor, Maybe, Maybe, double, double>>& p, bool with_stats) {
+  op("norm_leaky", [](const std::vector<std::tuple<Tensor, Maybe, Maybe, double, double>>& p, bool with_stats) {
     std::vector<Norm> jobs;
     for (const auto& [x, w, b, eps, slope] : p) jobs.push_back({x, given(w), given(b), eps, slope});
-    py::list r;
-    for (const Normed& n : norm_leaky(jobs, with_stats)) r.append(outs(n.y, n.mean, n.rstd));
+    std::vector<std::tuple<Maybe, Maybe, Maybe>> r;
+    for (const Normed& n : norm_leaky(jobs, with_stats)) r.push_back(outs(n.y, n.mean, n.rstd));
     return r;
   });
-  m.def("polarity_fwd", [](const Tensor& qg, const Tensor& kv, const Tensor& pe, const Tensor& scale, const Tensor& power, int64_t heads) {
+  op("polarity_fwd", [](const Tensor& qg, const Tensor& kv, const Tensor& pe, const Tensor& scale, const Tensor& power, int64_t heads) {
     return outs(polarity_fwd(qg, kv, pe, scale, power, heads));
   });
-  m.def("polarity_bwd", [](const Tensor& qg, const Tensor& kv, const Tensor& pe, const Tensor& scale, const Tensor& power, int64_t heads,
+  op("polarity_bwd", [](const Tensor& qg, const Tensor& kv, const Tensor& pe, const Tensor& scale, const Tensor& power, int64_t heads,
                            const Tensor& a, const Tensor& b, const Tensor& c, const Tensor& d, const Tensor& e, const Tensor& f) {
     return outs(polarity_bwd(qg, kv, pe, scale, power, heads, a, b, c, d, e, f));
   });
-  m.def("rotary_fwd", [](const Tensor& qk, const Tensor& x, const Tensor& rotations, int64_t heads) {
+  op("rotary_fwd", [](const Tensor& qk, const Tensor& x, const Tensor& rotations, int64_t heads) {
     return outs(rotary_fwd(qk, x, rotations, heads));
   });
-  m.def("rotary_bwd", [](const Tensor& qk, const Tensor& rotations, int64_t heads, const Tensor& a, const Tensor& b, const Tensor& c,
+  op("rotary_bwd", [](const Tensor& qk, const Tensor& rotations, int64_t heads, const Tensor& a, const Tensor& b, const Tensor& c,
                          const Tensor& d, const Tensor& e, const Tensor& f) {
     const auto r = rotary_bwd(qk, rotations, heads, a, b, c, d, e, f);
     return outs(r.first, r.second);
   });
-  m.def("merge_fwd", [](const Tensor& o, const Maybe& o2, const Tensor& local, const Maybe& gate) {
+  op("merge_fwd", [](const Tensor& o, const Maybe& o2, const Tensor& local, const Maybe& gate) {
     return merge_fwd(o, given(o2), local, given(gate));
   });
-  m.def("merge_bwd", [](const Tensor& dout, int64_t heads, bool halves, const Maybe& o, const Maybe& o2, const Maybe& local,
+  op("merge_bwd", [](const Tensor& dout, int64_t heads, bool halves, const Maybe& o, const Maybe& o2, const Maybe& local,
                         const Maybe& gate) {
     const MergeGrads r = merge_bwd(dout, heads, halves, given(o), given(o2), given(local), given(gate));
     return outs(r.o, r.o2, r.local, r.gate);
   });
-  m.def("interpolate_fwd", &interpolate_fwd);
-  m.def("interpolate_bwd", &interpolate_bwd);
-  m.def("focus_fwd", [](const Tensor& q, const Tensor& kv, const Tensor& pe, const Tensor& scale, int64_t heads) {
+  op("interpolate_fwd", &interpolate_fwd);
+  op("interpolate_bwd", &interpolate_bwd);
+  op("focus_fwd", [](const Tensor& q, const Tensor& kv, const Tensor& pe, const Tensor& scale, int64_t heads) {
     return outs(focus_fwd(q, kv, pe, scale, heads));
   });
-  m.def("focus_bwd", [](const Tensor& q, const Tensor& kv, const Tensor& pe, const Tensor& scale, int64_t heads, const Tensor& a,
+  op("focus_bwd", [](const Tensor& q, const Tensor& kv, const Tensor& pe, const Tensor& scale, int64_t heads, const Tensor& a,
                         const Tensor& b, const Tensor& c, const Tensor& d) { return outs(focus_bwd(q, kv, pe, scale, heads, a, b, c, d)); });
-  m.def("turn_fwd", [](const Tensor& q, const Tensor& k, const Tensor& weight, const Tensor& rotations) {
+  op("turn_fwd", [](const Tensor& q, const Tensor& k, const Tensor& weight, const Tensor& rotations) {
     return outs(turn_fwd(q, k, weight, rotations));
   });
-  m.def("turn_bwd", [](const Tensor& k, const Tensor& weight, const Tensor& rotations, const Tensor& a, const Tensor& b, const Tensor& c) {
+  op("turn_bwd", [](const Tensor& k, const Tensor& weight, const Tensor& rotations, const Tensor& a, const Tensor& b, const Tensor& c) {
     return outs(turn_bwd(k, weight, rotations, a, b, c));
   });
 
-  m.def("mlla_fwd", [](const Tensor& x, const std::vector<Maybe>& p, const Tensor& rotations, int64_t side, int64_t heads) {
+  op("mlla_fwd", [](const Tensor& x, const std::vector<Maybe>& p, const Tensor& rotations, int64_t side, int64_t heads) {
     return listed(mlla_fwd(x, given(p[0]), given(p[1]), given(p[2]), given(p[3]), rotations, side, heads));
   });
-  m.def("mlla_bwd", [](const Tensor& g, const Tensor& x, const Tensor& w, const Tensor& conv_w, const Tensor& rotations,
+  op("mlla_bwd", [](const Tensor& g, const Tensor& x, const Tensor& w, const Tensor& conv_w, const Tensor& rotations,
                        const std::vector<Tensor>& s, int64_t side, int64_t heads, const std::array<bool, 5>& need, bool kernel) {
     return listed(mlla_bwd(g, x, w, conv_w, rotations, s, side, heads, need, kernel));
   });
-  m.def("pola_fwd", [](const Tensor& x, const Tensor& src, const std::vector<Maybe>& p, double alpha, int64_t H, int64_t W, int64_t heads) {
+  op("pola_fwd", [](const Tensor& x, const Tensor& src, const std::vector<Maybe>& p, double alpha, int64_t H, int64_t W, int64_t heads) {
     return listed(pola_fwd(x, src, p, alpha, H, W, heads));
   });
-  m.def("pola_bwd", [](const Tensor& g, const Tensor& x, const Tensor& src, bool same, const std::vector<Maybe>& p,
+  op("pola_bwd", [](const Tensor& g, const Tensor& x, const Tensor& src, bool same, const std::vector<Maybe>& p,
                        const std::vector<Maybe>& s, double alpha, int64_t H, int64_t W, int64_t heads, const std::array<bool, 13>& need,
                        const std::array<bool, 3>& kernel) { return listed(pola_bwd(g, x, src, same, p, s, alpha, H, W, heads, need, kernel)); });
-  m.def("focused_fwd", [](const Tensor& x, const Tensor& src, const std::vector<Maybe>& p, int64_t H, int64_t W, int64_t heads) {
+  op("focused_fwd", [](const Tensor& x, const Tensor& src, const std::vector<Maybe>& p, int64_t H, int64_t W, int64_t heads) {
     return listed(focused_fwd(x, src, p, H, W, heads));
   });
-  m.def("focused_bwd", [](const Tensor& g, const Tensor& x, const Tensor& src, bool same, const std::vector<Maybe>& p,
+  op("focused_bwd", [](const Tensor& g, const Tensor& x, const Tensor& src, bool same, const std::vector<Maybe>& p,
                           const std::vector<Maybe>& s, int64_t H, int64_t W, int64_t heads, const std::array<bool, 12>& need,
                           const std::array<bool, 3>& kernel) { return listed(focused_bwd(g, x, src, same, p, s, H, W, heads, need, kernel)); });
-  m.def("linfusion_fwd", [](const Tensor& x, const Tensor& cu, const std::vector<Maybe>& p, const std::array<double, 2>& eps,
+  op("linfusion_fwd", [](const Tensor& x, const Tensor& cu, const std::vector<Maybe>& p, const std::array<double, 2>& eps,
                             const std::array<double, 2>& slope, int64_t heads, bool trains) {
     return listed(linfusion_fwd(x, cu, p, eps, slope, heads, trains));
   });
-  m.def("linfusion_bwd", [](const Tensor& g, const Tensor& x, const Tensor& cu, const std::vector<Maybe>& p, const std::vector<Maybe>& s,
+  op("linfusion_bwd", [](const Tensor& g, const Tensor& x, const Tensor& cu, const std::vector<Maybe>& p, const std::vector<Maybe>& s,
                             const std::array<double, 2>& slope, const std::array<bool, 21>& need, const std::array<bool, 8>& kernel) {
     return listed(linfusion_bwd(g, x, cu, p, s, slope, need, kernel));
   });

@@ -37,6 +37,7 @@ Tensors that are not contiguous or off a 16-byte boundary are copied first.
 import ctypes
 import importlib.util
 import os
+import threading
 
 import torch
 
@@ -144,7 +145,19 @@ _NATIVE = frozenset((
     "focused_fits", "linfusion_fits"))
 
 
+_native_lock = threading.Lock()
+_native = None
+
+
 def _load_native():
+    global _native
+    with _native_lock:  # (once: native calls do not hold the interpreter's lock)
+        if _native is None:
+            _native = _open_native()
+    return _native
+
+
+def _open_native():
     path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_lib", "fbla_torch.so")
     if not os.path.exists(path):
         raise RuntimeError(f"flash_bla: host library not found at {path}; build it with "

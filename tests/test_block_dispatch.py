@@ -3,6 +3,8 @@ launches a kernel.  A call that torch's operators refuse stays refused, one that
 import os
 import subprocess
 import sys
+import threading
+import time
 
 import pytest
 import torch
@@ -597,3 +599,29 @@ def test_numbers_of_heads_that_are_none_do_not_fit(heads):
                  lambda: _hip.chunk_reduce(heads4, heads4, heads4, heads), lambda: _hip.norm_leaky([(x[..., :0], None, None, 1e-5, 0.1)], False)):
         with pytest.raises(ValueError, match="positive"):
             call()
+
+
+def test_native_calls_let_other_threads_run():
+    """A call that takes a while (here a projection on the CPU, in front of a kernel that refuses its rows) does not hold the
+    interpreter's lock: with a switch interval that no call reaches, the other thread runs only while the lock is given up."""
+    x, w = torch.randn(1, 2048, 1024), torch.randn(2048, 1024)
+    args = (x, x, [w[:1024], None, w, None, x, x[:, :1], w, None, w, None], 32, 64, 4)
+    ticks, stop, interval = [0], threading.Event(), sys.getswitchinterval()
+
+    def tick():
+        while not stop.is_set():
+            ticks[0] += 1
+            time.sleep(0)
+    thread = threading.Thread(target=tick)
+    thread.start()
+    try:
+        sys.setswitchinterval(1000)
+        before = ticks[0]
+        with pytest.raises(ValueError, match="GPU"):
+            _hip.focused_fwd(*args)
+        during = ticks[0] - before
+    finally:
+        stop.set()
+        sys.setswitchinterval(interval)
+        thread.join()
+    assert during > 0
