@@ -10,11 +10,12 @@
 // into LDS, or by the transposing read where the contraction runs over W's rows); results leave through LDS as whole rows.
 // Sums are fp32 and rounded once, bias, `add` and the second product included.
 //
-// GPU us, the library / here (bf16, with bias; in brackets the input gradient): 200704 x 64 -> 128 24.1 / 16.9 (46 / 16.4), 50176 x 256
-// -> 512 33.2 / 30.6 (22.2 / 24.8), -> 256 14.6 / 16.8 (16.4 / 16.5), 3136 x 256 -> 512 6.2 / 5.6 (7.5 / 5.5), 1024 x 640 -> 640 6.4 / 6.4
-// (7.3 / 5.9), 8192 x 640 -> 640 13.2 / 14.5 (16.4 / 14.5), three of them in one launch 40 / 30.3.  Where the library's GEMM is faster by
-// itself (contractions of 512 and more over many tokens) the blocks keep it (`projects` in fbla_torch.cpp); elsewhere what
-// counts beside the GPU's time is that a launch here costs the host 4 us and a GEMM call of torch 17.  A first form with
+// GPU us in a captured graph, four sets of rows in turn, the library / here (bf16, with bias; in brackets the input gradient): 200704
+// x 64 -> 128 28.0 / 25.3 (54.3 / 19.3), 50176 x 256 -> 512 41.1 / 38.5 (25.7 / 31.8), -> 256 15.8 / 20.3 (17.6 / 19.6), 3136 x 256 -> 512
+// 6.5 / 5.8 (7.6 / 5.4), 1024 x 640 -> 640 6.3 / 6.3 (7.3 / 5.9), 8192 x 640 -> 640 14.4 / 16.8 (17.6 / 16.3), three of them in one launch
+// 42.6 / 37.1.  The blocks keep the library's GEMM where both sides of the weight are 512 and more and the product is large (`projects`
+// in fbla_torch.cpp, where the line and whom it favours are stated): a launch here costs the host 4 us, a GEMM call of torch 17, and
+// what the library is faster at by itself is paid back by the launches and passes that go into one here.  A first form with
 // branches around its loads waited for every step's rows (and looped over lanes for descriptors the compiler could not see to
 // be uniform): 15 % more throughout.  Blocks: LinFusion forward 8192 x 640 243 -> 142 us (with norm_leaky below, residual sums in
 // the products), MLLA step 64 x 56x56 x 64 414 -> 371, PolaFormer step 64 x 28x28 x 256 781 -> 750.

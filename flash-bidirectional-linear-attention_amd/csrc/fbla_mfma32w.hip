@@ -3,8 +3,11 @@
 // memory).  The plain operator, with or without the denominator, dense and packed; the decoupled
 // operator with such heads stays on the shape-generic kernels.  v_mfma_f32_32x32x2_f32, fp32
 // throughout: one instruction covers two values of the contraction index and takes 64 cycles, and a
-// token of a 128 x 128 head needs 8192 of them per compute unit and kernel against 1 KiB of rows, so
-// these kernels are bound by the matrix unit at about 60 % of the HBM rate.
+// token of a 128 x 128 head needs 8 of them against 1 KiB of rows: 112 us a product of B8-H16-T4096 at
+// the 153 TFLOP/s that a large fp32 product holds, at 2.2 to 2.4 GHz, for seconds.  The kernels take 172
+// to 198 us (two products in the two-job launch: 319): the matrix unit is busy 55 to 62 % (68 %) of the
+// time, at 2.4 GHz, and a wave waits 60 to 85 % of its cycles with two of them on a SIMD.  What bounds
+// them is that latency, not the matrix unit and not HBM.
 //
 //  state32w_kernel   S_part = K^T V and sum_t k_t over a token chunk.  A workgroup of four waves
 //                    shares the tokens; wave w owns the 64 x 64 block (w / 2, w % 2) of the state, so

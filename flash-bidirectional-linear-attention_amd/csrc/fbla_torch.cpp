@@ -634,10 +634,11 @@ std::array<Tensor, 3> turn_bwd(const Tensor& k_, const Tensor& weight_, const Te
 }
 
 // ---- blocks ---------------------------------------------------------------------------------------------------------------
-// A vision block between its input and its output as one call a direction: the projections' GEMMs (torch's) and the launches
-// above, in the order in which the block's Python steps issue them one by one, without a node of the autograd graph, a
-// Python call and their checks between them.  The gradient of a tensor that two steps read is accumulated by the second
-// step's GEMM instead of a launch of its own (12 us at 200704 x 64 and 50176 x 256 in bf16).
+// A vision block between its input and its output as one call a direction: what the block's Python steps do one by one, without
+// a node of the autograd graph, a Python call and their checks between them.  Projections are `project`'s or torch's GEMMs (the rule
+// below); the attention of 16-bit heads of 32 channels runs on the projections' rows (`on_rows`), other heads through the launches
+// above.  The gradient of a tensor that two steps read is accumulated by the second step's GEMM instead of a launch of its own (12
+// us at 200704 x 64 and 50176 x 256 in bf16).
 Tensor flat(const Tensor& t) { return t.reshape({-1, t.size(-1)}); }
 // Whether `project` takes a projection of these rows rather than torch's GEMM: 16-bit types within the entry point's limits
 // (fbla_project refuses others), unless both sides of the weight are 512 and more and the product is one of 4e9 multiply-adds and

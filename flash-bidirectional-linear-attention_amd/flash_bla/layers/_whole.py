@@ -3,14 +3,17 @@
 Issued step by step from Python, a block's training step on few tokens is bound by the host: every projection, feature map,
 operator and merge is a node of the autograd graph with its checks, its Python calls and its bookkeeping.  Where nothing
 looks between the steps - an ordinary eager call of the block's own class on plain modules, without hooks, of the shapes that
-all its fused steps take - the block is one node instead, whose forward and backward issue the same kernels in the same
-order.  Everything else runs step by step (`_steps` of the block), and so does a gradient that is to be differentiated again or
-that the kernels cannot read: it is composed by running the steps again on the node's inputs.
+all its fused steps take - the block is one node instead.  Its forward and backward do what the steps do, 16-bit types on kernels
+that only whole blocks have: projections with residuals and second products in their sums, the norm and activation between them
+(csrc/fbla_gemm.hip), and with heads of 32 channels PolaFormer's and MLLA's attention on the projections' rows (csrc/fbla_rows.hip).
+Everything else (autocast among it) runs step by step (`_steps` of the block), and so does a gradient that is to be differentiated
+again or that the kernels cannot read: it is composed by running the steps on what the node saved.
 
-Host time of a forward / a training step before (steps from Python through ctypes) and here, us, on a host in whose slower
-state a node of the graph that does nothing costs 63 us (33 in the other): mlla 107 / 301 -> 55 / 229, pola 195 / 614 -> 134 /
-470, with spatial reduction 352 / 1160 -> 250 / 940, focused 159 / 600 -> 106 / 445 (2 x 14x14 x 64 bf16), linfusion 245 / 1010 ->
-234 / 815 (1 x 16x16 x 320 fp16); what is left is the library's GEMM calls (17 us each, a launch of this package 4) and the graph.
+Host time of a forward / a training step, steps from Python through ctypes and here, us, in the slower of the host's two states
+(the faster one takes two thirds): mlla 107 / 450 -> 31 / 175, pola 198 / 800 -> 44 / 275, with spatial reduction 348 / 1280 -> 114 /
+590, focused 161 / 680 -> 57 / 310 (2 x 14x14 x 64 bf16), linfusion 249 / 1100 -> 74 / 500 (1 x 16x16 x 320 fp16).  What is left is the
+engine's hand-over to its thread (a node of the graph that does nothing costs 33 or 63 us there), torch's own modules and GEMM calls
+(17 us each, a launch of this package 4), and the launches.
 """
 import contextlib
 
