@@ -729,9 +729,9 @@ Tensor row_workspace(const fbla_block_attn& a, const Tensor& x) {
 std::vector<Tensor> mlla_fwd(const Tensor& x, const Tensor& w, const Tensor& b, const Tensor& conv_w, const Tensor& conv_b,
                              const Tensor& rotations, int64_t side, int64_t heads) {
   const NoGraph none;
-  const Tensor qk = linear(x, w, b), local = dwconv_fwd(x, conv_w, conv_b, side, side, false);
+  const Tensor qk = linear(x, w, b);
   if (on_rows(x, heads)) {
-    const Tensor xs = whole(x), rot = whole(rotations), out = like(local);
+    const Tensor local = dwconv_fwd(x, conv_w, conv_b, side, side, false), xs = whole(x), rot = whole(rotations), out = like(local);
     const RowState state = new_row_state(kRotary, x, heads);
     fbla_block_attn a = row_args(kRotary, qk, 0, qk, x.size(2), xs, 0, heads, state);
     const Tensor ws = row_workspace(a, x);
@@ -742,6 +742,7 @@ std::vector<Tensor> mlla_fwd(const Tensor& x, const Tensor& w, const Tensor& b, 
   }
   const auto [q, k, qr, kr, v] = rotary_fwd(qk, x, rotations, heads);
   const Attended a = la_fwd(q, k, v, qr, kr, 1.0 / x.size(1), 1e-6, FBLA_NORMALIZE | FBLA_DECOUPLED);
+  const Tensor local = dwconv_fwd(x, conv_w, conv_b, side, side, false);  // (last: the merge finds it in the caches)
   return {merge_fwd(a.o, Tensor(), local, Tensor()), qk, q, k, qr, kr, v, a.s, a.km};
 }
 
