@@ -640,19 +640,24 @@ std::array<Tensor, 3> turn_bwd(const Tensor& k_, const Tensor& weight_, const Te
 // above.  The gradient of a tensor that two steps read is accumulated by the second step's GEMM instead of a launch of its own (12
 // us at 200704 x 64 and 50176 x 256 in bf16).
 Tensor flat(const Tensor& t) { return t.reshape({-1, t.size(-1)}); }
-// Whether `project` takes a projection of these rows rather than torch's GEMM: 16-bit types within the entry point's limits
-// (fbla_project refuses others), unless both sides of the weight are 512 and more and the product is one of 4e9 multiply-adds and
-// more, where the library's deeper pipeline counts.  The line is drawn for a call by itself, host included: a call of the library
-// takes the host 17 us, one of ours 4 for up to three products.  GPU us of the library / here (bf16, with bias): 8192 x 640 -> 640
-// 14.4 / 16.8, three of them 42.6 / 37.1; 1024 x 1280 -> 1280 12.0 / 13.5; 4096 x 1280 -> 1280 21.5 / 26.1; 12544 x 512 -> 512 15.4 / 18.5,
-// -> 1024 20.7 / 28.5; 50176 x 256 -> 256 15.8 / 20.3, -> 512 41 / 38.5.  In a captured graph, which pays no host time, the products
-// below the line that the library is faster at cost up to 10 us more here (50176 x 512 -> 256 24.1 / 33.6).
-bool projects(const Tensor& x, const Tensor& w) {
+// Whether `project` takes products of these rows rather than torch's GEMM: 16-bit types within the entry point's limits
+// (fbla_project refuses others), unless the product is large enough for the library's deeper pipeline to count.  A call of the library
+// takes the host 17 us, one of ours 4 for up to three products, which small products do not hide.  GPU us of the library / here (bf16,
+// with bias, captured graph): a forward product by itself (`alone`) of whole 256-wide tiles, contractions of 128 and more, over 1.5e9
+// multiply-adds and up to 2^24 results is the library's: 50176 x 128 -> 256 13.4 / 16.7, 12544 x 256 -> 512 11.7 / 13.6, 25088 x 256 -> 256 11.6 / 13.7, 50176 x 256 -> 256
+// 16.4 / 20.9, x 512 -> 256 22.0 / 30.4, 12544 x 512 -> 512 15.7 / 18.7; more results 50176 x 256 -> 512 38.3 / 37.1, x 512 -> 512 62.0 / 58.9;
+// fewer products 8192 x 256 -> 512 8.3 / 8.8, 12544 x 256 -> 256 8.2 / 8.4, 4096 x 512 -> 512 9.4 / 8.1; other widths 12544 x 320 -> 320 11.2
+// / 9.8, 50176 x 320 -> 640 47.9 / 48.8, 8192 x 640 -> 640 14.9 / 17.4.  Several in a launch, an added tensor or a second product pay up to
+// 4e9 where both sides are 512 and more: three of 8192 x 640 -> 640 42.6 / 37.1, of 50176 x 256 -> 512 109 / 87; one of 4096 x 1280 -> 1280
+// 21.5 / 26.1.
+bool projects(const Tensor& x, const Tensor& w, bool alone = false) {
   constexpr int64_t kMostChannels = 1 << 16, kMostWeights = 1 << 29, kLongestRow = 1 << 22;  // of fbla_project
   if (x.element_size() != 2 || w.size(0) > kMostChannels || w.size(1) > kMostChannels || w.numel() > kMostWeights ||
       (x.dim() > 1 && x.stride(-2) > kLongestRow))
     return false;
-  const double work = (double)(x.numel() / x.size(-1)) * w.numel();
+  const int64_t tokens = x.numel() / x.size(-1);
+  const double work = (double)tokens * w.numel();
+  if (alone && work > 1.5e9 && w.size(1) >= 128 && w.size(0) % 256 == 0 && tokens * w.size(0) <= 1 << 24) return false;
   return w.size(0) < 512 || w.size(1) < 512 || work <= 4e9;
 }
 // y = x W^T + b (+ add) for one or more projections
@@ -661,7 +666,8 @@ struct Linear {
 };
 std::vector<Tensor> linears(const std::vector<Linear>& p) {
   bool own = p.size() <= 3;
-  for (const Linear& l : p) own = own && projects(l.x, l.w) && l.x.numel() / l.x.size(-1) == p[0].x.numel() / p[0].x.size(-1);
+  const bool alone = p.size() == 1 && !p[0].add.defined();
+  for (const Linear& l : p) own = own && projects(l.x, l.w, alone) && l.x.numel() / l.x.size(-1) == p[0].x.numel() / p[0].x.size(-1);
   std::vector<Tensor> r;
   if (own) {
     std::vector<Projection> jobs;
@@ -1320,6 +1326,7 @@ PYBIND11_MODULE(fbla_torch, m) {
   const py::object parameter = py::module_::import("torch.nn").attr("Parameter");
   m.def("plain_gpu_tensors", [parameter](py::handle x, py::args rest) { return plain_gpu_tensors(x, rest, parameter.ptr()); });
   m.def("untouched_modules", &untouched_modules);
+  m.def("projects", &projects);
   m.def("mlla_fits", &mlla_fits);
   m.def("pola_fits", &pola_fits);
   m.def("focused_fits", &focused_fits);

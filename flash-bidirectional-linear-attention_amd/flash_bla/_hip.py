@@ -17,6 +17,7 @@ library.  `lib()` is the library itself through ctypes.  There is no fallback: a
     dwconv_fwd(x, w, bias, H, W, flip=False) -> y, dwconv_grad(x, g, w, H, W, with_bias) -> dw, db
     linear_wgrad(g, x, with_bias) -> dw, db
     project([(a, w, bias, add, a2, w2), ...], rows_of_w) -> [a w^T + bias + add, ...] or (rows_of_w) [a w + a2 w2 + add, ...]
+    projects(x, w, alone) -> whether a whole block runs a product of these rows on `project` (and not on the library's GEMM)
     norm_leaky([(x, weight, bias, eps, slope), ...], with_stats) -> [(y, mean, rstd), ...]
     polarity_fwd(qg, kv, pe, scale, power, heads) -> q_same, q_opp, k_both, v
     polarity_bwd(qg, kv, pe, scale, power, heads, dq_same, dq_opp, dk_both, dv, dv_rows, dgate) -> dqg, dkv, dpe, dscale, dpower
@@ -141,7 +142,7 @@ _NATIVE = frozenset((
     "piecewise_supported", "piecewise_fwd", "elu1_fwd", "elu1_bwd", "dwconv_fwd", "dwconv_grad", "linear_wgrad", "project", "norm_leaky", "polarity_fwd",
     "polarity_bwd", "rotary_fwd", "rotary_bwd", "merge_fwd", "merge_bwd", "interpolate_fwd", "interpolate_bwd", "focus_fwd",
     "focus_bwd", "turn_fwd", "turn_bwd", "mlla_fwd", "mlla_bwd", "pola_fwd", "pola_bwd", "focused_fwd", "focused_bwd",
-    "linfusion_fwd", "linfusion_bwd", "dense_operands", "plain_gpu_tensors", "untouched_modules", "mlla_fits", "pola_fits",
+    "linfusion_fwd", "linfusion_bwd", "dense_operands", "plain_gpu_tensors", "untouched_modules", "projects", "mlla_fits", "pola_fits",
     "focused_fits", "linfusion_fits"))
 
 

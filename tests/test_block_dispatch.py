@@ -625,3 +625,15 @@ def test_native_calls_let_other_threads_run():
         sys.setswitchinterval(interval)
         thread.join()
     assert during > 0
+
+
+@pytest.mark.parametrize("tokens,K,N,alone,several", [
+    (50176, 256, 256, False, True), (50176, 128, 256, False, True), (12544, 512, 512, False, True), (12544, 256, 512, False, True),
+    (50176, 256, 512, True, True), (12544, 256, 256, True, True), (8192, 640, 640, True, True), (200704, 64, 128, True, True),
+    (4096, 1280, 1280, False, False), (12544, 512, 1024, False, False), (64, 64, 65544, False, False), (8, 40000, 20000, False, False)])
+def test_products_that_the_library_is_faster_at_are_left_to_it(tokens, K, N, alone, several):
+    """Large ones of whole tiles, by themselves; and what the kernel's entry point refuses."""
+    x, w = torch.empty(tokens, K, dtype=torch.half, device="meta"), torch.empty(N, K, dtype=torch.half, device="meta")
+    assert (_hip.projects(x, w, True), _hip.projects(x, w, False)) == (alone, several)
+    far = torch.empty_strided((4, K), ((1 << 22) + 8, 1), dtype=torch.half, device="meta")
+    assert not _hip.projects(far, w, False) and not _hip.projects(x.float(), w.float(), False)
