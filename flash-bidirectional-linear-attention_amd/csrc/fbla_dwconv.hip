@@ -24,7 +24,6 @@ namespace {
 constexpr int kThreads = 256;
 constexpr float kLargest = 3.40282347e38f;  // of fp32
 constexpr int kFinishParts = 32;    // threads that share the terms of one filter's gradient
-constexpr int kAtOnce = 2;          // channels of a lane that the gradient kernel holds as fp32 at a time
 constexpr int kBlockChannels = 64;  // channels of a workgroup: 128-byte (16-bit) or 256-byte (fp32) pieces of a row
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -165,14 +164,17 @@ __global__ __launch_bounds__(kThreads) void conv_kernel(Conv a, int strips_per_r
 // x + kx - P], the bias gradient in row K of ky = 0.  One tap row per workgroup (blockIdx.z): K * V accumulators per
 // lane, kept over all strips of the chunk, added over the workgroup's strips at the end in a fixed order (fp32: sums of g alone
 // and sums over chunks in 64 bits, so that the bias gradient is no further from exact than column sums in a tree).  The K
-// workgroups of a chunk fetch the same rows (out of the caches), what bounds it is the latency of a strip's loads: two of a lane's
-// channels are fp32 at a time, so that three waves fit a SIMD (all eight: 173 VGPRs at 5x5, two waves), and the grid
-// is the three workgroups a CU that run at once.  bf16: 64 x 28x28 x 256, 5x5, 46 -> 33 us (51 MB); 64 x 56x56 x 64, 3x3, 29 -> 22 us.
+// workgroups of a chunk fetch the same rows (out of the caches), what bounds it is the latency of a strip's loads.  16-bit types up to
+// 5x5: two of a lane's channels are fp32 at a time, so that three waves fit a SIMD (all eight: 173 VGPRs at 5x5, two waves), and the
+// grid is the three workgroups a CU that run at once.  bf16: 64 x 28x28 x 256, 5x5, 46 -> 33 us (51 MB); 64 x 56x56 x 64, 3x3, 29 -> 22 us.
+// fp32 has three or four waves as it is and 7x7 of 16 bits two either way: all channels at once and a grid of four workgroups a CU
+// (7x7, 64 x 28x28 x 256 bf16 59 us, 65 in parts with three a CU; fp32 77 and 90; 5x5, 64 x 28x28 x 64 fp32 22 and 25).
+template <typename T> constexpr bool grad_in_parts(int K) { return sizeof(T) == 2 && K < 7; }
 template <typename T, int K, int STRIP>
 __global__ __launch_bounds__(kThreads) void grad_kernel(Conv a, const T* __restrict__ g, int64_t g_batch, int64_t g_row,
                                                         float* __restrict__ partial, int strips_per_row, int nstrips) {
   constexpr int V = Lane<T>::kVec, P = K / 2, IN = STRIP + K - 1;
-  constexpr int kWaves = kThreads / 64;
+  constexpr int kWaves = kThreads / 64, kAtOnce = grad_in_parts<T>(K) ? 2 : V;
   const int ky = blockIdx.z, c0 = blockIdx.y * kBlockChannels;
   const int lane = threadIdx.x % Lane<T>::kLanes, worker = threadIdx.x / Lane<T>::kLanes;
   const int cl = lane * V, c = c0 + cl;
@@ -197,7 +199,7 @@ __global__ __launch_bounds__(kThreads) void grad_kernel(Conv a, const T* __restr
       Piece<T> gv[STRIP], in[IN];
       load_row<T, STRIP>(g + (int64_t)b * g_batch + (int64_t)y * a.W * g_row + c, g_row, x0, a.W, gv);
       load_row<T, IN>(xc + (int64_t)b * a.x_batch + (int64_t)(inside ? yy : y) * a.W * a.x_row, a.x_row, x0 - P, a.W, in);
-      if (ky == 0) {  // (no other workgroup's is kept)
+      if (kAtOnce == V || ky == 0) {  // (no other workgroup's is kept; the branch costs the kernels without parts registers)
 #pragma unroll
         for (int t = 0; t < STRIP; ++t)
 #pragma unroll
@@ -212,7 +214,7 @@ __global__ __launch_bounds__(kThreads) void grad_kernel(Conv a, const T* __restr
             for (int t = 0; t < STRIP; ++t)
 #pragma unroll
               for (int j = j0; j < j0 + kAtOnce; ++j) acc[kx][j] = fmaf((float)gv[t].e[j], (float)in[t + kx].e[j], acc[kx][j]);
-          __builtin_amdgcn_sched_barrier(0);
+          if constexpr (kAtOnce < V) __builtin_amdgcn_sched_barrier(0);
         }
       }
     }
@@ -313,13 +315,14 @@ __global__ __launch_bounds__(kThreads) void grad_finish_kernel(const float* __re
 // outputs of one lane: the strip length that leaves fewer unused columns in the last strip of a row
 int strip_for(int W) { return ((W + 6) / 7) * 7 < ((W + 7) / 8) * 8 ? 7 : 8; }
 
-// workgroups of the gradient kernel along the strips: over all tap rows and channel blocks about three per CU, what its registers
-// let run at once, and no more than there are strips (each chunk costs K * (K + 1) * C partial sums)
-int grad_chunks(const Conv& a, int K, int workers) {
+// workgroups of the gradient kernel along the strips: over all tap rows and channel blocks three per CU where it works in parts, what
+// its registers let run at once, else four, and no more than there are strips (each chunk costs K * (K + 1) * C partial sums)
+template <typename T> int grad_chunks(const Conv& a, int K) {
+  constexpr int workers = Lane<T>::kWorkers;
   const int s = strip_for(a.W);
   const int64_t nstrips = (int64_t)a.B * a.H * ((a.W + s - 1) / s);
   const int64_t share = (int64_t)K * ((a.C + kBlockChannels - 1) / kBlockChannels);
-  const int64_t want = 768 / share < 1 ? 1 : 768 / share;
+  const int64_t all = grad_in_parts<T>(K) ? 768 : 1024, want = all / share < 1 ? 1 : all / share;
   const int64_t most = (nstrips + workers - 1) / workers;
   return (int)(want < most ? want : most);
 }
@@ -335,7 +338,7 @@ template <typename T, int K, int STRIP>
 void launch_grad(const Conv& a, const void* g, int64_t g_batch, int64_t g_row, void* dw, void* db, float* partial,
                  hipStream_t st) {
   const int per_row = (a.W + STRIP - 1) / STRIP, nstrips = a.B * a.H * per_row;
-  const int chunks = grad_chunks(a, K, Lane<T>::kWorkers);
+  const int chunks = grad_chunks<T>(a, K);
   const dim3 grid((unsigned)chunks, (unsigned)((a.C + kBlockChannels - 1) / kBlockChannels), (unsigned)K);
   grad_kernel<T, K, STRIP><<<grid, dim3(kThreads), 0, st>>>(a, (const T*)g, g_batch, g_row, partial, per_row, nstrips);
   grad_finish_kernel<T><<<dim3((unsigned)(K * K + 1), (unsigned)cdiv64(a.Cw, kThreads / kFinishParts)), dim3(kThreads), 0, st>>>(
@@ -367,8 +370,9 @@ bool supported(int C, int Cw, int K, int dtype) {
 }
 
 size_t grad_workspace_bytes(const Conv& a, int K, int dtype) {
-  const int workers = dtype == kF32 ? Lane<float>::kWorkers : Lane<_Float16>::kWorkers;
-  return sizeof(float) * (size_t)grad_chunks(a, K, workers) * K * (K + 1) * a.C;
+  int64_t chunks = 0;
+  by_type(dtype, [&](auto t) { chunks = grad_chunks<decltype(t)>(a, K); });
+  return sizeof(float) * (size_t)chunks * K * (K + 1) * a.C;
 }
 
 void forward(const Conv& a, int K, int dtype, bool flip, hipStream_t st) {

@@ -98,6 +98,14 @@ def test_finer_chunks_do_not_take_a_forward_past_the_built_in_scratch(B, H, L, D
     assert need <= _hip.lib().fbla_static_scratch_bytes()
 
 
+@pytest.mark.parametrize("dtype,K,workgroups", [(_hip.F32, 3, 1024), (_hip.F32, 5, 1024), (_hip.F32, 7, 1024), (_hip.BF16, 7, 1024),
+                                                (_hip.F16, 7, 1024), (_hip.BF16, 5, 768), (_hip.F16, 3, 768)])
+def test_filter_gradients_fill_the_gpu_with_what_their_registers_allow(dtype, K, workgroups):
+    """One partial of K * (K + 1) sums a chunk; K tap rows and 4 blocks of channels share the workgroups."""
+    need = _hip.lib().fbla_dwconv_grad_workspace_bytes(64, 28, 28, 256, 32, K, dtype)
+    assert need == 4 * (workgroups // (4 * K)) * K * (K + 1) * 256
+
+
 class _Described(torch.Tensor):
     is_cuda = True
 
