@@ -823,8 +823,9 @@ std::vector<Tensor> pola_fwd(const Tensor& x, const Tensor& src, const std::vect
   const PolaWeights p = pola_weights(params);
   const int64_t N = x.size(1), n = src.size(1), C = x.size(2);
   const auto [qg, kv] = two_linears({x, p.q_w, p.q_b, Tensor()}, {src, p.kv_w, p.kv_b, Tensor()});
-  const LocalValues l = local_values(kv.narrow(2, C, C), N, p.conv_w, p.conv_b, H, W);
+  LocalValues l;
   if (on_rows(x, heads)) {
+    l = local_values(kv.narrow(2, C, C), N, p.conv_w, p.conv_b, H, W);
     const Tensor merged = like(l.local), pe = whole(p.pe), scale = whole(p.scale), power = whole(p.power);
     const RowState state = new_row_state(kPolarity, x, heads);
     fbla_block_attn a = row_args(kPolarity, qg, 0, kv, 0, kv, C, heads, state);
@@ -850,6 +851,7 @@ std::vector<Tensor> pola_fwd(const Tensor& x, const Tensor& src, const std::vect
     const Attended b = la_fwd(q_opp, k, v2, Tensor(), Tensor(), 1.0 / n, 1e-6, FBLA_NORMALIZE);
     o1 = a.o, s = a.s, km = a.km, o2 = b.o, s2 = b.s, km2 = b.km;
   }
+  l = local_values(kv.narrow(2, C, C), N, p.conv_w, p.conv_b, H, W);  // (last: the merge finds it in the caches)
   const Tensor merged = merge_fwd(o1, o2, l.local, qg.narrow(2, C, C));
   return {linear(merged, p.proj_w, p.proj_b), scale, sigmoid, power, qg, kv, q_same, q_opp, k, v, l.grid, l.local, o1, o2, s, km, s2,
           km2, v1, v2, merged};
@@ -930,8 +932,8 @@ std::vector<Tensor> focused_fwd(const Tensor& x, const Tensor& src, const std::v
   const NoGraph none;
   const FocusedWeights p = focused_weights(params);
   const int64_t N = x.size(1), n = src.size(1), C = x.size(2);
-  const Tensor scale = at::softplus(p.scale);
   const auto [q_rows, kv] = two_linears({x, p.q_w, p.q_b, Tensor()}, {src, p.kv_w, p.kv_b, Tensor()});
+  const Tensor scale = at::softplus(p.scale);
   const auto [q, k, v] = focus_fwd(q_rows, kv, p.pe, scale, heads);
   const Attended a = la_fwd(q, k, v, Tensor(), Tensor(), 1.0 / n, 1e-6, FBLA_NORMALIZE);
   const LocalValues l = local_values(kv.narrow(2, C, C), N, p.conv_w, p.conv_b, H, W);
