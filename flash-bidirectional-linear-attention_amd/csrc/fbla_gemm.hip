@@ -13,8 +13,8 @@
 // GPU us in a captured graph, four sets of rows in turn, the library / here (bf16, with bias; in brackets the input gradient): 200704
 // x 64 -> 128 28.0 / 25.3 (54.3 / 19.3), 50176 x 256 -> 512 41.1 / 38.5 (25.7 / 31.8), -> 256 15.8 / 20.3 (17.6 / 19.6), 3136 x 256 -> 512
 // 6.5 / 5.8 (7.6 / 5.4), 1024 x 640 -> 640 6.3 / 6.3 (7.3 / 5.9), 8192 x 640 -> 640 14.4 / 16.8 (17.6 / 16.3), three of them in one launch
-// 42.6 / 37.1.  The blocks keep the library's GEMM where it is the faster one by more than
-// its host time (`projects` in fbla_torch.cpp has the lines and both sides of each): a launch here costs the host 4 us, a GEMM call of
+// 42.6 / 37.1.  The blocks keep the library's GEMM where it is the faster one and long
+// enough to hide its host time (`projects` in fbla_torch.cpp has the lines and both sides of each): a launch here costs the host 4 us, a GEMM call of
 // torch 17, and launches and passes that go into one here pay back what the library is faster at by itself.  A first form with
 // branches around its loads waited for every step's rows (and looped over lanes for descriptors the compiler could not see to
 // be uniform): 15 % more throughout.  Blocks: LinFusion forward 8192 x 640 243 -> 142 us (with norm_leaky below, residual sums in

@@ -702,6 +702,14 @@ std::pair<Tensor, Tensor> weight_grad(const Tensor& g, const Tensor& x, bool wei
   const Tensor rows_ = flat(g);
   return {weight ? at::mm(rows_.t(), flat(x)) : Tensor(), bias ? rows_.sum(0) : Tensor()};
 }
+// Large blocks give up what nothing reads any more before they allocate what comes next, as the steps one by one do (inference, peak
+// without / with: LinFusion 32768 x 640 bf16 441 / 200 MB, FLatten 401408 x 256 with reduced keys 1622 / 935).  Rows of up to 64 MB do not:
+// kernels that write where others have just read were 2 to 5 % slower there (captured forward, FLatten 64 x 28x28 x 64 with reduced keys
+// bf16 109.6 / 114.2 us, 64 x 28x28 x 256 fp32 517 / 524), and the same from 98 MB on.
+bool spares(const Tensor& x) { return x.nbytes() >= size_t(64) << 20; }
+template <typename... T> void release(bool large, T&... t) {
+  if (large) ((t = Tensor()), ...);
+}
 struct NoGraph {  // (called inside an autograd function or without gradients: nothing is recorded)
   at::AutoDispatchBelowADInplaceOrView guard;
 };
@@ -733,9 +741,10 @@ Tensor row_workspace(const fbla_block_attn& a, const Tensor& x) {
 
 // layers/mlla.py: qk projection, rotary features, decoupled attention, positional convolution of the input
 std::vector<Tensor> mlla_fwd(const Tensor& x, const Tensor& w, const Tensor& b, const Tensor& conv_w, const Tensor& conv_b,
-                             const Tensor& rotations, int64_t side, int64_t heads) {
+                             const Tensor& rotations, int64_t side, int64_t heads, bool trains) {
   const NoGraph none;
-  const Tensor qk = linear(x, w, b);
+  const bool lean = !trains && spares(x);
+  Tensor qk = linear(x, w, b);
   if (on_rows(x, heads)) {
     const Tensor local = dwconv_fwd(x, conv_w, conv_b, side, side, false), xs = whole(x), rot = whole(rotations), out = like(local);
     const RowState state = new_row_state(kRotary, x, heads);
@@ -744,12 +753,17 @@ std::vector<Tensor> mlla_fwd(const Tensor& x, const Tensor& w, const Tensor& b, 
     a.local = ptr(local), a.rot = f32(rot), a.out = ptr(out), a.workspace = ptr(ws), a.workspace_bytes = ws.numel();
     const On on(x);
     check(api.fbla_block_attn_forward(&a, on.stream), "fbla_block_attn_forward");
+    if (!trains) return {out};
     return {out, qk, state.planes, state.km};
   }
-  const auto [q, k, qr, kr, v] = rotary_fwd(qk, x, rotations, heads);
+  auto [q, k, qr, kr, v] = rotary_fwd(qk, x, rotations, heads);
+  release(lean, qk);
   const Attended a = la_fwd(q, k, v, qr, kr, 1.0 / x.size(1), 1e-6, FBLA_NORMALIZE | FBLA_DECOUPLED);
+  release(lean, q, k, qr, kr, v);
   const Tensor local = dwconv_fwd(x, conv_w, conv_b, side, side, false);  // (last: the merge finds it in the caches)
-  return {merge_fwd(a.o, Tensor(), local, Tensor()), qk, q, k, qr, kr, v, a.s, a.km};
+  const Tensor out = merge_fwd(a.o, Tensor(), local, Tensor());
+  if (!trains) return {out};
+  return {out, qk, q, k, qr, kr, v, a.s, a.km};
 }
 
 // saved: what mlla_fwd returned after its output, or what saved-tensor hooks made of it (any strides).  need: x, w, b, conv_w, conv_b
@@ -775,8 +789,9 @@ std::vector<Tensor> mlla_bwd(const Tensor& g, const Tensor& x, const Tensor& w, 
       check(api.fbla_block_attn_backward_keys(&a, on.stream), "fbla_block_attn_backward_keys");
     } else {
       const Tensor q = saved.at(1), k = saved.at(2), qr = saved.at(3), kr = saved.at(4), v = saved.at(5);
-      const MergeGrads m = merge_bwd(g, heads, false, Tensor(), Tensor(), Tensor(), Tensor());
+      MergeGrads m = merge_bwd(g, heads, false, Tensor(), Tensor(), Tensor(), Tensor());
       const AttendedGrads d = la_bwd(q, k, v, qr, kr, m.o, saved.at(6), saved.at(7), 1.0 / x.size(1), 1e-6, FBLA_NORMALIZE | FBLA_DECOUPLED);
+      release(spares(x), m.o);
       std::tie(dqk, dx) = rotary_bwd(qk, rotations, heads, d.q, d.k, d.q_rope, d.k_rope, d.v, dlocal);
     }
     std::tie(dw, db) = weight_grad(dqk, x, need[1], need[2], kernel);
@@ -818,11 +833,12 @@ PolaWeights pola_weights(const std::vector<Maybe>& p) {
 
 // layers/polaformer.py up to the output projection.  src: the rows of the keys and values (x unless they were reduced)
 std::vector<Tensor> pola_fwd(const Tensor& x, const Tensor& src, const std::vector<Maybe>& params, double alpha, int64_t H, int64_t W,
-                             int64_t heads) {
+                             int64_t heads, bool trains) {
   const NoGraph none;
+  const bool lean = !trains && spares(x);
   const PolaWeights p = pola_weights(params);
   const int64_t N = x.size(1), n = src.size(1), C = x.size(2);
-  const auto [qg, kv] = two_linears({x, p.q_w, p.q_b, Tensor()}, {src, p.kv_w, p.kv_b, Tensor()});
+  auto [qg, kv] = two_linears({x, p.q_w, p.q_b, Tensor()}, {src, p.kv_w, p.kv_b, Tensor()});
   LocalValues l;
   if (on_rows(x, heads)) {
     l = local_values(kv.narrow(2, C, C), N, p.conv_w, p.conv_b, H, W);
@@ -836,10 +852,13 @@ std::vector<Tensor> pola_fwd(const Tensor& x, const Tensor& src, const std::vect
       const On on(x);
       check(api.fbla_block_attn_forward(&a, on.stream), "fbla_block_attn_forward");
     }
-    return {linear(merged, p.proj_w, p.proj_b), qg, kv, l.grid, l.local, state.planes, state.km, merged};
+    release(lean, qg, kv, l.grid, l.local);
+    const Tensor y = linear(merged, p.proj_w, p.proj_b);
+    if (!trains) return {y};
+    return {y, qg, kv, l.grid, l.local, state.planes, state.km, merged};
   }
   const Tensor scale = at::softplus(p.scale), sigmoid = at::sigmoid(p.power), power = at::add(at::mul(sigmoid, alpha), 1);
-  const auto [q_same, q_opp, k, v] = polarity_fwd(qg, kv, p.pe, scale, power, heads);
+  auto [q_same, q_opp, k, v] = polarity_fwd(qg, kv, p.pe, scale, power, heads);
   Tensor o1, o2, s, km, s2, km2, v1, v2;
   if (n == N && pair_supported(q_same, v)) {
     const Paired a = pair_fwd(q_same, q_opp, k, v, 1.0 / n, 1e-6);
@@ -851,9 +870,13 @@ std::vector<Tensor> pola_fwd(const Tensor& x, const Tensor& src, const std::vect
     const Attended b = la_fwd(q_opp, k, v2, Tensor(), Tensor(), 1.0 / n, 1e-6, FBLA_NORMALIZE);
     o1 = a.o, s = a.s, km = a.km, o2 = b.o, s2 = b.s, km2 = b.km;
   }
+  release(lean, q_same, q_opp, k, v, v1, v2);
   l = local_values(kv.narrow(2, C, C), N, p.conv_w, p.conv_b, H, W);  // (last: the merge finds it in the caches)
   const Tensor merged = merge_fwd(o1, o2, l.local, qg.narrow(2, C, C));
-  return {linear(merged, p.proj_w, p.proj_b), scale, sigmoid, power, qg, kv, q_same, q_opp, k, v, l.grid, l.local, o1, o2, s, km, s2,
+  release(lean, o1, o2, l.grid, l.local, qg, kv);
+  const Tensor y = linear(merged, p.proj_w, p.proj_b);
+  if (!trains) return {y};
+  return {y, scale, sigmoid, power, qg, kv, q_same, q_opp, k, v, l.grid, l.local, o1, o2, s, km, s2,
           km2, v1, v2, merged};
 }
 
@@ -871,7 +894,7 @@ std::vector<Tensor> pola_bwd(const Tensor& g, const Tensor& x, const Tensor& src
   std::vector<Tensor> r(2 + kPola);
   std::tie(r[11], r[12]) = weight_grad(g, merged, need[11], need[12], kernel[2]);
   if (std::none_of(need.begin(), need.begin() + 11, [](bool b) { return b; })) return r;
-  const Tensor dmerged = input_grad(g, p.proj_w);
+  Tensor dmerged = input_grad(g, p.proj_w);
   std::array<Tensor, 5> d;  // of qg, kv, pe, scale, power
   if (rows_) {
     const Tensor grid = at_(2), local = whole(at_(3)), pe = whole(p.pe), scale = whole(p.scale), power = whole(p.power), dlocal = like(dmerged);
@@ -895,10 +918,12 @@ std::vector<Tensor> pola_bwd(const Tensor& g, const Tensor& x, const Tensor& src
     check(api.fbla_block_attn_backward_keys(&a, on.stream), "fbla_block_attn_backward_keys");
   } else {
     const Tensor scale = at_(0), power = at_(2), q_same = at_(5), q_opp = at_(6), k = at_(7), v = at_(8), grid = at_(9), s = at_(13), km = at_(14), s2 = at_(15);
-    const MergeGrads m = merge_bwd(dmerged, heads, true, at_(11), at_(12), at_(10), qg.narrow(2, C, C));
+    MergeGrads m = merge_bwd(dmerged, heads, true, at_(11), at_(12), at_(10), qg.narrow(2, C, C));
+    release(spares(x), dmerged);
     if (need[9] || need[10]) std::tie(r[9], r[10]) = dwconv_grad(grid, m.local, p.conv_w, H, W, need[10]);
     if (std::none_of(need.begin(), need.begin() + 9, [](bool b) { return b; })) return r;
     const Tensor dv_rows = local_values_grad(m.local, n, p.conv_w, H, W);
+    release(spares(x), m.local);
     PairedGrads pd;
     if (!s2.defined()) {
       pd = pair_bwd(q_same, q_opp, k, v, m.o, m.o2, s, km, 1.0 / n, 1e-6);
@@ -907,6 +932,7 @@ std::vector<Tensor> pola_bwd(const Tensor& g, const Tensor& x, const Tensor& src
       const AttendedGrads b = la_bwd(q_opp, k, at_(18), Tensor(), Tensor(), m.o2, s2, at_(16), 1.0 / n, 1e-6, FBLA_NORMALIZE);
       pd = {a.q, b.q, at::add(a.k, b.k), at::cat({a.v, b.v}, -1)};
     }
+    release(spares(x), m.o, m.o2);
     d = polarity_bwd(qg, kv, p.pe, scale, power, heads, pd.q1, pd.q2, pd.k, pd.v, dv_rows, m.gate);
   }
   std::tie(r[0], r[1]) = two_input_grads(d[0], p.q_w, need[0], d[1], p.kv_w, same, need[1]);
@@ -928,17 +954,24 @@ FocusedWeights focused_weights(const std::vector<Maybe>& p) {
 }
 
 // layers/focused_la.py up to the output projection, as above
-std::vector<Tensor> focused_fwd(const Tensor& x, const Tensor& src, const std::vector<Maybe>& params, int64_t H, int64_t W, int64_t heads) {
+std::vector<Tensor> focused_fwd(const Tensor& x, const Tensor& src, const std::vector<Maybe>& params, int64_t H, int64_t W, int64_t heads,
+                                bool trains) {
   const NoGraph none;
+  const bool lean = !trains && spares(x);
   const FocusedWeights p = focused_weights(params);
   const int64_t N = x.size(1), n = src.size(1), C = x.size(2);
-  const auto [q_rows, kv] = two_linears({x, p.q_w, p.q_b, Tensor()}, {src, p.kv_w, p.kv_b, Tensor()});
+  auto [q_rows, kv] = two_linears({x, p.q_w, p.q_b, Tensor()}, {src, p.kv_w, p.kv_b, Tensor()});
   const Tensor scale = at::softplus(p.scale);
-  const auto [q, k, v] = focus_fwd(q_rows, kv, p.pe, scale, heads);
-  const Attended a = la_fwd(q, k, v, Tensor(), Tensor(), 1.0 / n, 1e-6, FBLA_NORMALIZE);
-  const LocalValues l = local_values(kv.narrow(2, C, C), N, p.conv_w, p.conv_b, H, W);
+  auto [q, k, v] = focus_fwd(q_rows, kv, p.pe, scale, heads);
+  release(lean, q_rows);
+  Attended a = la_fwd(q, k, v, Tensor(), Tensor(), 1.0 / n, 1e-6, FBLA_NORMALIZE);
+  release(lean, q, k, v);
+  LocalValues l = local_values(kv.narrow(2, C, C), N, p.conv_w, p.conv_b, H, W);
   const Tensor merged = merge_fwd(a.o, Tensor(), l.local, Tensor());
-  return {linear(merged, p.proj_w, p.proj_b), scale, q_rows, kv, q, k, v, l.grid, a.s, a.km, merged};
+  release(lean, a.o, l.local);
+  const Tensor y = linear(merged, p.proj_w, p.proj_b);
+  if (!trains) return {y};
+  return {y, scale, q_rows, kv, q, k, v, l.grid, a.s, a.km, merged};
 }
 
 std::vector<Tensor> focused_bwd(const Tensor& g, const Tensor& x, const Tensor& src, bool same, const std::vector<Maybe>& params,
@@ -954,12 +987,15 @@ std::vector<Tensor> focused_bwd(const Tensor& g, const Tensor& x, const Tensor& 
   std::vector<Tensor> r(2 + kFocused);
   std::tie(r[10], r[11]) = weight_grad(g, merged, need[10], need[11], kernel[2]);
   if (std::none_of(need.begin(), need.begin() + 10, [](bool b) { return b; })) return r;
-  const MergeGrads m = merge_bwd(input_grad(g, p.proj_w), heads, false, Tensor(), Tensor(), Tensor(), Tensor());
+  MergeGrads m = merge_bwd(input_grad(g, p.proj_w), heads, false, Tensor(), Tensor(), Tensor(), Tensor());
   if (need[8] || need[9]) std::tie(r[8], r[9]) = dwconv_grad(grid, m.local, p.conv_w, H, W, need[9]);
   if (std::none_of(need.begin(), need.begin() + 8, [](bool b) { return b; })) return r;
   const Tensor dv_rows = local_values_grad(m.local, n, p.conv_w, H, W);
-  const AttendedGrads d = la_bwd(q, k, v, Tensor(), Tensor(), m.o, s, km, 1.0 / n, 1e-6, FBLA_NORMALIZE);
+  release(spares(x), m.local);
+  AttendedGrads d = la_bwd(q, k, v, Tensor(), Tensor(), m.o, s, km, 1.0 / n, 1e-6, FBLA_NORMALIZE);
+  release(spares(x), m.o);
   const auto [dq, dkv, dpe, dscale] = focus_bwd(q_rows, kv, p.pe, scale, heads, d.q, d.k, d.v, dv_rows);
+  release(spares(x), d.q, d.k, d.v);
   std::tie(r[0], r[1]) = two_input_grads(dq, p.q_w, need[0], dkv, p.kv_w, same, need[1]);
   std::tie(r[2], r[3]) = weight_grad(dq, x, need[2], need[3], kernel[0]);
   std::tie(r[4], r[5]) = weight_grad(dkv, src, need[4], need[5], kernel[1]);
@@ -988,24 +1024,34 @@ LinFusionWeights linfusion_weights(const std::vector<Maybe>& p) {
 std::vector<Tensor> linfusion_fwd(const Tensor& x, const Tensor& cu, const std::vector<Maybe>& params, const std::array<double, 2>& eps,
                                   const std::array<double, 2>& slope, int64_t heads, bool trains) {
   const NoGraph none;
+  const bool lean = !trains && spares(x);
   const LinFusionWeights p = linfusion_weights(params);
   const int64_t B = x.size(0), N = x.size(1);
   const auto &pq = p.path[0], &pk = p.path[1];
-  const auto first = linears({{x, pq.in_w, pq.in_b, Tensor()}, {x, pk.in_w, pk.in_b, Tensor()}, {x, p.w[2], p.b[2], Tensor()}});
+  auto first = linears({{x, pq.in_w, pq.in_b, Tensor()}, {x, pk.in_w, pk.in_b, Tensor()}, {x, p.w[2], p.b[2], Tensor()}});
   std::vector<Normed> normed;
-  const Norm norms[2] = {{first[0], pq.norm_w, pq.norm_b, eps[0], slope[0]}, {first[1], pk.norm_w, pk.norm_b, eps[1], slope[1]}};
-  if (first[0].sizes() == first[1].sizes()) {
-    normed = norm_leaky({norms[0], norms[1]}, trains);
-  } else {
-    for (const Norm& n : norms) normed.push_back(norm_leaky({n}, trains)[0]);
+  {
+    const Norm norms[2] = {{first[0], pq.norm_w, pq.norm_b, eps[0], slope[0]}, {first[1], pk.norm_w, pk.norm_b, eps[1], slope[1]}};
+    if (first[0].sizes() == first[1].sizes()) {
+      normed = norm_leaky({norms[0], norms[1]}, trains);
+    } else {
+      for (const Norm& n : norms) normed.push_back(norm_leaky({n}, trains)[0]);
+    }
   }
-  const auto in = linears({{normed[0].y, pq.out_w, pq.out_b, x}, {normed[1].y, pk.out_w, pk.out_b, x}});
-  const auto qk = linears({{in[0], p.w[0], p.b[0], Tensor()}, {in[1], p.w[1], p.b[1], Tensor()}});
-  Tensor packed[3] = {qk[0], qk[1], first[2]};
-  for (Tensor& t : packed) t = t.view({B * N, heads, -1});
+  release(lean, first[0], first[1]);
+  auto in = linears({{normed[0].y, pq.out_w, pq.out_b, x}, {normed[1].y, pk.out_w, pk.out_b, x}});
+  release(lean, normed[0].y, normed[1].y);
+  Tensor packed[3];
+  {
+    const auto qk = linears({{in[0], p.w[0], p.b[0], Tensor()}, {in[1], p.w[1], p.b[1], Tensor()}});
+    for (int i = 0; i < 3; ++i) packed[i] = (i < 2 ? qk[i] : first[2]).view({B * N, heads, -1});
+  }
+  release(lean, in[0], in[1], first[2]);
   const Attended a = varlen_fwd(packed[0], packed[1], packed[2], cu, N, std::nullopt, 1e-4, FBLA_ELU1_QK);
+  release(lean, packed[0], packed[1], packed[2]);
   const Tensor o = a.o.view({B, N, -1});
   std::vector<Tensor> r{linear(o, p.proj_w, p.proj_b)};
+  if (!trains) return r;
   for (int i = 0; i < 2; ++i) r.insert(r.end(), {first[i], normed[i].mean, normed[i].rstd, normed[i].y, in[i]});
   r.insert(r.end(), {packed[0], packed[1], packed[2], a.s, a.km, o});
   return r;
@@ -1297,22 +1343,20 @@ PYBIND11_MODULE(fbla_torch, m) {
     return outs(turn_bwd(k, weight, rotations, a, b, c));
   });
 
-  op("mlla_fwd", [](const Tensor& x, const std::vector<Maybe>& p, const Tensor& rotations, int64_t side, int64_t heads) {
-    return listed(mlla_fwd(x, given(p[0]), given(p[1]), given(p[2]), given(p[3]), rotations, side, heads));
+  op("mlla_fwd", [](const Tensor& x, const std::vector<Maybe>& p, const Tensor& rotations, int64_t side, int64_t heads, bool trains) {
+    return listed(mlla_fwd(x, given(p[0]), given(p[1]), given(p[2]), given(p[3]), rotations, side, heads, trains));
   });
   op("mlla_bwd", [](const Tensor& g, const Tensor& x, const Tensor& w, const Tensor& conv_w, const Tensor& rotations,
                        const std::vector<Tensor>& s, int64_t side, int64_t heads, const std::array<bool, 5>& need, bool kernel) {
     return listed(mlla_bwd(g, x, w, conv_w, rotations, s, side, heads, need, kernel));
   });
-  op("pola_fwd", [](const Tensor& x, const Tensor& src, const std::vector<Maybe>& p, double alpha, int64_t H, int64_t W, int64_t heads) {
-    return listed(pola_fwd(x, src, p, alpha, H, W, heads));
-  });
+  op("pola_fwd", [](const Tensor& x, const Tensor& src, const std::vector<Maybe>& p, double alpha, int64_t H, int64_t W, int64_t heads,
+                    bool trains) { return listed(pola_fwd(x, src, p, alpha, H, W, heads, trains)); });
   op("pola_bwd", [](const Tensor& g, const Tensor& x, const Tensor& src, bool same, const std::vector<Maybe>& p,
                        const std::vector<Maybe>& s, double alpha, int64_t H, int64_t W, int64_t heads, const std::array<bool, 13>& need,
                        const std::array<bool, 3>& kernel) { return listed(pola_bwd(g, x, src, same, p, s, alpha, H, W, heads, need, kernel)); });
-  op("focused_fwd", [](const Tensor& x, const Tensor& src, const std::vector<Maybe>& p, int64_t H, int64_t W, int64_t heads) {
-    return listed(focused_fwd(x, src, p, H, W, heads));
-  });
+  op("focused_fwd", [](const Tensor& x, const Tensor& src, const std::vector<Maybe>& p, int64_t H, int64_t W, int64_t heads,
+                       bool trains) { return listed(focused_fwd(x, src, p, H, W, heads, trains)); });
   op("focused_bwd", [](const Tensor& g, const Tensor& x, const Tensor& src, bool same, const std::vector<Maybe>& p,
                           const std::vector<Maybe>& s, int64_t H, int64_t W, int64_t heads, const std::array<bool, 12>& need,
                           const std::array<bool, 3>& kernel) { return listed(focused_bwd(g, x, src, same, p, s, H, W, heads, need, kernel)); });

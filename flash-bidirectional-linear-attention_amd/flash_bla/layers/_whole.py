@@ -140,7 +140,7 @@ class _Mlla:
 
     def run(self, inputs, trains=True):
         *inputs, rotations = inputs
-        return _hip.mlla_fwd(inputs[0], inputs[1:], rotations, self.side, self.heads)
+        return _hip.mlla_fwd(inputs[0], inputs[1:], rotations, self.side, self.heads, trains)
 
     def run_backward(self, g, inputs, saved, need):
         x, w, b, conv_w, _, rotations = inputs
@@ -186,7 +186,7 @@ class _Pola(_Pvt):
 
     def run(self, inputs, trains=True):
         x, src, *p = inputs
-        return _hip.pola_fwd(x, x if src is None else src, p, self.alpha, self.H, self.W, self.heads)
+        return _hip.pola_fwd(x, x if src is None else src, p, self.alpha, self.H, self.W, self.heads, trains)
 
     def run_backward(self, g, inputs, saved, need):
         x, src, *p = inputs
@@ -200,7 +200,7 @@ class _Focused(_Pvt):
 
     def run(self, inputs, trains=True):
         x, src, *p = inputs
-        return _hip.focused_fwd(x, x if src is None else src, p, self.H, self.W, self.heads)
+        return _hip.focused_fwd(x, x if src is None else src, p, self.H, self.W, self.heads, trains)
 
     def run_backward(self, g, inputs, saved, need):
         x, src, *p = inputs

@@ -613,7 +613,7 @@ def test_native_calls_let_other_threads_run():
     """A call that takes a while (here a projection on the CPU, in front of a kernel that refuses its rows) does not hold the
     interpreter's lock: with a switch interval that no call reaches, the other thread runs only while the lock is given up."""
     x, w = torch.randn(1, 2048, 1024), torch.randn(2048, 1024)
-    args = (x, x, [w[:1024], None, w, None, x, x[:, :1], w, None, w, None], 32, 64, 4)
+    args = (x, x, [w[:1024], None, w, None, x, x[:, :1], w, None, w, None], 32, 64, 4, False)
     ticks, stop, interval = [0], threading.Event(), sys.getswitchinterval()
 
     def tick():

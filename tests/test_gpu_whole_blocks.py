@@ -254,3 +254,30 @@ def test_saved_tensors_that_come_back_elsewhere(name, counted):
     assert len(counted) == 2
     for a, b in zip(*grads):
         _close(a, b, torch.half)
+
+
+@pytest.mark.parametrize("dtype", [torch.half, torch.float])
+@pytest.mark.parametrize("make,side", [
+    (lambda: MambaLikeLinearAttention(128, (28, 28), 2), ()), (lambda: MambaLikeLinearAttention(128, (28, 28), 4), ()),
+    (lambda: PolaLinearAttention(128, 784, num_heads=2), (28, 28)), (lambda: PolaLinearAttention(128, 784, num_heads=4), (28, 28)),
+    (lambda: PolaLinearAttention(128, 784, num_heads=2, sr_ratio=2), (28, 28)),
+    (lambda: FocusedLinearAttention(128, 784, num_heads=2), (28, 28)),
+    (lambda: FocusedLinearAttention(128, 784, num_heads=2, sr_ratio=2), (28, 28)),
+    (lambda: GeneralizedLinearAttention(128, heads=2, dim_head=64), ())])
+def test_inference_holds_no_more_memory_than_the_steps(make, side, dtype, monkeypatch):
+    """Rows of 64 MB and more: what nothing reads any more is given up on the way."""
+    torch.manual_seed(0)
+    block = make().cuda().to(dtype)
+    if hasattr(block, "rope"):
+        block.rope.float()
+    x = torch.randn(336, 784, 128, device="cuda").to(dtype)
+
+    def peak(block):
+        with torch.no_grad():
+            block(x, *side)
+            torch.cuda.synchronize()
+            before = torch.cuda.memory_allocated()
+            torch.cuda.reset_peak_memory_stats()
+            block(x, *side)
+        return torch.cuda.max_memory_allocated() - before
+    assert peak(block) <= _steps(block, monkeypatch, peak) + (1 << 20)
