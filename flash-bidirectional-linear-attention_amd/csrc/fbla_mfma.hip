@@ -2544,9 +2544,10 @@ int state_chunk(const Prob& p, int dtype, bool block_stats) {
     if (direct) return direct;
   }
   const int whole = block_stats && padded(p) ? 0 : whole_state_chunk(p);
-  // 16-bit heads of two chunks, 32 workgroups and more: the consumers' prologues read twice the partials of chunks half as long
-  // (B1-H16-T512-D64 fp16 forward 17.6 us, 18.6 with four chunks; fp32, whose state kernel is longer, 24.1 and 21.6).
-  const bool two = dtype != kF32 && p.L <= 512 && (int64_t)p.N * p.H >= 16;
+  // 16-bit heads of two chunks: the consumers' prologues read twice the partials of chunks half as long (fp16 forward, us, two chunks /
+  // more: B1-H16-T512-D64 17.6 / 18.6, B1-H1-T512-D64 17.1 / 17.9, B1-H4-T296-D40 17.5 / 18.9; fp32, whose state kernel is longer, B1-H16-
+  // T512-D64 24.1 / 21.6).
+  const bool two = dtype != kF32 && p.L <= 512;
   return whole ? whole : chunk_for(p, per_cu, 1, block_stats || two ? 256 : least_state_chunk(p), 64, true);
 }
 

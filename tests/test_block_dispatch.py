@@ -89,6 +89,14 @@ def test_long_heads_are_not_cut_finer_than_their_partials_are_worth(H, L, D):
     assert need <= max(32, H * L // 256) * slot + 4096
 
 
+@pytest.mark.parametrize("H", [1, 4, 16])
+def test_short_16_bit_heads_keep_two_chunks(H):
+    """Up to 512 tokens of 64 x 64: two state partials a head (fp32: more)."""
+    slot = 4 * (64 * 64 + 64)
+    need = [_hip.lib().fbla_la_workspace_bytes(0, 1, H, 512, 64, 64, dtype, _hip.NORMALIZE) // slot for dtype in (_hip.BF16, _hip.F32)]
+    assert need[0] == 2 * H < need[1]
+
+
 @pytest.mark.parametrize("B,H,L,DK,DV,dtype,flags", [
     (3, 3, 1750, 110, 87, _hip.F16, 0), (4, 1, 1704, 126, 126, _hip.F32, 1), (8, 2, 648, 83, 114, _hip.BF16, 3),
     (1, 16, 689, 76, 123, _hip.F16, 3), (2, 2, 3520, 121, 84, _hip.BF16, 0), (7, 1, 1140, 125, 97, _hip.F32, 1)])
