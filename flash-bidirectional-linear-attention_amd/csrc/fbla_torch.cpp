@@ -643,13 +643,13 @@ Tensor flat(const Tensor& t) { return t.reshape({-1, t.size(-1)}); }
 // Whether `project` takes products of these rows rather than torch's GEMM: 16-bit types within the entry point's limits
 // (fbla_project refuses others), unless the product is large enough for the library's deeper pipeline to count.  A call of the library
 // takes the host 17 us, one of ours 4 for up to three products, which small products do not hide.  GPU us of the library / here (bf16,
-// with bias, captured graph): a forward product by itself (`alone`) of whole 256-wide tiles, contractions of 128 and more, over 1.5e9
-// multiply-adds and up to 2^24 results is the library's: 50176 x 128 -> 256 13.4 / 16.7, 12544 x 256 -> 512 11.7 / 13.6, 25088 x 256 -> 256 11.6 / 13.7, 50176 x 256 -> 256
-// 16.4 / 20.9, x 512 -> 256 22.0 / 30.4, 12544 x 512 -> 512 15.7 / 18.7; more results 50176 x 256 -> 512 38.3 / 37.1, x 512 -> 512 62.0 / 58.9;
-// fewer products 8192 x 256 -> 512 8.3 / 8.8, 12544 x 256 -> 256 8.2 / 8.4, 4096 x 512 -> 512 9.4 / 8.1; other widths 12544 x 320 -> 320 11.2
-// / 9.8, 50176 x 320 -> 640 47.9 / 48.8, 8192 x 640 -> 640 14.9 / 17.4.  Several in a launch, an added tensor or a second product pay up to
-// 4e9 where both sides are 512 and more: three of 8192 x 640 -> 640 42.6 / 37.1, of 50176 x 256 -> 512 109 / 87; one of 4096 x 1280 -> 1280
-// 21.5 / 26.1.
+// with bias, captured graph).  A forward product by itself (`alone`) of whole 256-wide tiles, contractions of 128 and more, over 1.5e9
+// multiply-adds and up to 2^24 results is the library's: 50176 x 128 -> 256 13.4 / 16.7, 12544 x 256 -> 512 11.7 / 13.6, 25088 x 256 ->
+// 256 11.6 / 13.7, 50176 x 256 -> 256 16.4 / 20.9, x 512 -> 256 22.0 / 30.4, 12544 x 512 -> 512 15.7 / 18.7.  More results: 50176 x 256 ->
+// 512 38.3 / 37.1, x 512 -> 512 62.0 / 58.9; fewer products: 8192 x 256 -> 512 8.3 / 8.8, 12544 x 256 -> 256 8.2 / 8.4, 4096 x 512 -> 512
+// 9.4 / 8.1; other widths: 12544 x 320 -> 320 11.2 / 9.8, 50176 x 320 -> 640 47.9 / 48.8, 8192 x 640 -> 640 14.9 / 17.4.  Several in a launch,
+// an added tensor or a second product pay up to 4e9 where both sides are 512 and more: three of 8192 x 640 -> 640 42.6 / 37.1, of 50176
+// x 256 -> 512 109 / 87; one of 4096 x 1280 -> 1280 21.5 / 26.1.
 bool projects(const Tensor& x, const Tensor& w, bool alone = false) {
   constexpr int64_t kMostChannels = 1 << 16, kMostWeights = 1 << 29, kLongestRow = 1 << 22;  // of fbla_project
   if (x.element_size() != 2 || w.size(0) > kMostChannels || w.size(1) > kMostChannels || w.numel() > kMostWeights ||
@@ -717,7 +717,9 @@ struct NoGraph {  // (called inside an autograd function or without gradients: n
 // The attention between the projections' rows and the block's, where the kernels of fbla_rows.hip take it: 16-bit types, heads of
 // 32 channels.  `rows` are the projections with queries (and keys) first in a row.
 constexpr int kPolarity = 0, kRotary = 1;
-bool on_rows(const Tensor& x, int64_t heads) { return x.element_size() == 2 && x.size(2) == 32 * heads && x.size(0) <= 65535 && x.size(1) <= 1 << 24 && heads <= 2048; }
+bool on_rows(const Tensor& x, int64_t heads) {
+  return x.element_size() == 2 && x.size(2) == 32 * heads && x.size(0) <= 65535 && x.size(1) <= 1 << 24 && heads <= 2048;
+}
 struct RowState {
   Tensor planes, km;
 };
@@ -917,7 +919,8 @@ std::vector<Tensor> pola_bwd(const Tensor& g, const Tensor& x, const Tensor& src
     const On on(x);
     check(api.fbla_block_attn_backward_keys(&a, on.stream), "fbla_block_attn_backward_keys");
   } else {
-    const Tensor scale = at_(0), power = at_(2), q_same = at_(5), q_opp = at_(6), k = at_(7), v = at_(8), grid = at_(9), s = at_(13), km = at_(14), s2 = at_(15);
+    const Tensor scale = at_(0), power = at_(2), q_same = at_(5), q_opp = at_(6), k = at_(7), v = at_(8), grid = at_(9), s = at_(13),
+                 km = at_(14), s2 = at_(15);
     MergeGrads m = merge_bwd(dmerged, heads, true, at_(11), at_(12), at_(10), qg.narrow(2, C, C));
     release(spares(x), dmerged);
     if (need[9] || need[10]) std::tie(r[9], r[10]) = dwconv_grad(grid, m.local, p.conv_w, H, W, need[10]);
@@ -1076,7 +1079,8 @@ std::vector<Tensor> linfusion_bwd(const Tensor& g, const Tensor& x, const Tensor
   Tensor dx = need[0] ? input_grad(d[2], p.w[2]) : Tensor();
   for (int i = 0; i < 2; ++i) {
     const auto& path = p.path[i];
-    const Tensor hidden = whole(at_(5 * i)), mean = whole(at_(5 * i + 1)), rstd = whole(at_(5 * i + 2)), normed = at_(5 * i + 3), in = at_(5 * i + 4);
+    const Tensor hidden = whole(at_(5 * i)), mean = whole(at_(5 * i + 1)), rstd = whole(at_(5 * i + 2)), normed = at_(5 * i + 3),
+                 in = at_(5 * i + 4);
     const int at0 = 1 + 6 * i;
     std::tie(r[13 + 2 * i], r[14 + 2 * i]) = weight_grad(d[i], in, need[13 + 2 * i], need[14 + 2 * i], kernel[4 + i]);
     const Tensor din = input_grad(d[i], p.w[i]);  // of x + residual
